@@ -5,16 +5,16 @@
 // (shaders/slang/raypipeline.slang:182); both are opaque. This file is the MI355X replacement.
 //
 // Build (all on the GPU, one stream):
-//   k_gather    indexed mesh -> per-triangle (v0, e1, e2), exact AABB, centroid-bounds atomics
+//   k_bounds    bounds of the triangles' AABB centers, index check
 //   k_morton    30-bit Morton code of the AABB center in the centroid bounds
 //   radix sort  (code, triangle) pairs, project-written (radix_sort.hip)
 //   k_karras    binary radix tree over the sorted codes (Karras 2012), ties broken by position; or, with
 //               VKRT_BUILDER_PLOC, agglomerative clustering over the sorted leaves (k_ploc_*)
-//   k_box_*     node boxes as unions over each node's leaf run (segment prefix/suffix unions and a sparse
-//               table of segment unions)
-//   k_layout    BVH2 nodes holding both children's boxes (64 B), subtrees of <= max_leaf_size
-//               triangles collapsed into leaves over the contiguous sorted range
-//   k_reorder   triangles in leaf order as 48-B records (v0, e1, e2, original index)
+//   k_leaves    triangles in leaf order, straight from the mesh: exact AABBs and 48-B records (v0, e1, e2,
+//               original index)
+//   k_box_*     unions of leaf boxes (segment prefix/suffix unions and a sparse table of segment unions)
+//   k_layout    BVH2 nodes holding both children's boxes (64 B), each the union over its leaf run; subtrees of
+//               <= max_leaf_size triangles collapsed into leaves over the contiguous sorted range
 //
 // Traversal: one ray per lane, front-to-back descent with a per-lane stack. Box tests are padded so
 // that a box is never culled when it holds a triangle the reference test accepts (see slab_interval),
@@ -46,70 +46,90 @@ __device__ __forceinline__ bool finite3(const vec3 &v)
     return __builtin_isfinite(v.x) && __builtin_isfinite(v.y) && __builtin_isfinite(v.z);
 }
 
-__device__ __forceinline__ void atomic_min_f(uint32_t *p, float v) { atomicMin(p, ordered_bits(v + 0.0f)); }
-__device__ __forceinline__ void atomic_max_f(uint32_t *p, float v) { atomicMax(p, ordered_bits(v + 0.0f)); }
-
-__device__ __forceinline__ float from_ordered(uint32_t b)
-{
-    uint32_t r = (b & 0x80000000u) ? (b & 0x7fffffffu) : ~b;
-    return __uint_as_float(r);
-}
-
 // ---------------------------------------------------------------------------------------------
 // build kernels
 // ---------------------------------------------------------------------------------------------
-__global__ void k_gather(const uint8_t *__restrict__ pos, uint32_t stride, const uint32_t *__restrict__ idx,
-                         uint32_t n_tri, uint32_t n_vert, float *__restrict__ pre, float *__restrict__ box,
-                         uint32_t *__restrict__ cbounds, uint32_t *__restrict__ err)
+//! an indexed mesh as the build reads it: vertex i's position at pos + i * stride
+struct mesh_view
 {
-    const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-    // the centroid bounds are reduced across the wave first and reach memory as one atomic per bound and wave
-    // (one per triangle serialized 1.8 M triangles' updates on six words: about 1.9 ms); lanes past the end
-    // stay in the wave for the reduction
-    float cmin[3] = {INFINITY, INFINITY, INFINITY}, cmax[3] = {-INFINITY, -INFINITY, -INFINITY};
-    if(j < n_tri)
+    const uint8_t *pos;
+    const uint32_t *idx;
+    uint32_t stride, n_tri, n_vert;
+};
+
+//! triangle j's vertices; an index past the vertices reads vertex 0 (and `ok` turns false: the build then fails)
+__device__ __forceinline__ void load_triangle(const mesh_view &m, uint32_t j, vec3 &v0, vec3 &v1, vec3 &v2, bool &ok)
+{
+    uint32_t i0 = m.idx[3 * (size_t)j], i1 = m.idx[3 * (size_t)j + 1], i2 = m.idx[3 * (size_t)j + 2];
+    ok = i0 < m.n_vert && i1 < m.n_vert && i2 < m.n_vert;
+    if(!ok) i0 = i1 = i2 = 0;
+    v0 = ld3(reinterpret_cast<const float *>(m.pos + (size_t)i0 * m.stride));
+    v1 = ld3(reinterpret_cast<const float *>(m.pos + (size_t)i1 * m.stride));
+    v2 = ld3(reinterpret_cast<const float *>(m.pos + (size_t)i2 * m.stride));
+}
+
+//! a triangle's exact box, lo xyz then hi xyz. A triangle with a non-finite vertex never yields a finite t (the
+//! reference test then produces NaN), so it gets an empty box and is never visited (returns false)
+__device__ __forceinline__ bool triangle_box(const vec3 &v0, const vec3 &v1, const vec3 &v2, float b[6])
+{
+    if(!(finite3(v0) && finite3(v1) && finite3(v2)))
     {
-        uint32_t i0 = idx[3 * (size_t)j], i1 = idx[3 * (size_t)j + 1], i2 = idx[3 * (size_t)j + 2];
-        if(i0 >= n_vert || i1 >= n_vert || i2 >= n_vert)
-        {
-            atomicOr(err, 1u);
-            i0 = i1 = i2 = 0;
-        }
-        vec3 v0 = ld3(reinterpret_cast<const float *>(pos + (size_t)i0 * stride));
-        vec3 v1 = ld3(reinterpret_cast<const float *>(pos + (size_t)i1 * stride));
-        vec3 v2 = ld3(reinterpret_cast<const float *>(pos + (size_t)i2 * stride));
-        vec3 e1 = v1 - v0, e2 = v2 - v0;
-        float *p = pre + 9 * (size_t)j;
-        p[0] = v0.x, p[1] = v0.y, p[2] = v0.z, p[3] = e1.x, p[4] = e1.y, p[5] = e1.z, p[6] = e2.x, p[7] = e2.y,
-        p[8] = e2.z;
-        float *b = box + 6 * (size_t)j;
-        if(finite3(v0) && finite3(v1) && finite3(v2))
-        {
-            vec3 lo{fminf(fminf(v0.x, v1.x), v2.x), fminf(fminf(v0.y, v1.y), v2.y), fminf(fminf(v0.z, v1.z), v2.z)};
-            vec3 hi{fmaxf(fmaxf(v0.x, v1.x), v2.x), fmaxf(fmaxf(v0.y, v1.y), v2.y), fmaxf(fmaxf(v0.z, v1.z), v2.z)};
-            b[0] = lo.x, b[1] = lo.y, b[2] = lo.z, b[3] = hi.x, b[4] = hi.y, b[5] = hi.z;
-            cmin[0] = cmax[0] = 0.5f * lo.x + 0.5f * hi.x;
-            cmin[1] = cmax[1] = 0.5f * lo.y + 0.5f * hi.y;
-            cmin[2] = cmax[2] = 0.5f * lo.z + 0.5f * hi.z;
-        }
-        else
-        {
-            // a triangle with a non-finite vertex never yields a finite t (the reference test then produces
-            // NaN), so it gets an empty box and is never visited
-            b[0] = b[1] = b[2] = FLT_MAX;
-            b[3] = b[4] = b[5] = -FLT_MAX;
-        }
+        b[0] = b[1] = b[2] = FLT_MAX;
+        b[3] = b[4] = b[5] = -FLT_MAX;
+        return false;
     }
-    for(int off = 32; off > 0; off >>= 1)
+    b[0] = fminf(fminf(v0.x, v1.x), v2.x), b[1] = fminf(fminf(v0.y, v1.y), v2.y), b[2] = fminf(fminf(v0.z, v1.z), v2.z);
+    b[3] = fmaxf(fmaxf(v0.x, v1.x), v2.x), b[4] = fmaxf(fmaxf(v0.y, v1.y), v2.y), b[5] = fmaxf(fmaxf(v0.z, v1.z), v2.z);
+    return true;
+}
+
+//! the bounds of the triangles' box centers, as one partial result per workgroup (k_morton combines them). No
+//! atomics: 1.8M triangles' wave minima meeting on six words of one line took 1.92 ms of the 13.4 ms build (an
+//! update of a line that every XCD writes costs 11 ns, one after the other). Two workgroups per CU keep the
+//! partials few enough for every k_morton workgroup to read them all.
+constexpr uint32_t BOUNDS_BLOCK = 512, BOUNDS_PARTIALS = 512;
+__global__ void __launch_bounds__(BOUNDS_BLOCK) k_bounds(mesh_view m, float *__restrict__ partial,
+                                                         uint32_t *__restrict__ err)
+{
+    __shared__ float part[6][BOUNDS_BLOCK / 64];
+    float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+    bool all_ok = true;
+    for(uint32_t j = blockIdx.x * BOUNDS_BLOCK + threadIdx.x; j < m.n_tri; j += gridDim.x * BOUNDS_BLOCK)
+    {
+        vec3 v0, v1, v2;
+        bool ok;
+        float b[6];
+        load_triangle(m, j, v0, v1, v2, ok);
+        all_ok = all_ok && ok;
+        if(!triangle_box(v0, v1, v2, b)) continue;
         for(int k = 0; k < 3; ++k)
         {
-            cmin[k] = fminf(cmin[k], __shfl_xor(cmin[k], off));
-            cmax[k] = fmaxf(cmax[k], __shfl_xor(cmax[k], off));
+            const float c = 0.5f * b[k] + 0.5f * b[3 + k];
+            lo[k] = fminf(lo[k], c);
+            hi[k] = fmaxf(hi[k], c);
         }
-    if((threadIdx.x & 63u) == 0 && cmin[0] <= cmax[0])
+    }
+    if(!all_ok) atomicOr(err, 1u);
+    for(int k = 0; k < 3; ++k)
     {
-        atomic_min_f(&cbounds[0], cmin[0]), atomic_min_f(&cbounds[1], cmin[1]), atomic_min_f(&cbounds[2], cmin[2]);
-        atomic_max_f(&cbounds[3], cmax[0]), atomic_max_f(&cbounds[4], cmax[1]), atomic_max_f(&cbounds[5], cmax[2]);
+        for(int off = 32; off > 0; off >>= 1)
+        {
+            lo[k] = fminf(lo[k], __shfl_xor(lo[k], off));
+            hi[k] = fmaxf(hi[k], __shfl_xor(hi[k], off));
+        }
+        if((threadIdx.x & 63u) == 0)
+        {
+            part[k][threadIdx.x >> 6] = lo[k];
+            part[3 + k][threadIdx.x >> 6] = hi[k];
+        }
+    }
+    __syncthreads();
+    if(threadIdx.x < 6)
+    {
+        float x = part[threadIdx.x][0];
+        for(uint32_t w = 1; w < BOUNDS_BLOCK / 64; ++w)
+            x = threadIdx.x < 3 ? fminf(x, part[threadIdx.x][w]) : fmaxf(x, part[threadIdx.x][w]);
+        partial[6 * blockIdx.x + threadIdx.x] = x;
     }
 }
 
@@ -123,19 +143,39 @@ __device__ __forceinline__ uint32_t spread10(uint32_t x)
     return x;
 }
 
-__global__ void k_morton(const float *__restrict__ box, uint32_t n, const uint32_t *__restrict__ cbounds,
-                         uint32_t *__restrict__ keys, uint32_t *__restrict__ vals)
+//! 30-bit Morton code of each triangle's box center in the bounds that the n_partial partial results give. The
+//! boxes are computed again from the mesh, which costs less than writing and reading them back would.
+__global__ void __launch_bounds__(256) k_morton(mesh_view m, const float *__restrict__ partial, uint32_t n_partial,
+                                                uint32_t *__restrict__ keys, uint32_t *__restrict__ vals)
 {
-    uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-    if(j >= n) return;
-    const float *b = box + 6 * (size_t)j;
+    __shared__ float part[6][4];
+    float cb[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    for(uint32_t p = threadIdx.x; p < n_partial; p += 256)
+        for(int a = 0; a < 6; ++a) cb[a] = a < 3 ? fminf(cb[a], partial[6 * p + a]) : fmaxf(cb[a], partial[6 * p + a]);
+    for(int a = 0; a < 6; ++a)
+    {
+        for(int off = 32; off > 0; off >>= 1)
+        {
+            const float o = __shfl_xor(cb[a], off);
+            cb[a] = a < 3 ? fminf(cb[a], o) : fmaxf(cb[a], o);
+        }
+        if((threadIdx.x & 63u) == 0) part[a][threadIdx.x >> 6] = cb[a];
+    }
+    __syncthreads();
+    const uint32_t j = blockIdx.x * 256 + threadIdx.x;
+    if(j >= m.n_tri) return;
+    vec3 v0, v1, v2;
+    bool ok;
+    float b[6];
+    load_triangle(m, j, v0, v1, v2, ok);
     uint32_t code = 0;
-    if(b[0] <= b[3])
+    if(triangle_box(v0, v1, v2, b))
     {
         uint32_t q[3];
         for(int a = 0; a < 3; ++a)
         {
-            float lo = from_ordered(cbounds[a]), hi = from_ordered(cbounds[3 + a]);
+            const float lo = fminf(fminf(part[a][0], part[a][1]), fminf(part[a][2], part[a][3]));
+            const float hi = fmaxf(fmaxf(part[3 + a][0], part[3 + a][1]), fmaxf(part[3 + a][2], part[3 + a][3]));
             float c = 0.5f * b[a] + 0.5f * b[3 + a];
             float ext = hi - lo;
             float f = ext > 0.f ? (c - lo) / ext : 0.5f;
@@ -191,19 +231,45 @@ __global__ void k_karras(const uint32_t *__restrict__ keys, int n, int2 *__restr
     if(i == 0) parent_int[0] = -1;
 }
 
-__global__ void k_sorted_boxes(const uint32_t *__restrict__ order, uint32_t n, const float *__restrict__ box,
-                               float *__restrict__ tbox)
-{
-    uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-    if(j >= n) return;
-    const float *s = box + 6 * (size_t)order[j];
-    float *d = tbox + 6 * (size_t)j;
-    for(int a = 0; a < 6; ++a) d[a] = s[a];
-}
-
+//! (box arrays are 8-byte aligned: three 8-byte accesses per box)
 __device__ __forceinline__ void load_box(const float *p, float b[6])
 {
-    for(int a = 0; a < 6; ++a) b[a] = p[a];
+    const float2 *q = reinterpret_cast<const float2 *>(p);
+    for(int a = 0; a < 3; ++a)
+    {
+        const float2 v = q[a];
+        b[2 * a] = v.x, b[2 * a + 1] = v.y;
+    }
+}
+
+__device__ __forceinline__ void store_box(float *p, const float b[6])
+{
+    float2 *q = reinterpret_cast<float2 *>(p);
+    for(int a = 0; a < 3; ++a) q[a] = make_float2(b[2 * a], b[2 * a + 1]);
+}
+
+//! the triangles in leaf order, straight from the mesh: their boxes, and with RECORDS the 48-B leaf records
+//! (v0, e1, e2, original index; the last two words are cleared)
+template<bool RECORDS>
+__global__ void __launch_bounds__(256) k_leaves(mesh_view m, const uint32_t *__restrict__ order,
+                                                float *__restrict__ tbox, float4 *__restrict__ tris)
+{
+    const uint32_t j = blockIdx.x * 256 + threadIdx.x;
+    if(j >= m.n_tri) return;
+    const uint32_t src = order[j];
+    vec3 v0, v1, v2;
+    bool ok;
+    float b[6];
+    load_triangle(m, src, v0, v1, v2, ok);
+    triangle_box(v0, v1, v2, b);
+    store_box(tbox + 6 * (size_t)j, b);
+    if constexpr(RECORDS)
+    {
+        const vec3 e1 = v1 - v0, e2 = v2 - v0;
+        tris[3 * (size_t)j + 0] = make_float4(v0.x, v0.y, v0.z, e1.x);
+        tris[3 * (size_t)j + 1] = make_float4(e1.y, e1.z, e2.x, e2.y);
+        tris[3 * (size_t)j + 2] = make_float4(e2.z, __uint_as_float(src), 0.f, 0.f);
+    }
 }
 
 //! Node boxes without a bottom-up hand-off. Every internal node covers a contiguous run [first, last] of the
@@ -261,14 +327,11 @@ __global__ void __launch_bounds__(BOX_SEG) k_box_scan(uint32_t n, const float *_
     }
     if(t < cnt)
     {
-        for(int k = 0; k < 6; ++k)
-        {
-            pre[6 * (size_t)j + k] = a[k];
-            suf[6 * (size_t)j + k] = b[k];
-        }
+        store_box(pre + 6 * (size_t)j, a);
+        store_box(suf + 6 * (size_t)j, b);
     }
     if(t == 0)
-        for(int k = 0; k < 6; ++k) seg[6 * (size_t)blockIdx.x + k] = b[k];// leaf 0's suffix: the segment
+        store_box(seg + 6 * (size_t)blockIdx.x, b);// leaf 0's suffix: the segment
 }
 
 //! sparse-table level k from level k - 1: entry i = union of entries i and i + 2^(k-1), for i + 2^k <= nseg
@@ -283,49 +346,51 @@ __global__ void k_box_sparse(uint32_t nseg, uint32_t k, float *__restrict__ tabl
     load_box(lo, a);
     load_box(hi, b);
     box_union(a, b);
-    for(int c = 0; c < 6; ++c) table[6 * ((size_t)k * nseg + i) + c] = a[c];
+    store_box(table + 6 * ((size_t)k * nseg + i), a);
 }
 
-__global__ void k_box_nodes(uint32_t ni, uint32_t n, uint32_t nseg, const uint2 *__restrict__ range,
-                            const float *__restrict__ tbox, const float *__restrict__ pre,
-                            const float *__restrict__ suf, const float *__restrict__ table, float *__restrict__ nbox)
+//! the leaves' boxes and their unions, as k_layout reads them
+struct leaf_unions
 {
-    const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-    if(p >= ni) return;
-    const uint2 r = range[p];
-    const uint32_t first = r.x, last = r.y, sf = first / BOX_SEG, sl = last / BOX_SEG;
-    float o[6], x[6];
+    const float *tbox, *pre, *suf, *table;
+    uint32_t n, nseg;
+};
+
+//! the union of leaf boxes first .. last
+__device__ __forceinline__ void run_box(const leaf_unions &l, uint32_t first, uint32_t last, float o[6])
+{
+    const uint32_t sf = first / BOX_SEG, sl = last / BOX_SEG;
+    float x[6];
     if(sf == sl)
     {
-        const bool at_end = last % BOX_SEG == BOX_SEG - 1 || last == n - 1;
-        if(first % BOX_SEG == 0) load_box(pre + 6 * (size_t)last, o);
-        else if(at_end) load_box(suf + 6 * (size_t)first, o);
+        const bool at_end = last % BOX_SEG == BOX_SEG - 1 || last == l.n - 1;
+        if(first % BOX_SEG == 0) load_box(l.pre + 6 * (size_t)last, o);
+        else if(at_end) load_box(l.suf + 6 * (size_t)first, o);
         else
         {
-            load_box(tbox + 6 * (size_t)first, o);
+            load_box(l.tbox + 6 * (size_t)first, o);
             for(uint32_t j = first + 1; j <= last; ++j)
             {
-                load_box(tbox + 6 * (size_t)j, x);
+                load_box(l.tbox + 6 * (size_t)j, x);
                 box_union(o, x);
             }
         }
     }
     else
     {
-        load_box(suf + 6 * (size_t)first, o);
-        load_box(pre + 6 * (size_t)last, x);
+        load_box(l.suf + 6 * (size_t)first, o);
+        load_box(l.pre + 6 * (size_t)last, x);
         box_union(o, x);
         if(sl > sf + 1)
         {
             const uint32_t lo = sf + 1, count = sl - 1 - lo + 1;
             const uint32_t k = 31u - __builtin_clz(count);
-            load_box(table + 6 * ((size_t)k * nseg + lo), x);
+            load_box(l.table + 6 * ((size_t)k * l.nseg + lo), x);
             box_union(o, x);
-            load_box(table + 6 * ((size_t)k * nseg + (sl - 1) - (1u << k) + 1), x);
+            load_box(l.table + 6 * ((size_t)k * l.nseg + (sl - 1) - (1u << k) + 1), x);
             box_union(o, x);
         }
     }
-    for(int c = 0; c < 6; ++c) nbox[6 * (size_t)p + c] = o[c];
 }
 
 //! the sparse table's depth for nseg segments: levels 0 .. floor(log2(nseg))
@@ -339,35 +404,36 @@ static uint32_t box_levels(uint32_t nseg)
 __device__ __forceinline__ float pad_lo(float x) { return x - fabsf(x) * BOX_PAD; }
 __device__ __forceinline__ float pad_hi(float x) { return x + fabsf(x) * BOX_PAD; }
 
-__global__ void k_layout(uint32_t n, const int2 *__restrict__ child, const uint2 *__restrict__ range,
-                         const float *__restrict__ nbox, const float *__restrict__ tbox, uint32_t max_leaf,
-                         vkrt_bvh_node *__restrict__ nodes)
+//! BVH2 node i from its children's leaf runs: child k's box is the union over its run (each node is one node's
+//! child, so no node's box is computed twice, and none is stored on its own)
+__global__ void __launch_bounds__(256) k_layout(leaf_unions l, const int2 *__restrict__ child,
+                                                const uint2 *__restrict__ range, uint32_t max_leaf,
+                                                vkrt_bvh_node *__restrict__ nodes)
 {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if(i + 1 >= n) return;
-    int2 c = child[i];
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if(i + 1 >= l.n) return;
+    const int2 c = child[i];
     float bx[2][6];
     int ref[2];
     const int cr[2] = {c.x, c.y};
     for(int k = 0; k < 2; ++k)
     {
         uint32_t first, last;
-        const float *src;
         if(cr[k] < 0)
         {
             first = last = ~cr[k];
-            src = tbox + 6 * (size_t)first;
+            load_box(l.tbox + 6 * (size_t)first, bx[k]);
         }
         else
         {
-            uint2 r = range[cr[k]];
-            first = r.x, last = r.y;
-            src = nbox + 6 * (size_t)cr[k];
+            const uint2 cr_range = range[cr[k]];
+            first = cr_range.x, last = cr_range.y;
+            run_box(l, first, last, bx[k]);
         }
-        uint32_t count = last - first + 1;
+        const uint32_t count = last - first + 1;
         ref[k] = (cr[k] < 0 || count <= max_leaf) ? ~static_cast<int>((first << 3) | (count - 1)) : cr[k];
-        for(int a = 0; a < 3; ++a) bx[k][a] = pad_lo(src[a]);
-        for(int a = 3; a < 6; ++a) bx[k][a] = pad_hi(src[a]);
+        for(int a = 0; a < 3; ++a) bx[k][a] = pad_lo(bx[k][a]);
+        for(int a = 3; a < 6; ++a) bx[k][a] = pad_hi(bx[k][a]);
     }
     vkrt_bvh_node nd;
     nd.a = make_float4(bx[0][0], bx[0][3], bx[0][1], bx[0][4]);
@@ -375,18 +441,6 @@ __global__ void k_layout(uint32_t n, const int2 *__restrict__ child, const uint2
     nd.c = make_float4(bx[0][2], bx[0][5], bx[1][2], bx[1][5]);
     nd.d = make_int4(ref[0], ref[1], 0, 0);
     nodes[i] = nd;
-}
-
-__global__ void k_reorder(const uint32_t *__restrict__ order, uint32_t n, const float *__restrict__ pre,
-                          float4 *__restrict__ tris)
-{
-    uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-    if(j >= n) return;
-    uint32_t src = order[j];
-    const float *p = pre + 9 * (size_t)src;
-    tris[3 * (size_t)j + 0] = make_float4(p[0], p[1], p[2], p[3]);
-    tris[3 * (size_t)j + 1] = make_float4(p[4], p[5], p[6], p[7]);
-    tris[3 * (size_t)j + 2] = make_float4(p[8], __uint_as_float(src), 0.f, 0.f);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -524,33 +578,27 @@ static void compute_stats(vkrt_bvh *bvh, hipStream_t s)
 
 static void build_topology_ploc(vkrt_ctx *ctx, vkrt_bvh *bvh);
 
-static void build_topology(vkrt_ctx *ctx, vkrt_bvh *bvh, const uint8_t *pos, uint32_t stride, const uint32_t *idx)
+static void build_topology(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh)
 {
     hipStream_t s = ctx->stream;
     const uint32_t n = bvh->n_tri;
-    bvh->pre.reserve((size_t)n * 9 * sizeof(float));
     bvh->tbox.reserve((size_t)n * 6 * sizeof(float));
     bvh->err.reserve(64);
-    // scratch: per-triangle boxes in input order + centroid bounds + sort keys/values + sort temp
+    // scratch: centroid bounds, sort keys, sort temp
     device_buffer &tmp = ctx->scratch[2];
-    const size_t box_bytes = (size_t)n * 6 * sizeof(float);
-    const size_t key_bytes = (size_t)n * sizeof(uint32_t);
-    tmp.reserve(box_bytes + 64 + key_bytes + radix_sort_temp_bytes(n));
-    float *box = tmp.as<float>();
-    uint32_t *cb = reinterpret_cast<uint32_t *>(tmp.as<uint8_t>() + box_bytes);
-    uint32_t *keys = reinterpret_cast<uint32_t *>(tmp.as<uint8_t>() + box_bytes + 64);
-    void *sort_tmp = tmp.as<uint8_t>() + box_bytes + 64 + key_bytes;
+    const size_t key_bytes = (size_t)n * sizeof(uint32_t), partial_bytes = BOUNDS_PARTIALS * 6 * sizeof(float);
+    tmp.reserve(partial_bytes + key_bytes + radix_sort_temp_bytes(n));
+    float *partial = tmp.as<float>();
+    uint32_t *keys = reinterpret_cast<uint32_t *>(tmp.as<uint8_t>() + partial_bytes);
+    void *sort_tmp = tmp.as<uint8_t>() + partial_bytes + key_bytes;
     bvh->order.reserve(key_bytes);
     uint32_t *order = bvh->order.as<uint32_t>();
 
-    uint32_t init[8] = {0xffffffffu, 0xffffffffu, 0xffffffffu, 0u, 0u, 0u, 0u, 0u};
-    VKRT_HIP(hipMemcpyAsync(cb, init, sizeof(init), hipMemcpyHostToDevice, s));
     VKRT_HIP(hipMemsetAsync(bvh->err.ptr, 0, 4, s));
-    k_gather<<<div_up(n, 256), 256, 0, s>>>(pos, stride, idx, n, bvh->n_vert, bvh->pre.as<float>(), box, cb,
-                                            bvh->err.as<uint32_t>());
-    k_morton<<<div_up(n, 256), 256, 0, s>>>(box, n, cb, keys, order);
+    const uint32_t n_partial = std::min(BOUNDS_PARTIALS, div_up(n, BOUNDS_BLOCK));
+    k_bounds<<<n_partial, BOUNDS_BLOCK, 0, s>>>(mesh, partial, bvh->err.as<uint32_t>());
+    k_morton<<<div_up(n, 256), 256, 0, s>>>(mesh, partial, n_partial, keys, order);
     radix_sort_pairs(s, keys, order, n, 30, sort_tmp);
-    k_sorted_boxes<<<div_up(n, 256), 256, 0, s>>>(order, n, box, bvh->tbox.as<float>());
     uint32_t err_host = 0;
     VKRT_HIP(hipMemcpyAsync(&err_host, bvh->err.ptr, 4, hipMemcpyDeviceToHost, s));
     if(n >= 2)
@@ -559,9 +607,12 @@ static void build_topology(vkrt_ctx *ctx, vkrt_bvh *bvh, const uint8_t *pos, uin
         bvh->child.reserve(ni * sizeof(int2));
         bvh->range.reserve(ni * sizeof(uint2));
         bvh->parent.reserve(((size_t)ni + n) * sizeof(int32_t));
-        bvh->nbox.reserve((size_t)ni * 6 * sizeof(float));
         int32_t *parent_int = bvh->parent.as<int32_t>(), *parent_leaf = parent_int + ni;
-        if(bvh->builder == VKRT_BUILDER_PLOC) build_topology_ploc(ctx, bvh);
+        if(bvh->builder == VKRT_BUILDER_PLOC)
+        {
+            k_leaves<false><<<div_up(n, 256), 256, 0, s>>>(mesh, order, bvh->tbox.as<float>(), nullptr);
+            build_topology_ploc(ctx, bvh);
+        }
         else
             k_karras<<<div_up(ni, 256), 256, 0, s>>>(keys, (int)n, bvh->child.as<int2>(), bvh->range.as<uint2>(),
                                                      parent_int, parent_leaf);
@@ -746,11 +797,9 @@ __global__ void k_ploc_dfs(uint32_t ni, uint32_t n, const int2 *__restrict__ chi
     }
 }
 
-//! leaves to depth-first order: the triangle order, sorted boxes, leaf parents and leaf child refs
+//! leaves to depth-first order: the triangle order and leaf child refs
 __global__ void k_ploc_permute(uint32_t ni, uint32_t n, const uint32_t *__restrict__ leaf_pos,
-                               const uint32_t *__restrict__ order_in, const float *__restrict__ tbox_in,
-                               const int32_t *__restrict__ parent_leaf_in, uint32_t *__restrict__ order_out,
-                               float *__restrict__ tbox_out, int32_t *__restrict__ parent_leaf_out,
+                               const uint32_t *__restrict__ order_in, uint32_t *__restrict__ order_out,
                                const int2 *__restrict__ child_in, int2 *__restrict__ child_out)
 {
     const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
@@ -759,8 +808,6 @@ __global__ void k_ploc_permute(uint32_t ni, uint32_t n, const uint32_t *__restri
         const uint32_t d = leaf_pos[k];
         if(d >= n) return;// only a malformed tree gets here; compute_stats rejects it
         order_out[d] = order_in[k];
-        for(int a = 0; a < 6; ++a) tbox_out[6 * (size_t)d + a] = tbox_in[6 * (size_t)k + a];
-        parent_leaf_out[d] = parent_leaf_in[k];
     }
     if(k < ni)
     {
@@ -918,8 +965,7 @@ static void build_topology_ploc(vkrt_ctx *ctx, vkrt_bvh *bvh)
     }
     VKRT_REQUIRE(base == ni, "PLOC did not build n - 1 nodes");
     // the cluster lists and flag arrays are free now: renumbered tree (root first), then depth-first leaf
-    // positions and ranges, then the permuted copies, which are copied back into the BVH's own arrays.
-    // lo[1] and hi[0] are adjacent (32 n bytes), enough for the 24 n bytes of permuted boxes
+    // positions and ranges, then the permuted copies
     int2 *child2 = reinterpret_cast<int2 *>(lo[0]);
     uint32_t *cnt2 = merge;
     int32_t *pint2 = reinterpret_cast<int32_t *>(moff);
@@ -927,24 +973,22 @@ static void build_topology_ploc(vkrt_ctx *ctx, vkrt_bvh *bvh)
     k_ploc_renumber<<<div_up(n, 256), 256, 0, s>>>(ni, n, child, cnt, parent_int, parent_leaf, child2, cnt2, pint2,
                                                    pleaf2);
     k_ploc_dfs<<<div_up(n, 256), 256, 0, s>>>(ni, n, child2, cnt2, pint2, pleaf2, leaf_pos, bvh->range.as<uint2>());
-    uint32_t *order_out = koff;
-    float *tbox_out = reinterpret_cast<float *>(lo[1]);
-    int32_t *pleaf_out = id[0];
-    int2 *child_out = reinterpret_cast<int2 *>(hi[1]);
-    k_ploc_permute<<<div_up(n, 256), 256, 0, s>>>(ni, n, leaf_pos, bvh->order.as<uint32_t>(), bvh->tbox.as<float>(),
-                                                  pleaf2, order_out, tbox_out, pleaf_out, child2, child_out);
-    VKRT_HIP(hipMemcpyAsync(bvh->order.ptr, order_out, (size_t)n * 4, hipMemcpyDeviceToDevice, s));
-    VKRT_HIP(hipMemcpyAsync(bvh->tbox.ptr, tbox_out, (size_t)n * 24, hipMemcpyDeviceToDevice, s));
-    VKRT_HIP(hipMemcpyAsync(parent_leaf, pleaf_out, (size_t)n * 4, hipMemcpyDeviceToDevice, s));
+    uint32_t *order_in = koff;
+    VKRT_HIP(hipMemcpyAsync(order_in, bvh->order.ptr, (size_t)n * 4, hipMemcpyDeviceToDevice, s));
+    k_ploc_permute<<<div_up(n, 256), 256, 0, s>>>(ni, n, leaf_pos, order_in, bvh->order.as<uint32_t>(), child2, child);
     VKRT_HIP(hipMemcpyAsync(parent_int, pint2, (size_t)ni * 4, hipMemcpyDeviceToDevice, s));
-    VKRT_HIP(hipMemcpyAsync(child, child_out, (size_t)ni * 8, hipMemcpyDeviceToDevice, s));
     VKRT_HIP(hipGetLastError());
 }
 
-static void build_bounds(vkrt_ctx *ctx, vkrt_bvh *bvh)
+//! the leaf records, the BVH2's nodes and the root, from the mesh and a topology: the last part of a build and the
+//! whole of a refit, which keeps the topology
+static void build_bounds(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh)
 {
     hipStream_t s = ctx->stream;
     const uint32_t n = bvh->n_tri;
+    bvh->tris.reserve((size_t)n * 3 * sizeof(float4));
+    k_leaves<true><<<div_up(n, 256), 256, 0, s>>>(mesh, bvh->order.as<uint32_t>(), bvh->tbox.as<float>(),
+                                                  bvh->tris.as<float4>());
     if(n >= 2)
     {
         const uint32_t ni = n - 1;
@@ -956,12 +1000,10 @@ static void build_bounds(vkrt_ctx *ctx, vkrt_bvh *bvh)
         k_box_scan<<<nseg, BOX_SEG, 0, s>>>(n, bvh->tbox.as<float>(), pre, suf, table);
         for(uint32_t k = 1; k < levels; ++k)
             k_box_sparse<<<div_up(nseg, 256), 256, 0, s>>>(nseg, k, table);
-        k_box_nodes<<<div_up(ni, 256), 256, 0, s>>>(ni, n, nseg, bvh->range.as<uint2>(), bvh->tbox.as<float>(), pre,
-                                                     suf, table, bvh->nbox.as<float>());
         bvh->n_nodes = ni;
         bvh->nodes.reserve((size_t)ni * sizeof(vkrt_bvh_node));
-        k_layout<<<div_up(ni, 256), 256, 0, s>>>(n, bvh->child.as<int2>(), bvh->range.as<uint2>(),
-                                                 bvh->nbox.as<float>(), bvh->tbox.as<float>(), bvh->max_leaf,
+        const leaf_unions l{bvh->tbox.as<float>(), pre, suf, table, n, nseg};
+        k_layout<<<div_up(ni, 256), 256, 0, s>>>(l, bvh->child.as<int2>(), bvh->range.as<uint2>(), bvh->max_leaf,
                                                  bvh->nodes.as<vkrt_bvh_node>());
         bvh->root_ref = (n <= bvh->max_leaf) ? ~static_cast<int>(n - 1) : 0;
     }
@@ -970,9 +1012,6 @@ static void build_bounds(vkrt_ctx *ctx, vkrt_bvh *bvh)
         bvh->n_nodes = 0;
         bvh->root_ref = ~0;// a leaf holding the single triangle
     }
-    bvh->tris.reserve((size_t)n * 3 * sizeof(float4));
-    k_reorder<<<div_up(n, 256), 256, 0, s>>>(bvh->order.as<uint32_t>(), n, bvh->pre.as<float>(),
-                                             bvh->tris.as<float4>());
     VKRT_HIP(hipGetLastError());
 }
 
@@ -1230,8 +1269,9 @@ int vkrt_bvh_build(vkrt_ctx *ctx, const float *positions, uint32_t n_vert, uint3
             const uint32_t *didx = input(ctx, 1, indices, (size_t)n_tri * 3, flags);
             VKRT_HIP(hipMemcpyAsync(bvh->indices.ptr, didx, (size_t)n_tri * 3 * sizeof(uint32_t),
                                     hipMemcpyDeviceToDevice, ctx->stream));
-            build_topology(ctx, bvh.get(), dpos, stride_bytes, bvh->indices.as<uint32_t>());
-            build_bounds(ctx, bvh.get());
+            const mesh_view mesh{dpos, bvh->indices.as<uint32_t>(), stride_bytes, n_tri, n_vert};
+            build_topology(ctx, bvh.get(), mesh);
+            build_bounds(ctx, bvh.get(), mesh);
             build_wide(ctx, bvh.get());
             VKRT_HIP(hipStreamSynchronize(ctx->stream));
         }
@@ -1249,18 +1289,9 @@ int vkrt_bvh_refit(vkrt_ctx *ctx, vkrt_bvh *bvh, const float *positions, uint32_
         if(bvh->empty) return;
         VKRT_REQUIRE(positions, "null positions");
         hipStream_t s = ctx->stream;
-        const uint32_t n = bvh->n_tri;
         const size_t pos_bytes = (size_t)(bvh->n_vert - 1) * stride_bytes + 12;
         const uint8_t *dpos = input(ctx, 0, reinterpret_cast<const uint8_t *>(positions), pos_bytes, flags);
-        device_buffer &tmp = ctx->scratch[2];
-        tmp.reserve((size_t)n * 6 * sizeof(float) + 64);
-        float *box = tmp.as<float>();
-        uint32_t *cb = reinterpret_cast<uint32_t *>(tmp.as<uint8_t>() + (size_t)n * 6 * sizeof(float));
-        VKRT_HIP(hipMemsetAsync(bvh->err.ptr, 0, 4, s));
-        k_gather<<<div_up(n, 256), 256, 0, s>>>(dpos, stride_bytes, bvh->indices.as<uint32_t>(), n, bvh->n_vert,
-                                                bvh->pre.as<float>(), box, cb, bvh->err.as<uint32_t>());
-        k_sorted_boxes<<<div_up(n, 256), 256, 0, s>>>(bvh->order.as<uint32_t>(), n, box, bvh->tbox.as<float>());
-        build_bounds(ctx, bvh);
+        build_bounds(ctx, bvh, mesh_view{dpos, bvh->indices.as<uint32_t>(), stride_bytes, bvh->n_tri, bvh->n_vert});
         refit_wide(ctx, bvh);
         VKRT_HIP(hipStreamSynchronize(s));
         refresh_info(bvh, s, false);
