@@ -1,0 +1,39 @@
+"""BVH builds and refits at the sizes where the build's tiles, segments and workgroups end: every invariant of
+vkrt_bvh_validate, and hits equal to brute force, before and after the vertices move."""
+import numpy as np
+import pytest
+
+import vierkant_amd as vk
+from parity import assert_hits_equal
+from vierkant_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+# leaf-box segments of 64, workgroups of 256, 512 and 1024, radix tiles, and the bounds pass's 512 x 512 grid
+SIZES = [1, 2, 3, 8, 9, 63, 64, 65, 129, 255, 256, 257, 511, 513, 1023, 1024, 1025, 2047, 2049, 4097, 65537, 262145]
+
+
+@pytest.mark.parametrize("builder", [vk.BUILDER_LBVH, vk.BUILDER_PLOC])
+@pytest.mark.parametrize("n_tri", SIZES)
+def test_build_and_refit_at_tile_edges(ctx, builder, n_tri):
+    rng = np.random.default_rng(n_tri)
+    corner = rng.uniform(-1, 1, (n_tri, 1, 3))
+    size = 2.0 * n_tri ** (-1 / 3)
+    pos = (corner + rng.uniform(-size, size, (n_tri, 3, 3))).astype(np.float32).reshape(-1, 3)
+    idx = rng.permutation(n_tri * 3).astype(np.uint32)
+    pos = np.ascontiguousarray(pos[np.argsort(idx)])
+    o = rng.uniform(-2, 2, (1000, 3)).astype(np.float32)
+    rays = W.make_rays(o, W.glm_normalize(rng.normal(size=(1000, 3)).astype(np.float32)))
+    for leaf, width in ((0, 0), (8, 0), (1, 2)):
+        bvh = ctx.bvh_build(pos, idx, builder=builder, max_leaf_size=leaf, width=width)
+        info = bvh.info()
+        assert info.n_tri == n_tri and info.depth <= 64
+        moved = pos + np.float32(0.25) * np.sin(3.0 * pos[:, ::-1]).astype(np.float32)
+        for p in (pos, moved):
+            if p is moved:
+                bvh.refit(p)
+            check = bvh.validate(p)
+            assert check["ok"], check
+            assert_hits_equal(ctx.trace_closest(bvh, rays), ctx.brute_closest(W.flat_triangles(p, idx), rays),
+                              f"{n_tri} triangles, leaf {leaf}, width {width}")
+        bvh.close()

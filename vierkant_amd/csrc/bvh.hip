@@ -197,8 +197,7 @@ __device__ __forceinline__ int delta(const uint32_t *__restrict__ keys, int n, i
 }
 
 //! Karras 2012 binary radix tree. child refs: >= 0 internal node, < 0 leaf at sorted position ~ref.
-__global__ void k_karras(const uint32_t *__restrict__ keys, int n, int2 *__restrict__ child, uint2 *__restrict__ range,
-                         int32_t *__restrict__ parent_int, int32_t *__restrict__ parent_leaf)
+__global__ void k_karras(const uint32_t *__restrict__ keys, int n, int2 *__restrict__ child, uint2 *__restrict__ range)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if(i >= n - 1) return;
@@ -224,11 +223,6 @@ __global__ void k_karras(const uint32_t *__restrict__ keys, int n, int2 *__restr
     int right = (last == gamma + 1) ? ~(gamma + 1) : gamma + 1;
     child[i] = make_int2(left, right);
     range[i] = make_uint2(first, last);
-    if(left < 0) parent_leaf[~left] = i;
-    else parent_int[left] = i;
-    if(right < 0) parent_leaf[~right] = i;
-    else parent_int[right] = i;
-    if(i == 0) parent_int[0] = -1;
 }
 
 //! (box arrays are 8-byte aligned: three 8-byte accesses per box)
@@ -446,68 +440,51 @@ __global__ void __launch_bounds__(256) k_layout(leaf_unions l, const int2 *__res
 // ---------------------------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------------------------
-//! build statistics over the final BVH2 nodes. A node stays internal in the layout when its run holds more
-//! than max_leaf triangles (every ancestor's run then does too), so those nodes and the root are the ones a
-//! traversal reaches. Each counts its depth up the parent chain (the root is 1), and adds its children's SAH
-//! terms (box area; a leaf's times its triangle count, divided by the root's area on the host), its leaf
-//! children and their depth. Sums go through a wave reduction and one atomic per wave.
-struct bvh_stats_dev
+//! what a build's kernels count and its host side reads: one block in device memory, cleared at the start of a
+//! build and copied to the context's pinned host memory by k_report (a kernel's store and the synchronization
+//! take 10 us; a copy into pageable memory took 25 us besides). Counters that many workgroups update lie on
+//! lines of their own.
+constexpr uint32_t MAX_LEVELS = STACK_SIZE + 2;// of the 4-wide collapse: each goes at least one binary level down
+struct bvh_state
 {
-    double sah;
-    uint32_t leaves, depth;
+    uint32_t err;// an index past the vertices
+    uint32_t pad0[31];
+    double sah;  // sum of the children's SAH terms (divided by the root's area on the host)
+    uint32_t pad1[30];
+    uint32_t leaves;
+    uint32_t pad2[31];
+    uint32_t depth;// of the binary tree, its root counting 1
+    uint32_t pad3[31];
+    uint32_t stack;// worst-case traversal stack of the 4-wide tree
+    uint32_t pad4[31];
+    uint32_t level[MAX_LEVELS + 2];// 4-wide nodes per level
+    vkrt_bvh_node root;
 };
 
-__device__ __forceinline__ double child_area(float lx, float hx, float ly, float hy, float lz, float hz)
+__global__ void __launch_bounds__(256) k_state_clear(bvh_state *__restrict__ st)
 {
-    const double dx = fmax(0.0, (double)hx - lx), dy = fmax(0.0, (double)hy - ly), dz = fmax(0.0, (double)hz - lz);
-    return 2.0 * (dx * dy + dy * dz + dz * dx);
+    uint32_t *w = reinterpret_cast<uint32_t *>(st);
+    for(uint32_t i = threadIdx.x; i < sizeof(bvh_state) / 4; i += 256) w[i] = 0u;
 }
 
-__global__ void k_stats(uint32_t ni, uint32_t max_leaf, const vkrt_bvh_node *__restrict__ nodes,
-                        const uint2 *__restrict__ range, const int32_t *__restrict__ parent_int,
-                        bvh_stats_dev *__restrict__ out)
+__global__ void __launch_bounds__(256) k_report(const bvh_state *__restrict__ st, const vkrt_bvh_node *__restrict__ nodes,
+                                                bvh_state *__restrict__ host)
 {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    double sah = 0.0;
-    uint32_t leaves = 0, depth = 0;
-    if(i < ni)
-    {
-        const uint2 r = range[i];
-        if(i == 0 || r.y - r.x + 1 > max_leaf)
-        {
-            // (past STACK_SIZE + 1 the walk stops: the host rejects any depth above STACK_SIZE)
-            uint32_t d = 1;
-            for(int32_t p = static_cast<int32_t>(i); p > 0 && d <= STACK_SIZE + 1; ++d) p = parent_int[p];
-            const vkrt_bvh_node nd = nodes[i];
-            const int32_t refs[2] = {nd.d.x, nd.d.y};
-            const double ar[2] = {child_area(nd.a.x, nd.a.y, nd.a.z, nd.a.w, nd.c.x, nd.c.y),
-                                  child_area(nd.b.x, nd.b.y, nd.b.z, nd.b.w, nd.c.z, nd.c.w)};
-            depth = d;
-            for(int k = 0; k < 2; ++k)
-            {
-                if(refs[k] >= 0) sah += ar[k];
-                else
-                {
-                    const uint32_t v = static_cast<uint32_t>(~refs[k]);
-                    sah += ((v & 7u) + 1) * ar[k];
-                    ++leaves;
-                    depth = d + 1;
-                }
-            }
-        }
-    }
-    for(int off = 32; off > 0; off >>= 1)
-    {
-        sah += __shfl_xor(sah, off);
-        leaves += __shfl_xor(leaves, off);
-        depth = max(depth, (uint32_t)__shfl_xor(depth, off));
-    }
-    if((threadIdx.x & 63u) == 0 && (leaves || depth))
-    {
-        atomicAdd(&out->sah, sah);
-        atomicAdd(&out->leaves, leaves);
-        atomicMax(&out->depth, depth);
-    }
+    const uint32_t *src = reinterpret_cast<const uint32_t *>(st);
+    uint32_t *dst = reinterpret_cast<uint32_t *>(host);
+    for(uint32_t i = threadIdx.x; i < offsetof(bvh_state, root) / 4; i += 256) dst[i] = src[i];
+    if(nodes && threadIdx.x < sizeof(vkrt_bvh_node) / 4)
+        dst[offsetof(bvh_state, root) / 4 + threadIdx.x] = reinterpret_cast<const uint32_t *>(nodes)[threadIdx.x];
+}
+
+//! the state as the host reads it, once everything queued before has run; with nodes, the root node too
+static const bvh_state &read_state(vkrt_ctx *ctx, const vkrt_bvh_node *nodes)
+{
+    bvh_state *host = ctx->pinned_as<bvh_state>();
+    k_report<<<1, 256, 0, ctx->stream>>>(ctx->state.as<bvh_state>(), nodes, host);
+    VKRT_HIP(hipGetLastError());
+    VKRT_HIP(hipStreamSynchronize(ctx->stream));
+    return *host;
 }
 
 //! the root's box from its two child boxes: rb as (lo, hi) pairs per axis, bounds as lo xyz then hi xyz
@@ -523,57 +500,32 @@ static void root_bounds(const vkrt_bvh_node &root, float rb[6], float bounds[6])
     }
 }
 
-static void compute_stats(vkrt_bvh *bvh, hipStream_t s)
+//! a single leaf's bounds (at most 8 triangles): the union of its triangles' boxes (tbox, in leaf order), padded
+//! like every node box
+static void single_leaf_info(vkrt_bvh *bvh, hipStream_t s)
 {
-    // depth and SAH cost from the final nodes (build-time statistics only)
     vkrt_bvh_info &info = bvh->info;
     info.depth = 1;
     info.sah_cost = 0.f;
     info.n_leaves = bvh->empty ? 0 : 1;
     if(bvh->empty) return;
-    if(bvh->root_ref < 0)
-    {
-        // a single leaf (at most 8 triangles): the union of its triangles' boxes (tbox, in leaf order),
-        // padded like every node box
-        const uint32_t v = static_cast<uint32_t>(~bvh->root_ref), first = v >> 3, count = (v & 7u) + 1;
-        std::vector<float> box(6 * (size_t)count);
-        VKRT_HIP(hipMemcpyAsync(box.data(), bvh->tbox.as<float>() + 6 * (size_t)first, box.size() * 4,
-                                hipMemcpyDeviceToHost, s));
-        VKRT_HIP(hipStreamSynchronize(s));
-        float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-        for(uint32_t k = 0; k < count; ++k)
-            for(int a = 0; a < 3; ++a)
-            {
-                lo[a] = std::min(lo[a], box[6 * (size_t)k + a]);
-                hi[a] = std::max(hi[a], box[6 * (size_t)k + 3 + a]);
-            }
+    const uint32_t v = static_cast<uint32_t>(~bvh->root_ref), first = v >> 3, count = (v & 7u) + 1;
+    std::vector<float> box(6 * (size_t)count);
+    VKRT_HIP(hipMemcpyAsync(box.data(), bvh->tbox.as<float>() + 6 * (size_t)first, box.size() * 4,
+                            hipMemcpyDeviceToHost, s));
+    VKRT_HIP(hipStreamSynchronize(s));
+    float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+    for(uint32_t k = 0; k < count; ++k)
         for(int a = 0; a < 3; ++a)
         {
-            info.bounds[a] = lo[a] - std::fabs(lo[a]) * BOX_PAD;
-            info.bounds[3 + a] = hi[a] + std::fabs(hi[a]) * BOX_PAD;
+            lo[a] = std::min(lo[a], box[6 * (size_t)k + a]);
+            hi[a] = std::max(hi[a], box[6 * (size_t)k + 3 + a]);
         }
-        return;
+    for(int a = 0; a < 3; ++a)
+    {
+        info.bounds[a] = lo[a] - std::fabs(lo[a]) * BOX_PAD;
+        info.bounds[3 + a] = hi[a] + std::fabs(hi[a]) * BOX_PAD;
     }
-    // the sums on the GPU (a wave reduction and one atomic per wave), the root node and the sums read back
-    bvh_stats_dev *dst = reinterpret_cast<bvh_stats_dev *>(bvh->err.as<uint8_t>() + 32);
-    VKRT_HIP(hipMemsetAsync(dst, 0, sizeof(bvh_stats_dev), s));
-    k_stats<<<div_up(bvh->n_nodes, 256), 256, 0, s>>>(bvh->n_nodes, bvh->max_leaf, bvh->nodes.as<vkrt_bvh_node>(),
-                                                      bvh->range.as<uint2>(), bvh->parent.as<int32_t>(), dst);
-    VKRT_HIP(hipGetLastError());
-    bvh_stats_dev st;
-    vkrt_bvh_node root;
-    VKRT_HIP(hipMemcpyAsync(&st, dst, sizeof st, hipMemcpyDeviceToHost, s));
-    VKRT_HIP(hipMemcpyAsync(&root, bvh->nodes.ptr, sizeof root, hipMemcpyDeviceToHost, s));
-    VKRT_HIP(hipStreamSynchronize(s));
-    float rb[6];
-    root_bounds(root, rb, info.bounds);
-    const double dx = std::max(0.0, (double)rb[1] - rb[0]), dy = std::max(0.0, (double)rb[3] - rb[2]),
-                 dz = std::max(0.0, (double)rb[5] - rb[4]);
-    const double root_area = std::max(1e-30, 2.0 * (dx * dy + dy * dz + dz * dx));
-    info.depth = std::max(1u, st.depth);
-    info.sah_cost = static_cast<float>(1.0 + st.sah / root_area);// 1: the root's own visit
-    info.n_leaves = st.leaves;
-    if(info.depth > (uint32_t)STACK_SIZE) throw error(VKRT_E_INTERNAL, "BVH deeper than the traversal stack");
 }
 
 static void build_topology_ploc(vkrt_ctx *ctx, vkrt_bvh *bvh);
@@ -583,7 +535,6 @@ static void build_topology(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh)
     hipStream_t s = ctx->stream;
     const uint32_t n = bvh->n_tri;
     bvh->tbox.reserve((size_t)n * 6 * sizeof(float));
-    bvh->err.reserve(64);
     // scratch: centroid bounds, sort keys, sort temp
     device_buffer &tmp = ctx->scratch[2];
     const size_t key_bytes = (size_t)n * sizeof(uint32_t), partial_bytes = BOUNDS_PARTIALS * 6 * sizeof(float);
@@ -594,32 +545,26 @@ static void build_topology(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh)
     bvh->order.reserve(key_bytes);
     uint32_t *order = bvh->order.as<uint32_t>();
 
-    VKRT_HIP(hipMemsetAsync(bvh->err.ptr, 0, 4, s));
+    bvh_state *st = ctx->state.as<bvh_state>();
+    k_state_clear<<<1, 256, 0, s>>>(st);
     const uint32_t n_partial = std::min(BOUNDS_PARTIALS, div_up(n, BOUNDS_BLOCK));
-    k_bounds<<<n_partial, BOUNDS_BLOCK, 0, s>>>(mesh, partial, bvh->err.as<uint32_t>());
+    k_bounds<<<n_partial, BOUNDS_BLOCK, 0, s>>>(mesh, partial, &st->err);
     k_morton<<<div_up(n, 256), 256, 0, s>>>(mesh, partial, n_partial, keys, order);
     radix_sort_pairs(s, keys, order, n, 30, sort_tmp);
-    uint32_t err_host = 0;
-    VKRT_HIP(hipMemcpyAsync(&err_host, bvh->err.ptr, 4, hipMemcpyDeviceToHost, s));
     if(n >= 2)
     {
         const uint32_t ni = n - 1;
         bvh->child.reserve(ni * sizeof(int2));
         bvh->range.reserve(ni * sizeof(uint2));
-        bvh->parent.reserve(((size_t)ni + n) * sizeof(int32_t));
-        int32_t *parent_int = bvh->parent.as<int32_t>(), *parent_leaf = parent_int + ni;
         if(bvh->builder == VKRT_BUILDER_PLOC)
         {
             k_leaves<false><<<div_up(n, 256), 256, 0, s>>>(mesh, order, bvh->tbox.as<float>(), nullptr);
             build_topology_ploc(ctx, bvh);
         }
         else
-            k_karras<<<div_up(ni, 256), 256, 0, s>>>(keys, (int)n, bvh->child.as<int2>(), bvh->range.as<uint2>(),
-                                                     parent_int, parent_leaf);
+            k_karras<<<div_up(ni, 256), 256, 0, s>>>(keys, (int)n, bvh->child.as<int2>(), bvh->range.as<uint2>());
     }
-    VKRT_HIP(hipStreamSynchronize(s));
     VKRT_HIP(hipGetLastError());
-    if(err_host) throw error(VKRT_E_INVALID_ARG, "triangle index out of range of the vertex count");
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -806,7 +751,7 @@ __global__ void k_ploc_permute(uint32_t ni, uint32_t n, const uint32_t *__restri
     if(k < n)
     {
         const uint32_t d = leaf_pos[k];
-        if(d >= n) return;// only a malformed tree gets here; compute_stats rejects it
+        if(d >= n) return;// only a malformed tree gets here; its depth is rejected
         order_out[d] = order_in[k];
     }
     if(k < ni)
@@ -917,7 +862,7 @@ static void build_topology_ploc(vkrt_ctx *ctx, vkrt_bvh *bvh)
     // working set: two cluster lists (ids, lo, hi), neighbours, flags and offsets, leaf counts, scan sums
     device_buffer &w = ctx->scratch[3];
     const size_t nb = div_up(n, 1024);
-    const size_t bytes = (size_t)n * (2 * 4 + 4 * 16 + 4 + 4 * 4 + 4) + (size_t)ni * 4 + nb * 4 + 512;
+    const size_t bytes = (size_t)n * (2 * 4 + 4 * 16 + 4 + 4 * 4 + 4 + 4) + (size_t)ni * 8 + nb * 4 + 512;
     w.reserve(bytes);
     uint8_t *q = w.as<uint8_t>();
     auto take = [&q](size_t b) {
@@ -937,10 +882,11 @@ static void build_topology_ploc(vkrt_ctx *ctx, vkrt_bvh *bvh)
     uint32_t *cnt = reinterpret_cast<uint32_t *>(take((size_t)ni * 4));
     uint32_t *sums = reinterpret_cast<uint32_t *>(take(nb * 4));
     uint32_t *totals = reinterpret_cast<uint32_t *>(take(16));
+    int32_t *parent_int = reinterpret_cast<int32_t *>(take((size_t)ni * 4));
+    int32_t *parent_leaf = reinterpret_cast<int32_t *>(take((size_t)n * 4));
     VKRT_REQUIRE(q <= w.as<uint8_t>() + bytes, "PLOC working set overrun");
 
     int2 *child = bvh->child.as<int2>();
-    int32_t *parent_int = bvh->parent.as<int32_t>(), *parent_leaf = parent_int + ni;
     k_ploc_init<<<div_up(n, 256), 256, 0, s>>>(bvh->tbox.as<float>(), n, id[0], lo[0], hi[0], parent_int, ni);
     uint32_t nc = n, base = 0;
     int cur = 0;
@@ -976,7 +922,6 @@ static void build_topology_ploc(vkrt_ctx *ctx, vkrt_bvh *bvh)
     uint32_t *order_in = koff;
     VKRT_HIP(hipMemcpyAsync(order_in, bvh->order.ptr, (size_t)n * 4, hipMemcpyDeviceToDevice, s));
     k_ploc_permute<<<div_up(n, 256), 256, 0, s>>>(ni, n, leaf_pos, order_in, bvh->order.as<uint32_t>(), child2, child);
-    VKRT_HIP(hipMemcpyAsync(parent_int, pint2, (size_t)ni * 4, hipMemcpyDeviceToDevice, s));
     VKRT_HIP(hipGetLastError());
 }
 
@@ -1051,74 +996,186 @@ __device__ __forceinline__ float half_area(const collapse_child &c)
     return dx * dy + dy * dz + dz * dx;
 }
 
-//! queue entries: (BVH2 node, BVH4 slot, stack depth on entry, -); counters: [0] BVH4 nodes allocated,
-//! [1] next queue size, [2] maximum stack depth
-__global__ void __launch_bounds__(256) k_collapse(const vkrt_bvh_node *__restrict__ n2, const int4 *__restrict__ in_q,
-                                                  uint32_t n_in, vkrt_bvh4_node *__restrict__ n4,
-                                                  int4 *__restrict__ out_q, uint32_t *__restrict__ counters)
+__device__ __forceinline__ double child_area(const collapse_child &c)
 {
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    if(t >= n_in) return;
-    const int4 item = in_q[t];
-    collapse_child ch[4];
-    const vkrt_bvh_node root = n2[item.x];
-    ch[0] = child_of(root, item.x, 0);
-    ch[1] = child_of(root, item.x, 1);
-    int cnt = 2;
-    while(cnt < 4)
+    const double dx = fmax(0.0, (double)c.hi[0] - c.lo[0]), dy = fmax(0.0, (double)c.hi[1] - c.lo[1]),
+                 dz = fmax(0.0, (double)c.hi[2] - c.lo[2]);
+    return 2.0 * (dx * dy + dy * dz + dz * dx);
+}
+
+//! one level of the collapse. The work item of 4-wide node i is queue[i] = (BVH2 node, stack depth on entry, the
+//! BVH2 node's depth): nodes are numbered level by level, so the queue's index is the node's. The level's
+//! nodes and its children's are st->level[0 .. level + 1]; a workgroup takes its children's slots with one
+//! atomic per 256 items (a child each took 63 us per level at 1.8M triangles on three words that every XCD
+//! writes), which also lays a node's children side by side. The grid may be larger or smaller than the level.
+//! A level opens every BVH2 node once, so the tree's depth, leaves and SAH terms are summed on the way (a pass of
+//! its own, climbing the parents for the depth, took 608 us). Nodes deeper than the stack end the descent: the
+//! build then fails. n4 null: the sums only.
+constexpr uint32_t COLLAPSE_BLOCK = 256, COLLAPSE_GRID = 1024;
+__global__ void __launch_bounds__(COLLAPSE_BLOCK) k_collapse(const vkrt_bvh_node *__restrict__ n2,
+                                                             int4 *__restrict__ queue, uint32_t level,
+                                                             vkrt_bvh4_node *__restrict__ n4,
+                                                             bvh_state *__restrict__ st)
+{
+    __shared__ uint32_t wave_sum[COLLAPSE_BLOCK / 64], slot_base;
+    __shared__ double wave_sah[COLLAPSE_BLOCK / 64];
+    __shared__ uint32_t wave_leaves[COLLAPSE_BLOCK / 64], wave_depth[COLLAPSE_BLOCK / 64],
+            wave_stack[COLLAPSE_BLOCK / 64];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    uint32_t first = 0;// the level's first node
+    for(uint32_t l = 0; l < level; ++l) first += st->level[l];
+    const uint32_t count = st->level[level], next = first + count;
+    double sah = 0.0;
+    uint32_t leaves = 0, depth = 0, stack = 0;
+    for(uint32_t base = blockIdx.x * COLLAPSE_BLOCK; base < count; base += gridDim.x * COLLAPSE_BLOCK)
     {
-        int best = -1;
-        float best_a = -1.0f;
-        for(int j = 0; j < cnt; ++j)
+        const bool active = base + threadIdx.x < count;
+        const uint32_t me = first + base + threadIdx.x;
+        collapse_child ch[4];
+        uint32_t ch_depth[4] = {0, 0, 0, 0};// depth of the BVH2 node each child came from
+        int cnt = 0;
+        uint32_t inner = 0, depth_here = 0;
+        if(active)
         {
-            if(ch[j].ref < 0) continue;
-            const float a = half_area(ch[j]);
-            if(a > best_a)
+            const int4 item = queue[me];
+            auto open = [&](int slot_a, int slot_b, int32_t node, uint32_t d) {
+                const vkrt_bvh_node nd = n2[node];
+                ch[slot_a] = child_of(nd, node, 0);
+                ch[slot_b] = child_of(nd, node, 1);
+                ch_depth[slot_a] = ch_depth[slot_b] = d;
+                depth = max(depth, d);
+                for(const int k: {slot_a, slot_b})
+                {
+                    const double a = child_area(ch[k]);
+                    if(ch[k].ref >= 0) sah += a;
+                    else
+                    {
+                        sah += ((static_cast<uint32_t>(~ch[k].ref) & 7u) + 1) * a;
+                        ++leaves;
+                        depth = max(depth, d + 1);
+                    }
+                }
+            };
+            open(0, 1, item.x, static_cast<uint32_t>(item.z));
+            cnt = 2;
+#pragma unroll
+            for(int step = 0; step < 2; ++step)
             {
-                best_a = a;
-                best = j;
+                int best = -1;
+                float best_a = -1.0f;
+#pragma unroll
+                for(int j = 0; j < 3; ++j)
+                {
+                    if(j >= cnt || ch[j].ref < 0) continue;
+                    const float a = half_area(ch[j]);
+                    if(a > best_a)
+                    {
+                        best_a = a;
+                        best = j;
+                    }
+                }
+                if(best < 0) break;
+                // (constant slots: an array indexed by `best` would live in scratch memory)
+                if(best == 0) open(0, 2 + step, ch[0].ref, ch_depth[0] + 1);
+                else if(best == 1) open(1, 2 + step, ch[1].ref, ch_depth[1] + 1);
+                else open(2, 3, ch[2].ref, ch_depth[2] + 1);
+                ++cnt;
             }
+            depth_here = static_cast<uint32_t>(item.y) + (cnt - 1);
+            stack = max(stack, depth_here);
+#pragma unroll
+            for(int j = 0; j < 4; ++j)
+                inner += j < cnt && ch[j].ref >= 0 && ch_depth[j] <= (uint32_t)STACK_SIZE ? 1u : 0u;
         }
-        if(best < 0) break;
-        const int32_t opened = ch[best].ref;
-        const vkrt_bvh_node nd = n2[opened];
-        ch[best] = child_of(nd, opened, 0);
-        ch[cnt] = child_of(nd, opened, 1);
-        ++cnt;
+        // the children's slots: an exclusive scan over the workgroup and one atomic
+        uint32_t sum = inner;
+        for(int off = 1; off < 64; off <<= 1)
+        {
+            const uint32_t y = __shfl_up(sum, off);
+            if(lane >= (uint32_t)off) sum += y;
+        }
+        if(lane == 63) wave_sum[wave] = sum;
+        __syncthreads();
+        uint32_t before = 0, total = 0;
+        for(uint32_t w = 0; w < COLLAPSE_BLOCK / 64; ++w)
+        {
+            before += w < wave ? wave_sum[w] : 0u;
+            total += wave_sum[w];
+        }
+        if(threadIdx.x == 0) slot_base = next + (total ? atomicAdd(&st->level[level + 1], total) : 0u);
+        __syncthreads();
+        uint32_t slot = slot_base + before + sum - inner;
+        if(active)
+        {
+            vkrt_bvh4_node out;
+            float lo[3][4], hi[3][4];
+            int32_t refs[4], srcs[4];
+#pragma unroll
+            for(int j = 0; j < 4; ++j)
+            {
+                srcs[j] = j < cnt ? ch[j].src : -1;
+                for(int a = 0; a < 3; ++a)
+                {
+                    lo[a][j] = j < cnt ? ch[j].lo[a] : 0.0f;
+                    hi[a][j] = j < cnt ? ch[j].hi[a] : 0.0f;
+                }
+                refs[j] = EMPTY_CHILD;
+                if(j >= cnt) continue;
+                if(ch[j].ref < 0) refs[j] = ch[j].ref;
+                else if(ch_depth[j] <= (uint32_t)STACK_SIZE)
+                {
+                    refs[j] = static_cast<int32_t>(slot);
+                    queue[slot++] = make_int4(ch[j].ref, static_cast<int32_t>(depth_here),
+                                              static_cast<int32_t>(ch_depth[j] + 1), 0);
+                }
+            }
+            out.lox = make_float4(lo[0][0], lo[0][1], lo[0][2], lo[0][3]);
+            out.hix = make_float4(hi[0][0], hi[0][1], hi[0][2], hi[0][3]);
+            out.loy = make_float4(lo[1][0], lo[1][1], lo[1][2], lo[1][3]);
+            out.hiy = make_float4(hi[1][0], hi[1][1], hi[1][2], hi[1][3]);
+            out.loz = make_float4(lo[2][0], lo[2][1], lo[2][2], lo[2][3]);
+            out.hiz = make_float4(hi[2][0], hi[2][1], hi[2][2], hi[2][3]);
+            out.child = make_int4(refs[0], refs[1], refs[2], refs[3]);
+            out.src = make_int4(srcs[0], srcs[1], srcs[2], srcs[3]);
+            if(n4) n4[me] = out;
+        }
     }
-    const int32_t depth_here = item.z + (cnt - 1);
-    atomicMax(&counters[2], static_cast<uint32_t>(depth_here));
-    vkrt_bvh4_node out;
-    float lo[3][4], hi[3][4];
-    int32_t refs[4], srcs[4];
-    for(int j = 0; j < 4; ++j)
+    if(blockIdx.x * COLLAPSE_BLOCK >= count) return;// (the whole workgroup: it had no item)
+    for(int off = 32; off > 0; off >>= 1)
     {
-        srcs[j] = j < cnt ? ch[j].src : -1;
-        for(int a = 0; a < 3; ++a)
-        {
-            lo[a][j] = j < cnt ? ch[j].lo[a] : 0.0f;
-            hi[a][j] = j < cnt ? ch[j].hi[a] : 0.0f;
-        }
-        refs[j] = EMPTY_CHILD;
-        if(j >= cnt) continue;
-        if(ch[j].ref < 0) refs[j] = ch[j].ref;
-        else
-        {
-            const uint32_t slot = atomicAdd(&counters[0], 1u);
-            refs[j] = static_cast<int32_t>(slot);
-            const uint32_t q = atomicAdd(&counters[1], 1u);
-            out_q[q] = make_int4(ch[j].ref, static_cast<int32_t>(slot), depth_here, 0);
-        }
+        sah += __shfl_xor(sah, off);
+        leaves += __shfl_xor(leaves, off);
+        depth = max(depth, (uint32_t)__shfl_xor(depth, off));
+        stack = max(stack, (uint32_t)__shfl_xor(stack, off));
     }
-    out.lox = make_float4(lo[0][0], lo[0][1], lo[0][2], lo[0][3]);
-    out.hix = make_float4(hi[0][0], hi[0][1], hi[0][2], hi[0][3]);
-    out.loy = make_float4(lo[1][0], lo[1][1], lo[1][2], lo[1][3]);
-    out.hiy = make_float4(hi[1][0], hi[1][1], hi[1][2], hi[1][3]);
-    out.loz = make_float4(lo[2][0], lo[2][1], lo[2][2], lo[2][3]);
-    out.hiz = make_float4(hi[2][0], hi[2][1], hi[2][2], hi[2][3]);
-    out.child = make_int4(refs[0], refs[1], refs[2], refs[3]);
-    out.src = make_int4(srcs[0], srcs[1], srcs[2], srcs[3]);
-    n4[item.y] = out;
+    if(lane == 0)
+    {
+        wave_sah[wave] = sah;
+        wave_leaves[wave] = leaves;
+        wave_depth[wave] = depth;
+        wave_stack[wave] = stack;
+    }
+    __syncthreads();
+    if(threadIdx.x == 0)
+    {
+        for(uint32_t w = 1; w < COLLAPSE_BLOCK / 64; ++w)
+        {
+            sah += wave_sah[w];
+            leaves += wave_leaves[w];
+            depth = max(depth, wave_depth[w]);
+            stack = max(stack, wave_stack[w]);
+        }
+        atomicAdd(&st->sah, sah);
+        if(leaves) atomicAdd(&st->leaves, leaves);
+        atomicMax(&st->depth, depth);
+        atomicMax(&st->stack, stack);
+    }
+}
+
+__global__ void k_collapse_root(int4 *__restrict__ queue, bvh_state *__restrict__ st)
+{
+    queue[0] = make_int4(0, 0, 1, 0);
+    st->level[0] = 1u;
 }
 
 //! refit of the 4-wide layout: every used child slot re-reads its box from the BVH2 node it was collapsed
@@ -1155,77 +1212,90 @@ static void refit_wide(vkrt_ctx *ctx, vkrt_bvh *bvh)
     VKRT_HIP(hipGetLastError());
 }
 
-//! collapse the BVH2 into the BVH4 used for traversal; keeps the BVH2 path when the worst-case stack
-//! depth of the collapse exceeds STACK_SIZE
+//! the end of a build: the BVH2 collapsed into the BVH4 used for traversal (kept off when its worst-case stack
+//! depth exceeds STACK_SIZE), the tree's statistics, and what the kernels before found wrong
 static void build_wide(vkrt_ctx *ctx, vkrt_bvh *bvh)
 {
     hipStream_t s = ctx->stream;
     bvh->wide = false;
     bvh->n_nodes4 = 0;
     bvh->stack4 = 0;
-    if(bvh->empty || !bvh->allow_wide) return;
+    auto check_indices = [](const bvh_state &st) {
+        if(st.err) throw error(VKRT_E_INVALID_ARG, "triangle index out of range of the vertex count");
+    };
     if(bvh->root_ref < 0)
     {
+        check_indices(read_state(ctx, nullptr));
         bvh->root4 = bvh->root_ref;// a single leaf
-        bvh->wide = true;
+        bvh->wide = bvh->allow_wide;
+        single_leaf_info(bvh, s);
         return;
     }
-    const size_t cap = std::max<uint32_t>(1u, bvh->n_nodes);
-    bvh->nodes4.reserve(cap * sizeof(vkrt_bvh4_node));
-    bvh->collapse_q[0].reserve(cap * sizeof(int4));
-    bvh->collapse_q[1].reserve(cap * sizeof(int4));
-    bvh->collapse_cnt.reserve(64);
-    uint32_t *cnt = bvh->collapse_cnt.as<uint32_t>();
-    const uint32_t init[4] = {1u, 0u, 0u, 0u};
-    VKRT_HIP(hipMemcpyAsync(cnt, init, sizeof init, hipMemcpyHostToDevice, s));
-    const int4 root_item = make_int4(bvh->root_ref, 0, 0, 0);
-    VKRT_HIP(hipMemcpyAsync(bvh->collapse_q[0].ptr, &root_item, sizeof root_item, hipMemcpyHostToDevice, s));
-    uint32_t n_in = 1;
-    int cur = 0;
-    while(n_in)
+    // (a 4-wide node takes in at least one node of the binary tree)
+    const size_t cap = bvh->n_nodes;
+    ctx->scratch[2].reserve(cap * sizeof(int4));
+    int4 *queue = ctx->scratch[2].as<int4>();
+    vkrt_bvh4_node *n4 = nullptr;
+    if(bvh->allow_wide)
     {
-        VKRT_HIP(hipMemsetAsync(cnt + 1, 0, 4, s));
-        k_collapse<<<div_up(n_in, 256), 256, 0, s>>>(bvh->nodes.as<vkrt_bvh_node>(), bvh->collapse_q[cur].as<int4>(),
-                                                     n_in, bvh->nodes4.as<vkrt_bvh4_node>(),
-                                                     bvh->collapse_q[cur ^ 1].as<int4>(), cnt);
-        VKRT_HIP(hipGetLastError());
-        uint32_t next = 0;
-        VKRT_HIP(hipMemcpyAsync(&next, cnt + 1, 4, hipMemcpyDeviceToHost, s));
-        VKRT_HIP(hipStreamSynchronize(s));
-        n_in = next;
-        cur ^= 1;
+        ctx->scratch[3].reserve(cap * sizeof(vkrt_bvh4_node));
+        n4 = ctx->scratch[3].as<vkrt_bvh4_node>();
     }
-    uint32_t host_cnt[4];
-    VKRT_HIP(hipMemcpyAsync(host_cnt, cnt, sizeof host_cnt, hipMemcpyDeviceToHost, s));
-    VKRT_HIP(hipStreamSynchronize(s));
-    bvh->n_nodes4 = host_cnt[0];
-    bvh->stack4 = host_cnt[2];
+    const vkrt_bvh_node *n2 = bvh->nodes.as<vkrt_bvh_node>();
+    bvh_state *st = ctx->state.as<bvh_state>();
+    k_collapse_root<<<1, 1, 0, s>>>(queue, st);
+    // the levels are launched without asking how many there are: as many as balanced trees of this size have and
+    // some more (a level that is not there costs its launch, 2 us), then in turns until the last one is empty
+    uint32_t level = 0, todo = 6;
+    for(size_t k = 1; k < cap; k *= 4) ++todo;
+    const bvh_state *got = nullptr;
+    while(true)
+    {
+        for(uint32_t stop = std::min(level + todo, MAX_LEVELS); level < stop; ++level)
+        {
+            const uint64_t most = std::min<uint64_t>(cap, level < 16 ? 1ull << (2 * level) : cap);
+            k_collapse<<<std::min(COLLAPSE_GRID, div_up(most, COLLAPSE_BLOCK)), COLLAPSE_BLOCK, 0, s>>>(n2, queue, level,
+                                                                                                         n4, st);
+        }
+        got = &read_state(ctx, n2);
+        check_indices(*got);
+        if(got->depth > (uint32_t)STACK_SIZE) throw error(VKRT_E_INTERNAL, "BVH deeper than the traversal stack");
+        if(got->level[level] == 0) break;
+        VKRT_REQUIRE(level < MAX_LEVELS, "BVH4 collapse did not end");
+        todo = 4;
+    }
+    uint64_t total = 0;
+    for(uint32_t l = 0; l < level; ++l) total += got->level[l];
+    VKRT_REQUIRE(total <= cap, "BVH4 collapse overflow");
+    vkrt_bvh_info &info = bvh->info;
+    float rb[6];
+    root_bounds(got->root, rb, info.bounds);
+    const double dx = std::max(0.0, (double)rb[1] - rb[0]), dy = std::max(0.0, (double)rb[3] - rb[2]),
+                 dz = std::max(0.0, (double)rb[5] - rb[4]);
+    const double root_area = std::max(1e-30, 2.0 * (dx * dy + dy * dz + dz * dx));
+    info.depth = std::max(1u, got->depth);
+    info.sah_cost = static_cast<float>(1.0 + got->sah / root_area);// 1: the root's own visit
+    info.n_leaves = got->leaves;
+    if(!bvh->allow_wide) return;
+    bvh->n_nodes4 = static_cast<uint32_t>(total);
+    bvh->stack4 = got->stack;
     bvh->root4 = 0;
-    VKRT_REQUIRE(bvh->n_nodes4 <= cap, "BVH4 collapse overflow");
+    // the nodes move from the scratch, sized for the most there could be, into an array of their number
+    const size_t bytes = (size_t)bvh->n_nodes4 * sizeof(vkrt_bvh4_node);
+    bvh->nodes4.reserve(bytes);
+    VKRT_HIP(hipMemcpyAsync(bvh->nodes4.ptr, n4, bytes, hipMemcpyDeviceToDevice, s));
     // the 4-wide walk addresses nodes with 32-bit byte offsets (node4_intervals)
-    bvh->wide = bvh->stack4 <= (uint32_t)STACK_SIZE &&
-                (uint64_t)bvh->n_nodes4 * sizeof(vkrt_bvh4_node) <= 0xffffffffull;
+    bvh->wide = bvh->stack4 <= (uint32_t)STACK_SIZE && (uint64_t)bytes <= 0xffffffffull;
 }
 
-//! the info block after a build (stats: depth, leaf count and SAH cost from all nodes, read back to the host)
-//! or after a refit, which keeps the topology: only the bounds change, read from the root node
-static void refresh_info(vkrt_bvh *bvh, hipStream_t s, bool stats)
+//! the rest of the info block after a build or a refit
+static void refresh_info(vkrt_bvh *bvh)
 {
     bvh->info.n_tri = bvh->n_tri;
     bvh->info.n_nodes = bvh->n_nodes;
     bvh->info.device_bytes = bvh->nodes.bytes + bvh->tris.bytes + bvh->nodes4.bytes;
     bvh->info.n_wide_nodes = bvh->wide ? bvh->n_nodes4 : 0;
     bvh->info.wide_stack = bvh->stack4;
-    if(stats || bvh->empty || bvh->root_ref < 0)
-    {
-        compute_stats(bvh, s);// (a single leaf or an empty BVH reads no node array)
-        return;
-    }
-    vkrt_bvh_node root;
-    VKRT_HIP(hipMemcpyAsync(&root, bvh->nodes.ptr, sizeof root, hipMemcpyDeviceToHost, s));
-    VKRT_HIP(hipStreamSynchronize(s));
-    float rb[6];
-    root_bounds(root, rb, bvh->info.bounds);
 }
 
 }// namespace vkrt
@@ -1262,6 +1332,7 @@ int vkrt_bvh_build(vkrt_ctx *ctx, const float *positions, uint32_t n_vert, uint3
         bvh->ploc_radius = params ? params->ploc_radius : 0u;
         if(n_tri)
         {
+            ctx->state.reserve(sizeof(bvh_state));
             const size_t pos_bytes = (size_t)(n_vert - 1) * stride_bytes + 12;
             const uint8_t *dpos =
                     input(ctx, 0, reinterpret_cast<const uint8_t *>(positions), pos_bytes, flags);
@@ -1275,8 +1346,9 @@ int vkrt_bvh_build(vkrt_ctx *ctx, const float *positions, uint32_t n_vert, uint3
             build_wide(ctx, bvh.get());
             VKRT_HIP(hipStreamSynchronize(ctx->stream));
         }
+        else single_leaf_info(bvh.get(), ctx->stream);
         bvh->info.build_ms = std::chrono::duration<float, std::milli>(std::chrono::steady_clock::now() - t_start).count();
-        refresh_info(bvh.get(), ctx->stream, true);
+        refresh_info(bvh.get());
         *out = bvh.release();
     });
 }
@@ -1288,13 +1360,20 @@ int vkrt_bvh_refit(vkrt_ctx *ctx, vkrt_bvh *bvh, const float *positions, uint32_
         VKRT_REQUIRE(stride_bytes >= 12 && stride_bytes % 4 == 0, "stride must be >= 12 and a multiple of 4");
         if(bvh->empty) return;
         VKRT_REQUIRE(positions, "null positions");
+        ctx->state.reserve(sizeof(bvh_state));
         hipStream_t s = ctx->stream;
         const size_t pos_bytes = (size_t)(bvh->n_vert - 1) * stride_bytes + 12;
         const uint8_t *dpos = input(ctx, 0, reinterpret_cast<const uint8_t *>(positions), pos_bytes, flags);
         build_bounds(ctx, bvh, mesh_view{dpos, bvh->indices.as<uint32_t>(), stride_bytes, bvh->n_tri, bvh->n_vert});
         refit_wide(ctx, bvh);
-        VKRT_HIP(hipStreamSynchronize(s));
-        refresh_info(bvh, s, false);
+        if(bvh->root_ref < 0) single_leaf_info(bvh, s);
+        else
+        {
+            // the topology stays, and with it depth, leaves and SAH cost: only the bounds change
+            float rb[6];
+            root_bounds(read_state(ctx, bvh->nodes.as<vkrt_bvh_node>()).root, rb, bvh->info.bounds);
+        }
+        refresh_info(bvh);
     });
 }
 

@@ -35,11 +35,11 @@ struct vkrt_bvh
     bool empty = true;
     vkrt::device_buffer nodes, tris;
     // the 4-wide collapse used by traversal when its worst-case stack fits (wide == true)
-    vkrt::device_buffer nodes4, collapse_q[2], collapse_cnt;
+    vkrt::device_buffer nodes4;
     int32_t root4 = 0;
     uint32_t n_nodes4 = 0, stack4 = 0;
     bool wide = false, allow_wide = true;
-    vkrt::device_buffer indices, order, child, range, parent, tbox, err;
+    vkrt::device_buffer indices, order, child, range, tbox;
     vkrt_bvh_info info{};
 };
 

@@ -37,6 +37,7 @@ int vkrt_create(int device, void *hip_stream, vkrt_ctx **out)
         if(arch.rfind("gfx950", 0) != 0)
             throw vkrt::error(VKRT_E_UNSUPPORTED, "libvkrt is built for gfx950 only; device is " + arch);
         vkrt::noalloc_scratch_init(ctx);
+        VKRT_HIP(hipHostMalloc(&ctx->pinned, vkrt_ctx::PINNED_BYTES));
     });
     if(rc != VKRT_OK)
     {
@@ -55,6 +56,8 @@ void vkrt_destroy(vkrt_ctx *ctx)
     if(ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     for(auto &b: ctx->staging) b.release();
     for(auto &b: ctx->scratch) b.release();
+    ctx->state.release();
+    if(ctx->pinned) (void)hipHostFree(ctx->pinned);
     if(ctx->own_stream && ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
 }

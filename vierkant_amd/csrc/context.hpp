@@ -94,6 +94,16 @@ struct vkrt_ctx
     vkrt::device_buffer staging[8];
     //! scratch for multi-pass kernels (keys, counters)
     vkrt::device_buffer scratch[4];
+    //! counters of a call's kernels, and the pinned host block they are read through
+    vkrt::device_buffer state;
+    void *pinned = nullptr;
+    static constexpr size_t PINNED_BYTES = 4096;
+    template<class T>
+    T *pinned_as() const
+    {
+        static_assert(sizeof(T) <= PINNED_BYTES);
+        return static_cast<T *>(pinned);
+    }
     //! this device's address of the allocation-free entry point's file-scope scratch array
     void *noalloc_scratch = nullptr;
 };
