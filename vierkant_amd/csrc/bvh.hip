@@ -72,15 +72,14 @@ __device__ __forceinline__ void load_triangle(const mesh_view &m, uint32_t j, ve
 //! reference test then produces NaN), so it gets an empty box and is never visited (returns false)
 __device__ __forceinline__ bool triangle_box(const vec3 &v0, const vec3 &v1, const vec3 &v2, float b[6])
 {
-    if(!(finite3(v0) && finite3(v1) && finite3(v2)))
-    {
-        b[0] = b[1] = b[2] = FLT_MAX;
-        b[3] = b[4] = b[5] = -FLT_MAX;
-        return false;
-    }
-    b[0] = fminf(fminf(v0.x, v1.x), v2.x), b[1] = fminf(fminf(v0.y, v1.y), v2.y), b[2] = fminf(fminf(v0.z, v1.z), v2.z);
-    b[3] = fmaxf(fmaxf(v0.x, v1.x), v2.x), b[4] = fmaxf(fmaxf(v0.y, v1.y), v2.y), b[5] = fmaxf(fmaxf(v0.z, v1.z), v2.z);
-    return true;
+    const bool finite = finite3(v0) && finite3(v1) && finite3(v2);
+    b[0] = finite ? fminf(fminf(v0.x, v1.x), v2.x) : FLT_MAX;
+    b[1] = finite ? fminf(fminf(v0.y, v1.y), v2.y) : FLT_MAX;
+    b[2] = finite ? fminf(fminf(v0.z, v1.z), v2.z) : FLT_MAX;
+    b[3] = finite ? fmaxf(fmaxf(v0.x, v1.x), v2.x) : -FLT_MAX;
+    b[4] = finite ? fmaxf(fmaxf(v0.y, v1.y), v2.y) : -FLT_MAX;
+    b[5] = finite ? fmaxf(fmaxf(v0.z, v1.z), v2.z) : -FLT_MAX;
+    return finite;
 }
 
 //! the bounds of the triangles' box centers, as one partial result per workgroup (k_morton combines them). No
@@ -242,28 +241,24 @@ __device__ __forceinline__ void store_box(float *p, const float b[6])
     for(int a = 0; a < 3; ++a) q[a] = make_float2(b[2 * a], b[2 * a + 1]);
 }
 
-//! the triangles in leaf order, straight from the mesh: their boxes, and with RECORDS the 48-B leaf records
-//! (v0, e1, e2, original index; the last two words are cleared)
-template<bool RECORDS>
+//! the triangles in leaf order, straight from the mesh: their boxes and the 48-B leaf records (v0, e1, e2, original
+//! index; the last two words are cleared)
 __global__ void __launch_bounds__(256) k_leaves(mesh_view m, const uint32_t *__restrict__ order,
                                                 float *__restrict__ tbox, float4 *__restrict__ tris)
 {
     const uint32_t j = blockIdx.x * 256 + threadIdx.x;
     if(j >= m.n_tri) return;
-    const uint32_t src = order[j];
+    const uint32_t src = min(order[j], m.n_tri - 1u);// (a malformed tree, rejected for its depth, leaves gaps)
     vec3 v0, v1, v2;
     bool ok;
     float b[6];
     load_triangle(m, src, v0, v1, v2, ok);
     triangle_box(v0, v1, v2, b);
     store_box(tbox + 6 * (size_t)j, b);
-    if constexpr(RECORDS)
-    {
-        const vec3 e1 = v1 - v0, e2 = v2 - v0;
-        tris[3 * (size_t)j + 0] = make_float4(v0.x, v0.y, v0.z, e1.x);
-        tris[3 * (size_t)j + 1] = make_float4(e1.y, e1.z, e2.x, e2.y);
-        tris[3 * (size_t)j + 2] = make_float4(e2.z, __uint_as_float(src), 0.f, 0.f);
-    }
+    const vec3 e1 = v1 - v0, e2 = v2 - v0;
+    tris[3 * (size_t)j + 0] = make_float4(v0.x, v0.y, v0.z, e1.x);
+    tris[3 * (size_t)j + 1] = make_float4(e1.y, e1.z, e2.x, e2.y);
+    tris[3 * (size_t)j + 2] = make_float4(e2.z, __uint_as_float(src), 0.f, 0.f);
 }
 
 //! Node boxes without a bottom-up hand-off. Every internal node covers a contiguous run [first, last] of the
@@ -444,6 +439,10 @@ __global__ void __launch_bounds__(256) k_layout(leaf_unions l, const int2 *__res
 //! build and copied to the context's pinned host memory by k_report (a kernel's store and the synchronization
 //! take 10 us; a copy into pageable memory took 25 us besides). Counters that many workgroups update lie on
 //! lines of their own.
+struct ploc_round
+{
+    uint32_t nc, base, buf;// clusters, nodes made so far, which of the two lists holds the clusters
+};
 constexpr uint32_t MAX_LEVELS = STACK_SIZE + 2;// of the 4-wide collapse: each goes at least one binary level down
 struct bvh_state
 {
@@ -458,6 +457,8 @@ struct bvh_state
     uint32_t stack;// worst-case traversal stack of the 4-wide tree
     uint32_t pad4[31];
     uint32_t level[MAX_LEVELS + 2];// 4-wide nodes per level
+    ploc_round ploc[2];            // the clusters before an even and an odd round
+    uint32_t ploc_left, ploc_nodes;// clusters left and nodes made after the last tail
     vkrt_bvh_node root;
 };
 
@@ -528,7 +529,7 @@ static void single_leaf_info(vkrt_bvh *bvh, hipStream_t s)
     }
 }
 
-static void build_topology_ploc(vkrt_ctx *ctx, vkrt_bvh *bvh);
+static void build_topology_ploc(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh, const uint32_t *sorted);
 
 static void build_topology(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh)
 {
@@ -538,12 +539,14 @@ static void build_topology(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh)
     // scratch: centroid bounds, sort keys, sort temp
     device_buffer &tmp = ctx->scratch[2];
     const size_t key_bytes = (size_t)n * sizeof(uint32_t), partial_bytes = BOUNDS_PARTIALS * 6 * sizeof(float);
-    tmp.reserve(partial_bytes + key_bytes + radix_sort_temp_bytes(n));
+    tmp.reserve(partial_bytes + 2 * key_bytes + radix_sort_temp_bytes(n));
     float *partial = tmp.as<float>();
     uint32_t *keys = reinterpret_cast<uint32_t *>(tmp.as<uint8_t>() + partial_bytes);
-    void *sort_tmp = tmp.as<uint8_t>() + partial_bytes + key_bytes;
+    void *sort_tmp = tmp.as<uint8_t>() + partial_bytes + 2 * key_bytes;
     bvh->order.reserve(key_bytes);
-    uint32_t *order = bvh->order.as<uint32_t>();
+    // PLOC puts the sorted triangles into an order of its own
+    const bool ploc = bvh->builder == VKRT_BUILDER_PLOC && n >= 2;
+    uint32_t *order = ploc ? keys + n : bvh->order.as<uint32_t>();
 
     bvh_state *st = ctx->state.as<bvh_state>();
     k_state_clear<<<1, 256, 0, s>>>(st);
@@ -556,11 +559,7 @@ static void build_topology(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh)
         const uint32_t ni = n - 1;
         bvh->child.reserve(ni * sizeof(int2));
         bvh->range.reserve(ni * sizeof(uint2));
-        if(bvh->builder == VKRT_BUILDER_PLOC)
-        {
-            k_leaves<false><<<div_up(n, 256), 256, 0, s>>>(mesh, order, bvh->tbox.as<float>(), nullptr);
-            build_topology_ploc(ctx, bvh);
-        }
+        if(ploc) build_topology_ploc(ctx, bvh, mesh, order);
         else
             k_karras<<<div_up(ni, 256), 256, 0, s>>>(keys, (int)n, bvh->child.as<int2>(), bvh->range.as<uint2>());
     }
@@ -572,82 +571,364 @@ static void build_topology(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh)
 // cluster finds, within PLOC_RADIUS positions of the sorted list, the cluster whose merged box has the
 // smallest surface area; mutual nearest neighbours merge into a new node at the lower position, and the list
 // is compacted. Pairs are ordered by (area, lower position, higher position), so the globally smallest pair
-// is always mutual and every round merges. Internal nodes are numbered in merge order, then renumbered so the
-// root is node 0 and parents precede children; leaves are finally put in depth-first order so that every
-// subtree covers a contiguous range, which the leaf collapse of k_layout and the refit rely on.
+// is always mutual and every round merges. Nodes are numbered down from n - 2 in merge order, so the root is
+// node 0 and parents precede children; leaves are finally put in depth-first order so that every subtree
+// covers a contiguous range, which the leaf collapse of k_layout and the refit rely on.
+//
+// A 1.8M-triangle build takes 64 rounds, 30 of them over fewer than 1,024 clusters, so what a round costs besides
+// its work decides: two launches a round, with no count read by the host, and the last rounds in one workgroup
+// that keeps its clusters in LDS (nine launches and a host round trip a round took 5.0 ms; now 1.1 ms).
 // ---------------------------------------------------------------------------------------------
 constexpr int PLOC_RADIUS = 16;    // default search radius
 constexpr int PLOC_MAX_RADIUS = 32;
 constexpr int PLOC_BLOCK = 256;
-constexpr uint32_t PLOC_MAX_DEPTH = 4096;// bound of the upward walks; deeper trees are rejected after layout
+constexpr int PLOC_SPAN = 4 * PLOC_BLOCK;// positions whose neighbour a workgroup finds: its tile and a radius each side
+constexpr uint32_t PLOC_TAIL = 1024;     // clusters that one workgroup finishes
+constexpr uint32_t PLOC_MAX_CLIMB = 4096;// bound of the upward walks; deeper trees are rejected after the collapse
 
-__device__ __forceinline__ float merged_half_area(const float4 &alo, const float4 &ahi, const float4 &blo,
-                                                  const float4 &bhi)
+//! the positions of a tile whose neighbours' neighbours are inside the workgroup's span
+__host__ __device__ constexpr uint32_t ploc_tile(int radius) { return PLOC_SPAN - 2 * radius; }
+
+//! what a cluster does in a round: merge with the cluster `code` positions on, or one of these
+constexpr int8_t PLOC_GONE = 0, PLOC_STAYS = -128;
+
+//! the two cluster lists: box corners, with the cluster's node (a leaf: ~position) in lo.w and its leaf count in
+//! hi.w, as bits
+struct ploc_lists
 {
-    const float dx = fmaxf(ahi.x, bhi.x) - fminf(alo.x, blo.x);
-    const float dy = fmaxf(ahi.y, bhi.y) - fminf(alo.y, blo.y);
-    const float dz = fmaxf(ahi.z, bhi.z) - fminf(alo.z, blo.z);
+    float4 *lo[2], *hi[2];
+};
+
+//! the tree under construction: node k's children, leaf count and parent
+struct ploc_tree
+{
+    int2 *child;
+    uint32_t *cnt;
+    int32_t *parent;
+    uint32_t ni;
+};
+
+__device__ __forceinline__ float merged_half_area(const float2 a[3], const float2 b[3])
+{
+    const float dx = fmaxf(a[0].y, b[0].y) - fminf(a[0].x, b[0].x);
+    const float dy = fmaxf(a[1].y, b[1].y) - fminf(a[1].x, b[1].x);
+    const float dz = fmaxf(a[2].y, b[2].y) - fminf(a[2].x, b[2].x);
     return dx * dy + dy * dz + dz * dx;
 }
 
-__global__ void k_ploc_init(const float *__restrict__ tbox, uint32_t n, int32_t *__restrict__ cl_id,
-                            float4 *__restrict__ lo, float4 *__restrict__ hi, int32_t *__restrict__ parent_int,
-                            uint32_t ni)
+__global__ void __launch_bounds__(256) k_ploc_init(mesh_view m, const uint32_t *__restrict__ order, float4 *__restrict__ lo,
+                                                   float4 *__restrict__ hi, bvh_state *__restrict__ st)
 {
-    const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-    if(j < ni) parent_int[j] = -1;
-    if(j >= n) return;
-    const float *b = tbox + 6 * (size_t)j;
-    cl_id[j] = ~static_cast<int32_t>(j);
-    lo[j] = make_float4(b[0], b[1], b[2], 0.f);
-    hi[j] = make_float4(b[3], b[4], b[5], 0.f);
+    const uint32_t j = blockIdx.x * 256 + threadIdx.x;
+    if(j == 0) st->ploc[0] = ploc_round{m.n_tri, 0u, 0u};
+    if(j >= m.n_tri) return;
+    vec3 v0, v1, v2;
+    bool ok;
+    float b[6];
+    load_triangle(m, order[j], v0, v1, v2, ok);
+    triangle_box(v0, v1, v2, b);
+    lo[j] = make_float4(b[0], b[1], b[2], __int_as_float(~static_cast<int32_t>(j)));
+    hi[j] = make_float4(b[3], b[4], b[5], __uint_as_float(1u));
 }
 
-//! nearest neighbour of every cluster within the window; ties go to the smallest position, which is the
-//! smallest pair in (area, lower, higher) order
-__global__ void __launch_bounds__(PLOC_BLOCK) k_ploc_nn(const float4 *__restrict__ lo, const float4 *__restrict__ hi,
-                                                        uint32_t nc, int radius, int32_t *__restrict__ nn)
+//! node `id` over clusters a and b (their node and leaf count); returns its leaf count
+__device__ __forceinline__ uint32_t ploc_node(const ploc_tree &t, int32_t id, int32_t a, int32_t b, uint32_t na, uint32_t nb)
 {
-    __shared__ float4 slo[PLOC_BLOCK + 2 * PLOC_MAX_RADIUS], shi[PLOC_BLOCK + 2 * PLOC_MAX_RADIUS];
-    const int base = static_cast<int>(blockIdx.x * PLOC_BLOCK) - radius;
-    for(int k = threadIdx.x; k < PLOC_BLOCK + 2 * radius; k += PLOC_BLOCK)
+    t.child[id] = make_int2(a, b);
+    t.cnt[id] = na + nb;
+    if(a >= 0) t.parent[a] = id;
+    if(b >= 0) t.parent[b] = id;
+    return na + nb;
+}
+
+//! the nearest neighbour of every cluster within the window (ties go to the smallest position, which is the
+//! smallest pair in (area, lower, higher) order), and what each cluster does: code, and per tile the clusters kept
+//! and merged. A thread takes four neighbouring positions, so a box read from LDS serves four of them (one position
+//! a thread read 64 16-B words each, 180 us for 1.8M clusters); boxes lie by position mod 4, so that a wave's
+//! reads are consecutive. RADIUS 0: the radius is the argument.
+template<int RADIUS>
+__global__ void __launch_bounds__(PLOC_BLOCK) k_ploc_nn(const bvh_state *__restrict__ st, uint32_t parity, int radius_arg,
+                                                        ploc_lists l, int8_t *__restrict__ code,
+                                                        uint32_t *__restrict__ counts)
+{
+    constexpr int QUARTER = (PLOC_SPAN + 2 * PLOC_MAX_RADIUS) / 4;
+    __shared__ float2 box[3][4 * QUARTER];
+    __shared__ int16_t nn[PLOC_SPAN];
+    __shared__ uint32_t wave_count[PLOC_BLOCK / 64];
+    const int radius = RADIUS ? RADIUS : radius_arg;
+    const ploc_round round = st->ploc[parity];
+    const int nc = static_cast<int>(round.nc), tile = static_cast<int>(ploc_tile(radius));
+    const int start = static_cast<int>(blockIdx.x) * tile;
+    if(round.nc <= PLOC_TAIL || start >= nc) return;
+    const float4 *__restrict__ lo = l.lo[round.buf], *__restrict__ hi = l.hi[round.buf];
+    const int span0 = start - radius;// the position of nn[0]
+    for(int s = threadIdx.x; s < PLOC_SPAN + 2 * radius; s += PLOC_BLOCK)
     {
-        const int g = base + k;
-        if(g >= 0 && g < static_cast<int>(nc))
-        {
-            slo[k] = lo[g];
-            shi[k] = hi[g];
-        }
+        const int j = span0 - radius + s;
+        if(j < 0 || j >= nc) continue;
+        const float4 a = lo[j], b = hi[j];
+        const int slot = (s & 3) * QUARTER + (s >> 2);
+        box[0][slot] = make_float2(a.x, b.x);
+        box[1][slot] = make_float2(a.y, b.y);
+        box[2][slot] = make_float2(a.z, b.z);
     }
     __syncthreads();
-    const int i = static_cast<int>(blockIdx.x * PLOC_BLOCK + threadIdx.x);
-    if(i >= static_cast<int>(nc)) return;
-    const int li = threadIdx.x + radius;
-    float best = 0.f;
-    int bj = -1;
-    for(int o = -radius; o <= radius; ++o)
-    {
-        const int j = i + o;
-        if(o == 0 || j < 0 || j >= static_cast<int>(nc)) continue;
-        const float d = merged_half_area(slo[li], shi[li], slo[li + o], shi[li + o]);
-        if(bj < 0 || d < best)
+    const int t = static_cast<int>(threadIdx.x);
+    auto load = [&](int c, float2 v[3]) {
+        const int slot = (c & 3) * QUARTER + t + (c >> 2);
+        v[0] = box[0][slot], v[1] = box[1][slot], v[2] = box[2][slot];
+    };
+    float2 own[4][3];
+    for(int k = 0; k < 4; ++k) load(k + radius, own[k]);
+    float best[4] = {0.f, 0.f, 0.f, 0.f};
+    int best_c[4] = {-1, -1, -1, -1};
+    const int j0 = span0 - radius + 4 * t;
+    auto step = [&](int c) {
+        const int j = j0 + c;
+        const bool there = j >= 0 && j < nc;
+        float2 v[3];
+        load(c, v);
+#pragma unroll
+        for(int k = 0; k < 4; ++k)
         {
-            best = d;
-            bj = j;
+            const int o = c - radius - k;
+            if(o < -radius || o > radius || o == 0) continue;
+            const float d = merged_half_area(own[k], v);
+            if(there && (best_c[k] < 0 || d < best[k]))
+            {
+                best[k] = d;
+                best_c[k] = c;
+            }
         }
+    };
+    if constexpr(RADIUS != 0)
+    {
+#pragma unroll
+        for(int c = 0; c < 2 * RADIUS + 4; ++c) step(c);
     }
-    nn[i] = bj;
+    else
+        for(int c = 0; c < 2 * radius + 4; ++c) step(c);
+    for(int k = 0; k < 4; ++k) nn[4 * t + k] = static_cast<int16_t>(4 * t + best_c[k] - radius);
+    __syncthreads();
+    uint32_t kept = 0, merged = 0;
+    for(int m = 0; m < 4; ++m)
+    {
+        const int i = t + m * PLOC_BLOCK;
+        const bool mine = i >= radius && i < PLOC_SPAN - radius && span0 + i < nc;
+        int8_t what = PLOC_GONE;
+        if(mine)
+        {
+            const int j = nn[i];
+            const bool mutual = nn[j] == i;
+            what = !mutual ? PLOC_STAYS : (i < j ? static_cast<int8_t>(j - i) : PLOC_GONE);
+            code[span0 + i] = what;
+        }
+        kept += __popcll(__ballot(mine && what != PLOC_GONE));
+        merged += __popcll(__ballot(mine && what > 0));
+    }
+    if((threadIdx.x & 63u) == 0) wave_count[threadIdx.x >> 6] = kept | (merged << 16);
+    __syncthreads();
+    if(threadIdx.x == 0)
+        counts[blockIdx.x] = (wave_count[0] + wave_count[1]) + (wave_count[2] + wave_count[3]);
 }
 
-__global__ void k_ploc_flags(const int32_t *__restrict__ nn, uint32_t nc, uint32_t *__restrict__ merge,
-                             uint32_t *__restrict__ keep)
+//! the round's merges and the compacted list. A tile's place is the sum of the tiles before it, which every
+//! workgroup adds up for itself (at most 1,900 of them at 1.8M clusters, from L2): no scan launches and no waiting.
+__global__ void __launch_bounds__(PLOC_BLOCK) k_ploc_merge(bvh_state *__restrict__ st, uint32_t parity, int radius,
+                                                           ploc_lists l, const int8_t *__restrict__ code,
+                                                           const uint32_t *__restrict__ counts, ploc_tree tree)
 {
-    const int i = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
-    if(i >= static_cast<int>(nc)) return;
-    const int j = nn[i];
-    const bool mutual = nn[j] == i;
-    merge[i] = (mutual && i < j) ? 1u : 0u;
-    keep[i] = (mutual && i > j) ? 0u : 1u;
+    __shared__ uint32_t wave_kept[PLOC_BLOCK / 64], wave_merged[PLOC_BLOCK / 64], wave_sum[PLOC_BLOCK / 64];
+    const ploc_round round = st->ploc[parity];
+    const uint32_t tile = ploc_tile(radius), start = blockIdx.x * tile;
+    if(round.nc <= PLOC_TAIL)
+    {
+        if(blockIdx.x == 0 && threadIdx.x == 0) st->ploc[parity ^ 1u] = round;// left to the tail
+        return;
+    }
+    if(start >= round.nc) return;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    uint32_t kept = 0, merged = 0;// of the tiles before
+    for(uint32_t b = threadIdx.x; b < blockIdx.x; b += PLOC_BLOCK)
+    {
+        const uint32_t c = counts[b];
+        kept += c & 0xffffu;
+        merged += c >> 16;
+    }
+    for(int off = 32; off > 0; off >>= 1)
+    {
+        kept += __shfl_xor(kept, off);
+        merged += __shfl_xor(merged, off);
+    }
+    int8_t what[4];
+    uint32_t mine = 0;// kept | merged << 16 of this thread's four positions
+    for(uint32_t k = 0; k < 4; ++k)
+    {
+        const uint32_t p = 4 * threadIdx.x + k;
+        what[k] = p < tile && start + p < round.nc ? code[start + p] : PLOC_GONE;
+        mine += (what[k] != PLOC_GONE ? 1u : 0u) + (what[k] > 0 ? 0x10000u : 0u);
+    }
+    uint32_t scan = mine;
+    for(int off = 1; off < 64; off <<= 1)
+    {
+        const uint32_t y = __shfl_up(scan, off);
+        if(lane >= (uint32_t)off) scan += y;
+    }
+    if(lane == 63) wave_sum[wave] = scan;
+    if(lane == 0)
+    {
+        wave_kept[wave] = kept;
+        wave_merged[wave] = merged;
+    }
+    __syncthreads();
+    kept = (wave_kept[0] + wave_kept[1]) + (wave_kept[2] + wave_kept[3]);
+    merged = (wave_merged[0] + wave_merged[1]) + (wave_merged[2] + wave_merged[3]);
+    uint32_t before = scan - mine, total = 0;
+    for(uint32_t w = 0; w < PLOC_BLOCK / 64; ++w)
+    {
+        before += w < wave ? wave_sum[w] : 0u;
+        total += wave_sum[w];
+    }
+    if(start + tile >= round.nc && threadIdx.x == 0)
+        st->ploc[parity ^ 1u] = ploc_round{kept + (total & 0xffffu), round.base + merged + (total >> 16), round.buf ^ 1u};
+    const float4 *__restrict__ lo = l.lo[round.buf], *__restrict__ hi = l.hi[round.buf];
+    float4 *__restrict__ out_lo = l.lo[round.buf ^ 1u], *__restrict__ out_hi = l.hi[round.buf ^ 1u];
+    uint32_t pos = kept + (before & 0xffffu), made = round.base + merged + (before >> 16);
+    for(uint32_t k = 0; k < 4; ++k)
+    {
+        if(what[k] == PLOC_GONE) continue;
+        const uint32_t i = start + 4 * threadIdx.x + k;
+        float4 a = lo[i], b = hi[i];
+        if(what[k] > 0)
+        {
+            const float4 c = lo[i + what[k]], d = hi[i + what[k]];
+            const int32_t id = static_cast<int32_t>(tree.ni - 1u - made);
+            ++made;
+            const uint32_t n = ploc_node(tree, id, __float_as_int(a.w), __float_as_int(c.w), __float_as_uint(b.w),
+                                         __float_as_uint(d.w));
+            a = make_float4(fminf(a.x, c.x), fminf(a.y, c.y), fminf(a.z, c.z), __int_as_float(id));
+            b = make_float4(fmaxf(b.x, d.x), fmaxf(b.y, d.y), fmaxf(b.z, d.z), __uint_as_float(n));
+        }
+        out_lo[pos] = a;
+        out_hi[pos] = b;
+        ++pos;
+    }
+}
+
+//! every remaining round of at most PLOC_TAIL clusters in one workgroup, one cluster a thread (three barriers a
+//! round, 1.5 us, against the two launches of the kernels above)
+__global__ void __launch_bounds__(PLOC_TAIL) k_ploc_tail(bvh_state *__restrict__ st, uint32_t parity, int radius,
+                                                         ploc_lists l, ploc_tree tree)
+{
+    __shared__ float2 box[3][PLOC_TAIL];
+    __shared__ int32_t node[PLOC_TAIL];
+    __shared__ uint32_t leaves[PLOC_TAIL];
+    __shared__ int16_t nn[PLOC_TAIL];
+    __shared__ uint32_t wave_sum[PLOC_TAIL / 64];
+    const ploc_round round = st->ploc[parity];
+    const int i = static_cast<int>(threadIdx.x);
+    if(round.nc > PLOC_TAIL)
+    {
+        if(i == 0) st->ploc_left = round.nc;
+        return;
+    }
+    int nc = static_cast<int>(round.nc);
+    uint32_t base = round.base;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    float2 me[3];
+    int32_t id = 0;
+    uint32_t n = 0;
+    if(i < nc)
+    {
+        const float4 a = l.lo[round.buf][i], b = l.hi[round.buf][i];
+        me[0] = make_float2(a.x, b.x), me[1] = make_float2(a.y, b.y), me[2] = make_float2(a.z, b.z);
+        id = __float_as_int(a.w);
+        n = __float_as_uint(b.w);
+        for(int k = 0; k < 3; ++k) box[k][i] = me[k];
+        node[i] = id;
+        leaves[i] = n;
+    }
+    __syncthreads();
+    while(nc > 1)
+    {
+        const bool active = i < nc;
+        int best_j = -1;
+        if(active)
+        {
+            float best = 0.f;
+            const int first = max(0, i - radius), last = min(nc - 1, i + radius);
+            for(int j = first; j <= last; ++j)
+            {
+                if(j == i) continue;
+                const float2 v[3] = {box[0][j], box[1][j], box[2][j]};
+                const float d = merged_half_area(me, v);
+                if(best_j < 0 || d < best)
+                {
+                    best = d;
+                    best_j = j;
+                }
+            }
+            nn[i] = static_cast<int16_t>(best_j);
+        }
+        __syncthreads();
+        const bool mutual = active && nn[best_j] == i;
+        const bool merges = mutual && i < best_j, keep = active && !(mutual && i > best_j);
+        float2 other[3];
+        int32_t other_id = 0;
+        uint32_t other_n = 0;
+        if(merges)
+        {
+            for(int k = 0; k < 3; ++k) other[k] = box[k][best_j];
+            other_id = node[best_j];
+            other_n = leaves[best_j];
+        }
+        const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+        const uint64_t km = __ballot(keep), mm = __ballot(merges);
+        if(lane == 0) wave_sum[wave] = __popcll(km) | (static_cast<uint32_t>(__popcll(mm)) << 16);
+        __syncthreads();
+        uint32_t before = 0, total = 0;
+        for(uint32_t w = 0; w < PLOC_TAIL / 64; ++w)
+        {
+            before += w < wave ? wave_sum[w] : 0u;
+            total += wave_sum[w];
+        }
+        if(merges)
+        {
+            const int32_t made = static_cast<int32_t>(tree.ni - 1u - (base + (before >> 16) + __popcll(mm & below)));
+            n = ploc_node(tree, made, id, other_id, n, other_n);
+            id = made;
+            for(int k = 0; k < 3; ++k)
+                me[k] = make_float2(fminf(me[k].x, other[k].x), fmaxf(me[k].y, other[k].y));
+        }
+        if((total >> 16) == 0u)
+        {
+            // every round merges the smallest pair at least, unless areas are NaN (an infinite extent times zero):
+            // the build then fails
+            if(i == 0) st->ploc_left = 0u;
+            return;
+        }
+        const int to = static_cast<int>((before & 0xffffu) + __popcll(km & below));
+        if(keep)
+        {
+            for(int k = 0; k < 3; ++k) box[k][to] = me[k];
+            node[to] = id;
+            leaves[to] = n;
+        }
+        nc = static_cast<int>(total & 0xffffu);
+        base += total >> 16;
+        __syncthreads();
+        if(i < nc)
+        {
+            for(int k = 0; k < 3; ++k) me[k] = box[k][i];
+            id = node[i];
+            n = leaves[i];
+        }
+    }
+    if(i == 0)
+    {
+        st->ploc_left = 1u;
+        st->ploc_nodes = base;
+    }
 }
 
 __device__ __forceinline__ uint32_t leaf_count(const uint32_t *__restrict__ cnt, int32_t ref)
@@ -655,214 +936,63 @@ __device__ __forceinline__ uint32_t leaf_count(const uint32_t *__restrict__ cnt,
     return ref < 0 ? 1u : cnt[ref];
 }
 
-__global__ void k_ploc_merge(const int32_t *__restrict__ nn, uint32_t nc, const uint32_t *__restrict__ merge,
-                             const uint32_t *__restrict__ moff, const uint32_t *__restrict__ keep,
-                             const uint32_t *__restrict__ koff, uint32_t base, const int32_t *__restrict__ cl_id,
-                             const float4 *__restrict__ lo, const float4 *__restrict__ hi,
-                             int32_t *__restrict__ out_id, float4 *__restrict__ out_lo, float4 *__restrict__ out_hi,
-                             int2 *__restrict__ child, uint32_t *__restrict__ cnt, int32_t *__restrict__ parent_int,
-                             int32_t *__restrict__ parent_leaf)
+//! the depth-first position of the first leaf of nodes a .. b - 1: the leaf counts of all left siblings on the way
+//! up to a node before a, whose position an earlier launch found (parents precede children). Launched over
+//! ranges that grow eightfold, so a climb is a few steps (up to the root from everywhere took 199 us)
+__global__ void __launch_bounds__(256) k_ploc_first(uint32_t a, uint32_t b, ploc_tree tree, uint32_t *__restrict__ first)
 {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if(i >= nc || !keep[i]) return;
-    const uint32_t pos = koff[i];
-    if(!merge[i])
+    const uint32_t k = a + blockIdx.x * 256 + threadIdx.x;
+    if(k >= b) return;
+    uint32_t off = 0;
+    int32_t cur = static_cast<int32_t>(k);
+    for(uint32_t step = 0; cur > 0 && step < PLOC_MAX_CLIMB; ++step)
     {
-        out_id[pos] = cl_id[i];
-        out_lo[pos] = lo[i];
-        out_hi[pos] = hi[i];
-        return;
-    }
-    const uint32_t j = static_cast<uint32_t>(nn[i]);
-    const int32_t id = static_cast<int32_t>(base + moff[i]);
-    const int32_t a = cl_id[i], b = cl_id[j];
-    child[id] = make_int2(a, b);
-    cnt[id] = leaf_count(cnt, a) + leaf_count(cnt, b);
-    if(a < 0) parent_leaf[~a] = id;
-    else parent_int[a] = id;
-    if(b < 0) parent_leaf[~b] = id;
-    else parent_int[b] = id;
-    const float4 la = lo[i], lb = lo[j], ha = hi[i], hb = hi[j];
-    out_id[pos] = id;
-    out_lo[pos] = make_float4(fminf(la.x, lb.x), fminf(la.y, lb.y), fminf(la.z, lb.z), 0.f);
-    out_hi[pos] = make_float4(fmaxf(ha.x, hb.x), fmaxf(ha.y, hb.y), fmaxf(ha.z, hb.z), 0.f);
-}
-
-//! internal node k becomes ni - 1 - k: the last merge (the root) is node 0 and parents precede children
-__global__ void k_ploc_renumber(uint32_t ni, uint32_t n, const int2 *__restrict__ child, const uint32_t *__restrict__ cnt,
-                                const int32_t *__restrict__ parent_int, const int32_t *__restrict__ parent_leaf,
-                                int2 *__restrict__ child2, uint32_t *__restrict__ cnt2, int32_t *__restrict__ parent_int2,
-                                int32_t *__restrict__ parent_leaf2)
-{
-    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    auto map = [ni](int32_t r) { return r < 0 ? r : static_cast<int32_t>(ni - 1u) - r; };
-    if(k < ni)
-    {
-        const uint32_t nk = ni - 1u - k;
-        const int2 c = child[k];
-        child2[nk] = make_int2(map(c.x), map(c.y));
-        cnt2[nk] = cnt[k];
-        parent_int2[nk] = parent_int[k] < 0 ? -1 : map(parent_int[k]);
-    }
-    if(k < n) parent_leaf2[k] = map(parent_leaf[k]);
-}
-
-//! depth-first position of every leaf and the first position of every internal node's range: the leaf
-//! counts of all left siblings on the way up
-__global__ void k_ploc_dfs(uint32_t ni, uint32_t n, const int2 *__restrict__ child, const uint32_t *__restrict__ cnt,
-                           const int32_t *__restrict__ parent_int, const int32_t *__restrict__ parent_leaf,
-                           uint32_t *__restrict__ leaf_pos, uint2 *__restrict__ range)
-{
-    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    if(k < n)
-    {
-        uint32_t off = 0;
-        int32_t cur = ~static_cast<int32_t>(k), node = parent_leaf[k];
-        for(uint32_t step = 0; node >= 0 && step < PLOC_MAX_DEPTH; ++step)
+        const int32_t up = tree.parent[cur];
+        const int2 c = tree.child[up];
+        if(c.y == cur) off += leaf_count(tree.cnt, c.x);
+        cur = up;
+        if(cur > 0 && static_cast<uint32_t>(cur) < a)
         {
-            const int2 c = child[node];
-            if(c.y == cur) off += leaf_count(cnt, c.x);
-            cur = node;
-            node = parent_int[node];
+            off += first[cur];
+            break;
         }
-        leaf_pos[k] = off;
     }
-    if(k < ni)
-    {
-        uint32_t off = 0;
-        int32_t cur = static_cast<int32_t>(k), node = parent_int[k];
-        for(uint32_t step = 0; node >= 0 && step < PLOC_MAX_DEPTH; ++step)
-        {
-            const int2 c = child[node];
-            if(c.y == cur) off += leaf_count(cnt, c.x);
-            cur = node;
-            node = parent_int[node];
-        }
-        range[k] = make_uint2(off, off + cnt[k] - 1u);
-    }
+    first[k] = off;
 }
 
-//! leaves to depth-first order: the triangle order and leaf child refs
-__global__ void k_ploc_permute(uint32_t ni, uint32_t n, const uint32_t *__restrict__ leaf_pos,
-                               const uint32_t *__restrict__ order_in, uint32_t *__restrict__ order_out,
-                               const int2 *__restrict__ child_in, int2 *__restrict__ child_out)
+//! the leaves in depth-first order: each node's range, its leaf children's positions and their triangles
+__global__ void __launch_bounds__(256) k_ploc_emit(ploc_tree tree, const uint32_t *__restrict__ first,
+                                                   const uint32_t *__restrict__ order_in, uint32_t *__restrict__ order_out,
+                                                   uint2 *__restrict__ range)
 {
-    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    if(k < n)
+    const uint32_t k = blockIdx.x * 256 + threadIdx.x;
+    if(k >= tree.ni) return;
+    const uint32_t f = first[k];
+    range[k] = make_uint2(f, f + tree.cnt[k] - 1u);
+    int2 c = tree.child[k];
+    const uint32_t right = f + leaf_count(tree.cnt, c.x);
+    if(c.x < 0)
     {
-        const uint32_t d = leaf_pos[k];
-        if(d >= n) return;// only a malformed tree gets here; its depth is rejected
-        order_out[d] = order_in[k];
+        order_out[f] = order_in[~c.x];
+        c.x = ~static_cast<int32_t>(f);
     }
-    if(k < ni)
+    if(c.y < 0)
     {
-        const int2 c = child_in[k];
-        auto map = [leaf_pos](int32_t r) { return r < 0 ? ~static_cast<int32_t>(leaf_pos[~r]) : r; };
-        child_out[k] = make_int2(map(c.x), map(c.y));
+        order_out[right] = order_in[~c.y];
+        c.y = ~static_cast<int32_t>(right);
     }
+    tree.child[k] = c;
 }
 
-__global__ void __launch_bounds__(1024) k_scan_local(const uint32_t *__restrict__ in, uint32_t n,
-                                                     uint32_t *__restrict__ out, uint32_t *__restrict__ block_sums)
-{
-    __shared__ uint32_t wsum[16];
-    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const uint32_t i = blockIdx.x * 1024 + threadIdx.x;
-    const uint32_t x = i < n ? in[i] : 0u;
-    uint32_t sc = x;
-    for(int off = 1; off < 64; off <<= 1)
-    {
-        const uint32_t y = __shfl_up(sc, off);
-        if(lane >= (uint32_t)off) sc += y;
-    }
-    if(lane == 63) wsum[wave] = sc;
-    __syncthreads();
-    if(threadIdx.x < 16)
-    {
-        const uint32_t w = wsum[threadIdx.x];
-        uint32_t acc = w;
-        for(int off = 1; off < 16; off <<= 1)
-        {
-            const uint32_t y = __shfl_up(acc, off, 16);
-            if(threadIdx.x >= (uint32_t)off) acc += y;
-        }
-        wsum[threadIdx.x] = acc - w;
-        if(threadIdx.x == 15) block_sums[blockIdx.x] = acc;
-    }
-    __syncthreads();
-    if(i < n) out[i] = wsum[wave] + sc - x;
-}
-
-//! exclusive scan of the per-block sums in one workgroup, 1024 at a time with a running carry
-__global__ void __launch_bounds__(1024) k_scan_blocks(uint32_t *__restrict__ data, uint32_t n)
-{
-    __shared__ uint32_t wsum[16];
-    __shared__ uint32_t carry;
-    if(threadIdx.x == 0) carry = 0;
-    __syncthreads();
-    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for(uint32_t base = 0; base < n; base += 1024)
-    {
-        const uint32_t i = base + threadIdx.x;
-        const uint32_t x = i < n ? data[i] : 0u;
-        uint32_t sc = x;
-        for(int off = 1; off < 64; off <<= 1)
-        {
-            const uint32_t y = __shfl_up(sc, off);
-            if(lane >= (uint32_t)off) sc += y;
-        }
-        if(lane == 63) wsum[wave] = sc;
-        __syncthreads();
-        if(threadIdx.x < 16)
-        {
-            const uint32_t w = wsum[threadIdx.x];
-            uint32_t acc = w;
-            for(int off = 1; off < 16; off <<= 1)
-            {
-                const uint32_t y = __shfl_up(acc, off, 16);
-                if(threadIdx.x >= (uint32_t)off) acc += y;
-            }
-            wsum[threadIdx.x] = acc - w;
-        }
-        __syncthreads();
-        const uint32_t c = carry;
-        if(i < n) data[i] = c + wsum[wave] + sc - x;
-        __syncthreads();
-        if(threadIdx.x == 1023) carry = c + wsum[wave] + sc;
-        __syncthreads();
-    }
-}
-
-__global__ void __launch_bounds__(1024) k_scan_add(const uint32_t *__restrict__ in, uint32_t n,
-                                                   uint32_t *__restrict__ out, const uint32_t *__restrict__ block_off,
-                                                   uint32_t *__restrict__ total)
-{
-    const uint32_t i = blockIdx.x * 1024 + threadIdx.x;
-    if(i >= n) return;
-    const uint32_t v = out[i] + block_off[blockIdx.x];
-    out[i] = v;
-    if(i == n - 1) *total = v + in[i];
-}
-
-//! exclusive prefix sum of n values; *total receives the sum. block_sums holds div_up(n, 1024) entries
-static void exclusive_scan(hipStream_t s, const uint32_t *in, uint32_t *out, uint32_t n, uint32_t *block_sums,
-                           uint32_t *total)
-{
-    const uint32_t nb = div_up(n, 1024);
-    k_scan_local<<<nb, 1024, 0, s>>>(in, n, out, block_sums);
-    k_scan_blocks<<<1, 1024, 0, s>>>(block_sums, nb);
-    k_scan_add<<<nb, 1024, 0, s>>>(in, n, out, block_sums, total);
-}
-
-static void build_topology_ploc(vkrt_ctx *ctx, vkrt_bvh *bvh)
+static void build_topology_ploc(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh, const uint32_t *sorted)
 {
     hipStream_t s = ctx->stream;
-    const uint32_t radius = bvh->ploc_radius ? bvh->ploc_radius : PLOC_RADIUS;
-    const uint32_t n = bvh->n_tri, ni = n - 1;
-    // working set: two cluster lists (ids, lo, hi), neighbours, flags and offsets, leaf counts, scan sums
+    const int radius = bvh->ploc_radius ? static_cast<int>(bvh->ploc_radius) : PLOC_RADIUS;
+    const uint32_t n = bvh->n_tri, ni = n - 1, tiles = div_up(n, ploc_tile(radius));
+    // working set: two cluster lists, what each cluster does, counts per tile, the tree's counts, parents and
+    // first leaves
     device_buffer &w = ctx->scratch[3];
-    const size_t nb = div_up(n, 1024);
-    const size_t bytes = (size_t)n * (2 * 4 + 4 * 16 + 4 + 4 * 4 + 4 + 4) + (size_t)ni * 8 + nb * 4 + 512;
+    const size_t bytes = (size_t)n * 65 + (size_t)tiles * 4 + (size_t)ni * 12 + 512;
     w.reserve(bytes);
     uint8_t *q = w.as<uint8_t>();
     auto take = [&q](size_t b) {
@@ -870,58 +1000,54 @@ static void build_topology_ploc(vkrt_ctx *ctx, vkrt_bvh *bvh)
         q += (b + 15) & ~size_t(15);
         return r;
     };
-    int32_t *id[2] = {reinterpret_cast<int32_t *>(take((size_t)n * 4)), reinterpret_cast<int32_t *>(take((size_t)n * 4))};
-    float4 *lo[2] = {reinterpret_cast<float4 *>(take((size_t)n * 16)), reinterpret_cast<float4 *>(take((size_t)n * 16))};
-    float4 *hi[2] = {reinterpret_cast<float4 *>(take((size_t)n * 16)), reinterpret_cast<float4 *>(take((size_t)n * 16))};
-    int32_t *nn = reinterpret_cast<int32_t *>(take((size_t)n * 4));
-    uint32_t *merge = reinterpret_cast<uint32_t *>(take((size_t)n * 4));
-    uint32_t *moff = reinterpret_cast<uint32_t *>(take((size_t)n * 4));
-    uint32_t *keep = reinterpret_cast<uint32_t *>(take((size_t)n * 4));
-    uint32_t *koff = reinterpret_cast<uint32_t *>(take((size_t)n * 4));
-    uint32_t *leaf_pos = reinterpret_cast<uint32_t *>(take((size_t)n * 4));
-    uint32_t *cnt = reinterpret_cast<uint32_t *>(take((size_t)ni * 4));
-    uint32_t *sums = reinterpret_cast<uint32_t *>(take(nb * 4));
-    uint32_t *totals = reinterpret_cast<uint32_t *>(take(16));
-    int32_t *parent_int = reinterpret_cast<int32_t *>(take((size_t)ni * 4));
-    int32_t *parent_leaf = reinterpret_cast<int32_t *>(take((size_t)n * 4));
+    ploc_lists l;
+    for(int k = 0; k < 2; ++k)
+    {
+        l.lo[k] = reinterpret_cast<float4 *>(take((size_t)n * 16));
+        l.hi[k] = reinterpret_cast<float4 *>(take((size_t)n * 16));
+    }
+    int8_t *code = reinterpret_cast<int8_t *>(take(n));
+    uint32_t *counts = reinterpret_cast<uint32_t *>(take((size_t)tiles * 4));
+    ploc_tree tree{bvh->child.as<int2>(), reinterpret_cast<uint32_t *>(take((size_t)ni * 4)),
+                   reinterpret_cast<int32_t *>(take((size_t)ni * 4)), ni};
+    uint32_t *first = reinterpret_cast<uint32_t *>(take((size_t)ni * 4));
     VKRT_REQUIRE(q <= w.as<uint8_t>() + bytes, "PLOC working set overrun");
 
-    int2 *child = bvh->child.as<int2>();
-    k_ploc_init<<<div_up(n, 256), 256, 0, s>>>(bvh->tbox.as<float>(), n, id[0], lo[0], hi[0], parent_int, ni);
-    uint32_t nc = n, base = 0;
-    int cur = 0;
-    uint32_t rounds = 0;
-    while(nc > 1)
+    bvh_state *st = ctx->state.as<bvh_state>();
+    k_ploc_init<<<div_up(n, 256), 256, 0, s>>>(mesh, sorted, l.lo[0], l.hi[0], st);
+    // rounds are launched without asking how many clusters are left: as many as a list that shrinks by a fifth each
+    // time needs (a round with too few clusters passes them on, 4 us), the tail, and eight more at a time while
+    // the tail finds too many
+    uint32_t round = 0, nc = n, todo = 0;
+    for(double k = n; k > PLOC_TAIL; k *= 0.82) ++todo;
+    while(true)
     {
-        VKRT_REQUIRE(++rounds <= n, "PLOC made no progress");
-        k_ploc_nn<<<div_up(nc, PLOC_BLOCK), PLOC_BLOCK, 0, s>>>(lo[cur], hi[cur], nc, static_cast<int>(radius), nn);
-        k_ploc_flags<<<div_up(nc, 256), 256, 0, s>>>(nn, nc, merge, keep);
-        exclusive_scan(s, merge, moff, nc, sums, totals);
-        exclusive_scan(s, keep, koff, nc, sums, totals + 1);
-        k_ploc_merge<<<div_up(nc, 256), 256, 0, s>>>(nn, nc, merge, moff, keep, koff, base, id[cur], lo[cur], hi[cur],
-                                                     id[cur ^ 1], lo[cur ^ 1], hi[cur ^ 1], child, cnt, parent_int,
-                                                     parent_leaf);
-        uint32_t t[2];
-        VKRT_HIP(hipMemcpyAsync(t, totals, 8, hipMemcpyDeviceToHost, s));
-        VKRT_HIP(hipStreamSynchronize(s));
-        VKRT_REQUIRE(t[0] >= 1 && t[1] == nc - t[0], "PLOC round inconsistent");
-        base += t[0];
-        nc = t[1];
-        cur ^= 1;
+        const uint32_t grid = div_up(nc, ploc_tile(radius));// (the list never grows)
+        for(uint32_t stop = round + todo; round < stop; ++round)
+        {
+            if(radius == PLOC_RADIUS)
+                k_ploc_nn<PLOC_RADIUS><<<grid, PLOC_BLOCK, 0, s>>>(st, round & 1u, radius, l, code, counts);
+            else
+                k_ploc_nn<0><<<grid, PLOC_BLOCK, 0, s>>>(st, round & 1u, radius, l, code, counts);
+            k_ploc_merge<<<grid, PLOC_BLOCK, 0, s>>>(st, round & 1u, radius, l, code, counts, tree);
+        }
+        k_ploc_tail<<<1, PLOC_TAIL, 0, s>>>(st, round & 1u, radius, l, tree);
+        const bvh_state &got = read_state(ctx, nullptr);
+        VKRT_REQUIRE(got.ploc_left >= 1 && got.ploc_left < nc, "PLOC made no progress");
+        nc = got.ploc_left;
+        if(nc == 1)
+        {
+            VKRT_REQUIRE(got.ploc_nodes == ni, "PLOC did not build n - 1 nodes");
+            break;
+        }
+        todo = 8;
     }
-    VKRT_REQUIRE(base == ni, "PLOC did not build n - 1 nodes");
-    // the cluster lists and flag arrays are free now: renumbered tree (root first), then depth-first leaf
-    // positions and ranges, then the permuted copies
-    int2 *child2 = reinterpret_cast<int2 *>(lo[0]);
-    uint32_t *cnt2 = merge;
-    int32_t *pint2 = reinterpret_cast<int32_t *>(moff);
-    int32_t *pleaf2 = reinterpret_cast<int32_t *>(keep);
-    k_ploc_renumber<<<div_up(n, 256), 256, 0, s>>>(ni, n, child, cnt, parent_int, parent_leaf, child2, cnt2, pint2,
-                                                   pleaf2);
-    k_ploc_dfs<<<div_up(n, 256), 256, 0, s>>>(ni, n, child2, cnt2, pint2, pleaf2, leaf_pos, bvh->range.as<uint2>());
-    uint32_t *order_in = koff;
-    VKRT_HIP(hipMemcpyAsync(order_in, bvh->order.ptr, (size_t)n * 4, hipMemcpyDeviceToDevice, s));
-    k_ploc_permute<<<div_up(n, 256), 256, 0, s>>>(ni, n, leaf_pos, order_in, bvh->order.as<uint32_t>(), child2, child);
+    for(uint32_t a = 0, b = 1024; a < ni; a = b, b *= 8)
+    {
+        const uint32_t stop = std::min(b, ni);
+        k_ploc_first<<<div_up(stop - a, 256), 256, 0, s>>>(a, stop, tree, first);
+    }
+    k_ploc_emit<<<div_up(ni, 256), 256, 0, s>>>(tree, first, sorted, bvh->order.as<uint32_t>(), bvh->range.as<uint2>());
     VKRT_HIP(hipGetLastError());
 }
 
@@ -932,7 +1058,7 @@ static void build_bounds(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh)
     hipStream_t s = ctx->stream;
     const uint32_t n = bvh->n_tri;
     bvh->tris.reserve((size_t)n * 3 * sizeof(float4));
-    k_leaves<true><<<div_up(n, 256), 256, 0, s>>>(mesh, bvh->order.as<uint32_t>(), bvh->tbox.as<float>(),
+    k_leaves<<<div_up(n, 256), 256, 0, s>>>(mesh, bvh->order.as<uint32_t>(), bvh->tbox.as<float>(),
                                                   bvh->tris.as<float4>());
     if(n >= 2)
     {
