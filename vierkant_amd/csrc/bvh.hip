@@ -323,19 +323,30 @@ __global__ void __launch_bounds__(BOX_SEG) k_box_scan(uint32_t n, const float *_
         store_box(seg + 6 * (size_t)blockIdx.x, b);// leaf 0's suffix: the segment
 }
 
-//! sparse-table level k from level k - 1: entry i = union of entries i and i + 2^(k-1), for i + 2^k <= nseg
-__global__ void k_box_sparse(uint32_t nseg, uint32_t k, float *__restrict__ table)
+//! sparse-table levels k .. k + 2 from level k - 1: entry i of level k + d is the union of 2^(d + 1) entries of level
+//! k - 1, 2^(k - 1) apart, while the last of them is inside (i + 2^(k + d) <= nseg). Three levels a launch: the
+//! table of 1.8M leaves has 15, and a launch each took 3 us of which the work was a fraction.
+constexpr uint32_t SPARSE_LEVELS = 3;
+__global__ void __launch_bounds__(256) k_box_sparse(uint32_t nseg, uint32_t k, uint32_t levels, float *__restrict__ table)
 {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t half = 1u << (k - 1);
-    if((size_t)i + 2 * half > nseg) return;
-    const float *lo = table + 6 * ((size_t)(k - 1) * nseg + i);
-    const float *hi = table + 6 * ((size_t)(k - 1) * nseg + i + half);
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    const uint32_t step = 1u << (k - 1);
+    if((size_t)i + 2 * step > nseg) return;
+    const float *from = table + 6 * ((size_t)(k - 1) * nseg + i);
     float a[6], b[6];
-    load_box(lo, a);
-    load_box(hi, b);
-    box_union(a, b);
-    store_box(table + 6 * ((size_t)k * nseg + i), a);
+    load_box(from, a);
+    uint32_t taken = 1;
+    for(uint32_t d = 0; d < SPARSE_LEVELS && k + d < levels; ++d)
+    {
+        const uint32_t want = 2u << d;
+        if((size_t)i + (size_t)want * step > nseg) return;
+        for(; taken < want; ++taken)
+        {
+            load_box(from + 6 * (size_t)taken * step, b);
+            box_union(a, b);
+        }
+        store_box(table + 6 * ((size_t)(k + d) * nseg + i), a);
+    }
 }
 
 //! the leaves' boxes and their unions, as k_layout reads them
@@ -1069,8 +1080,8 @@ static void build_bounds(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh)
         w.reserve(((size_t)2 * n + (size_t)levels * nseg) * 6 * sizeof(float));
         float *pre = w.as<float>(), *suf = pre + 6 * (size_t)n, *table = suf + 6 * (size_t)n;
         k_box_scan<<<nseg, BOX_SEG, 0, s>>>(n, bvh->tbox.as<float>(), pre, suf, table);
-        for(uint32_t k = 1; k < levels; ++k)
-            k_box_sparse<<<div_up(nseg, 256), 256, 0, s>>>(nseg, k, table);
+        for(uint32_t k = 1; k < levels; k += SPARSE_LEVELS)
+            k_box_sparse<<<div_up(nseg, 256), 256, 0, s>>>(nseg, k, levels, table);
         bvh->n_nodes = ni;
         bvh->nodes.reserve((size_t)ni * sizeof(vkrt_bvh_node));
         const leaf_unions l{bvh->tbox.as<float>(), pre, suf, table, n, nseg};
