@@ -26,6 +26,7 @@
 #include <cmath>
 #include <cstring>
 #include <memory>
+#include <utility>
 #include <vector>
 
 #include "context.hpp"
@@ -514,7 +515,7 @@ static void root_bounds(const vkrt_bvh_node &root, float rb[6], float bounds[6])
 
 //! a single leaf's bounds (at most 8 triangles): the union of its triangles' boxes (tbox, in leaf order), padded
 //! like every node box
-static void single_leaf_info(vkrt_bvh *bvh, hipStream_t s)
+static void single_leaf_info(vkrt_bvh *bvh, const float *tbox, hipStream_t s)
 {
     vkrt_bvh_info &info = bvh->info;
     info.depth = 1;
@@ -523,8 +524,7 @@ static void single_leaf_info(vkrt_bvh *bvh, hipStream_t s)
     if(bvh->empty) return;
     const uint32_t v = static_cast<uint32_t>(~bvh->root_ref), first = v >> 3, count = (v & 7u) + 1;
     std::vector<float> box(6 * (size_t)count);
-    VKRT_HIP(hipMemcpyAsync(box.data(), bvh->tbox.as<float>() + 6 * (size_t)first, box.size() * 4,
-                            hipMemcpyDeviceToHost, s));
+    VKRT_HIP(hipMemcpyAsync(box.data(), tbox + 6 * (size_t)first, box.size() * 4, hipMemcpyDeviceToHost, s));
     VKRT_HIP(hipStreamSynchronize(s));
     float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
     for(uint32_t k = 0; k < count; ++k)
@@ -546,7 +546,6 @@ static void build_topology(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh)
 {
     hipStream_t s = ctx->stream;
     const uint32_t n = bvh->n_tri;
-    bvh->tbox.reserve((size_t)n * 6 * sizeof(float));
     // scratch: centroid bounds, sort keys, sort temp
     device_buffer &tmp = ctx->scratch[2];
     const size_t key_bytes = (size_t)n * sizeof(uint32_t), partial_bytes = BOUNDS_PARTIALS * 6 * sizeof(float);
@@ -554,7 +553,6 @@ static void build_topology(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh)
     float *partial = tmp.as<float>();
     uint32_t *keys = reinterpret_cast<uint32_t *>(tmp.as<uint8_t>() + partial_bytes);
     void *sort_tmp = tmp.as<uint8_t>() + partial_bytes + 2 * key_bytes;
-    bvh->order.reserve(key_bytes);
     // PLOC puts the sorted triangles into an order of its own
     const bool ploc = bvh->builder == VKRT_BUILDER_PLOC && n >= 2;
     uint32_t *order = ploc ? keys + n : bvh->order.as<uint32_t>();
@@ -568,8 +566,6 @@ static void build_topology(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh)
     if(n >= 2)
     {
         const uint32_t ni = n - 1;
-        bvh->child.reserve(ni * sizeof(int2));
-        bvh->range.reserve(ni * sizeof(uint2));
         if(ploc) build_topology_ploc(ctx, bvh, mesh, order);
         else
             k_karras<<<div_up(ni, 256), 256, 0, s>>>(keys, (int)n, bvh->child.as<int2>(), bvh->range.as<uint2>());
@@ -1062,15 +1058,49 @@ static void build_topology_ploc(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &m
     VKRT_HIP(hipGetLastError());
 }
 
+//! the BVH's memory, all but the 4-wide nodes, whose number only the collapse tells
+static void allocate(vkrt_bvh *bvh)
+{
+    const size_t n = bvh->n_tri, ni = n - 1;
+    const std::pair<vkrt_bvh::part *, size_t> parts[vkrt_bvh::PARTS] = {
+            {&bvh->nodes, ni * sizeof(vkrt_bvh_node)}, {&bvh->tris, n * 3 * sizeof(float4)},
+            {&bvh->indices, n * 3 * sizeof(uint32_t)}, {&bvh->order, n * sizeof(uint32_t)},
+            {&bvh->child, ni * sizeof(int2)},          {&bvh->range, ni * sizeof(uint2)}};
+    size_t total = 0;
+    for(const auto &[p, bytes]: parts)
+    {
+        p->bytes = std::max<size_t>(bytes, 256);
+        total += (p->bytes + 255) & ~size_t(255);
+    }
+    // below about 2 MiB the runtime hands out parts of a block it keeps (1 us, against 70 us for allocating and
+    // freeing 4 MB), so the parts of a small BVH stay apart
+    const bool apart = bvh->nodes.bytes < (2u << 20);
+    if(!apart) bvh->memory[0].reserve(total);
+    uint8_t *at = bvh->memory[0].as<uint8_t>();
+    for(size_t k = 0; k < std::size(parts); ++k)
+    {
+        vkrt_bvh::part &p = *parts[k].first;
+        if(apart)
+        {
+            bvh->memory[k].reserve(p.bytes);
+            p.ptr = bvh->memory[k].ptr;
+            continue;
+        }
+        p.ptr = at;
+        at += (p.bytes + 255) & ~size_t(255);
+    }
+}
+
 //! the leaf records, the BVH2's nodes and the root, from the mesh and a topology: the last part of a build and the
 //! whole of a refit, which keeps the topology
 static void build_bounds(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh)
 {
     hipStream_t s = ctx->stream;
     const uint32_t n = bvh->n_tri;
-    bvh->tris.reserve((size_t)n * 3 * sizeof(float4));
-    k_leaves<<<div_up(n, 256), 256, 0, s>>>(mesh, bvh->order.as<uint32_t>(), bvh->tbox.as<float>(),
-                                                  bvh->tris.as<float4>());
+    // (the sort's scratch is done with; a single leaf's box is read back from here)
+    ctx->scratch[2].reserve((size_t)n * 6 * sizeof(float));
+    float *tbox = ctx->scratch[2].as<float>();
+    k_leaves<<<div_up(n, 256), 256, 0, s>>>(mesh, bvh->order.as<uint32_t>(), tbox, bvh->tris.as<float4>());
     if(n >= 2)
     {
         const uint32_t ni = n - 1;
@@ -1079,12 +1109,11 @@ static void build_bounds(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh)
         device_buffer &w = ctx->scratch[3];
         w.reserve(((size_t)2 * n + (size_t)levels * nseg) * 6 * sizeof(float));
         float *pre = w.as<float>(), *suf = pre + 6 * (size_t)n, *table = suf + 6 * (size_t)n;
-        k_box_scan<<<nseg, BOX_SEG, 0, s>>>(n, bvh->tbox.as<float>(), pre, suf, table);
+        k_box_scan<<<nseg, BOX_SEG, 0, s>>>(n, tbox, pre, suf, table);
         for(uint32_t k = 1; k < levels; k += SPARSE_LEVELS)
             k_box_sparse<<<div_up(nseg, 256), 256, 0, s>>>(nseg, k, levels, table);
         bvh->n_nodes = ni;
-        bvh->nodes.reserve((size_t)ni * sizeof(vkrt_bvh_node));
-        const leaf_unions l{bvh->tbox.as<float>(), pre, suf, table, n, nseg};
+        const leaf_unions l{tbox, pre, suf, table, n, nseg};
         k_layout<<<div_up(ni, 256), 256, 0, s>>>(l, bvh->child.as<int2>(), bvh->range.as<uint2>(), bvh->max_leaf,
                                                  bvh->nodes.as<vkrt_bvh_node>());
         bvh->root_ref = (n <= bvh->max_leaf) ? ~static_cast<int>(n - 1) : 0;
@@ -1365,7 +1394,7 @@ static void build_wide(vkrt_ctx *ctx, vkrt_bvh *bvh)
         check_indices(read_state(ctx, nullptr));
         bvh->root4 = bvh->root_ref;// a single leaf
         bvh->wide = bvh->allow_wide;
-        single_leaf_info(bvh, s);
+        single_leaf_info(bvh, ctx->scratch[2].as<float>(), s);
         return;
     }
     // (a 4-wide node takes in at least one node of the binary tree)
@@ -1473,7 +1502,7 @@ int vkrt_bvh_build(vkrt_ctx *ctx, const float *positions, uint32_t n_vert, uint3
             const size_t pos_bytes = (size_t)(n_vert - 1) * stride_bytes + 12;
             const uint8_t *dpos =
                     input(ctx, 0, reinterpret_cast<const uint8_t *>(positions), pos_bytes, flags);
-            bvh->indices.reserve((size_t)n_tri * 3 * sizeof(uint32_t));
+            allocate(bvh.get());
             const uint32_t *didx = input(ctx, 1, indices, (size_t)n_tri * 3, flags);
             VKRT_HIP(hipMemcpyAsync(bvh->indices.ptr, didx, (size_t)n_tri * 3 * sizeof(uint32_t),
                                     hipMemcpyDeviceToDevice, ctx->stream));
@@ -1483,7 +1512,7 @@ int vkrt_bvh_build(vkrt_ctx *ctx, const float *positions, uint32_t n_vert, uint3
             build_wide(ctx, bvh.get());
             VKRT_HIP(hipStreamSynchronize(ctx->stream));
         }
-        else single_leaf_info(bvh.get(), ctx->stream);
+        else single_leaf_info(bvh.get(), nullptr, ctx->stream);
         bvh->info.build_ms = std::chrono::duration<float, std::milli>(std::chrono::steady_clock::now() - t_start).count();
         refresh_info(bvh.get());
         *out = bvh.release();
@@ -1503,7 +1532,7 @@ int vkrt_bvh_refit(vkrt_ctx *ctx, vkrt_bvh *bvh, const float *positions, uint32_
         const uint8_t *dpos = input(ctx, 0, reinterpret_cast<const uint8_t *>(positions), pos_bytes, flags);
         build_bounds(ctx, bvh, mesh_view{dpos, bvh->indices.as<uint32_t>(), stride_bytes, bvh->n_tri, bvh->n_vert});
         refit_wide(ctx, bvh);
-        if(bvh->root_ref < 0) single_leaf_info(bvh, s);
+        if(bvh->root_ref < 0) single_leaf_info(bvh, ctx->scratch[2].as<float>(), s);
         else
         {
             // the topology stays, and with it depth, leaves and SAH cost: only the bounds change
