@@ -10,7 +10,7 @@
 //   k_pt_trace   per queued path: closest hit through the BVH, back faces culled while the path is in air
 //   k_pt_shade   per queued path: the bounce's RNG hash, miss (sky) or closest-hit shading (emission,
 //                sample_disney, throughput, media stack, Russian roulette); survivors are appended to the
-//                next queue with one wave ballot + one atomic per wave; finished paths add their radiance
+//                next queue with one atomic per workgroup; finished paths add their radiance
 //                to the pixel's sample sum
 //   k_pt_resolve per pixel: mean over the batch's samples, running mean over batches, pixel_data_t
 //
@@ -47,7 +47,15 @@ constexpr uint32_t VERTEX_F4 = 7;  // training vertex: 4 float4 of features + (e
 constexpr uint32_t SHADOW_F4 = 6;  // shadow record: ray o, d; (radiance, mis weight); (F, cos); (beta, pdf);
                                    // (pixel, training vertex, -, -)
 constexpr uint32_t NO_VERTEX = 0xffffffffu;
-constexpr uint32_t TRAIN_COUNTERS = 8;// offset of the training stream's counters
+// counters, each on a 128-B line of its own: updates of one line that every XCD writes take 11 ns each, one after
+// the other
+constexpr uint32_t COUNTER_LINE = 32;
+constexpr uint32_t C_QUEUE = 0;                     // the two queues' sizes
+constexpr uint32_t C_SEGMENTS = 2 * COUNTER_LINE;   // path segments (64-bit)
+constexpr uint32_t C_QUERIES = 3 * COUNTER_LINE;    // cache queries
+constexpr uint32_t C_RECORDS = 4 * COUNTER_LINE;    // training records
+constexpr uint32_t C_SHADOW = 5 * COUNTER_LINE;     // next-event shadow rays of a depth
+constexpr uint32_t TRAIN_COUNTERS = 6 * COUNTER_LINE;// offset of the training stream's counters
 constexpr int PT_BLOCK = 256;
 constexpr int PT_LDS = 16;
 // the closest-hit trace of the queued paths: the trace kernels' launch shape (64 lanes per workgroup; the
@@ -59,7 +67,7 @@ constexpr uint32_t PT_TRACE_CHUNK = 8;
 // kernel claiming tiles of PT_TRACE_BLOCK paths from per-XCD queues at counter + PT_CLAIMS and the shadow
 // kernel striding over its records; measured on the room scene (1920x1080, 64 spp, depth 8) it is slower,
 // 230 ms against 192 ms a frame: the hardware dispatcher hands out tiles faster than the claim atomics.
-constexpr uint32_t PT_CLAIMS = 64;            // word offset of the trace kernel's claim counters
+constexpr uint32_t PT_CLAIMS = 2 * TRAIN_COUNTERS;// word offset of the trace kernel's claim counters
 constexpr uint32_t PT_COUNTER_WORDS = PT_CLAIMS + CLAIM_COUNTERS;
 constexpr uint32_t PT_TRACE_WAVES_PER_SIMD = 6;// the trace kernel's register cap (amdgpu_waves_per_eu): 80 VGPRs
 // the filter-free trace kernel fits 64 VGPRs with no spill: 8 waves per SIMD instead of 7 (room, 64 spp at
@@ -160,15 +168,14 @@ struct pt_buffers
     float4 *acc;            // sum of the batch's sample radiance (rgb), coverage
     uint4 *info;            // first-hit depth bits, normal, object id, albedo
     uint32_t *queue[2];
-    uint32_t *counter;      // [0], [1]: queue sizes; [2..3]: segment count (64-bit); [4]: cache queries;
-                            // [5]: training records; [6]: shadow rays. Training paths of the cache mode run on
-                            // their own stream with the same layout at counter + TRAIN_COUNTERS
+    uint32_t *counter;      // counters (C_*); training paths of the cache mode run on their own stream with the
+                            // same layout at counter + TRAIN_COUNTERS
     uint32_t *train_queue;  // the training paths' first queue (cache mode)
     vkrt_pixel *pixels;
     float4 *qrec;           // cache queries (QUERY_F4 float4 each)
     float4 *tvtx;           // training paths' vertices [path][depth] (VERTEX_F4 float4 each)
     float4 *trec, *ttgt;    // training records (4 float4) and targets
-    float4 *shadow;         // next-event shadow rays of one depth (SHADOW_F4 float4 each), count in counter[6]
+    float4 *shadow;         // next-event shadow rays of one depth (SHADOW_F4 float4 each), count in C_SHADOW
     float2 *cone;           // ray cone per path: spread angle, width
     uint32_t *hit_inst;     // instanced scenes: the instance of each path's hit
 };
@@ -341,10 +348,10 @@ __global__ void __launch_bounds__(PT_BLOCK) k_pt_begin(pt_frame f, pt_buffers b,
     const uint32_t n_train = f.cache_on ? f.n_train_paths : 0u;
     if(p == 0)
     {
-        b.counter[0] = f.n_pix - n_train;
-        b.counter[4] = 0u;
-        b.counter[5] = 0u;
-        b.counter[TRAIN_COUNTERS] = n_train;
+        b.counter[C_QUEUE] = f.n_pix - n_train;
+        b.counter[C_QUERIES] = 0u;
+        b.counter[C_RECORDS] = 0u;
+        b.counter[TRAIN_COUNTERS + C_QUEUE] = n_train;
     }
     if(p >= f.n_pix) return;
     const uint32_t x = p % f.width, y = p / f.width;
@@ -409,7 +416,10 @@ __global__ void __launch_bounds__(PT_BLOCK) k_pt_begin(pt_frame f, pt_buffers b,
     }
 }
 
-__global__ void __launch_bounds__(PT_BLOCK) k_pt_zero(uint32_t *c) { c[threadIdx.x] = 0u; }
+__global__ void __launch_bounds__(PT_BLOCK) k_pt_zero(uint32_t *c, uint32_t n)
+{
+    for(uint32_t i = threadIdx.x; i < n; i += PT_BLOCK) c[i] = 0u;
+}
 
 //! before a depth: the next queue, the shadow-ray count and the trace kernel's claim counters start at zero
 //! (one thread per claim counter)
@@ -417,8 +427,8 @@ __global__ void k_pt_reset_depth(uint32_t *c, int next)
 {
     if(threadIdx.x == 0)
     {
-        c[next] = 0u;
-        c[6] = 0u;
+        c[C_QUEUE + next * COUNTER_LINE] = 0u;
+        c[C_SHADOW] = 0u;
     }
     c[PT_CLAIMS + threadIdx.x * COUNTER_STRIDE] = 0u;
 }
@@ -476,7 +486,7 @@ k_pt_trace(const vkrt_bvh_node *__restrict__ nodes, const float4 *__restrict__ t
            uint32_t depth, pt_tlas tl)
 {
     __shared__ int32_t smem[PT_LDS * PT_TRACE_BLOCK];
-    const uint32_t count = b.counter[in];
+    const uint32_t count = b.counter[C_QUEUE + in * COUNTER_LINE];
     const uint32_t tiles = (count + PT_TRACE_BLOCK - 1) / PT_TRACE_BLOCK;
     const uint32_t home = blockIdx.x % XCDS;
     uint32_t queue = 0;
@@ -954,79 +964,81 @@ __device__ __forceinline__ void shade_path(const pt_frame &f, const pt_buffers &
     }
 }
 
+//! the slots of a workgroup's flagged threads in a list whose size is *counter: a ballot per wave, the waves' counts
+//! in LDS, one atomic
+struct append_slots
+{
+    uint32_t wave_count[PT_BLOCK / 64], base;
+};
+
+__device__ __forceinline__ uint32_t append_slot(append_slots &sh, bool flag, uint32_t *counter)
+{
+    const uint64_t mask = __ballot(flag);
+    const uint32_t lane = __lane_id(), wave = threadIdx.x >> 6;
+    if(lane == 0) sh.wave_count[wave] = static_cast<uint32_t>(__popcll(mask));
+    __syncthreads();
+    if(threadIdx.x == 0)
+    {
+        uint32_t total = 0;
+        for(uint32_t w = 0; w < PT_BLOCK / 64; ++w) total += sh.wave_count[w];
+        if(total) sh.base = atomicAdd(counter, total);
+    }
+    __syncthreads();
+    uint32_t slot = sh.base + static_cast<uint32_t>(__popcll(mask & (lane == 0 ? 0ull : (~0ull >> (64 - lane)))));
+    for(uint32_t w = 0; w < wave; ++w) slot += sh.wave_count[w];
+    return slot;
+}
+
 //! queue entry q of a depth (inactive past the count): shade_path, then survivors, cache queries and shadow
-//! rays are appended with one ballot and one atomic per wave each
+//! rays are appended with one atomic per workgroup each. (With one per wave, and another for the segment count on
+//! the same line, a full-HD frame's 32,400 waves spent 600 us at the first depth, all of it in the atomics' queue.)
 template<bool LIGHTS, bool INST>
 __device__ __forceinline__ void shade_queue_entry(const pt_frame &f, const pt_buffers &b, const pt_scene_dev &s,
                                                   uint32_t depth, int in, uint32_t q, uint32_t count)
 {
-    const bool active = q < count;
+    __shared__ append_slots sh[3];
     bool alive = false;
     bool to_cache = false;
     bool need_shadow = false;
     float4 shadow_rec[SHADOW_F4];
     float4 qfeat[QUERY_F4];
     uint32_t p = 0;
-    if(active)
+    if(q < count)
     {
         p = b.queue[in][q];
         shade_path<LIGHTS, INST>(f, b, s, depth, p, alive, to_cache, need_shadow, shadow_rec, qfeat);
     }
-    // append survivors to the next queue: one ballot and one atomic per wave
-    const uint64_t mask = __ballot(alive);
-    const uint32_t lane = __lane_id();
-    const uint64_t n_active = __ballot(active);
-    uint32_t base = 0;
-    if(lane == 0)
+    if(q == 0) atomicAdd(reinterpret_cast<unsigned long long *>(&b.counter[C_SEGMENTS]), (unsigned long long)count);
+    const uint32_t next = append_slot(sh[0], alive, &b.counter[C_QUEUE + (in ^ 1) * COUNTER_LINE]);
+    if(alive) b.queue[in ^ 1][next] = p;
+    if(f.cache_on && depth == f.cache_depth)
     {
-        if(mask) base = atomicAdd(&b.counter[in ^ 1], static_cast<uint32_t>(__popcll(mask)));
-        if(n_active) atomicAdd(reinterpret_cast<unsigned long long *>(&b.counter[2]), (unsigned long long)__popcll(n_active));
-    }
-    base = __shfl(base, 0);
-    if(alive)
-    {
-        const uint64_t below = lane == 0 ? 0ull : (mask & (~0ull >> (64 - lane)));
-        b.queue[in ^ 1][base + __popcll(below)] = p;
-    }
-    // cache queries: one ballot and one atomic per wave
-    const uint64_t qmask = __ballot(to_cache);
-    if(qmask)
-    {
-        uint32_t qbase = 0;
-        if(lane == 0) qbase = atomicAdd(&b.counter[4], static_cast<uint32_t>(__popcll(qmask)));
-        qbase = __shfl(qbase, 0);
+        const uint32_t slot = append_slot(sh[1], to_cache, &b.counter[C_QUERIES]);
         if(to_cache)
         {
-            const uint64_t below = lane == 0 ? 0ull : (qmask & (~0ull >> (64 - lane)));
-            float4 *dst = b.qrec + (size_t)(qbase + __popcll(below)) * QUERY_F4;
+            float4 *dst = b.qrec + (size_t)slot * QUERY_F4;
             for(uint32_t k = 0; k < QUERY_F4; ++k) dst[k] = qfeat[k];
         }
     }
-    // next-event shadow rays: one ballot and one atomic per wave
-    const uint64_t smask = __ballot(need_shadow);
-    if(smask)
+    if(LIGHTS)
     {
-        uint32_t sbase = 0;
-        if(lane == 0) sbase = atomicAdd(&b.counter[6], static_cast<uint32_t>(__popcll(smask)));
-        sbase = __shfl(sbase, 0);
+        const uint32_t slot = append_slot(sh[2], need_shadow, &b.counter[C_SHADOW]);
         if(need_shadow)
         {
-            const uint64_t below = lane == 0 ? 0ull : (smask & (~0ull >> (64 - lane)));
-            float4 *dst = b.shadow + (size_t)(sbase + __popcll(below)) * SHADOW_F4;
+            float4 *dst = b.shadow + (size_t)slot * SHADOW_F4;
             for(uint32_t k = 0; k < SHADOW_F4; ++k) dst[k] = shadow_rec[k];
         }
     }
 }
 
-//! one depth of shading over a compacted queue; survivors, cache queries and shadow rays are appended with
-//! one ballot and one atomic per wave each
+//! one depth of shading over a compacted queue
 //! (one tile per workgroup over a grid that covers every pixel: a grid-striding loop here keeps more values
 //! live across iterations, 190 VGPRs against 161, and drops the kernel from 3 waves per SIMD to 2)
 template<bool LIGHTS, bool INST>
 __global__ void __launch_bounds__(PT_BLOCK) k_pt_shade(pt_frame f, pt_buffers b, pt_scene_dev s, uint32_t depth,
                                                        int in)
 {
-    const uint32_t count = b.counter[in];
+    const uint32_t count = b.counter[C_QUEUE + in * COUNTER_LINE];
     const uint32_t first = blockIdx.x * PT_BLOCK;
     if(first < count) shade_queue_entry<LIGHTS, INST>(f, b, s, depth, in, first + threadIdx.x, count);
 }
@@ -1049,7 +1061,7 @@ __global__ void __launch_bounds__(PT_BLOCK) k_pt_train_targets(pt_frame f, pt_bu
         const vec3 L{e.x + w.x * Lin.x, e.y + w.y * Lin.y, e.z + w.z * Lin.z};
         Lin = vec3{g.x + L.x, g.y + L.y, g.z + L.z};
         if(kind != 1u) continue;
-        const uint32_t k = atomicAdd(&b.counter[5], 1u);
+        const uint32_t k = atomicAdd(&b.counter[C_RECORDS], 1u);
         if(k >= f.train_max) continue;
         float4 *r = b.trec + (size_t)k * 4;
         r[0] = tv[d * VERTEX_F4 + 0];
@@ -1491,7 +1503,7 @@ __attribute__((amdgpu_waves_per_eu(INST || F::active ? 1 : PT_SHADOW_PLAIN_WAVES
                                                         pt_buffers b, F flt, pt_tlas tl)
 {
     __shared__ int32_t smem[PT_LDS * PT_BLOCK];
-    const uint32_t count = b.counter[6];
+    const uint32_t count = b.counter[C_SHADOW];
     for(uint32_t i = blockIdx.x * PT_BLOCK + threadIdx.x; i < count; i += gridDim.x * PT_BLOCK)
     {
         const float4 *rec = b.shadow + (size_t)i * SHADOW_F4;
@@ -1515,7 +1527,7 @@ __global__ void __launch_bounds__(PT_BLOCK) k_pt_train_paths(const vkrt_bvh_node
 {
     __shared__ int32_t smem[PT_LDS * PT_BLOCK];
     const uint32_t q = blockIdx.x * PT_BLOCK + threadIdx.x;
-    if(q >= b.counter[0]) return;
+    if(q >= b.counter[C_QUEUE]) return;
     const uint32_t p = b.queue[0][q];
     const alpha_filter flt{s.idx, s.uv, s.mats, s.tex, s.texels, f.disable_material != 0u};
     const alpha_filter shadow_flt{s.idx, s.uv, s.mats, s.tex, s.texels, false};
@@ -1534,7 +1546,7 @@ __global__ void __launch_bounds__(PT_BLOCK) k_pt_train_paths(const vkrt_bvh_node
                                             smem + threadIdx.x, shadow_flt, tl);
         if(!alive) break;
     }
-    atomicAdd(reinterpret_cast<unsigned long long *>(&b.counter[2]), (unsigned long long)segments);
+    atomicAdd(reinterpret_cast<unsigned long long *>(&b.counter[C_SEGMENTS]), (unsigned long long)segments);
 }
 
 //! the deep-bounce tail: the paths alive at depth d0 (queue `in`) finish in one lane each, trace, shade and
@@ -1555,7 +1567,7 @@ __global__ void __launch_bounds__(PT_BLOCK) k_pt_finish(const vkrt_bvh_node *__r
     if(threadIdx.x == 0) s_segments = 0ull;
     __syncthreads();
     const uint32_t q = blockIdx.x * PT_BLOCK + threadIdx.x;
-    const uint32_t count = b.counter[in];
+    const uint32_t count = b.counter[C_QUEUE + in * COUNTER_LINE];
     uint32_t segments = 0;
     if(q < count)
     {
@@ -1578,7 +1590,7 @@ __global__ void __launch_bounds__(PT_BLOCK) k_pt_finish(const vkrt_bvh_node *__r
     if(segments) atomicAdd(&s_segments, (unsigned long long)segments);
     __syncthreads();
     if(threadIdx.x == 0 && s_segments)
-        atomicAdd(reinterpret_cast<unsigned long long *>(&b.counter[2]), s_segments);
+        atomicAdd(reinterpret_cast<unsigned long long *>(&b.counter[C_SEGMENTS]), s_segments);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -2010,7 +2022,7 @@ static void trace_batch(vkrt_pt *pt, const vkrt_camera &cam, uint32_t seed)
         });
     };
     VKRT_HIP(hipEventRecord(pt->ev0, s));
-    k_pt_zero<<<1, 2 * TRAIN_COUNTERS, 0, s>>>(b.counter);
+    k_pt_zero<<<1, PT_BLOCK, 0, s>>>(b.counter, 2 * TRAIN_COUNTERS);
     for(uint32_t sample = 0; sample < f.num_samples; ++sample)
     {
         uint32_t main_depths = f.max_depth;
@@ -2051,7 +2063,7 @@ static void trace_batch(vkrt_pt *pt, const vkrt_camera &cam, uint32_t seed)
             if(f.train_max)
             {
                 k_pt_train_targets<<<tgrid, PT_BLOCK, 0, pt->train_stream>>>(f, b);
-                rc::train(pt->rc, b.trec, 4, b.ttgt, f.train_max, false, b.counter + 5, pt->train_stream);
+                rc::train(pt->rc, b.trec, 4, b.ttgt, f.train_max, false, b.counter + C_RECORDS, pt->train_stream);
             }
             VKRT_HIP(hipGetLastError());
             VKRT_HIP(hipEventRecord(pt->ev_join, pt->train_stream));
@@ -2076,15 +2088,15 @@ static void trace_batch(vkrt_pt *pt, const vkrt_camera &cam, uint32_t seed)
         if(f.cache_on)
         {
             if(fork) VKRT_HIP(hipStreamWaitEvent(s, pt->ev_join, 0));
-            rc::query(pt->rc, b.qrec, QUERY_F4, f.n_pix, nullptr, b.acc, b.counter + 4);
+            rc::query(pt->rc, b.qrec, QUERY_F4, f.n_pix, nullptr, b.acc, b.counter + C_QUERIES);
         }
     }
     k_pt_resolve<<<blocks, PT_BLOCK, 0, s>>>(f, b);
     VKRT_HIP(hipEventRecord(pt->ev1, s));
     VKRT_HIP(hipGetLastError());
     uint64_t seg[2] = {0, 0};
-    VKRT_HIP(hipMemcpyAsync(&seg[0], b.counter + 2, 8, hipMemcpyDeviceToHost, s));
-    VKRT_HIP(hipMemcpyAsync(&seg[1], b.counter + TRAIN_COUNTERS + 2, 8, hipMemcpyDeviceToHost, s));
+    VKRT_HIP(hipMemcpyAsync(&seg[0], b.counter + C_SEGMENTS, 8, hipMemcpyDeviceToHost, s));
+    VKRT_HIP(hipMemcpyAsync(&seg[1], b.counter + TRAIN_COUNTERS + C_SEGMENTS, 8, hipMemcpyDeviceToHost, s));
     VKRT_HIP(hipStreamSynchronize(s));
     float ms = 0.f;
     VKRT_HIP(hipEventElapsedTime(&ms, pt->ev0, pt->ev1));
