@@ -269,7 +269,7 @@ int vkrt_batch_create(vkrt_ctx *ctx, const vkrt_batch_item *items, uint32_t n_it
             d.empty = it.bvh->empty ? 1u : 0u;
             d.n_rays = it.n_rays;
             d.root4 = it.bvh->root4;
-            d.wide = it.bvh->wide ? 1u : 0u;
+            d.wide = it.bvh->wide && it.bvh->joint ? 1u : 0u;
             b->items.push_back(d);
             b->n_rays.push_back(it.n_rays);
             b->total_rays += it.n_rays;

@@ -10,7 +10,7 @@
 //   radix sort  (code, triangle) pairs, project-written (radix_sort.hip)
 //   k_karras    binary radix tree over the sorted codes (Karras 2012), ties broken by position; or, with
 //               VKRT_BUILDER_PLOC, agglomerative clustering over the sorted leaves (k_ploc_*)
-//   k_leaves    triangles in leaf order, straight from the mesh: exact AABBs and 48-B records (v0, e1, e2,
+//   k_leaves    triangles in leaf order, straight from the mesh: exact AABBs and 64-B records (v0, e1, e2,
 //               original index)
 //   k_box_*     unions of leaf boxes (segment prefix/suffix unions and a sparse table of segment unions)
 //   k_layout    BVH2 nodes holding both children's boxes (64 B), each the union over its leaf run; subtrees of
@@ -242,8 +242,9 @@ __device__ __forceinline__ void store_box(float *p, const float b[6])
     for(int a = 0; a < 3; ++a) q[a] = make_float2(b[2 * a], b[2 * a + 1]);
 }
 
-//! the triangles in leaf order, straight from the mesh: their boxes and the 48-B leaf records (v0, e1, e2, original
-//! index; the last two words are cleared)
+//! the triangles in leaf order, straight from the mesh: their boxes (BOXES) and leaf records (RECORDS; the material
+//! and flags are cleared)
+template<bool BOXES, bool RECORDS>
 __global__ void __launch_bounds__(256) k_leaves(mesh_view m, const uint32_t *__restrict__ order,
                                                 float *__restrict__ tbox, float4 *__restrict__ tris)
 {
@@ -252,14 +253,22 @@ __global__ void __launch_bounds__(256) k_leaves(mesh_view m, const uint32_t *__r
     const uint32_t src = min(order[j], m.n_tri - 1u);// (a malformed tree, rejected for its depth, leaves gaps)
     vec3 v0, v1, v2;
     bool ok;
-    float b[6];
     load_triangle(m, src, v0, v1, v2, ok);
-    triangle_box(v0, v1, v2, b);
-    store_box(tbox + 6 * (size_t)j, b);
-    const vec3 e1 = v1 - v0, e2 = v2 - v0;
-    tris[3 * (size_t)j + 0] = make_float4(v0.x, v0.y, v0.z, e1.x);
-    tris[3 * (size_t)j + 1] = make_float4(e1.y, e1.z, e2.x, e2.y);
-    tris[3 * (size_t)j + 2] = make_float4(e2.z, __uint_as_float(src), 0.f, 0.f);
+    if constexpr(BOXES)
+    {
+        float b[6];
+        triangle_box(v0, v1, v2, b);
+        store_box(tbox + 6 * (size_t)j, b);
+    }
+    if constexpr(RECORDS)
+    {
+        const vec3 e1 = v1 - v0, e2 = v2 - v0;
+        float4 *t = tris + (TRI_BYTES / 16) * (size_t)j;
+        t[0] = make_float4(v0.x, v0.y, v0.z, e1.x);
+        t[1] = make_float4(e1.y, e1.z, e2.x, e2.y);
+        t[2] = make_float4(e2.z, __uint_as_float(src), 0.f, 0.f);
+        t[3] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
 }
 
 //! Node boxes without a bottom-up hand-off. Every internal node covers a contiguous run [first, last] of the
@@ -1058,14 +1067,14 @@ static void build_topology_ploc(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &m
     VKRT_HIP(hipGetLastError());
 }
 
-//! the BVH's memory, all but the 4-wide nodes, whose number only the collapse tells
+//! the BVH's memory, all but what traversal walks (the 4-wide nodes' number only the collapse tells)
 static void allocate(vkrt_bvh *bvh)
 {
     const size_t n = bvh->n_tri, ni = n - 1;
     const std::pair<vkrt_bvh::part *, size_t> parts[vkrt_bvh::PARTS] = {
-            {&bvh->nodes, ni * sizeof(vkrt_bvh_node)}, {&bvh->tris, n * 3 * sizeof(float4)},
-            {&bvh->indices, n * 3 * sizeof(uint32_t)}, {&bvh->order, n * sizeof(uint32_t)},
-            {&bvh->child, ni * sizeof(int2)},          {&bvh->range, ni * sizeof(uint2)}};
+            {&bvh->nodes, ni * sizeof(vkrt_bvh_node)}, {&bvh->indices, n * 3 * sizeof(uint32_t)},
+            {&bvh->order, n * sizeof(uint32_t)},       {&bvh->child, ni * sizeof(int2)},
+            {&bvh->range, ni * sizeof(uint2)}};
     size_t total = 0;
     for(const auto &[p, bytes]: parts)
     {
@@ -1091,8 +1100,9 @@ static void allocate(vkrt_bvh *bvh)
     }
 }
 
-//! the leaf records, the BVH2's nodes and the root, from the mesh and a topology: the last part of a build and the
-//! whole of a refit, which keeps the topology
+//! the BVH2's nodes and the root from the mesh and a topology; with RECORDS (a refit, which keeps the topology)
+//! the leaf records as well
+template<bool RECORDS>
 static void build_bounds(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh)
 {
     hipStream_t s = ctx->stream;
@@ -1100,7 +1110,8 @@ static void build_bounds(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh)
     // (the sort's scratch is done with; a single leaf's box is read back from here)
     ctx->scratch[2].reserve((size_t)n * 6 * sizeof(float));
     float *tbox = ctx->scratch[2].as<float>();
-    k_leaves<<<div_up(n, 256), 256, 0, s>>>(mesh, bvh->order.as<uint32_t>(), tbox, bvh->tris.as<float4>());
+    k_leaves<true, RECORDS><<<div_up(n, 256), 256, 0, s>>>(mesh, bvh->order.as<uint32_t>(), tbox,
+                                                           bvh->tris.as<float4>());
     if(n >= 2)
     {
         const uint32_t ni = n - 1;
@@ -1378,9 +1389,27 @@ static void refit_wide(vkrt_ctx *ctx, vkrt_bvh *bvh)
     VKRT_HIP(hipGetLastError());
 }
 
+//! what traversal walks: room for the 4-wide nodes and, after them, the leaf records, written from the mesh
+static void build_walk(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh)
+{
+    const size_t node_bytes = (size_t)bvh->n_nodes4 * sizeof(vkrt_bvh4_node);
+    const size_t tri_bytes = (size_t)bvh->n_tri * TRI_BYTES;
+    // (a step at the last leaf reads one record past it)
+    const size_t total = node_bytes + tri_bytes + TRI_BYTES;
+    bvh->walk.reserve(total);
+    bvh->nodes4.ptr = bvh->walk.ptr;
+    bvh->nodes4.bytes = node_bytes;
+    bvh->tris.ptr = bvh->walk.as<uint8_t>() + node_bytes;
+    bvh->tris.bytes = tri_bytes;
+    bvh->joint = total <= 0xffffffffull;
+    k_leaves<false, true><<<div_up(bvh->n_tri, 256), 256, 0, ctx->stream>>>(mesh, bvh->order.as<uint32_t>(), nullptr,
+                                                                            bvh->tris.as<float4>());
+    VKRT_HIP(hipGetLastError());
+}
+
 //! the end of a build: the BVH2 collapsed into the BVH4 used for traversal (kept off when its worst-case stack
 //! depth exceeds STACK_SIZE), the tree's statistics, and what the kernels before found wrong
-static void build_wide(vkrt_ctx *ctx, vkrt_bvh *bvh)
+static void build_wide(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh)
 {
     hipStream_t s = ctx->stream;
     bvh->wide = false;
@@ -1392,6 +1421,7 @@ static void build_wide(vkrt_ctx *ctx, vkrt_bvh *bvh)
     if(bvh->root_ref < 0)
     {
         check_indices(read_state(ctx, nullptr));
+        build_walk(ctx, bvh, mesh);
         bvh->root4 = bvh->root_ref;// a single leaf
         bvh->wide = bvh->allow_wide;
         single_leaf_info(bvh, ctx->scratch[2].as<float>(), s);
@@ -1442,16 +1472,16 @@ static void build_wide(vkrt_ctx *ctx, vkrt_bvh *bvh)
     info.depth = std::max(1u, got->depth);
     info.sah_cost = static_cast<float>(1.0 + got->sah / root_area);// 1: the root's own visit
     info.n_leaves = got->leaves;
+    const uint32_t stack4 = got->stack;
+    if(bvh->allow_wide) bvh->n_nodes4 = static_cast<uint32_t>(total);
+    build_walk(ctx, bvh, mesh);
     if(!bvh->allow_wide) return;
-    bvh->n_nodes4 = static_cast<uint32_t>(total);
-    bvh->stack4 = got->stack;
+    bvh->stack4 = stack4;
     bvh->root4 = 0;
     // the nodes move from the scratch, sized for the most there could be, into an array of their number
-    const size_t bytes = (size_t)bvh->n_nodes4 * sizeof(vkrt_bvh4_node);
-    bvh->nodes4.reserve(bytes);
-    VKRT_HIP(hipMemcpyAsync(bvh->nodes4.ptr, n4, bytes, hipMemcpyDeviceToDevice, s));
+    VKRT_HIP(hipMemcpyAsync(bvh->nodes4.ptr, n4, bvh->nodes4.bytes, hipMemcpyDeviceToDevice, s));
     // the 4-wide walk addresses nodes with 32-bit byte offsets (node4_intervals)
-    bvh->wide = bvh->stack4 <= (uint32_t)STACK_SIZE && (uint64_t)bytes <= 0xffffffffull;
+    bvh->wide = bvh->stack4 <= (uint32_t)STACK_SIZE && (uint64_t)bvh->nodes4.bytes <= 0xffffffffull;
 }
 
 //! the rest of the info block after a build or a refit
@@ -1508,8 +1538,8 @@ int vkrt_bvh_build(vkrt_ctx *ctx, const float *positions, uint32_t n_vert, uint3
                                     hipMemcpyDeviceToDevice, ctx->stream));
             const mesh_view mesh{dpos, bvh->indices.as<uint32_t>(), stride_bytes, n_tri, n_vert};
             build_topology(ctx, bvh.get(), mesh);
-            build_bounds(ctx, bvh.get(), mesh);
-            build_wide(ctx, bvh.get());
+            build_bounds<false>(ctx, bvh.get(), mesh);
+            build_wide(ctx, bvh.get(), mesh);
             VKRT_HIP(hipStreamSynchronize(ctx->stream));
         }
         else single_leaf_info(bvh.get(), nullptr, ctx->stream);
@@ -1530,7 +1560,7 @@ int vkrt_bvh_refit(vkrt_ctx *ctx, vkrt_bvh *bvh, const float *positions, uint32_
         hipStream_t s = ctx->stream;
         const size_t pos_bytes = (size_t)(bvh->n_vert - 1) * stride_bytes + 12;
         const uint8_t *dpos = input(ctx, 0, reinterpret_cast<const uint8_t *>(positions), pos_bytes, flags);
-        build_bounds(ctx, bvh, mesh_view{dpos, bvh->indices.as<uint32_t>(), stride_bytes, bvh->n_tri, bvh->n_vert});
+        build_bounds<true>(ctx, bvh, mesh_view{dpos, bvh->indices.as<uint32_t>(), stride_bytes, bvh->n_tri, bvh->n_vert});
         refit_wide(ctx, bvh);
         if(bvh->root_ref < 0) single_leaf_info(bvh, ctx->scratch[2].as<float>(), s);
         else
@@ -1568,7 +1598,7 @@ int vkrt_bvh_validate(vkrt_ctx *ctx, const vkrt_bvh *bvh, const float *positions
         std::vector<uint8_t> h_nodes, h_nodes4, h_tris, h_idx, h_pos;
         fetch(bvh->nodes.ptr, (size_t)bvh->n_nodes * sizeof(vkrt_bvh_node), true, h_nodes);
         if(bvh->wide) fetch(bvh->nodes4.ptr, (size_t)bvh->n_nodes4 * sizeof(vkrt_bvh4_node), true, h_nodes4);
-        fetch(bvh->tris.ptr, (size_t)n * 3 * sizeof(float4), true, h_tris);
+        fetch(bvh->tris.ptr, (size_t)n * TRI_BYTES, true, h_tris);
         fetch(bvh->indices.ptr, (size_t)n * 3 * sizeof(uint32_t), true, h_idx);
         fetch(positions, (size_t)(bvh->n_vert - 1) * stride_bytes + 12, (flags & VKRT_DEVICE_PTRS) != 0, h_pos);
         VKRT_HIP(hipStreamSynchronize(s));
@@ -1604,7 +1634,7 @@ int vkrt_bvh_validate(vkrt_ctx *ctx, const vkrt_bvh *bvh, const float *positions
             {
                 ++out->tris_reached;
                 uint32_t orig;
-                std::memcpy(&orig, &tris[3 * (size_t)k + 2].y, 4);
+                std::memcpy(&orig, &tris[(TRI_BYTES / 16) * (size_t)k + 2].y, 4);
                 if(orig >= n)
                 {
                     ++out->bad_refs;

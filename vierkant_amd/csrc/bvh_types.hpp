@@ -46,11 +46,15 @@ struct vkrt_bvh
     bool empty = true;
     // one allocation holds everything whose size the triangle count gives: freeing a large one takes 250 to 500 us
     // (eight of them, 1.7 of the 4.1 ms that a 1.8M-triangle build and its destruction took)
-    static constexpr int PARTS = 6;
+    static constexpr int PARTS = 5;
     vkrt::device_buffer memory[PARTS];// (or one each, for a small BVH)
-    part nodes, tris;
-    // the 4-wide collapse used by traversal when its worst-case stack fits (wide == true)
-    vkrt::device_buffer nodes4;
+    part nodes;
+    // the 4-wide collapse, used by traversal when its worst-case stack fits (wide == true), and after it the leaf
+    // records: one allocation, so that a walk reaches both with 32-bit offsets from one base (joint == true unless
+    // it passes 4 GiB)
+    vkrt::device_buffer walk;
+    part nodes4, tris;
+    bool joint = true;
     int32_t root4 = 0;
     uint32_t n_nodes4 = 0, stack4 = 0;
     bool wide = false, allow_wide = true;
@@ -68,6 +72,9 @@ constexpr float BOX_PAD = 0x1p-16f; // relative growth of every stored box coord
 constexpr float T_PAD = 0x1p-16f;   // relative growth of every slab interval
 constexpr uint32_t TRI_TWO_SIDED = 1u;// flag bit in a leaf triangle record: never culled as a back face
 constexpr uint32_t TRI_ALPHA_MASK = 2u;// flag bit: the record's material is alpha-masked (any-hit test)
+//! a leaf record: v0, e1, e2 (nine floats), original triangle index, material, flags, and a gap of 16 B. At 64 B two
+//! records lie like the seven 16-B words of a 4-wide node (see fetch7), and none crosses a 64-B line
+constexpr uint32_t TRI_BYTES = 64;
 constexpr int32_t EMPTY_CHILD = 0x7fffffff;// unused BVH4 child slot (no node index reaches it)
 
 }// namespace vkrt

@@ -1182,7 +1182,7 @@ __device__ float4 transmittance_walk(const vkrt_bvh_node *__restrict__ nodes2, i
                 leaf_decode(ref, first, count);
                 for(uint32_t k = 0; k < count; ++k)
                 {
-                    const float4 *tr = tris + 3 * (size_t)(first + k);
+                    const float4 *tr = tris + (TRI_BYTES / 16) * (size_t)(first + k);
                     const float4 p0 = tr[0], p1 = tr[1], p2 = tr[2];
                     const bool two_sided = (__float_as_uint(p2.w) & TRI_TWO_SIDED) != 0u;
                     float t, u, v;
@@ -1340,7 +1340,7 @@ __device__ float4 transmittance_walk_scene(const pt_tlas &tl, const gpu_material
                 leaf_decode(ref, first, count);
                 for(uint32_t k = 0; k < count; ++k)
                 {
-                    const size_t tb = 48 * (size_t)(first + k);
+                    const size_t tb = (size_t)TRI_BYTES * (first + k);
                     const float4 p0 = load_global_f4(tris, tb), p1 = load_global_f4(tris, tb + 16),
                                  p2 = load_global_f4(tris, tb + 32);
                     const bool two_sided = (__float_as_uint(p2.w) & TRI_TWO_SIDED) != 0u;
@@ -1676,14 +1676,14 @@ __global__ void k_pt_tag(float4 *__restrict__ tris, uint32_t n, const uint32_t *
 {
     const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
     if(j >= n) return;
-    float4 r = tris[3 * (size_t)j + 2];
+    float4 r = tris[(TRI_BYTES / 16) * (size_t)j + 2];
     const uint32_t prim = __float_as_uint(r.y) + prim_offset;
     r.y = __uint_as_float(prim);
     const uint32_t mat = object_material[tri_object[prim]];
     r.z = __uint_as_float(mat);
     r.w = __uint_as_float((mats[mat].sheen.w != 0.f ? TRI_TWO_SIDED : 0u) |
                           (mats[mat].tex.y != VKRT_ALPHA_OPAQUE ? TRI_ALPHA_MASK : 0u));
-    tris[3 * (size_t)j + 2] = r;
+    tris[(TRI_BYTES / 16) * (size_t)j + 2] = r;
 }
 
 }// namespace vkrt
@@ -1969,7 +1969,7 @@ static void trace_batch(vkrt_pt *pt, const vkrt_camera &cam, uint32_t seed)
     const vkrt_bvh4_node *nodes4 = bvh ? bvh->nodes4.as<vkrt_bvh4_node>() : nullptr;
     const float4 *tris = bvh ? bvh->tris.as<float4>() : nullptr;
     const int32_t root_ref = bvh ? bvh->root_ref : 0, root4 = bvh ? bvh->root4 : 0;
-    const bool flat_empty = bvh ? bvh->empty : true, wide = bvh ? bvh->wide : false;
+    const bool flat_empty = bvh ? bvh->empty : true, wide = bvh && bvh->wide && bvh->joint;
     // one depth of a queue of paths: trace, shade, and the shadow rays of next-event estimation
     // scenes with no alpha-tested material take the trace and shadow kernels without the any-hit filter
     const bool alpha = pt->any_alpha;
@@ -2559,7 +2559,7 @@ int vkrt_pt_trace_transmittance(vkrt_pt *pt, const vkrt_ray *rays, uint32_t n, f
         {
             const vkrt_bvh *b = pt->bvh;
             k_pt_transmittance<false><<<div_up(n, PT_BLOCK), PT_BLOCK, 0, ctx->stream>>>(
-                    b->nodes.as<vkrt_bvh_node>(), b->root_ref, b->nodes4.as<vkrt_bvh4_node>(), b->root4, b->wide,
+                    b->nodes.as<vkrt_bvh_node>(), b->root_ref, b->nodes4.as<vkrt_bvh4_node>(), b->root4, b->wide && b->joint,
                     b->empty, b->tris.as<float4>(), pt->mats.as<gpu_material>(), r4, n, cull, dout, flt, pt->tlas);
         }
         VKRT_HIP(hipGetLastError());

@@ -55,7 +55,7 @@ __device__ __forceinline__ bool mesh_leaf(const float4 *__restrict__ tris, int32
     bool found = false;
     for(uint32_t k = 0; k < count; ++k)
     {
-        const size_t tb = 48 * (size_t)(first + k);
+        const size_t tb = (size_t)TRI_BYTES * (first + k);
         const float4 p0 = load_global_f4(tris, tb), p1 = load_global_f4(tris, tb + 16),
                      p2 = load_global_f4(tris, tb + 32);
         float t, u, v;

@@ -56,7 +56,8 @@ template<bool ANY, int BLOCK>
 static void launch_block(vkrt_ctx *ctx, const vkrt_trace_config &cfg, const vkrt_bvh *bvh, const float4 *rays,
                          uint32_t n, void *out)
 {
-    const bool p = cfg.traversal == VKRT_TRAVERSAL_POSTPONED;
+    // (the step loop reaches nodes and records from one base with 32-bit offsets; the other loop has one for each)
+    const bool p = cfg.traversal == VKRT_TRAVERSAL_POSTPONED || !bvh->joint;
     const uint32_t x = cfg.xcd_chunk;
     hipStream_t s = ctx->stream;
     switch(cfg.lds_stack_depth)
