@@ -37,3 +37,27 @@ def test_build_and_refit_at_tile_edges(ctx, builder, n_tri):
             assert_hits_equal(ctx.trace_closest(bvh, rays), ctx.brute_closest(W.flat_triangles(p, idx), rays),
                               f"{n_tri} triangles, leaf {leaf}, width {width}")
         bvh.close()
+
+
+@pytest.mark.parametrize("builder", [vk.BUILDER_LBVH, vk.BUILDER_PLOC])
+@pytest.mark.parametrize("segments", [8, 64, 128])
+def test_more_wide_nodes_than_expected(ctx, builder, segments):
+    """a regular grid with one triangle a leaf has two 4-wide nodes per three triangles, more than a build makes room
+    for at first: the collapse is done again, and the tree is as good as any"""
+    pos, idx = vk.plane(4.0, 4.0, segments, segments)
+    rng = np.random.default_rng(segments)
+    o = rng.uniform(-2, 2, (1000, 3)).astype(np.float32)
+    o[:, 1] = 2.0
+    d = W.glm_normalize(np.column_stack([rng.uniform(-.5, .5, 1000), -np.ones(1000), rng.uniform(-.5, .5, 1000)])
+                        .astype(np.float32))
+    rays = W.make_rays(o, d)
+    bvh = ctx.bvh_build(pos, idx, builder=builder, max_leaf_size=1)
+    info = bvh.info()
+    assert info.n_wide_nodes > 0.6 * info.n_tri and info.n_leaves == info.n_tri
+    for lift in (0.0, 0.5):
+        p = pos + np.float32([0.0, lift, 0.0]) * np.sin(pos[:, :1])
+        if lift:
+            bvh.refit(p)
+        assert bvh.validate(p)["ok"]
+        assert_hits_equal(ctx.trace_closest(bvh, rays), ctx.brute_closest(W.flat_triangles(p, idx), rays), f"{lift}")
+    bvh.close()

@@ -25,6 +25,7 @@
 #include <chrono>
 #include <cmath>
 #include <cstring>
+#include <initializer_list>
 #include <memory>
 #include <utility>
 #include <vector>
@@ -242,9 +243,9 @@ __device__ __forceinline__ void store_box(float *p, const float b[6])
     for(int a = 0; a < 3; ++a) q[a] = make_float2(b[2 * a], b[2 * a + 1]);
 }
 
-//! the triangles in leaf order, straight from the mesh: their boxes (BOXES) and leaf records (RECORDS; the material
-//! and flags are cleared)
-template<bool BOXES, bool RECORDS>
+//! the triangles in leaf order, straight from the mesh: their leaf records (material and flags cleared) and, with
+//! BOXES, their boxes
+template<bool BOXES>
 __global__ void __launch_bounds__(256) k_leaves(mesh_view m, const uint32_t *__restrict__ order,
                                                 float *__restrict__ tbox, float4 *__restrict__ tris)
 {
@@ -260,15 +261,12 @@ __global__ void __launch_bounds__(256) k_leaves(mesh_view m, const uint32_t *__r
         triangle_box(v0, v1, v2, b);
         store_box(tbox + 6 * (size_t)j, b);
     }
-    if constexpr(RECORDS)
-    {
-        const vec3 e1 = v1 - v0, e2 = v2 - v0;
-        float4 *t = tris + (TRI_BYTES / 16) * (size_t)j;
-        t[0] = make_float4(v0.x, v0.y, v0.z, e1.x);
-        t[1] = make_float4(e1.y, e1.z, e2.x, e2.y);
-        t[2] = make_float4(e2.z, __uint_as_float(src), 0.f, 0.f);
-        t[3] = make_float4(0.f, 0.f, 0.f, 0.f);
-    }
+    const vec3 e1 = v1 - v0, e2 = v2 - v0;
+    float4 *t = tris + (TRI_BYTES / 16) * (size_t)j;
+    t[0] = make_float4(v0.x, v0.y, v0.z, e1.x);
+    t[1] = make_float4(e1.y, e1.z, e2.x, e2.y);
+    t[2] = make_float4(e2.z, __uint_as_float(src), 0.f, 0.f);
+    t[3] = make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
 //! Node boxes without a bottom-up hand-off. Every internal node covers a contiguous run [first, last] of the
@@ -480,7 +478,8 @@ struct bvh_state
     uint32_t level[MAX_LEVELS + 2];// 4-wide nodes per level
     ploc_round ploc[2];            // the clusters before an even and an odd round
     uint32_t ploc_left, ploc_nodes;// clusters left and nodes made after the last tail
-    vkrt_bvh_node root;
+    vkrt_bvh_node root;  // of the binary tree, where one is given
+    vkrt_bvh4_node root4;// of the 4-wide tree
 };
 
 __global__ void __launch_bounds__(256) k_state_clear(bvh_state *__restrict__ st)
@@ -490,36 +489,25 @@ __global__ void __launch_bounds__(256) k_state_clear(bvh_state *__restrict__ st)
 }
 
 __global__ void __launch_bounds__(256) k_report(const bvh_state *__restrict__ st, const vkrt_bvh_node *__restrict__ nodes,
-                                                bvh_state *__restrict__ host)
+                                                const vkrt_bvh4_node *__restrict__ nodes4, bvh_state *__restrict__ host)
 {
     const uint32_t *src = reinterpret_cast<const uint32_t *>(st);
     uint32_t *dst = reinterpret_cast<uint32_t *>(host);
     for(uint32_t i = threadIdx.x; i < offsetof(bvh_state, root) / 4; i += 256) dst[i] = src[i];
     if(nodes && threadIdx.x < sizeof(vkrt_bvh_node) / 4)
         dst[offsetof(bvh_state, root) / 4 + threadIdx.x] = reinterpret_cast<const uint32_t *>(nodes)[threadIdx.x];
+    if(nodes4 && threadIdx.x < sizeof(vkrt_bvh4_node) / 4)
+        dst[offsetof(bvh_state, root4) / 4 + threadIdx.x] = reinterpret_cast<const uint32_t *>(nodes4)[threadIdx.x];
 }
 
-//! the state as the host reads it, once everything queued before has run; with nodes, the root node too
-static const bvh_state &read_state(vkrt_ctx *ctx, const vkrt_bvh_node *nodes)
+//! the state as the host reads it, once everything queued before has run; the root nodes of what is given too
+static const bvh_state &read_state(vkrt_ctx *ctx, const vkrt_bvh_node *nodes, const vkrt_bvh4_node *nodes4)
 {
     bvh_state *host = ctx->pinned_as<bvh_state>();
-    k_report<<<1, 256, 0, ctx->stream>>>(ctx->state.as<bvh_state>(), nodes, host);
+    k_report<<<1, 256, 0, ctx->stream>>>(ctx->state.as<bvh_state>(), nodes, nodes4, host);
     VKRT_HIP(hipGetLastError());
     VKRT_HIP(hipStreamSynchronize(ctx->stream));
     return *host;
-}
-
-//! the root's box from its two child boxes: rb as (lo, hi) pairs per axis, bounds as lo xyz then hi xyz
-static void root_bounds(const vkrt_bvh_node &root, float rb[6], float bounds[6])
-{
-    const float r[6] = {std::min(root.a.x, root.b.x), std::max(root.a.y, root.b.y), std::min(root.a.z, root.b.z),
-                        std::max(root.a.w, root.b.w), std::min(root.c.x, root.c.z), std::max(root.c.y, root.c.w)};
-    for(int a = 0; a < 6; ++a) rb[a] = r[a];
-    for(int a = 0; a < 3; ++a)
-    {
-        bounds[a] = r[2 * a];
-        bounds[3 + a] = r[2 * a + 1];
-    }
 }
 
 //! a single leaf's bounds (at most 8 triangles): the union of its triangles' boxes (tbox, in leaf order), padded
@@ -549,9 +537,18 @@ static void single_leaf_info(vkrt_bvh *bvh, const float *tbox, hipStream_t s)
     }
 }
 
-static void build_topology_ploc(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh, const uint32_t *sorted);
+//! the binary tree a build works on
+struct binary_tree
+{
+    vkrt_bvh_node *nodes;
+    int2 *child;
+    uint2 *range;// the run of leaves below each node
+};
 
-static void build_topology(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh)
+static void build_topology_ploc(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh, const binary_tree &bin,
+                                const uint32_t *sorted);
+
+static void build_topology(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh, const binary_tree &bin)
 {
     hipStream_t s = ctx->stream;
     const uint32_t n = bvh->n_tri;
@@ -575,9 +572,9 @@ static void build_topology(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh)
     if(n >= 2)
     {
         const uint32_t ni = n - 1;
-        if(ploc) build_topology_ploc(ctx, bvh, mesh, order);
+        if(ploc) build_topology_ploc(ctx, bvh, mesh, bin, order);
         else
-            k_karras<<<div_up(ni, 256), 256, 0, s>>>(keys, (int)n, bvh->child.as<int2>(), bvh->range.as<uint2>());
+            k_karras<<<div_up(ni, 256), 256, 0, s>>>(keys, (int)n, bin.child, bin.range);
     }
     VKRT_HIP(hipGetLastError());
 }
@@ -1000,7 +997,8 @@ __global__ void __launch_bounds__(256) k_ploc_emit(ploc_tree tree, const uint32_
     tree.child[k] = c;
 }
 
-static void build_topology_ploc(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh, const uint32_t *sorted)
+static void build_topology_ploc(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh, const binary_tree &bin,
+                                const uint32_t *sorted)
 {
     hipStream_t s = ctx->stream;
     const int radius = bvh->ploc_radius ? static_cast<int>(bvh->ploc_radius) : PLOC_RADIUS;
@@ -1024,7 +1022,7 @@ static void build_topology_ploc(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &m
     }
     int8_t *code = reinterpret_cast<int8_t *>(take(n));
     uint32_t *counts = reinterpret_cast<uint32_t *>(take((size_t)tiles * 4));
-    ploc_tree tree{bvh->child.as<int2>(), reinterpret_cast<uint32_t *>(take((size_t)ni * 4)),
+    ploc_tree tree{bin.child, reinterpret_cast<uint32_t *>(take((size_t)ni * 4)),
                    reinterpret_cast<int32_t *>(take((size_t)ni * 4)), ni};
     uint32_t *first = reinterpret_cast<uint32_t *>(take((size_t)ni * 4));
     VKRT_REQUIRE(q <= w.as<uint8_t>() + bytes, "PLOC working set overrun");
@@ -1048,7 +1046,7 @@ static void build_topology_ploc(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &m
             k_ploc_merge<<<grid, PLOC_BLOCK, 0, s>>>(st, round & 1u, radius, l, code, counts, tree);
         }
         k_ploc_tail<<<1, PLOC_TAIL, 0, s>>>(st, round & 1u, radius, l, tree);
-        const bvh_state &got = read_state(ctx, nullptr);
+        const bvh_state &got = read_state(ctx, nullptr, nullptr);
         VKRT_REQUIRE(got.ploc_left >= 1 && got.ploc_left < nc, "PLOC made no progress");
         nc = got.ploc_left;
         if(nc == 1)
@@ -1063,78 +1061,69 @@ static void build_topology_ploc(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &m
         const uint32_t stop = std::min(b, ni);
         k_ploc_first<<<div_up(stop - a, 256), 256, 0, s>>>(a, stop, tree, first);
     }
-    k_ploc_emit<<<div_up(ni, 256), 256, 0, s>>>(tree, first, sorted, bvh->order.as<uint32_t>(), bvh->range.as<uint2>());
+    k_ploc_emit<<<div_up(ni, 256), 256, 0, s>>>(tree, first, sorted, bvh->order.as<uint32_t>(), bin.range);
     VKRT_HIP(hipGetLastError());
 }
 
-//! the BVH's memory, all but what traversal walks (the 4-wide nodes' number only the collapse tells)
-static void allocate(vkrt_bvh *bvh)
+//! parts of one allocation, one after the other, each at a multiple of 256 B
+static void place(device_buffer &mem, std::initializer_list<std::pair<vkrt_bvh::part *, size_t>> parts)
 {
-    const size_t n = bvh->n_tri, ni = n - 1;
-    const std::pair<vkrt_bvh::part *, size_t> parts[vkrt_bvh::PARTS] = {
-            {&bvh->nodes, ni * sizeof(vkrt_bvh_node)}, {&bvh->indices, n * 3 * sizeof(uint32_t)},
-            {&bvh->order, n * sizeof(uint32_t)},       {&bvh->child, ni * sizeof(int2)},
-            {&bvh->range, ni * sizeof(uint2)}};
     size_t total = 0;
+    for(const auto &[p, bytes]: parts) total += (bytes + 255) & ~size_t(255);
+    mem.reserve(total);
+    uint8_t *at = mem.as<uint8_t>();
     for(const auto &[p, bytes]: parts)
     {
-        p->bytes = std::max<size_t>(bytes, 256);
-        total += (p->bytes + 255) & ~size_t(255);
-    }
-    // below about 2 MiB the runtime hands out parts of a block it keeps (1 us, against 70 us for allocating and
-    // freeing 4 MB), so the parts of a small BVH stay apart
-    const bool apart = bvh->nodes.bytes < (2u << 20);
-    if(!apart) bvh->memory[0].reserve(total);
-    uint8_t *at = bvh->memory[0].as<uint8_t>();
-    for(size_t k = 0; k < std::size(parts); ++k)
-    {
-        vkrt_bvh::part &p = *parts[k].first;
-        if(apart)
-        {
-            bvh->memory[k].reserve(p.bytes);
-            p.ptr = bvh->memory[k].ptr;
-            continue;
-        }
-        p.ptr = at;
-        at += (p.bytes + 255) & ~size_t(255);
+        p->ptr = at;
+        p->bytes = bytes;
+        at += (bytes + 255) & ~size_t(255);
     }
 }
 
-//! the BVH2's nodes and the root from the mesh and a topology; with RECORDS (a refit, which keeps the topology)
-//! the leaf records as well
-template<bool RECORDS>
-static void build_bounds(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh)
+//! the BVH's memory, with room for node_cap 4-wide nodes
+static void allocate(vkrt_bvh *bvh, uint32_t node_cap)
+{
+    const size_t n = bvh->n_tri;
+    // (a step at the last leaf reads one record past it)
+    place(bvh->memory, {{&bvh->nodes4, (size_t)node_cap * sizeof(vkrt_bvh4_node)}, {&bvh->tris, (n + 1) * TRI_BYTES},
+                        {&bvh->indices, n * 3 * sizeof(uint32_t)}, {&bvh->order, n * sizeof(uint32_t)},
+                        {&bvh->wide_range, node_cap * sizeof(uint2)}});
+    bvh->node_cap = node_cap;
+    bvh->joint = static_cast<size_t>(bvh->tris.as<uint8_t>() - bvh->nodes4.as<uint8_t>()) + bvh->tris.bytes <= 0xffffffffull;
+}
+
+//! how many 4-wide nodes a build makes room for before it knows: measured over heightfields, spheres, the room and
+//! triangle soups, both builders, a triangle takes 0.42 to 0.53 of a node at one triangle a leaf, 0.25 to 0.31 at two,
+//! 0.15 to 0.20 at four and 0.07 to 0.11 at eight. A tree that needs more (a regular grid at one triangle a leaf:
+//! 0.67) is collapsed again into a larger allocation. Knowing the place beforehand saves the build a copy of the
+//! nodes and a second pass over the mesh, and the allocation overlaps the kernels queued before it.
+static uint32_t node_guess(const vkrt_bvh *bvh)
+{
+    const double per_tri = 0.07 + 0.5 / bvh->max_leaf;
+    return static_cast<uint32_t>(std::min<double>(bvh->n_tri, bvh->n_tri * per_tri + 8));
+}
+
+//! leaf records and boxes from the mesh, and the boxes' unions (in scratch): the start of a refit and, after the
+//! topology, of a build
+static leaf_unions leaf_pass(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh)
 {
     hipStream_t s = ctx->stream;
     const uint32_t n = bvh->n_tri;
     // (the sort's scratch is done with; a single leaf's box is read back from here)
     ctx->scratch[2].reserve((size_t)n * 6 * sizeof(float));
     float *tbox = ctx->scratch[2].as<float>();
-    k_leaves<true, RECORDS><<<div_up(n, 256), 256, 0, s>>>(mesh, bvh->order.as<uint32_t>(), tbox,
-                                                           bvh->tris.as<float4>());
-    if(n >= 2)
-    {
-        const uint32_t ni = n - 1;
-        // scratch: per-leaf prefix and suffix unions, then the segments' sparse table
-        const uint32_t nseg = div_up(n, BOX_SEG), levels = box_levels(nseg);
-        device_buffer &w = ctx->scratch[3];
-        w.reserve(((size_t)2 * n + (size_t)levels * nseg) * 6 * sizeof(float));
-        float *pre = w.as<float>(), *suf = pre + 6 * (size_t)n, *table = suf + 6 * (size_t)n;
-        k_box_scan<<<nseg, BOX_SEG, 0, s>>>(n, tbox, pre, suf, table);
-        for(uint32_t k = 1; k < levels; k += SPARSE_LEVELS)
-            k_box_sparse<<<div_up(nseg, 256), 256, 0, s>>>(nseg, k, levels, table);
-        bvh->n_nodes = ni;
-        const leaf_unions l{tbox, pre, suf, table, n, nseg};
-        k_layout<<<div_up(ni, 256), 256, 0, s>>>(l, bvh->child.as<int2>(), bvh->range.as<uint2>(), bvh->max_leaf,
-                                                 bvh->nodes.as<vkrt_bvh_node>());
-        bvh->root_ref = (n <= bvh->max_leaf) ? ~static_cast<int>(n - 1) : 0;
-    }
-    else
-    {
-        bvh->n_nodes = 0;
-        bvh->root_ref = ~0;// a leaf holding the single triangle
-    }
+    k_leaves<true><<<div_up(n, 256), 256, 0, s>>>(mesh, bvh->order.as<uint32_t>(), tbox, bvh->tris.as<float4>());
+    if(n < 2) return leaf_unions{tbox, nullptr, nullptr, nullptr, n, 0u};
+    // per-leaf prefix and suffix unions, then the segments' sparse table
+    const uint32_t nseg = div_up(n, BOX_SEG), levels = box_levels(nseg);
+    device_buffer &w = ctx->scratch[3];
+    w.reserve(((size_t)2 * n + (size_t)levels * nseg) * 6 * sizeof(float));
+    float *pre = w.as<float>(), *suf = pre + 6 * (size_t)n, *table = suf + 6 * (size_t)n;
+    k_box_scan<<<nseg, BOX_SEG, 0, s>>>(n, tbox, pre, suf, table);
+    for(uint32_t k = 1; k < levels; k += SPARSE_LEVELS)
+        k_box_sparse<<<div_up(nseg, 256), 256, 0, s>>>(nseg, k, levels, table);
     VKRT_HIP(hipGetLastError());
+    return leaf_unions{tbox, pre, suf, table, n, nseg};
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1148,16 +1137,14 @@ static void build_bounds(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh)
 struct collapse_child
 {
     int32_t ref;
-    int32_t src;// (BVH2 parent node << 1) | side: where the box is stored, re-read by a refit
     float lo[3], hi[3];
 };
 
-__device__ __forceinline__ collapse_child child_of(const vkrt_bvh_node &nd, int32_t node, int k)
+__device__ __forceinline__ collapse_child child_of(const vkrt_bvh_node &nd, int k)
 {
     collapse_child c;
     const float4 xy = k == 0 ? nd.a : nd.b;
     c.ref = k == 0 ? nd.d.x : nd.d.y;
-    c.src = (node << 1) | k;
     c.lo[0] = xy.x;
     c.hi[0] = xy.y;
     c.lo[1] = xy.z;
@@ -1187,12 +1174,14 @@ __device__ __forceinline__ double child_area(const collapse_child &c)
 //! writes), which also lays a node's children side by side. The grid may be larger or smaller than the level.
 //! A level opens every BVH2 node once, so the tree's depth, leaves and SAH terms are summed on the way (a pass of
 //! its own, climbing the parents for the depth, took 608 us). Nodes deeper than the stack end the descent: the
-//! build then fails. n4 null: the sums only.
+//! build then fails. Nodes at or past n4_cap are counted and queued but not written (with n4_cap 0 a build wants the
+//! sums only); n4_range[i] is the run of leaves below node i.
 constexpr uint32_t COLLAPSE_BLOCK = 256, COLLAPSE_GRID = 1024;
 __global__ void __launch_bounds__(COLLAPSE_BLOCK) k_collapse(const vkrt_bvh_node *__restrict__ n2,
-                                                             int4 *__restrict__ queue, uint32_t level,
+                                                             const uint2 *__restrict__ range, int4 *__restrict__ queue,
+                                                             uint32_t level, uint32_t n4_cap,
                                                              vkrt_bvh4_node *__restrict__ n4,
-                                                             bvh_state *__restrict__ st)
+                                                             uint2 *__restrict__ n4_range, bvh_state *__restrict__ st)
 {
     __shared__ uint32_t wave_sum[COLLAPSE_BLOCK / 64], slot_base;
     __shared__ double wave_sah[COLLAPSE_BLOCK / 64];
@@ -1212,13 +1201,15 @@ __global__ void __launch_bounds__(COLLAPSE_BLOCK) k_collapse(const vkrt_bvh_node
         uint32_t ch_depth[4] = {0, 0, 0, 0};// depth of the BVH2 node each child came from
         int cnt = 0;
         uint32_t inner = 0, depth_here = 0;
+        int32_t node_here = 0;
         if(active)
         {
             const int4 item = queue[me];
+            node_here = item.x;
             auto open = [&](int slot_a, int slot_b, int32_t node, uint32_t d) {
                 const vkrt_bvh_node nd = n2[node];
-                ch[slot_a] = child_of(nd, node, 0);
-                ch[slot_b] = child_of(nd, node, 1);
+                ch[slot_a] = child_of(nd, 0);
+                ch[slot_b] = child_of(nd, 1);
                 ch_depth[slot_a] = ch_depth[slot_b] = d;
                 depth = max(depth, d);
                 for(const int k: {slot_a, slot_b})
@@ -1286,11 +1277,10 @@ __global__ void __launch_bounds__(COLLAPSE_BLOCK) k_collapse(const vkrt_bvh_node
         {
             vkrt_bvh4_node out;
             float lo[3][4], hi[3][4];
-            int32_t refs[4], srcs[4];
+            int32_t refs[4];
 #pragma unroll
             for(int j = 0; j < 4; ++j)
             {
-                srcs[j] = j < cnt ? ch[j].src : -1;
                 for(int a = 0; a < 3; ++a)
                 {
                     lo[a][j] = j < cnt ? ch[j].lo[a] : 0.0f;
@@ -1313,8 +1303,12 @@ __global__ void __launch_bounds__(COLLAPSE_BLOCK) k_collapse(const vkrt_bvh_node
             out.loz = make_float4(lo[2][0], lo[2][1], lo[2][2], lo[2][3]);
             out.hiz = make_float4(hi[2][0], hi[2][1], hi[2][2], hi[2][3]);
             out.child = make_int4(refs[0], refs[1], refs[2], refs[3]);
-            out.src = make_int4(srcs[0], srcs[1], srcs[2], srcs[3]);
-            if(n4) n4[me] = out;
+            out.pad = make_int4(0, 0, 0, 0);
+            if(me < n4_cap)
+            {
+                n4[me] = out;
+                n4_range[me] = range[node_here];
+            }
         }
     }
     if(blockIdx.x * COLLAPSE_BLOCK >= count) return;// (the whole workgroup: it had no item)
@@ -1355,106 +1349,91 @@ __global__ void k_collapse_root(int4 *__restrict__ queue, bvh_state *__restrict_
     st->level[0] = 1u;
 }
 
-//! refit of the 4-wide layout: every used child slot re-reads its box from the BVH2 node it was collapsed
-//! from (the BVH2 keeps its topology and node numbering on refit), so the collapse's shape, its worst-case
-//! stack depth and the choice of the 4-wide walk stay what the build recorded
-__global__ void k_wide_refit(const vkrt_bvh_node *__restrict__ n2, uint32_t n4_count, vkrt_bvh4_node *__restrict__ n4)
+//! refit of the 4-wide layout, a thread per child slot: a child's box is the union over its run of leaves, as when
+//! the tree was built, so the collapse's shape, its worst-case stack depth and the choice of the 4-wide walk stay
+//! what the build recorded
+__global__ void __launch_bounds__(256) k_wide_refit(leaf_unions l, uint32_t n4_count, const uint2 *__restrict__ n4_range,
+                                                    vkrt_bvh4_node *__restrict__ n4)
 {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t i = (blockIdx.x * 256 + threadIdx.x) >> 2, j = threadIdx.x & 3u;
     if(i >= n4_count) return;
-    vkrt_bvh4_node nd = n4[i];
-    float *lox = &nd.lox.x, *hix = &nd.hix.x, *loy = &nd.loy.x, *hiy = &nd.hiy.x, *loz = &nd.loz.x, *hiz = &nd.hiz.x;
-    const int32_t src[4] = {nd.src.x, nd.src.y, nd.src.z, nd.src.w};
+    const int32_t ref = reinterpret_cast<const int32_t *>(&n4[i].child)[j];
+    if(ref == EMPTY_CHILD) return;
+    uint2 r;
+    if(ref >= 0) r = n4_range[ref];
+    else
+    {
+        uint32_t count;
+        const uint32_t v = static_cast<uint32_t>(~ref);
+        r.x = v >> 3;
+        count = (v & 7u) + 1u;
+        r.y = r.x + count - 1u;
+    }
+    float b[6];
+    run_box(l, r.x, r.y, b);
+    float *f = reinterpret_cast<float *>(&n4[i]) + j;// lox hix loy hiy loz hiz, four floats each
+    for(int a = 0; a < 3; ++a)
+    {
+        f[8 * a] = pad_lo(b[a]);
+        f[8 * a + 4] = pad_hi(b[3 + a]);
+    }
+}
+
+//! the root's box from its two child boxes: rb as (lo, hi) pairs per axis, bounds as lo xyz then hi xyz
+static void root_bounds(const vkrt_bvh_node &root, float rb[6], float bounds[6])
+{
+    const float r[6] = {std::min(root.a.x, root.b.x), std::max(root.a.y, root.b.y), std::min(root.a.z, root.b.z),
+                        std::max(root.a.w, root.b.w), std::min(root.c.x, root.c.z), std::max(root.c.y, root.c.w)};
+    for(int a = 0; a < 6; ++a) rb[a] = r[a];
+    for(int a = 0; a < 3; ++a)
+    {
+        bounds[a] = r[2 * a];
+        bounds[3 + a] = r[2 * a + 1];
+    }
+}
+
+//! a root's box from its used children
+static void root_bounds(const vkrt_bvh4_node &root, float bounds[6])
+{
+    const float *planes[6] = {&root.lox.x, &root.loy.x, &root.loz.x, &root.hix.x, &root.hiy.x, &root.hiz.x};
+    const int32_t child[4] = {root.child.x, root.child.y, root.child.z, root.child.w};
+    bool first = true;
     for(int j = 0; j < 4; ++j)
     {
-        if(src[j] < 0) continue;
-        const vkrt_bvh_node p = n2[src[j] >> 1];
-        const collapse_child c = child_of(p, src[j] >> 1, src[j] & 1);
-        lox[j] = c.lo[0];
-        hix[j] = c.hi[0];
-        loy[j] = c.lo[1];
-        hiy[j] = c.hi[1];
-        loz[j] = c.lo[2];
-        hiz[j] = c.hi[2];
+        if(child[j] == EMPTY_CHILD) continue;
+        for(int a = 0; a < 6; ++a)
+            bounds[a] = first ? planes[a][j] : (a < 3 ? std::min(bounds[a], planes[a][j]) : std::max(bounds[a], planes[a][j]));
+        first = false;
     }
-    n4[i] = nd;
 }
 
-//! refreshes the boxes of an existing 4-wide layout after the BVH2 was refitted (no change of shape)
-static void refit_wide(vkrt_ctx *ctx, vkrt_bvh *bvh)
-{
-    if(bvh->empty || !bvh->wide || bvh->root4 < 0 || bvh->n_nodes4 == 0) return;
-    k_wide_refit<<<div_up(bvh->n_nodes4, 256), 256, 0, ctx->stream>>>(bvh->nodes.as<vkrt_bvh_node>(), bvh->n_nodes4,
-                                                                       bvh->nodes4.as<vkrt_bvh4_node>());
-    VKRT_HIP(hipGetLastError());
-}
-
-//! what traversal walks: room for the 4-wide nodes and, after them, the leaf records, written from the mesh
-static void build_walk(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh)
-{
-    const size_t node_bytes = (size_t)bvh->n_nodes4 * sizeof(vkrt_bvh4_node);
-    const size_t tri_bytes = (size_t)bvh->n_tri * TRI_BYTES;
-    // (a step at the last leaf reads one record past it)
-    const size_t total = node_bytes + tri_bytes + TRI_BYTES;
-    bvh->walk.reserve(total);
-    bvh->nodes4.ptr = bvh->walk.ptr;
-    bvh->nodes4.bytes = node_bytes;
-    bvh->tris.ptr = bvh->walk.as<uint8_t>() + node_bytes;
-    bvh->tris.bytes = tri_bytes;
-    bvh->joint = total <= 0xffffffffull;
-    k_leaves<false, true><<<div_up(bvh->n_tri, 256), 256, 0, ctx->stream>>>(mesh, bvh->order.as<uint32_t>(), nullptr,
-                                                                            bvh->tris.as<float4>());
-    VKRT_HIP(hipGetLastError());
-}
-
-//! the end of a build: the BVH2 collapsed into the BVH4 used for traversal (kept off when its worst-case stack
-//! depth exceeds STACK_SIZE), the tree's statistics, and what the kernels before found wrong
-static void build_wide(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh)
+//! the BVH2 collapsed into the BVH4 used for traversal and the tree's statistics; false when the nodes did not fit
+//! (n_nodes4 then says how many there are)
+static bool collapse(vkrt_ctx *ctx, vkrt_bvh *bvh, const binary_tree &bin)
 {
     hipStream_t s = ctx->stream;
-    bvh->wide = false;
-    bvh->n_nodes4 = 0;
-    bvh->stack4 = 0;
-    auto check_indices = [](const bvh_state &st) {
-        if(st.err) throw error(VKRT_E_INVALID_ARG, "triangle index out of range of the vertex count");
-    };
-    if(bvh->root_ref < 0)
-    {
-        check_indices(read_state(ctx, nullptr));
-        build_walk(ctx, bvh, mesh);
-        bvh->root4 = bvh->root_ref;// a single leaf
-        bvh->wide = bvh->allow_wide;
-        single_leaf_info(bvh, ctx->scratch[2].as<float>(), s);
-        return;
-    }
     // (a 4-wide node takes in at least one node of the binary tree)
-    const size_t cap = bvh->n_nodes;
-    ctx->scratch[2].reserve(cap * sizeof(int4));
+    const uint32_t most_nodes = bvh->n_nodes, cap = bvh->allow_wide ? bvh->node_cap : 0u;
+    ctx->scratch[2].reserve((size_t)most_nodes * sizeof(int4));
     int4 *queue = ctx->scratch[2].as<int4>();
-    vkrt_bvh4_node *n4 = nullptr;
-    if(bvh->allow_wide)
-    {
-        ctx->scratch[3].reserve(cap * sizeof(vkrt_bvh4_node));
-        n4 = ctx->scratch[3].as<vkrt_bvh4_node>();
-    }
-    const vkrt_bvh_node *n2 = bvh->nodes.as<vkrt_bvh_node>();
     bvh_state *st = ctx->state.as<bvh_state>();
     k_collapse_root<<<1, 1, 0, s>>>(queue, st);
     // the levels are launched without asking how many there are: as many as balanced trees of this size have and
     // some more (a level that is not there costs its launch, 2 us), then in turns until the last one is empty
     uint32_t level = 0, todo = 6;
-    for(size_t k = 1; k < cap; k *= 4) ++todo;
+    for(size_t k = 1; k < most_nodes; k *= 4) ++todo;
     const bvh_state *got = nullptr;
     while(true)
     {
         for(uint32_t stop = std::min(level + todo, MAX_LEVELS); level < stop; ++level)
         {
-            const uint64_t most = std::min<uint64_t>(cap, level < 16 ? 1ull << (2 * level) : cap);
-            k_collapse<<<std::min(COLLAPSE_GRID, div_up(most, COLLAPSE_BLOCK)), COLLAPSE_BLOCK, 0, s>>>(n2, queue, level,
-                                                                                                         n4, st);
+            const uint64_t most = std::min<uint64_t>(most_nodes, level < 16 ? 1ull << (2 * level) : most_nodes);
+            k_collapse<<<std::min(COLLAPSE_GRID, div_up(most, COLLAPSE_BLOCK)), COLLAPSE_BLOCK, 0, s>>>(
+                    bin.nodes, bin.range, queue, level, cap, bvh->nodes4.as<vkrt_bvh4_node>(),
+                    bvh->wide_range.as<uint2>(), st);
         }
-        got = &read_state(ctx, n2);
-        check_indices(*got);
+        got = &read_state(ctx, bin.nodes, nullptr);
+        if(got->err) throw error(VKRT_E_INVALID_ARG, "triangle index out of range of the vertex count");
         if(got->depth > (uint32_t)STACK_SIZE) throw error(VKRT_E_INTERNAL, "BVH deeper than the traversal stack");
         if(got->level[level] == 0) break;
         VKRT_REQUIRE(level < MAX_LEVELS, "BVH4 collapse did not end");
@@ -1462,7 +1441,7 @@ static void build_wide(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh)
     }
     uint64_t total = 0;
     for(uint32_t l = 0; l < level; ++l) total += got->level[l];
-    VKRT_REQUIRE(total <= cap, "BVH4 collapse overflow");
+    VKRT_REQUIRE(total <= most_nodes, "BVH4 collapse overflow");
     vkrt_bvh_info &info = bvh->info;
     float rb[6];
     root_bounds(got->root, rb, info.bounds);
@@ -1472,16 +1451,59 @@ static void build_wide(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh)
     info.depth = std::max(1u, got->depth);
     info.sah_cost = static_cast<float>(1.0 + got->sah / root_area);// 1: the root's own visit
     info.n_leaves = got->leaves;
-    const uint32_t stack4 = got->stack;
-    if(bvh->allow_wide) bvh->n_nodes4 = static_cast<uint32_t>(total);
-    build_walk(ctx, bvh, mesh);
-    if(!bvh->allow_wide) return;
-    bvh->stack4 = stack4;
+    if(!bvh->allow_wide) return true;
+    bvh->n_nodes4 = static_cast<uint32_t>(total);
+    bvh->stack4 = got->stack;
     bvh->root4 = 0;
-    // the nodes move from the scratch, sized for the most there could be, into an array of their number
-    VKRT_HIP(hipMemcpyAsync(bvh->nodes4.ptr, n4, bvh->nodes4.bytes, hipMemcpyDeviceToDevice, s));
+    return total <= cap;
+}
+
+//! the end of a build: the leaves, the binary tree, and its collapse (kept off when its worst-case stack depth exceeds
+//! STACK_SIZE)
+static void build_tree(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh, const binary_tree &bin)
+{
+    hipStream_t s = ctx->stream;
+    const uint32_t n = bvh->n_tri;
+    const leaf_unions leaves = leaf_pass(ctx, bvh, mesh);
+    bvh->n_nodes = n - 1u;
+    bvh->root_ref = n <= bvh->max_leaf ? ~static_cast<int>(n - 1u) : 0;
+    if(n >= 2)
+        k_layout<<<div_up(n - 1u, 256), 256, 0, s>>>(leaves, bin.child, bin.range, bvh->max_leaf, bin.nodes);
+    VKRT_HIP(hipGetLastError());
+    if(bvh->root_ref < 0)
+    {
+        if(read_state(ctx, nullptr, nullptr).err)
+            throw error(VKRT_E_INVALID_ARG, "triangle index out of range of the vertex count");
+        bvh->root4 = bvh->root_ref;// a single leaf
+        bvh->wide = bvh->allow_wide;
+        single_leaf_info(bvh, ctx->scratch[2].as<float>(), s);
+        return;
+    }
+    if(!collapse(ctx, bvh, bin))
+    {
+        // more nodes than there was room for: the same again in a larger allocation
+        device_buffer old = std::move(bvh->memory);
+        const vkrt_bvh::part indices = bvh->indices, order = bvh->order;
+        allocate(bvh, bvh->n_nodes4);
+        VKRT_HIP(hipMemcpyAsync(bvh->indices.ptr, indices.ptr, indices.bytes, hipMemcpyDeviceToDevice, s));
+        VKRT_HIP(hipMemcpyAsync(bvh->order.ptr, order.ptr, order.bytes, hipMemcpyDeviceToDevice, s));
+        mesh_view moved = mesh;
+        moved.idx = bvh->indices.as<uint32_t>();
+        k_leaves<false><<<div_up(n, 256), 256, 0, s>>>(moved, bvh->order.as<uint32_t>(), nullptr, bvh->tris.as<float4>());
+        k_state_clear<<<1, 256, 0, s>>>(ctx->state.as<bvh_state>());
+        VKRT_REQUIRE(collapse(ctx, bvh, bin), "BVH4 collapse overflow");
+    }
     // the 4-wide walk addresses nodes with 32-bit byte offsets (node4_intervals)
-    bvh->wide = bvh->stack4 <= (uint32_t)STACK_SIZE && (uint64_t)bvh->nodes4.bytes <= 0xffffffffull;
+    bvh->wide = bvh->allow_wide && bvh->stack4 <= (uint32_t)STACK_SIZE &&
+                (uint64_t)bvh->n_nodes4 * sizeof(vkrt_bvh4_node) <= 0xffffffffull;
+    if(bvh->wide && bvh->joint) return;
+    // the binary tree stays where traversal or a refit uses it
+    const size_t ni = n - 1u;
+    place(bvh->binary, {{&bvh->nodes, ni * sizeof(vkrt_bvh_node)}, {&bvh->child, ni * sizeof(int2)},
+                        {&bvh->range, ni * sizeof(uint2)}});
+    VKRT_HIP(hipMemcpyAsync(bvh->nodes.ptr, bin.nodes, bvh->nodes.bytes, hipMemcpyDeviceToDevice, s));
+    VKRT_HIP(hipMemcpyAsync(bvh->child.ptr, bin.child, bvh->child.bytes, hipMemcpyDeviceToDevice, s));
+    VKRT_HIP(hipMemcpyAsync(bvh->range.ptr, bin.range, bvh->range.bytes, hipMemcpyDeviceToDevice, s));
 }
 
 //! the rest of the info block after a build or a refit
@@ -1489,7 +1511,8 @@ static void refresh_info(vkrt_bvh *bvh)
 {
     bvh->info.n_tri = bvh->n_tri;
     bvh->info.n_nodes = bvh->n_nodes;
-    bvh->info.device_bytes = bvh->nodes.bytes + bvh->tris.bytes + bvh->nodes4.bytes;
+    bvh->info.device_bytes = bvh->nodes.bytes + (uint64_t)bvh->n_tri * TRI_BYTES +
+                             (uint64_t)bvh->n_nodes4 * sizeof(vkrt_bvh4_node);
     bvh->info.n_wide_nodes = bvh->wide ? bvh->n_nodes4 : 0;
     bvh->info.wide_stack = bvh->stack4;
 }
@@ -1532,14 +1555,20 @@ int vkrt_bvh_build(vkrt_ctx *ctx, const float *positions, uint32_t n_vert, uint3
             const size_t pos_bytes = (size_t)(n_vert - 1) * stride_bytes + 12;
             const uint8_t *dpos =
                     input(ctx, 0, reinterpret_cast<const uint8_t *>(positions), pos_bytes, flags);
-            allocate(bvh.get());
             const uint32_t *didx = input(ctx, 1, indices, (size_t)n_tri * 3, flags);
+            // the binary tree is scratch: most builds keep only its collapse
+            const size_t ni = n_tri - 1u, node_bytes = (ni * sizeof(vkrt_bvh_node) + 255) & ~size_t(255),
+                         child_bytes = (ni * sizeof(int2) + 255) & ~size_t(255);
+            ctx->scratch[4].reserve(node_bytes + child_bytes + ni * sizeof(uint2));
+            uint8_t *tree = ctx->scratch[4].as<uint8_t>();
+            const binary_tree bin{reinterpret_cast<vkrt_bvh_node *>(tree), reinterpret_cast<int2 *>(tree + node_bytes),
+                                  reinterpret_cast<uint2 *>(tree + node_bytes + child_bytes)};
+            allocate(bvh.get(), bvh->allow_wide ? node_guess(bvh.get()) : 0u);
             VKRT_HIP(hipMemcpyAsync(bvh->indices.ptr, didx, (size_t)n_tri * 3 * sizeof(uint32_t),
                                     hipMemcpyDeviceToDevice, ctx->stream));
             const mesh_view mesh{dpos, bvh->indices.as<uint32_t>(), stride_bytes, n_tri, n_vert};
-            build_topology(ctx, bvh.get(), mesh);
-            build_bounds<false>(ctx, bvh.get(), mesh);
-            build_wide(ctx, bvh.get(), mesh);
+            build_topology(ctx, bvh.get(), mesh, bin);
+            build_tree(ctx, bvh.get(), mesh, bin);
             VKRT_HIP(hipStreamSynchronize(ctx->stream));
         }
         else single_leaf_info(bvh.get(), nullptr, ctx->stream);
@@ -1560,14 +1589,24 @@ int vkrt_bvh_refit(vkrt_ctx *ctx, vkrt_bvh *bvh, const float *positions, uint32_
         hipStream_t s = ctx->stream;
         const size_t pos_bytes = (size_t)(bvh->n_vert - 1) * stride_bytes + 12;
         const uint8_t *dpos = input(ctx, 0, reinterpret_cast<const uint8_t *>(positions), pos_bytes, flags);
-        build_bounds<true>(ctx, bvh, mesh_view{dpos, bvh->indices.as<uint32_t>(), stride_bytes, bvh->n_tri, bvh->n_vert});
-        refit_wide(ctx, bvh);
+        const leaf_unions leaves = leaf_pass(
+                ctx, bvh, mesh_view{dpos, bvh->indices.as<uint32_t>(), stride_bytes, bvh->n_tri, bvh->n_vert});
         if(bvh->root_ref < 0) single_leaf_info(bvh, ctx->scratch[2].as<float>(), s);
         else
         {
-            // the topology stays, and with it depth, leaves and SAH cost: only the bounds change
+            // the topology stays, and with it depth, leaves and SAH cost: only the boxes and bounds change
+            vkrt_bvh4_node *n4 = bvh->wide ? bvh->nodes4.as<vkrt_bvh4_node>() : nullptr;
+            vkrt_bvh_node *n2 = bvh->nodes.as<vkrt_bvh_node>();
+            if(n4)
+                k_wide_refit<<<div_up((uint64_t)bvh->n_nodes4 * 4, 256), 256, 0, s>>>(leaves, bvh->n_nodes4,
+                                                                                     bvh->wide_range.as<uint2>(), n4);
+            if(n2)
+                k_layout<<<div_up(bvh->n_nodes, 256), 256, 0, s>>>(leaves, bvh->child.as<int2>(), bvh->range.as<uint2>(),
+                                                                   bvh->max_leaf, n2);
+            const bvh_state &got = read_state(ctx, n2, n4);
             float rb[6];
-            root_bounds(read_state(ctx, bvh->nodes.as<vkrt_bvh_node>()).root, rb, bvh->info.bounds);
+            if(n4) root_bounds(got.root4, bvh->info.bounds);
+            else root_bounds(got.root, rb, bvh->info.bounds);
         }
         refresh_info(bvh);
     });
@@ -1596,8 +1635,8 @@ int vkrt_bvh_validate(vkrt_ctx *ctx, const vkrt_bvh *bvh, const float *positions
             VKRT_HIP(hipMemcpyAsync(dst.data(), src, bytes, device ? hipMemcpyDeviceToHost : hipMemcpyHostToHost, s));
         };
         std::vector<uint8_t> h_nodes, h_nodes4, h_tris, h_idx, h_pos;
-        fetch(bvh->nodes.ptr, (size_t)bvh->n_nodes * sizeof(vkrt_bvh_node), true, h_nodes);
         if(bvh->wide) fetch(bvh->nodes4.ptr, (size_t)bvh->n_nodes4 * sizeof(vkrt_bvh4_node), true, h_nodes4);
+        else if(bvh->root_ref >= 0) fetch(bvh->nodes.ptr, (size_t)bvh->n_nodes * sizeof(vkrt_bvh_node), true, h_nodes);
         fetch(bvh->tris.ptr, (size_t)n * TRI_BYTES, true, h_tris);
         fetch(bvh->indices.ptr, (size_t)n * 3 * sizeof(uint32_t), true, h_idx);
         fetch(positions, (size_t)(bvh->n_vert - 1) * stride_bytes + 12, (flags & VKRT_DEVICE_PTRS) != 0, h_pos);

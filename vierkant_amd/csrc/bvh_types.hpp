@@ -22,7 +22,7 @@ struct vkrt_bvh4_node
 {
     float4 lox, hix, loy, hiy, loz, hiz;
     int4 child;// >= 0 BVH4 node, < 0 leaf (the BVH2 leaf encoding), EMPTY_CHILD unused
-    int4 src;  // per slot (BVH2 node << 1) | side holding the child's box, -1 unused (read by a refit only)
+    int4 pad;
 };
 
 struct vkrt_bvh
@@ -44,21 +44,21 @@ struct vkrt_bvh
     uint32_t ploc_radius = 0;// 0: default
     int32_t root_ref = 0;
     bool empty = true;
-    // one allocation holds everything whose size the triangle count gives: freeing a large one takes 250 to 500 us
-    // (eight of them, 1.7 of the 4.1 ms that a 1.8M-triangle build and its destruction took)
-    static constexpr int PARTS = 5;
-    vkrt::device_buffer memory[PARTS];// (or one each, for a small BVH)
-    part nodes;
-    // the 4-wide collapse, used by traversal when its worst-case stack fits (wide == true), and after it the leaf
-    // records: one allocation, so that a walk reaches both with 32-bit offsets from one base (joint == true unless
-    // it passes 4 GiB)
-    vkrt::device_buffer walk;
-    part nodes4, tris;
+    // One allocation holds the 4-wide collapse, used by traversal when its worst-case stack fits (wide == true), the
+    // leaf records behind it, so that a walk reaches both with 32-bit offsets from one base (joint == true unless
+    // they pass 4 GiB), and what a refit needs: the mesh's indices, the leaves' order and the run of leaves below
+    // each 4-wide node. (Freeing a large allocation takes 250 to 500 us: eight of them took 1.7 of the 4.1 ms that
+    // building and destroying a 1.8M-triangle BVH took.)
+    vkrt::device_buffer memory;
+    part nodes4, tris, indices, order, wide_range;
+    uint32_t node_cap = 0;// 4-wide nodes there is room for
+    // the binary tree with its children and runs, kept only where traversal walks it: no 4-wide collapse, or not joint
+    vkrt::device_buffer binary;
+    part nodes, child, range;
     bool joint = true;
     int32_t root4 = 0;
     uint32_t n_nodes4 = 0, stack4 = 0;
     bool wide = false, allow_wide = true;
-    part indices, order, child, range;
     vkrt_bvh_info info{};
 };
 

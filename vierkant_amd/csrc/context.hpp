@@ -93,7 +93,7 @@ struct vkrt_ctx
     //! staging slots for host-pointer calls (inputs/outputs copied through these)
     vkrt::device_buffer staging[8];
     //! scratch for multi-pass kernels (keys, counters)
-    vkrt::device_buffer scratch[4];
+    vkrt::device_buffer scratch[5];
     //! counters of a call's kernels, and the pinned host block they are read through
     vkrt::device_buffer state;
     void *pinned = nullptr;

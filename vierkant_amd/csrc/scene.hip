@@ -272,7 +272,7 @@ struct tlas_builder
         nd.loz = make_float4(lo_[2][0], lo_[2][1], lo_[2][2], lo_[2][3]);
         nd.hiz = make_float4(hi_[2][0], hi_[2][1], hi_[2][2], hi_[2][3]);
         nd.child = make_int4(ch[0], ch[1], ch[2], ch[3]);
-        nd.src = make_int4(-1, -1, -1, -1);
+        nd.pad = make_int4(0, 0, 0, 0);
         return static_cast<int32_t>(slot);
     }
 };
