@@ -476,6 +476,7 @@ struct bvh_state
     uint32_t stack;// worst-case traversal stack of the 4-wide tree
     uint32_t pad4[31];
     uint32_t level[MAX_LEVELS + 2];// 4-wide nodes per level
+    uint32_t top_levels;           // levels that the collapse's first launch took
     ploc_round ploc[2];            // the clusters before an even and an odd round
     uint32_t ploc_left, ploc_nodes;// clusters left and nodes made after the last tail
     vkrt_bvh_node root;  // of the binary tree, where one is given
@@ -1176,7 +1177,10 @@ __device__ __forceinline__ double child_area(const collapse_child &c)
 //! its own, climbing the parents for the depth, took 608 us). Nodes deeper than the stack end the descent: the
 //! build then fails. Nodes at or past n4_cap are counted and queued but not written (with n4_cap 0 a build wants the
 //! sums only); n4_range[i] is the run of leaves below node i.
+//! TOP: one workgroup takes the levels from the root on while they fit it (five in a full tree; a launch each took
+//! 8 us); `level` otherwise counts from the first level it left.
 constexpr uint32_t COLLAPSE_BLOCK = 256, COLLAPSE_GRID = 1024;
+template<bool TOP>
 __global__ void __launch_bounds__(COLLAPSE_BLOCK) k_collapse(const vkrt_bvh_node *__restrict__ n2,
                                                              const uint2 *__restrict__ range, int4 *__restrict__ queue,
                                                              uint32_t level, uint32_t n4_cap,
@@ -1188,130 +1192,161 @@ __global__ void __launch_bounds__(COLLAPSE_BLOCK) k_collapse(const vkrt_bvh_node
     __shared__ uint32_t wave_leaves[COLLAPSE_BLOCK / 64], wave_depth[COLLAPSE_BLOCK / 64],
             wave_stack[COLLAPSE_BLOCK / 64];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    uint32_t first = 0;// the level's first node
-    for(uint32_t l = 0; l < level; ++l) first += st->level[l];
-    const uint32_t count = st->level[level], next = first + count;
     double sah = 0.0;
     uint32_t leaves = 0, depth = 0, stack = 0;
-    for(uint32_t base = blockIdx.x * COLLAPSE_BLOCK; base < count; base += gridDim.x * COLLAPSE_BLOCK)
+    uint32_t first = 0, count = 1;// the level's first node and its nodes
+    if constexpr(TOP)
     {
-        const bool active = base + threadIdx.x < count;
-        const uint32_t me = first + base + threadIdx.x;
-        collapse_child ch[4];
-        uint32_t ch_depth[4] = {0, 0, 0, 0};// depth of the BVH2 node each child came from
-        int cnt = 0;
-        uint32_t inner = 0, depth_here = 0;
-        int32_t node_here = 0;
-        if(active)
+        level = 0;
+        if(threadIdx.x == 0)
         {
-            const int4 item = queue[me];
-            node_here = item.x;
-            auto open = [&](int slot_a, int slot_b, int32_t node, uint32_t d) {
-                const vkrt_bvh_node nd = n2[node];
-                ch[slot_a] = child_of(nd, 0);
-                ch[slot_b] = child_of(nd, 1);
-                ch_depth[slot_a] = ch_depth[slot_b] = d;
-                depth = max(depth, d);
-                for(const int k: {slot_a, slot_b})
-                {
-                    const double a = child_area(ch[k]);
-                    if(ch[k].ref >= 0) sah += a;
-                    else
-                    {
-                        sah += ((static_cast<uint32_t>(~ch[k].ref) & 7u) + 1) * a;
-                        ++leaves;
-                        depth = max(depth, d + 1);
-                    }
-                }
-            };
-            open(0, 1, item.x, static_cast<uint32_t>(item.z));
-            cnt = 2;
-#pragma unroll
-            for(int step = 0; step < 2; ++step)
-            {
-                int best = -1;
-                float best_a = -1.0f;
-#pragma unroll
-                for(int j = 0; j < 3; ++j)
-                {
-                    if(j >= cnt || ch[j].ref < 0) continue;
-                    const float a = half_area(ch[j]);
-                    if(a > best_a)
-                    {
-                        best_a = a;
-                        best = j;
-                    }
-                }
-                if(best < 0) break;
-                // (constant slots: an array indexed by `best` would live in scratch memory)
-                if(best == 0) open(0, 2 + step, ch[0].ref, ch_depth[0] + 1);
-                else if(best == 1) open(1, 2 + step, ch[1].ref, ch_depth[1] + 1);
-                else open(2, 3, ch[2].ref, ch_depth[2] + 1);
-                ++cnt;
-            }
-            depth_here = static_cast<uint32_t>(item.y) + (cnt - 1);
-            stack = max(stack, depth_here);
-#pragma unroll
-            for(int j = 0; j < 4; ++j)
-                inner += j < cnt && ch[j].ref >= 0 && ch_depth[j] <= (uint32_t)STACK_SIZE ? 1u : 0u;
+            queue[0] = make_int4(0, 0, 1, 0);
+            st->level[0] = 1u;
         }
-        // the children's slots: an exclusive scan over the workgroup and one atomic
-        uint32_t sum = inner;
-        for(int off = 1; off < 64; off <<= 1)
-        {
-            const uint32_t y = __shfl_up(sum, off);
-            if(lane >= (uint32_t)off) sum += y;
-        }
-        if(lane == 63) wave_sum[wave] = sum;
         __syncthreads();
-        uint32_t before = 0, total = 0;
-        for(uint32_t w = 0; w < COLLAPSE_BLOCK / 64; ++w)
-        {
-            before += w < wave ? wave_sum[w] : 0u;
-            total += wave_sum[w];
-        }
-        if(threadIdx.x == 0) slot_base = next + (total ? atomicAdd(&st->level[level + 1], total) : 0u);
-        __syncthreads();
-        uint32_t slot = slot_base + before + sum - inner;
-        if(active)
-        {
-            vkrt_bvh4_node out;
-            float lo[3][4], hi[3][4];
-            int32_t refs[4];
-#pragma unroll
-            for(int j = 0; j < 4; ++j)
-            {
-                for(int a = 0; a < 3; ++a)
-                {
-                    lo[a][j] = j < cnt ? ch[j].lo[a] : 0.0f;
-                    hi[a][j] = j < cnt ? ch[j].hi[a] : 0.0f;
-                }
-                refs[j] = EMPTY_CHILD;
-                if(j >= cnt) continue;
-                if(ch[j].ref < 0) refs[j] = ch[j].ref;
-                else if(ch_depth[j] <= (uint32_t)STACK_SIZE)
-                {
-                    refs[j] = static_cast<int32_t>(slot);
-                    queue[slot++] = make_int4(ch[j].ref, static_cast<int32_t>(depth_here),
-                                              static_cast<int32_t>(ch_depth[j] + 1), 0);
-                }
-            }
-            out.lox = make_float4(lo[0][0], lo[0][1], lo[0][2], lo[0][3]);
-            out.hix = make_float4(hi[0][0], hi[0][1], hi[0][2], hi[0][3]);
-            out.loy = make_float4(lo[1][0], lo[1][1], lo[1][2], lo[1][3]);
-            out.hiy = make_float4(hi[1][0], hi[1][1], hi[1][2], hi[1][3]);
-            out.loz = make_float4(lo[2][0], lo[2][1], lo[2][2], lo[2][3]);
-            out.hiz = make_float4(hi[2][0], hi[2][1], hi[2][2], hi[2][3]);
-            out.child = make_int4(refs[0], refs[1], refs[2], refs[3]);
-            out.pad = make_int4(0, 0, 0, 0);
-            if(me < n4_cap)
-            {
-                n4[me] = out;
-                n4_range[me] = range[node_here];
-            }
-        }
     }
-    if(blockIdx.x * COLLAPSE_BLOCK >= count) return;// (the whole workgroup: it had no item)
+    else
+    {
+        // (each lane reads a level's count: a loop over them waited for one after the other)
+        level += st->top_levels;
+        if(level >= MAX_LEVELS) return;
+        uint32_t sum = lane < level ? st->level[lane] : 0u;
+        if(lane + 64u < level) sum += st->level[lane + 64u];
+        for(int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+        first = sum;
+        count = st->level[level];
+    }
+    while(true)
+    {
+        const uint32_t next = first + count;
+        for(uint32_t base = blockIdx.x * COLLAPSE_BLOCK; base < count; base += gridDim.x * COLLAPSE_BLOCK)
+        {
+            const bool active = base + threadIdx.x < count;
+            const uint32_t me = first + base + threadIdx.x;
+            collapse_child ch[4];
+            uint32_t ch_depth[4] = {0, 0, 0, 0};// depth of the BVH2 node each child came from
+            int cnt = 0;
+            uint32_t inner = 0, depth_here = 0;
+            int32_t node_here = 0;
+            if(active)
+            {
+                const int4 item = queue[me];
+                node_here = item.x;
+                auto open = [&](int slot_a, int slot_b, int32_t node, uint32_t d) {
+                    const vkrt_bvh_node nd = n2[node];
+                    ch[slot_a] = child_of(nd, 0);
+                    ch[slot_b] = child_of(nd, 1);
+                    ch_depth[slot_a] = ch_depth[slot_b] = d;
+                    depth = max(depth, d);
+                    for(const int k: {slot_a, slot_b})
+                    {
+                        const double a = child_area(ch[k]);
+                        if(ch[k].ref >= 0) sah += a;
+                        else
+                        {
+                            sah += ((static_cast<uint32_t>(~ch[k].ref) & 7u) + 1) * a;
+                            ++leaves;
+                            depth = max(depth, d + 1);
+                        }
+                    }
+                };
+                open(0, 1, item.x, static_cast<uint32_t>(item.z));
+                cnt = 2;
+    #pragma unroll
+                for(int step = 0; step < 2; ++step)
+                {
+                    int best = -1;
+                    float best_a = -1.0f;
+    #pragma unroll
+                    for(int j = 0; j < 3; ++j)
+                    {
+                        if(j >= cnt || ch[j].ref < 0) continue;
+                        const float a = half_area(ch[j]);
+                        if(a > best_a)
+                        {
+                            best_a = a;
+                            best = j;
+                        }
+                    }
+                    if(best < 0) break;
+                    // (constant slots: an array indexed by `best` would live in scratch memory)
+                    if(best == 0) open(0, 2 + step, ch[0].ref, ch_depth[0] + 1);
+                    else if(best == 1) open(1, 2 + step, ch[1].ref, ch_depth[1] + 1);
+                    else open(2, 3, ch[2].ref, ch_depth[2] + 1);
+                    ++cnt;
+                }
+                depth_here = static_cast<uint32_t>(item.y) + (cnt - 1);
+                stack = max(stack, depth_here);
+    #pragma unroll
+                for(int j = 0; j < 4; ++j)
+                    inner += j < cnt && ch[j].ref >= 0 && ch_depth[j] <= (uint32_t)STACK_SIZE ? 1u : 0u;
+            }
+            // the children's slots: an exclusive scan over the workgroup and one atomic
+            uint32_t sum = inner;
+            for(int off = 1; off < 64; off <<= 1)
+            {
+                const uint32_t y = __shfl_up(sum, off);
+                if(lane >= (uint32_t)off) sum += y;
+            }
+            if(lane == 63) wave_sum[wave] = sum;
+            __syncthreads();
+            uint32_t before = 0, total = 0;
+            for(uint32_t w = 0; w < COLLAPSE_BLOCK / 64; ++w)
+            {
+                before += w < wave ? wave_sum[w] : 0u;
+                total += wave_sum[w];
+            }
+            if(threadIdx.x == 0) slot_base = next + (total ? atomicAdd(&st->level[level + 1], total) : 0u);
+            __syncthreads();
+            uint32_t slot = slot_base + before + sum - inner;
+            if(active)
+            {
+                vkrt_bvh4_node out;
+                float lo[3][4], hi[3][4];
+                int32_t refs[4];
+    #pragma unroll
+                for(int j = 0; j < 4; ++j)
+                {
+                    for(int a = 0; a < 3; ++a)
+                    {
+                        lo[a][j] = j < cnt ? ch[j].lo[a] : 0.0f;
+                        hi[a][j] = j < cnt ? ch[j].hi[a] : 0.0f;
+                    }
+                    refs[j] = EMPTY_CHILD;
+                    if(j >= cnt) continue;
+                    if(ch[j].ref < 0) refs[j] = ch[j].ref;
+                    else if(ch_depth[j] <= (uint32_t)STACK_SIZE)
+                    {
+                        refs[j] = static_cast<int32_t>(slot);
+                        queue[slot++] = make_int4(ch[j].ref, static_cast<int32_t>(depth_here),
+                                                  static_cast<int32_t>(ch_depth[j] + 1), 0);
+                    }
+                }
+                out.lox = make_float4(lo[0][0], lo[0][1], lo[0][2], lo[0][3]);
+                out.hix = make_float4(hi[0][0], hi[0][1], hi[0][2], hi[0][3]);
+                out.loy = make_float4(lo[1][0], lo[1][1], lo[1][2], lo[1][3]);
+                out.hiy = make_float4(hi[1][0], hi[1][1], hi[1][2], hi[1][3]);
+                out.loz = make_float4(lo[2][0], lo[2][1], lo[2][2], lo[2][3]);
+                out.hiz = make_float4(hi[2][0], hi[2][1], hi[2][2], hi[2][3]);
+                out.child = make_int4(refs[0], refs[1], refs[2], refs[3]);
+                out.pad = make_int4(0, 0, 0, 0);
+                if(me < n4_cap)
+                {
+                    n4[me] = out;
+                    n4_range[me] = range[node_here];
+                }
+            }
+        }
+        if constexpr(!TOP) break;
+        // the next level, when there is one and it fits (its nodes' queue entries are this workgroup's own stores)
+        __syncthreads();
+        ++level;
+        first = next;
+        count = __hip_atomic_load(&st->level[level], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if(count == 0 || count > COLLAPSE_BLOCK) break;
+    }
+    if(TOP && threadIdx.x == 0) st->top_levels = level;
+    if(!TOP && blockIdx.x * COLLAPSE_BLOCK >= count) return;// (the whole workgroup: it had no item)
     for(int off = 32; off > 0; off >>= 1)
     {
         sah += __shfl_xor(sah, off);
@@ -1341,12 +1376,6 @@ __global__ void __launch_bounds__(COLLAPSE_BLOCK) k_collapse(const vkrt_bvh_node
         atomicMax(&st->depth, depth);
         atomicMax(&st->stack, stack);
     }
-}
-
-__global__ void k_collapse_root(int4 *__restrict__ queue, bvh_state *__restrict__ st)
-{
-    queue[0] = make_int4(0, 0, 1, 0);
-    st->level[0] = 1u;
 }
 
 //! refit of the 4-wide layout, a thread per child slot: a child's box is the union over its run of leaves, as when
@@ -1417,30 +1446,32 @@ static bool collapse(vkrt_ctx *ctx, vkrt_bvh *bvh, const binary_tree &bin)
     ctx->scratch[2].reserve((size_t)most_nodes * sizeof(int4));
     int4 *queue = ctx->scratch[2].as<int4>();
     bvh_state *st = ctx->state.as<bvh_state>();
-    k_collapse_root<<<1, 1, 0, s>>>(queue, st);
-    // the levels are launched without asking how many there are: as many as balanced trees of this size have and
+    vkrt_bvh4_node *n4 = bvh->nodes4.as<vkrt_bvh4_node>();
+    uint2 *n4_range = bvh->wide_range.as<uint2>();
+    k_collapse<true><<<1, COLLAPSE_BLOCK, 0, s>>>(bin.nodes, bin.range, queue, 0u, cap, n4, n4_range, st);
+    // the other levels are launched without asking how many there are: as many as balanced trees of this size have and
     // some more (a level that is not there costs its launch, 2 us), then in turns until the last one is empty
-    uint32_t level = 0, todo = 6;
+    uint32_t level = 0, todo = 2;
     for(size_t k = 1; k < most_nodes; k *= 4) ++todo;
     const bvh_state *got = nullptr;
     while(true)
     {
-        for(uint32_t stop = std::min(level + todo, MAX_LEVELS); level < stop; ++level)
+        for(uint32_t stop = level + todo; level < stop; ++level)
         {
-            const uint64_t most = std::min<uint64_t>(most_nodes, level < 16 ? 1ull << (2 * level) : most_nodes);
-            k_collapse<<<std::min(COLLAPSE_GRID, div_up(most, COLLAPSE_BLOCK)), COLLAPSE_BLOCK, 0, s>>>(
-                    bin.nodes, bin.range, queue, level, cap, bvh->nodes4.as<vkrt_bvh4_node>(),
-                    bvh->wide_range.as<uint2>(), st);
+            // (the first of them has a parent level of at most COLLAPSE_BLOCK nodes)
+            const uint64_t most =
+                    std::min<uint64_t>(most_nodes, level < 12 ? 4ull * COLLAPSE_BLOCK << (2 * level) : most_nodes);
+            k_collapse<false><<<std::min(COLLAPSE_GRID, div_up(most, COLLAPSE_BLOCK)), COLLAPSE_BLOCK, 0, s>>>(
+                    bin.nodes, bin.range, queue, level, cap, n4, n4_range, st);
         }
         got = &read_state(ctx, bin.nodes, nullptr);
         if(got->err) throw error(VKRT_E_INVALID_ARG, "triangle index out of range of the vertex count");
         if(got->depth > (uint32_t)STACK_SIZE) throw error(VKRT_E_INTERNAL, "BVH deeper than the traversal stack");
-        if(got->level[level] == 0) break;
-        VKRT_REQUIRE(level < MAX_LEVELS, "BVH4 collapse did not end");
+        if(got->top_levels + level >= MAX_LEVELS || got->level[got->top_levels + level] == 0) break;
         todo = 4;
     }
     uint64_t total = 0;
-    for(uint32_t l = 0; l < level; ++l) total += got->level[l];
+    for(uint32_t l = 0; l < MAX_LEVELS; ++l) total += got->level[l];
     VKRT_REQUIRE(total <= most_nodes, "BVH4 collapse overflow");
     vkrt_bvh_info &info = bvh->info;
     float rb[6];
