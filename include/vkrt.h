@@ -666,9 +666,10 @@ int vkrt_pt_set_lights(vkrt_pt *pt, const vkrt_light *lights, uint32_t n);
 /* Launch shape of the path tracer's kernels (no counterpart in the reference, whose RT pipeline schedules
  * itself). mode FULL_GRID (the default): one workgroup per tile of the pixel count at every depth, the tiles
  * past the live queue returning at once; PERSISTENT: the per-depth trace and shadow kernels are fixed grids of
- * the workgroups the GPU holds at once that claim the live queue's tiles with atomics. tail_depth (>= 1;
- * default VKRT_PT_TAIL_DEPTH_DEFAULT): outside the radiance-cache mode the paths alive at that depth finish in
- * one lane each, every remaining depth in one kernel; VKRT_PT_NO_TAIL keeps one launch per depth to the end.
+ * the workgroups the GPU holds at once that claim the live queue's tiles with atomics. tail_depth (>= 1,
+ * VKRT_PT_TAIL_DEPTH_DEFAULT for large images): outside the radiance-cache mode the paths alive at that depth finish in
+ * one lane each, every remaining depth in one kernel; VKRT_PT_NO_TAIL keeps one launch per depth to the end. A
+ * tracer on which this was never called chooses the depth by the number of pixels.
  * Every combination gives the same image bit for bit. */
 enum
 {

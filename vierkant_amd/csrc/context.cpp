@@ -30,6 +30,7 @@ int vkrt_create(int device, void *hip_stream, vkrt_ctx **out)
             VKRT_HIP(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
             ctx->own_stream = true;
         }
+        VKRT_HIP(hipStreamCreateWithFlags(&ctx->side_stream, hipStreamNonBlocking));
         hipDeviceProp_t prop{};
         VKRT_HIP(hipGetDeviceProperties(&prop, device));
         ctx->cu_count = prop.multiProcessorCount;
@@ -41,6 +42,7 @@ int vkrt_create(int device, void *hip_stream, vkrt_ctx **out)
     });
     if(rc != VKRT_OK)
     {
+        if(ctx->side_stream) (void)hipStreamDestroy(ctx->side_stream);
         if(ctx->own_stream && ctx->stream) (void)hipStreamDestroy(ctx->stream);
         delete ctx;
         return rc;
@@ -54,10 +56,12 @@ void vkrt_destroy(vkrt_ctx *ctx)
     if(!ctx) return;
     (void)hipSetDevice(ctx->device);
     if(ctx->stream) (void)hipStreamSynchronize(ctx->stream);
+    if(ctx->side_stream) (void)hipStreamSynchronize(ctx->side_stream);
     for(auto &b: ctx->staging) b.release();
     for(auto &b: ctx->scratch) b.release();
     ctx->state.release();
     if(ctx->pinned) (void)hipHostFree(ctx->pinned);
+    if(ctx->side_stream) (void)hipStreamDestroy(ctx->side_stream);
     if(ctx->own_stream && ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
 }

@@ -86,6 +86,10 @@ struct vkrt_ctx
     int device = 0;
     hipStream_t stream = nullptr;
     bool own_stream = false;
+    //! work that runs beside the context's stream (training paths, the second half of a path tracer's pixels). Made with
+    //! the context and shared by its objects: streams that come to share a hardware queue run one after the other, with
+    //! a barrier at every change (a tracer whose second stream did took 27 ms a frame instead of 21)
+    hipStream_t side_stream = nullptr;
     std::string last_error;
     int cu_count = 256;
     // fastest shape of the block x LDS depth x loop x XCD chunk sweep on MI355X (1.8M-triangle scene)

@@ -68,7 +68,8 @@ constexpr uint32_t PT_TRACE_CHUNK = 8;
 // kernel striding over its records; measured on the room scene (1920x1080, 64 spp, depth 8) it is slower,
 // 230 ms against 192 ms a frame: the hardware dispatcher hands out tiles faster than the claim atomics.
 constexpr uint32_t PT_CLAIMS = 2 * TRAIN_COUNTERS;// word offset of the trace kernel's claim counters
-constexpr uint32_t PT_COUNTER_WORDS = PT_CLAIMS + CLAIM_COUNTERS;
+constexpr uint32_t PT_COUNTER_WORDS = PT_CLAIMS + CLAIM_COUNTERS;// of one pixel group
+constexpr uint32_t PT_MAX_GROUPS = 2;
 constexpr uint32_t PT_TRACE_WAVES_PER_SIMD = 6;// the trace kernel's register cap (amdgpu_waves_per_eu): 80 VGPRs
 // the filter-free trace kernel fits 64 VGPRs with no spill: 8 waves per SIMD instead of 7 (room, 64 spp at
 // 1080p: 170.9 ms against 174.2)
@@ -79,7 +80,7 @@ constexpr uint32_t PT_SHADOW_PLAIN_WAVES_PER_SIMD = 5;
 // the two-level walk's cap: 96 VGPRs and 5 spilled instead of 80 and 14 (instanced room, 16 spp at 1080p:
 // 68.2 ms against 69.9 at 6 waves and 70.5 at 4)
 constexpr uint32_t PT_TRACE_INST_WAVES_PER_SIMD = 5;
-constexpr uint32_t PT_TAIL_DEPTH = VKRT_PT_TAIL_DEPTH_DEFAULT;// survivors at this depth finish in one lane each
+constexpr uint32_t PT_TAIL_AUTO = 0;// no tail depth was set: by the number of pixels (shape_of)
 
 //! f32tof16 / f16tof32 round trip (round to nearest even) of the media stack's packed ior
 __host__ __device__ inline float round_half(float x)
@@ -340,20 +341,11 @@ struct alpha_filter
 __device__ __forceinline__ vec3 xyz(const float4 &f) { return vec3{f.x, f.y, f.z}; }
 __device__ __forceinline__ float frac(float x) { return x - floorf(x); }
 
-__global__ void __launch_bounds__(PT_BLOCK) k_pt_begin(pt_frame f, pt_buffers b, uint32_t sample)
+//! the start of pixel p's path of a sample: the pixel's RNG state and sample offset (first sample), the lens sample,
+//! the camera ray and a fresh path state with the given flags
+__device__ __forceinline__ void begin_path(const pt_frame &f, const pt_buffers &b, uint32_t sample, uint32_t p,
+                                           uint32_t flags)
 {
-    const uint32_t p = blockIdx.x * PT_BLOCK + threadIdx.x;
-    // in the cache mode every train_stride-th pixel (from train_offset) traces a training path, queued on
-    // its own; the others keep their order in the main queue
-    const uint32_t n_train = f.cache_on ? f.n_train_paths : 0u;
-    if(p == 0)
-    {
-        b.counter[C_QUEUE] = f.n_pix - n_train;
-        b.counter[C_QUERIES] = 0u;
-        b.counter[C_RECORDS] = 0u;
-        b.counter[TRAIN_COUNTERS + C_QUEUE] = n_train;
-    }
-    if(p >= f.n_pix) return;
     const uint32_t x = p % f.width, y = p / f.width;
     uint4 st = b.state[p];
     float offset;
@@ -376,18 +368,7 @@ __global__ void __launch_bounds__(PT_BLOCK) k_pt_begin(pt_frame f, pt_buffers b,
     xi.x = rnd(rng);
     xi.y = rnd(rng);
     st.x = rng;
-    st.y = 0u;// media index 0, no regularization, no caustic marker
-    if(f.cache_on && p % f.train_stride == f.train_offset)
-    {
-        st.y = F_TRAIN;
-        float4 *tv = b.tvtx + (size_t)(p / f.train_stride) * f.max_depth * VERTEX_F4;
-        for(uint32_t d = 0; d < f.max_depth; ++d)
-        {
-            tv[d * VERTEX_F4 + 4] = make_float4(0.f, 0.f, 0.f, 0.f);
-            tv[d * VERTEX_F4 + 5] = make_float4(0.f, 0.f, 0.f, 0.f);
-            tv[d * VERTEX_F4 + 6] = make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-    }
+    st.y = flags;// media index 0, no regularization, no caustic marker
     b.state[p] = st;
 
     // camera_ray (raypipeline.slang:58-89), perspective branch, in the camera's own basis
@@ -407,8 +388,38 @@ __global__ void __launch_bounds__(PT_BLOCK) k_pt_begin(pt_frame f, pt_buffers b,
     b.iors[p] = make_float4(1.f, 1.f, 1.f, 1.f);
     if(f.any_volume) b.media[p] = make_uint2(0xffffffffu, 0xffffffffu);
     b.cone[p] = make_float2(f.cone_spread, 0.f);
-    if(n_train == 0u) b.queue[0][p] = p;
-    else if(st.y & F_TRAIN) b.train_queue[(p - f.train_offset) / f.train_stride] = p;
+}
+
+//! pixels first .. first + n - 1: the whole image, or one of the pixel groups of a batch without a cache
+__global__ void __launch_bounds__(PT_BLOCK) k_pt_begin(pt_frame f, pt_buffers b, uint32_t sample, uint32_t first,
+                                                       uint32_t n)
+{
+    const uint32_t q = blockIdx.x * PT_BLOCK + threadIdx.x, p = first + q;
+    // in the cache mode every train_stride-th pixel (from train_offset) traces a training path, queued on
+    // its own; the others keep their order in the main queue
+    const uint32_t n_train = f.cache_on ? f.n_train_paths : 0u;
+    if(q == 0)
+    {
+        b.counter[C_QUEUE] = n - n_train;
+        b.counter[C_QUERIES] = 0u;
+        b.counter[C_RECORDS] = 0u;
+        b.counter[TRAIN_COUNTERS + C_QUEUE] = n_train;
+    }
+    if(q >= n) return;
+    const bool train = f.cache_on && p % f.train_stride == f.train_offset;
+    if(train)
+    {
+        float4 *tv = b.tvtx + (size_t)(p / f.train_stride) * f.max_depth * VERTEX_F4;
+        for(uint32_t d = 0; d < f.max_depth; ++d)
+        {
+            tv[d * VERTEX_F4 + 4] = make_float4(0.f, 0.f, 0.f, 0.f);
+            tv[d * VERTEX_F4 + 5] = make_float4(0.f, 0.f, 0.f, 0.f);
+            tv[d * VERTEX_F4 + 6] = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    }
+    begin_path(f, b, sample, p, train ? F_TRAIN : 0u);
+    if(n_train == 0u) b.queue[0][q] = p;
+    else if(train) b.train_queue[(p - f.train_offset) / f.train_stride] = p;
     else
     {
         const uint32_t below = p > f.train_offset ? (p - f.train_offset - 1u) / f.train_stride + 1u : 0u;
@@ -1549,43 +1560,66 @@ __global__ void __launch_bounds__(PT_BLOCK) k_pt_train_paths(const vkrt_bvh_node
     atomicAdd(reinterpret_cast<unsigned long long *>(&b.counter[C_SEGMENTS]), (unsigned long long)segments);
 }
 
-//! the deep-bounce tail: the paths alive at depth d0 (queue `in`) finish in one lane each, trace, shade and
-//! shadow ray at every remaining depth with no kernel boundary between depths. Past the first few depths the
-//! live queue fills a fraction of the GPU and each per-depth launch lasts as long as its slowest wave's
-//! traversal (a chain of dependent node loads); here a wave's lanes run their depths back to back and the
-//! waves overlap. Each path performs the operations of the per-depth kernels in the same order (trace, shade,
-//! shadow ray, next depth), so the image is bit for bit the same.
+//! one path from depth d0 on, in one lane: trace, shade and shadow ray at every remaining depth; returns the
+//! segments traced
 template<bool LIGHTS, class F, bool INST>
+__device__ __forceinline__ uint32_t finish_path(const vkrt_bvh_node *__restrict__ nodes2, const float4 *__restrict__ tris,
+                                                int32_t root2, bool empty, const vkrt_bvh4_node *__restrict__ nodes4,
+                                                int32_t root4, bool wide, const pt_frame &f, const pt_buffers &b,
+                                                const pt_scene_dev &s, const F &flt, const F &shadow_flt, uint32_t d0,
+                                                uint32_t p, int32_t *smem, const pt_tlas &tl)
+{
+    uint32_t segments = 0;
+    for(uint32_t depth = d0; depth < f.max_depth; ++depth)
+    {
+        trace_path<PT_BLOCK, F, INST>(nodes2, tris, root2, empty, nodes4, root4, wide, b, p, smem, flt, depth, tl);
+        bool alive = false, to_cache = false, need_shadow = false;
+        float4 shadow_rec[SHADOW_F4];
+        float4 qfeat[QUERY_F4];
+        shade_path<LIGHTS, INST>(f, b, s, depth, p, alive, to_cache, need_shadow, shadow_rec, qfeat);
+        ++segments;
+        if(LIGHTS && need_shadow)
+            shadow_path<F, INST>(nodes2, root2, nodes4, root4, wide, empty, tris, s.mats, f, b, shadow_rec, smem,
+                                 shadow_flt, tl);
+        if(!alive) break;
+    }
+    return segments;
+}
+
+//! The deep-bounce tail, SAMPLES false: the paths alive at depth d0 (queue `in`) finish in one lane each, every
+//! remaining depth with no kernel boundary between depths. Past the first few depths the live queue fills a fraction
+//! of the GPU and each per-depth launch lasts as long as its slowest wave's traversal (a chain of dependent node
+//! loads); here a wave's lanes run their depths back to back and the waves overlap. SAMPLES true: the same from the
+//! camera on, for every sample of pixels d0 .. d0 + n - 1, a lane each: a small image fills so little of the GPU
+//! that every launch is such a tail (see shape_of). Each path performs the operations of the per-depth kernels in
+//! the same order (trace, shade, shadow ray, next depth), so the image is bit for bit the same.
+template<bool LIGHTS, class F, bool INST, bool SAMPLES>
 __global__ void __launch_bounds__(PT_BLOCK) k_pt_finish(const vkrt_bvh_node *__restrict__ nodes2,
                                                         const float4 *__restrict__ tris, int32_t root2, bool empty,
                                                         const vkrt_bvh4_node *__restrict__ nodes4, int32_t root4,
                                                         bool wide, pt_frame f, pt_buffers b, pt_scene_dev s, F flt,
-                                                        F shadow_flt, uint32_t d0, int in, pt_tlas tl)
+                                                        F shadow_flt, uint32_t d0, int in, uint32_t n, pt_tlas tl)
 {
     __shared__ int32_t smem[PT_LDS * PT_BLOCK];
     __shared__ unsigned long long s_segments;
     if(threadIdx.x == 0) s_segments = 0ull;
     __syncthreads();
     const uint32_t q = blockIdx.x * PT_BLOCK + threadIdx.x;
-    const uint32_t count = b.counter[C_QUEUE + in * COUNTER_LINE];
+    const uint32_t count = SAMPLES ? n : b.counter[C_QUEUE + in * COUNTER_LINE];
     uint32_t segments = 0;
     if(q < count)
     {
-        const uint32_t p = b.queue[in][q];
-        for(uint32_t depth = d0; depth < f.max_depth; ++depth)
-        {
-            trace_path<PT_BLOCK, F, INST>(nodes2, tris, root2, empty, nodes4, root4, wide, b, p, smem + threadIdx.x,
-                                          flt, depth, tl);
-            bool alive = false, to_cache = false, need_shadow = false;
-            float4 shadow_rec[SHADOW_F4];
-            float4 qfeat[QUERY_F4];
-            shade_path<LIGHTS, INST>(f, b, s, depth, p, alive, to_cache, need_shadow, shadow_rec, qfeat);
-            ++segments;
-            if(LIGHTS && need_shadow)
-                shadow_path<F, INST>(nodes2, root2, nodes4, root4, wide, empty, tris, s.mats, f, b, shadow_rec,
-                                     smem + threadIdx.x, shadow_flt, tl);
-            if(!alive) break;
-        }
+        const uint32_t p = SAMPLES ? d0 + q : b.queue[in][q];
+        if constexpr(SAMPLES)
+            for(uint32_t sample = 0; sample < f.num_samples; ++sample)
+            {
+                begin_path(f, b, sample, p, 0u);
+                segments += finish_path<LIGHTS, F, INST>(nodes2, tris, root2, empty, nodes4, root4, wide, f, b, s, flt,
+                                                         shadow_flt, 0u, p, smem + threadIdx.x, tl);
+            }
+        else
+            segments = finish_path<LIGHTS, F, INST>(nodes2, tris, root2, empty, nodes4, root4, wide, f, b, s, flt,
+                                                    shadow_flt, d0, p, smem + threadIdx.x, tl);
     }
     if(segments) atomicAdd(&s_segments, (unsigned long long)segments);
     __syncthreads();
@@ -1696,7 +1730,7 @@ struct vkrt_pt
     vkrt_ctx *ctx = nullptr;
     vkrt_pt_settings settings{};
     int launch_mode = VKRT_PT_LAUNCH_FULL_GRID;// per-depth launch shape (vkrt_pt_set_launch_mode)
-    uint32_t tail_depth = vkrt::PT_TAIL_DEPTH;  // survivors at this depth finish in one lane (k_pt_finish)
+    uint32_t tail_depth = vkrt::PT_TAIL_AUTO;   // survivors at this depth finish in one lane (k_pt_finish)
     bool any_alpha = false;                    // some material is alpha-tested (MASK or BLEND)
     bool any_volume = false;                   // some material has an interior medium
     // instanced scenes (vkrt_pt_set_instanced_scene): one BVH per mesh, the top level over the instances, per
@@ -1720,8 +1754,7 @@ struct vkrt_pt
     vkrt::device_buffer ray_o, ray_d, hit, beta, rad, state, iors, media, acc, info, queue0, queue1, counter, pixels, cone;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     // the cache mode's training paths: their own queues, traced on a second stream beside the main paths
-    hipStream_t train_stream = nullptr;
-    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+    hipEvent_t ev_fork = nullptr, ev_join = nullptr;// the side stream's fork from the context's and its return
     vkrt::device_buffer train_queue0, train_queue1;
     vkrt_pt_stats stats{};
     // radiance cache (not owned) and its per-sample buffers
@@ -1785,7 +1818,7 @@ static void resize_storage(vkrt_pt *pt, uint32_t w, uint32_t h)
     pt->info.reserve(n * 16);
     pt->queue0.reserve(n * 4);
     pt->queue1.reserve(n * 4);
-    pt->counter.reserve(PT_COUNTER_WORDS * sizeof(uint32_t));
+    pt->counter.reserve(PT_MAX_GROUPS * PT_COUNTER_WORDS * sizeof(uint32_t));
     pt->pixels.reserve(n * sizeof(vkrt_pixel));
     VKRT_HIP(hipMemsetAsync(pt->pixels.ptr, 0, n * sizeof(vkrt_pixel), pt->ctx->stream));
     pt->width = w;
@@ -1920,9 +1953,35 @@ static F filter_of(const alpha_filter &a)
     else return F{};
 }
 
+//! How a batch without a cache is launched: pixel groups (one on the side stream), and the depth from which paths
+//! finish in one lane (0: from the camera on, every sample, in one launch).
+//!
+//! A per-depth launch lasts at least as long as its longest ray (150 us, lit 190), so the fewer pixels share it the
+//! earlier the one-lane kernel is the better one, although it holds only 2 waves per SIMD, 131,072 lanes of 256 CUs.
+//! Measured on the room, ms a sample at tail depths 0, 1, 2, 3, 4, unlit and lit:
+//!     57,600 pixels  .44 .59 .70 .77 .82   1.32 1.69 2.00 2.27 2.52
+//!    230,400         .77 .58 .69 .81 .89   2.39 1.91 2.11 2.43 2.75
+//!    515,823        1.11 .97 .73 .85 .96   3.39 2.93 2.28 2.54 2.88
+//!    921,600          - 1.60 1.15 .95 1.05    - 4.35 3.40 2.79 3.09
+//!  2,073,600          - 2.94 2.08 1.65 1.49   - 8.42 6.01 4.70 4.16
+//! Two groups, one tracing its last long paths while the other fills the chip, gain from about a million pixels on
+//! (921,600 pixels .95 -> .92 and 2.79 -> 2.73 ms, 2,073,600 1.49 -> 1.35 and 4.16 -> 3.77) and cost below (230,400
+//! .58 -> .61). Three gain 2 % more there.
+struct batch_shape
+{
+    uint32_t groups, tail;
+};
+
+static batch_shape shape_of(const vkrt_pt *pt, uint32_t n_pix)
+{
+    const uint32_t lanes = static_cast<uint32_t>(pt->ctx->cu_count) * 4u * 2u * 64u;
+    const uint32_t tail = n_pix <= lanes ? 0u : n_pix <= 5 * lanes / 2 ? 1u : n_pix <= 5 * lanes ? 2u : n_pix <= 10 * lanes ? 3u : 4u;
+    return batch_shape{n_pix <= 5 * lanes ? 1u : PT_MAX_GROUPS, pt->tail_depth == PT_TAIL_AUTO ? tail : pt->tail_depth};
+}
+
 static void trace_batch(vkrt_pt *pt, const vkrt_camera &cam, uint32_t seed)
 {
-    hipStream_t s = pt->ctx->stream;
+    hipStream_t s = pt->ctx->stream, side = pt->ctx->side_stream;
     pt_frame f = make_frame(pt, cam, seed);
     pt_buffers b = buffers(pt);
     const pt_scene_dev sc = scene_dev(pt);
@@ -1984,7 +2043,29 @@ static void trace_batch(vkrt_pt *pt, const vkrt_camera &cam, uint32_t seed)
         VKRT_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, block, 0));
         return full ? cap : std::min<uint32_t>(cus * static_cast<uint32_t>(std::max(per_cu, 1)), cap);
     };
-    const uint32_t trace_full = div_up(f.n_pix, PT_TRACE_BLOCK);
+    // the batch's pixel groups (one in the cache mode, whose second stream is the training paths')
+    const batch_shape shape = shape_of(pt, f.n_pix);
+    const uint32_t n_groups = f.cache_on ? 1u : shape.groups;
+    struct group
+    {
+        uint32_t first, n, blocks, trace_grid, shadow_grid;
+        hipStream_t stream;
+        pt_buffers b;
+    };
+    group groups[PT_MAX_GROUPS];
+    for(uint32_t g = 0; g < n_groups; ++g)
+    {
+        group &r = groups[g];
+        r.first = static_cast<uint32_t>((uint64_t)f.n_pix * g / n_groups);
+        r.n = static_cast<uint32_t>((uint64_t)f.n_pix * (g + 1) / n_groups) - r.first;
+        r.blocks = div_up(r.n, PT_BLOCK);
+        r.stream = g ? side : s;
+        r.b = b;
+        r.b.queue[0] += r.first;
+        r.b.queue[1] += r.first;
+        r.b.counter += g * PT_COUNTER_WORDS;
+        if(r.b.shadow) r.b.shadow += (size_t)r.first * SHADOW_F4;
+    }
     // compile-time variants: any-hit filter or none, flat or instanced scene
     const bool inst = pt->instanced;
     const pt_tlas tl = pt->tlas;
@@ -1996,64 +2077,102 @@ static void trace_batch(vkrt_pt *pt, const vkrt_camera &cam, uint32_t seed)
         if(alpha) by_inst(std::true_type{});
         else by_inst(std::false_type{});
     };
-    uint32_t trace_grid = 0, shadow_grid = 0;
     variant([&](auto a, auto in_) {
         using F = std::conditional_t<decltype(a)::value, alpha_filter, keep_all>;
-        trace_grid = resident(k_pt_trace<F, decltype(in_)::value>, PT_TRACE_BLOCK, trace_full);
-        shadow_grid = resident(k_pt_shadow<F, decltype(in_)::value>, PT_BLOCK, blocks);
+        for(uint32_t g = 0; g < n_groups; ++g)
+        {
+            groups[g].trace_grid =
+                    resident(k_pt_trace<F, decltype(in_)::value>, PT_TRACE_BLOCK, div_up(groups[g].n, PT_TRACE_BLOCK));
+            groups[g].shadow_grid = resident(k_pt_shadow<F, decltype(in_)::value>, PT_BLOCK, groups[g].blocks);
+        }
     });
-    auto depth_step = [&](hipStream_t st, const pt_buffers &bb, uint32_t depth, int in) {
+    auto depth_step = [&](const group &g, uint32_t depth, int in) {
+        const pt_buffers &bb = g.b;
+        hipStream_t st = g.stream;
         k_pt_reset_depth<<<1, XCDS, 0, st>>>(bb.counter, in ^ 1);
         variant([&](auto a, auto in_) {
             using F = std::conditional_t<decltype(a)::value, alpha_filter, keep_all>;
             constexpr bool I = decltype(in_)::value;
-            k_pt_trace<F, I><<<trace_grid, PT_TRACE_BLOCK, 0, st>>>(nodes2, tris, root_ref, flat_empty, nodes4,
-                                                                    root4, wide, bb, in, filter_of<F>(flt),
-                                                                    depth, tl);
+            k_pt_trace<F, I><<<g.trace_grid, PT_TRACE_BLOCK, 0, st>>>(nodes2, tris, root_ref, flat_empty, nodes4,
+                                                                      root4, wide, bb, in, filter_of<F>(flt),
+                                                                      depth, tl);
             if(f.n_lights)
             {
-                k_pt_shade<true, I><<<blocks, PT_BLOCK, 0, st>>>(f, bb, sc, depth, in);
-                k_pt_shadow<F, I><<<shadow_grid, PT_BLOCK, 0, st>>>(nodes2, root_ref, nodes4, root4,
-                                                                    wide, flat_empty, tris, sc.mats, f, bb,
-                                                                    filter_of<F>(shadow_flt), tl);
+                k_pt_shade<true, I><<<g.blocks, PT_BLOCK, 0, st>>>(f, bb, sc, depth, in);
+                k_pt_shadow<F, I><<<g.shadow_grid, PT_BLOCK, 0, st>>>(nodes2, root_ref, nodes4, root4,
+                                                                      wide, flat_empty, tris, sc.mats, f, bb,
+                                                                      filter_of<F>(shadow_flt), tl);
             }
             else
-                k_pt_shade<false, I><<<blocks, PT_BLOCK, 0, st>>>(f, bb, sc, depth, in);
+                k_pt_shade<false, I><<<g.blocks, PT_BLOCK, 0, st>>>(f, bb, sc, depth, in);
+        });
+    };
+    // the survivors at the tail depth finish in one lane each; from depth 0 on, all samples in one launch
+    auto finish = [&](const group &g, uint32_t depth) {
+        const int in = static_cast<int>(depth & 1u);
+        variant([&](auto a, auto in_) {
+            using F = std::conditional_t<decltype(a)::value, alpha_filter, keep_all>;
+            constexpr bool I = decltype(in_)::value;
+            auto launch = [&](auto lights, auto samples) {
+                k_pt_finish<decltype(lights)::value, F, I, decltype(samples)::value>
+                        <<<g.blocks, PT_BLOCK, 0, g.stream>>>(nodes2, tris, root_ref, flat_empty, nodes4, root4, wide, f,
+                                                              g.b, sc, filter_of<F>(flt), filter_of<F>(shadow_flt),
+                                                              depth ? depth : g.first, in, g.n, tl);
+            };
+            if(f.n_lights && depth) launch(std::true_type{}, std::false_type{});
+            else if(f.n_lights) launch(std::true_type{}, std::true_type{});
+            else if(depth) launch(std::false_type{}, std::false_type{});
+            else launch(std::false_type{}, std::true_type{});
         });
     };
     VKRT_HIP(hipEventRecord(pt->ev0, s));
-    k_pt_zero<<<1, PT_BLOCK, 0, s>>>(b.counter, 2 * TRAIN_COUNTERS);
-    for(uint32_t sample = 0; sample < f.num_samples; ++sample)
+    k_pt_zero<<<1, PT_BLOCK, 0, s>>>(b.counter, n_groups * PT_COUNTER_WORDS);
+    if(n_groups > 1)
+    {
+        VKRT_HIP(hipEventRecord(pt->ev_fork, s));
+        VKRT_HIP(hipStreamWaitEvent(side, pt->ev_fork, 0));
+    }
+    const bool whole = !f.cache_on && shape.tail == 0u;
+    for(uint32_t g = 0; whole && g < n_groups; ++g) finish(groups[g], 0u);
+    for(uint32_t sample = 0; !whole && sample < f.num_samples; ++sample)
     {
         uint32_t main_depths = f.max_depth;
-        if(f.cache_on)
+        if(!f.cache_on)
         {
-            // training pixels move every sample: offset from the batch seed and the sample index
-            f.train_offset = xxhash32(seed, sample) % f.train_stride;
-            f.n_train_paths = f.train_offset < f.n_pix ? div_up(f.n_pix - f.train_offset, f.train_stride) : 0u;
-            // paths other than training paths end at the cache depth
-            main_depths = std::min(f.max_depth, f.cache_depth + 1u);
+            // every pixel's samples are a chain of their own, so the groups never wait for each other: while one
+            // traces its last long paths, another fills the chip
+            const uint32_t per_depth = std::min(main_depths, shape.tail);
+            for(uint32_t g = 0; g < n_groups; ++g)
+            {
+                const group &r = groups[g];
+                k_pt_begin<<<r.blocks, PT_BLOCK, 0, r.stream>>>(f, r.b, sample, r.first, r.n);
+                for(uint32_t depth = 0; depth < per_depth; ++depth) depth_step(r, depth, static_cast<int>(depth & 1u));
+                if(per_depth < main_depths) finish(r, per_depth);
+            }
+            continue;
         }
-        k_pt_begin<<<blocks, PT_BLOCK, 0, s>>>(f, b, sample);
-        const bool fork = f.cache_on && f.n_train_paths;
-        // the deep-bounce tail (not in the cache mode, whose main paths end at the cache depth and queue cache
-        // queries): the survivors at tail_depth finish in one lane each
-        const uint32_t per_depth = f.cache_on ? main_depths : std::min(main_depths, pt->tail_depth);
+        // the cache mode. Training pixels move every sample: offset from the batch seed and the sample index
+        f.train_offset = xxhash32(seed, sample) % f.train_stride;
+        f.n_train_paths = f.train_offset < f.n_pix ? div_up(f.n_pix - f.train_offset, f.train_stride) : 0u;
+        // paths other than training paths end at the cache depth (and queue cache queries: no tail)
+        main_depths = std::min(f.max_depth, f.cache_depth + 1u);
+        k_pt_begin<<<blocks, PT_BLOCK, 0, s>>>(f, b, sample, 0u, f.n_pix);
+        const bool fork = f.n_train_paths != 0u;
         if(fork) VKRT_HIP(hipEventRecord(pt->ev_fork, s));
         // the first depth is queued before the training stream's launches, so the main stream does not wait
         // for the host to queue them
-        if(per_depth > 0) depth_step(s, b, 0, 0);
+        depth_step(groups[0], 0, 0);
         if(fork)
         {
             // the training paths' long, narrow tail is latency-bound: it runs on the second stream while the
             // main stream traces the full-width depths, followed there by the training step (targets, gradients,
             // Adam), which no main-path kernel reads before the cache query; the query waits for it, so the
             // main paths terminate into the cache as trained on this sample's training paths
-            VKRT_HIP(hipStreamWaitEvent(pt->train_stream, pt->ev_fork, 0));
+            VKRT_HIP(hipStreamWaitEvent(side, pt->ev_fork, 0));
             const uint32_t tgrid = div_up(f.n_train_paths, PT_BLOCK);
             auto train = [&](auto lights, auto in_) {
                 k_pt_train_paths<decltype(lights)::value, decltype(in_)::value>
-                        <<<tgrid, PT_BLOCK, 0, pt->train_stream>>>(nodes2, tris, root_ref, flat_empty, nodes4,
+                        <<<tgrid, PT_BLOCK, 0, side>>>(nodes2, tris, root_ref, flat_empty, nodes4,
                                                                    root4, wide, f, bt, sc, tl);
             };
             if(f.n_lights && inst) train(std::true_type{}, std::true_type{});
@@ -2062,47 +2181,40 @@ static void trace_batch(vkrt_pt *pt, const vkrt_camera &cam, uint32_t seed)
             else train(std::false_type{}, std::false_type{});
             if(f.train_max)
             {
-                k_pt_train_targets<<<tgrid, PT_BLOCK, 0, pt->train_stream>>>(f, b);
-                rc::train(pt->rc, b.trec, 4, b.ttgt, f.train_max, false, b.counter + C_RECORDS, pt->train_stream);
+                k_pt_train_targets<<<tgrid, PT_BLOCK, 0, side>>>(f, b);
+                rc::train(pt->rc, b.trec, 4, b.ttgt, f.train_max, false, b.counter + C_RECORDS, side);
             }
             VKRT_HIP(hipGetLastError());
-            VKRT_HIP(hipEventRecord(pt->ev_join, pt->train_stream));
+            VKRT_HIP(hipEventRecord(pt->ev_join, side));
         }
-        for(uint32_t depth = 1; depth < per_depth; ++depth) depth_step(s, b, depth, static_cast<int>(depth & 1u));
-        if(per_depth < main_depths && per_depth > 0)
-        {
-            const int in = static_cast<int>(per_depth & 1u);
-            variant([&](auto a, auto in_) {
-                using F = std::conditional_t<decltype(a)::value, alpha_filter, keep_all>;
-                constexpr bool I = decltype(in_)::value;
-                if(f.n_lights)
-                    k_pt_finish<true, F, I><<<blocks, PT_BLOCK, 0, s>>>(
-                        nodes2, tris, root_ref, flat_empty, nodes4, root4, wide, f, b, sc,
-                        filter_of<F>(flt), filter_of<F>(shadow_flt), per_depth, in, tl);
-                else
-                    k_pt_finish<false, F, I><<<blocks, PT_BLOCK, 0, s>>>(
-                        nodes2, tris, root_ref, flat_empty, nodes4, root4, wide, f, b, sc,
-                        filter_of<F>(flt), filter_of<F>(shadow_flt), per_depth, in, tl);
-            });
-        }
-        if(f.cache_on)
-        {
-            if(fork) VKRT_HIP(hipStreamWaitEvent(s, pt->ev_join, 0));
-            rc::query(pt->rc, b.qrec, QUERY_F4, f.n_pix, nullptr, b.acc, b.counter + C_QUERIES);
-        }
+        for(uint32_t depth = 1; depth < main_depths; ++depth) depth_step(groups[0], depth, static_cast<int>(depth & 1u));
+        if(fork) VKRT_HIP(hipStreamWaitEvent(s, pt->ev_join, 0));
+        rc::query(pt->rc, b.qrec, QUERY_F4, f.n_pix, nullptr, b.acc, b.counter + C_QUERIES);
+    }
+    if(n_groups > 1)
+    {
+        VKRT_HIP(hipEventRecord(pt->ev_join, side));
+        VKRT_HIP(hipStreamWaitEvent(s, pt->ev_join, 0));
     }
     k_pt_resolve<<<blocks, PT_BLOCK, 0, s>>>(f, b);
     VKRT_HIP(hipEventRecord(pt->ev1, s));
     VKRT_HIP(hipGetLastError());
-    uint64_t seg[2] = {0, 0};
-    VKRT_HIP(hipMemcpyAsync(&seg[0], b.counter + C_SEGMENTS, 8, hipMemcpyDeviceToHost, s));
-    VKRT_HIP(hipMemcpyAsync(&seg[1], b.counter + TRAIN_COUNTERS + C_SEGMENTS, 8, hipMemcpyDeviceToHost, s));
+    std::vector<uint32_t> counters(n_groups * PT_COUNTER_WORDS);
+    VKRT_HIP(hipMemcpyAsync(counters.data(), b.counter, counters.size() * 4, hipMemcpyDeviceToHost, s));
     VKRT_HIP(hipStreamSynchronize(s));
+    uint64_t segments = 0;
+    for(uint32_t g = 0; g < n_groups; ++g)
+        for(const uint32_t at: {C_SEGMENTS, TRAIN_COUNTERS + C_SEGMENTS})
+        {
+            uint64_t n = 0;
+            std::memcpy(&n, &counters[g * PT_COUNTER_WORDS + at], sizeof n);
+            segments += n;
+        }
     float ms = 0.f;
     VKRT_HIP(hipEventElapsedTime(&ms, pt->ev0, pt->ev1));
     pt->stats.raytrace_ms = ms;
     pt->stats.traced = 1;
-    pt->stats.segments = seg[0] + seg[1];
+    pt->stats.segments = segments;
     pt->stats.samples = (uint64_t)f.n_pix * f.num_samples;
 }
 
@@ -2132,7 +2244,6 @@ int vkrt_pt_create(vkrt_ctx *ctx, const vkrt_pt_settings *settings, uint32_t see
         VKRT_HIP(hipEventCreate(&pt->ev1));
         VKRT_HIP(hipEventCreateWithFlags(&pt->ev_fork, hipEventDisableTiming));
         VKRT_HIP(hipEventCreateWithFlags(&pt->ev_join, hipEventDisableTiming));
-        VKRT_HIP(hipStreamCreateWithFlags(&pt->train_stream, hipStreamNonBlocking));
         *out = pt.release();
     });
 }
@@ -2147,13 +2258,12 @@ void vkrt_pt_destroy(vkrt_pt *pt)
     if(!pt) return;
     (void)hipSetDevice(pt->ctx->device);
     (void)hipStreamSynchronize(pt->ctx->stream);
-    if(pt->train_stream) (void)hipStreamSynchronize(pt->train_stream);
+    (void)hipStreamSynchronize(pt->ctx->side_stream);
     release_scene_accel(pt);
     if(pt->ev0) (void)hipEventDestroy(pt->ev0);
     if(pt->ev1) (void)hipEventDestroy(pt->ev1);
     if(pt->ev_fork) (void)hipEventDestroy(pt->ev_fork);
     if(pt->ev_join) (void)hipEventDestroy(pt->ev_join);
-    if(pt->train_stream) (void)hipStreamDestroy(pt->train_stream);
     delete pt;
 }
 
