@@ -1,10 +1,12 @@
 // radiance_cache.hip - kernels and C ABI of the neural radiance cache (layout and methods: radiance_cache.hpp).
 //
-//   k_rc_query    per wave 4 x 16 samples: hash-grid + SH encoding in registers, 6 MFMA layers, output
+//   k_rc_encode   per record and table level: hash-grid features, each XCD reading two levels of its own
+//   k_rc_query    per wave 4 x 16 samples: inputs in registers, 6 MFMA layers, output
 //   k_rc_train    per block 64 samples per iteration: forward (activations to LDS), relative L2 loss,
-//                 back-propagation, weight gradients contracted over the samples in LDS, hash-grid gradient
-//                 scattered with packed fp16x2 atomics (one per corner, loss-scaled by a power of two);
-//                 per-block weight gradients written to a partial buffer
+//                 back-propagation, weight gradients contracted over the samples in LDS; per-block weight
+//                 gradients written to a partial buffer, feature gradients per record
+//   k_rc_scatter  per record and table level: hash-grid gradient scattered with packed fp16x2 atomics (one per
+//                 corner, loss-scaled by a power of two), each XCD writing two levels of its own
 //   k_rc_adam_mlp per weight: sum of the block partials in block order (deterministic), Adam, bf16 swizzles
 //   k_rc_adam_grid per grid parameter: Adam where the gradient is non-zero, fp16 copy for the encoder
 #include <algorithm>
@@ -12,6 +14,7 @@
 #include <memory>
 #include <vector>
 
+#include "kernels.hpp"
 #include "radiance_cache.hpp"
 
 namespace vkrt::rc
@@ -32,10 +35,46 @@ __device__ __forceinline__ void load_record(const float4 *records, uint32_t stri
     rec[3] = r[3];
 }
 
+//! a record's position word, read past the caches' least recently used order
+__device__ __forceinline__ float4 load_position(const float4 *rec)
+{
+    const f32x4 v = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(rec));
+    return make_float4(v[0], v[1], v[2], v[3]);
+}
+
+//! the records' features, two threads per record and two levels (see xcd_level). Bound by the
+//! line fills of the L1s, four per record and level: 262,144 random records take 100 us (140 with the eight corners asked
+//! for one after the other, whatever the L2s held), and the network's pass 26 us, where one kernel that read all levels
+//! in every wave took 184. *loss, if given, is set to zero.
+constexpr uint32_t ENC_BLOCK = 256, ENC_RECORDS = ENC_BLOCK / 2;
+__global__ void __launch_bounds__(ENC_BLOCK) k_rc_encode(cache_dev c, const float4 *__restrict__ records,
+                                                         uint32_t stride_f4, uint32_t n_host,
+                                                         const uint32_t *__restrict__ n_dev,
+                                                         bf16x2 *__restrict__ enc, size_t enc_stride,
+                                                         float *__restrict__ loss)
+{
+    if(loss && blockIdx.x == 0 && threadIdx.x == 0) *loss = 0.0f;
+    const uint32_t n = n_dev ? min(*n_dev, n_host) : n_host;
+    const uint32_t i = (blockIdx.x / XCDS) * ENC_RECORDS + threadIdx.x / 2, dx = threadIdx.x & 1u;
+    float p[3] = {0.f, 0.f, 0.f};
+    if(i < n) unit_position(c.g, load_position(records + (size_t)i * stride_f4), p);
+#pragma unroll
+    for(uint32_t k = 0; k < 2; ++k)
+    {
+        const uint32_t level = xcd_level(blockIdx.x % XCDS, k);
+        const bf16x2 e = encode_level(c, level, p, dx, i < n);
+        // (streamed past the L2's tables)
+        if(i < n && dx == 0)
+            __builtin_nontemporal_store(__builtin_bit_cast(uint32_t, e),
+                                        reinterpret_cast<uint32_t *>(enc + level * enc_stride + i));
+    }
+}
+
 __global__ void __launch_bounds__(QUERY_BLOCK) k_rc_query(cache_dev c, const float4 *__restrict__ records,
                                                           uint32_t stride_f4, uint32_t n_host,
-                                                          const uint32_t *__restrict__ n_dev, float4 *__restrict__ out,
-                                                          float4 *__restrict__ pixel_acc)
+                                                          const uint32_t *__restrict__ n_dev,
+                                                          const bf16x2 *__restrict__ enc, size_t enc_stride,
+                                                          float4 *__restrict__ out, float4 *__restrict__ pixel_acc)
 {
     const uint32_t n = n_dev ? *n_dev : n_host;
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
@@ -47,17 +86,14 @@ __global__ void __launch_bounds__(QUERY_BLOCK) k_rc_query(cache_dev c, const flo
     for(int t = 0; t < QUERY_TILES; ++t)
     {
         const uint32_t i = base + 16 * t + (lane & 15u);
-        float v[16];
         if(i < n)
         {
             float4 rec[4];
             load_record(records, stride_f4, i, rec);
-            encode_group(c, rec, group, v);
+            input_group(enc + i, enc_stride, rec, group, b[t]);
         }
         else
-            for(int k = 0; k < 16; ++k) v[k] = 0.0f;
-        b[t][0] = pack8(v);
-        b[t][1] = pack8(v + 8);
+            for(int j = 0; j < 8; ++j) b[t][0][j] = b[t][1][j] = static_cast<__bf16>(0.0f);
     }
     f32x4 y[QUERY_TILES];
     mlp_forward<QUERY_TILES>(c.w_fwd, lane, b, y);
@@ -87,8 +123,9 @@ __global__ void __launch_bounds__(QUERY_BLOCK) k_rc_query(cache_dev c, const flo
 __global__ void __launch_bounds__(TRAIN_BLOCK) k_rc_train(cache_dev c, const float4 *__restrict__ records,
                                                           uint32_t stride_f4, const float4 *__restrict__ targets,
                                                           uint32_t n_cap, const uint32_t *__restrict__ n_dev,
-                                                          half2v *__restrict__ grid_grad, float grad_scale,
-                                                          float *__restrict__ partials, float *__restrict__ loss_sum)
+                                                          const bf16x2 *__restrict__ enc, float2 *__restrict__ enc_grad,
+                                                          size_t enc_stride, float *__restrict__ partials,
+                                                          float *__restrict__ loss_sum)
 {
     // sample count: n_cap, or the device counter clamped to n_cap
     const uint32_t n = n_dev ? min(*n_dev, n_cap) : n_cap;
@@ -96,7 +133,6 @@ __global__ void __launch_bounds__(TRAIN_BLOCK) k_rc_train(cache_dev c, const flo
     __shared__ __bf16 dzs[WIDTH][LDS_ROW];          // the current layer's output gradient, [feature][sample]
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, group = lane >> 4, col = lane & 15u;
     const uint32_t m_local = 16 * wave + col;
-    const size_t table = size_t(1) << c.g.log2_t;
 
     f32x4 dw[N_HIDDEN][4];// W1..W5: row tile = wave, column tiles 0..3
     f32x4 dw6 = {0.f, 0.f, 0.f, 0.f};
@@ -111,19 +147,18 @@ __global__ void __launch_bounds__(TRAIN_BLOCK) k_rc_train(cache_dev c, const flo
     {
         const uint32_t m = it * TRAIN_SAMPLES + m_local;
         const bool valid = m < n;
-        float4 rec[4];
-        float v[16];
+        bf16x8 b[2];
         if(valid)
         {
+            float4 rec[4];
             load_record(records, stride_f4, m, rec);
-            encode_group(c, rec, group, v);
+            input_group(enc + m, enc_stride, rec, group, b);
         }
         else
-            for(int k = 0; k < 16; ++k) v[k] = 0.0f;
+            for(int j = 0; j < 8; ++j) b[0][j] = b[1][j] = static_cast<__bf16>(0.0f);
         __syncthreads();// the previous iteration's readers of act / dzs are done
 #pragma unroll
-        for(int k = 0; k < 16; ++k) act[0][16 * group + k][m_local] = static_cast<__bf16>(v[k]);
-        bf16x8 b[2] = {pack8(v), pack8(v + 8)};
+        for(int k = 0; k < 16; ++k) act[0][16 * group + k][m_local] = b[k / 8][k % 8];
 
         // ---- forward -------------------------------------------------------------------------------
         uint32_t relu_mask[N_HIDDEN];
@@ -231,31 +266,13 @@ __global__ void __launch_bounds__(TRAIN_BLOCK) k_rc_train(cache_dev c, const flo
             }
         }
 
-        // ---- hash-grid gradient: dh now holds dL/dx0; lane groups 0 and 1 carry the grid features -----
+        // ---- feature gradients: dh now holds dL/dx0; lane groups 0 and 1 carry the grid features ------
         if(valid && group < 2)
-        {
-            float p[3];
-            unit_position(c.g, rec[0], p);
 #pragma unroll
             for(int r = 0; r < 4; ++r)
 #pragma unroll
                 for(int h = 0; h < 2; ++h)
-                {
-                    const uint32_t level = 4 * r + 2 * group + h;
-                    const float g0 = dh[r][2 * h], g1 = dh[r][2 * h + 1];
-                    if(g0 == 0.0f && g1 == 0.0f) continue;
-                    uint32_t idx[8];
-                    float w[8];
-                    level_corners(c.g, level, p, idx, w);
-                    const float s0 = g0 * grad_scale, s1 = g1 * grad_scale;
-#pragma unroll
-                    for(int k = 0; k < 8; ++k)
-                    {
-                        const half2v val = {static_cast<_Float16>(w[k] * s0), static_cast<_Float16>(w[k] * s1)};
-                        __builtin_amdgcn_global_atomic_fadd_v2f16(grid_grad + (level * table + idx[k]), val);
-                    }
-                }
-        }
+                    enc_grad[(4 * r + 2 * group + h) * enc_stride + m] = make_float2(dh[r][2 * h], dh[r][2 * h + 1]);
     }
 
     // ---- per-block weight gradients, logical [out][in] layout ------------------------------------------
@@ -281,6 +298,40 @@ __global__ void __launch_bounds__(TRAIN_BLOCK) k_rc_train(cache_dev c, const flo
     if(lane == 0) atomicAdd(loss_sum, loss_lane);
 }
 
+//! the hash-grid gradient of the records' feature gradients, two threads per record and two levels as in k_rc_encode: an
+//! entry's updates then meet in one L2, and a corner's with its neighbour's in one request (16,384 records: 61 us, 114
+//! with a corner a lane)
+__global__ void __launch_bounds__(ENC_BLOCK) k_rc_scatter(cache_dev c, const float4 *__restrict__ records,
+                                                          uint32_t stride_f4, uint32_t n_cap,
+                                                          const uint32_t *__restrict__ n_dev,
+                                                          const float2 *__restrict__ enc_grad, size_t enc_stride,
+                                                          half2v *__restrict__ grid_grad, float grad_scale)
+{
+    const uint32_t n = n_dev ? min(*n_dev, n_cap) : n_cap;
+    const uint32_t i = (blockIdx.x / XCDS) * ENC_RECORDS + threadIdx.x / 2, dx = threadIdx.x & 1u;
+    if(i >= n) return;
+    float p[3];
+    unit_position(c.g, load_position(records + (size_t)i * stride_f4), p);
+#pragma unroll
+    for(uint32_t k = 0; k < 2; ++k)
+    {
+        const uint32_t level = xcd_level(blockIdx.x % XCDS, k);
+        const float2 g = enc_grad[level * enc_stride + i];
+        if(g.x == 0.0f && g.y == 0.0f) continue;
+        uint32_t idx[4];
+        float w[4];
+        level_corners(c.g, level, p, dx, idx, w);
+        half2v *table = grid_grad + ((size_t)level << c.g.log2_t);
+        const float s0 = g.x * grad_scale, s1 = g.y * grad_scale;
+#pragma unroll
+        for(int j = 0; j < 4; ++j)
+        {
+            const half2v val = {static_cast<_Float16>(w[j] * s0), static_cast<_Float16>(w[j] * s1)};
+            __builtin_amdgcn_global_atomic_fadd_v2f16(table + idx[j], val);
+        }
+    }
+}
+
 struct adam_consts
 {
     float lr, beta1, beta2, eps, c1, c2;// c1 = 1 / (1 - beta1^t), c2 = 1 / (1 - beta2^t)
@@ -302,22 +353,29 @@ __device__ __forceinline__ void publish_weight(uint32_t k, float w, __bf16 *w_fw
     w_bwd[bwd_pos(layer, out, in)] = static_cast<__bf16>(w);
 }
 
-__global__ void k_rc_adam_mlp(float *__restrict__ master, float *__restrict__ mom, float *__restrict__ vel,
-                              float *__restrict__ grad_out, const float *__restrict__ partials, uint32_t n_blocks,
-                              adam_consts a, int apply, __bf16 *__restrict__ w_fwd, __bf16 *__restrict__ w_bwd)
+//! MLP_K weights a workgroup; the partials of blocks j mod 8 are summed by thread row j, the eight sums combined in a
+//! fixed order: deterministic. The step's loss goes to pinned host memory on the way. (All eight sums by one thread per weight left 172 CUs idle: 15.5 us, 5.4 now.)
+constexpr uint32_t MLP_K = 32, MLP_SUMS = 8;
+__global__ void __launch_bounds__(MLP_K *MLP_SUMS) k_rc_adam_mlp(float *__restrict__ master, float *__restrict__ mom,
+                                                                 float *__restrict__ vel, float *__restrict__ grad_out,
+                                                                 const float *__restrict__ partials, uint32_t n_blocks,
+                                                                 adam_consts a, int apply, __bf16 *__restrict__ w_fwd,
+                                                                 __bf16 *__restrict__ w_bwd,
+                                                                 const float *__restrict__ loss,
+                                                                 float *__restrict__ host_loss)
 {
-    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    if(k >= N_MLP) return;
-    // eight independent partial sums (blocks b = j mod 8), combined in a fixed order: deterministic
-    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    uint32_t b = 0;
-    for(; b + 8 <= n_blocks; b += 8)
-#pragma unroll
-        for(int j = 0; j < 8; ++j) acc[j] = acc[j] + partials[(size_t)(b + j) * N_MLP + k];
-#pragma unroll
-    for(int j = 0; j < 8; ++j)
-        if(b + j < n_blocks) acc[j] = acc[j] + partials[(size_t)(b + j) * N_MLP + k];
-    const float g = ((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7]));
+    static_assert(N_MLP % MLP_K == 0);
+    if(blockIdx.x == 0 && threadIdx.x == 0) *host_loss = *loss;
+    __shared__ float sum[MLP_SUMS][MLP_K];
+    const uint32_t col = threadIdx.x % MLP_K, j = threadIdx.x / MLP_K, k = blockIdx.x * MLP_K + col;
+    float s = 0.f;
+#pragma unroll 8
+    for(uint32_t b = j; b < n_blocks; b += MLP_SUMS) s = s + partials[(size_t)b * N_MLP + k];
+    sum[j][col] = s;
+    __syncthreads();
+    if(j != 0) return;
+    const float g = ((sum[0][col] + sum[1][col]) + (sum[2][col] + sum[3][col])) +
+                    ((sum[4][col] + sum[5][col]) + (sum[6][col] + sum[7][col]));
     grad_out[k] = g;
     if(!apply || g == 0.0f) return;
     float p = master[k], m = mom[k], v = vel[k];
@@ -335,25 +393,27 @@ __global__ void k_rc_publish_mlp(const float *__restrict__ master, __bf16 *__res
 }
 
 //! (the gradient entries it reads as non-zero are set back to zero, so the next step starts from a clear buffer
-//! without a fill)
-__global__ void k_rc_adam_grid(float *__restrict__ master, float *__restrict__ mom, float *__restrict__ vel,
-                               _Float16 *__restrict__ grad, float inv_scale, __half *__restrict__ stored,
-                               uint64_t n, adam_consts a)
+//! without a fill). A thread takes a table entry, whose two features are touched together
+__global__ void __launch_bounds__(256) k_rc_adam_grid(float2 *__restrict__ master, float2 *__restrict__ mom,
+                                                      float2 *__restrict__ vel, uint32_t *__restrict__ grad,
+                                                      float inv_scale, __half2 *__restrict__ stored, uint64_t n,
+                                                      adam_consts a)
 {
-    const uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t k = (uint64_t)blockIdx.x * 256 + threadIdx.x;
     if(k >= n) return;
-    const _Float16 raw = grad[k];
-    if(raw == static_cast<_Float16>(0.0f)) return;
-    grad[k] = static_cast<_Float16>(0.0f);
-    const float g = static_cast<float>(raw) * inv_scale;
-    // untouched entries keep their parameters and moments; a non-finite (overflowed) gradient is dropped
-    if(g == 0.0f || !isfinite(g)) return;
-    float p = master[k], m = mom[k], v = vel[k];
-    adam_update(p, m, v, g, a);
+    const uint32_t raw = grad[k];
+    if(!(raw & 0x7fff7fffu)) return;// (a negative zero is a zero)
+    grad[k] = 0u;
+    const half2v h = __builtin_bit_cast(half2v, raw);
+    const float g[2] = {static_cast<float>(h[0]) * inv_scale, static_cast<float>(h[1]) * inv_scale};
+    float2 p = master[k], m = mom[k], v = vel[k];
+    // untouched features keep their parameters and moments; a non-finite (overflowed) gradient is dropped
+    if(g[0] != 0.0f && isfinite(g[0])) adam_update(p.x, m.x, v.x, g[0], a);
+    if(g[1] != 0.0f && isfinite(g[1])) adam_update(p.y, m.y, v.y, g[1], a);
     master[k] = p;
     mom[k] = m;
     vel[k] = v;
-    stored[k] = __float2half_rn(p);
+    stored[k] = __floats2half2_rn(p.x, p.y);
 }
 
 __global__ void k_rc_store_grid(const float *__restrict__ master, __half *__restrict__ stored, uint64_t n)
@@ -416,13 +476,24 @@ void train(vkrt_rc *c, const float4 *records, uint32_t stride_f4, const float4 *
     if(!c->grid_grad_clear) fill(s, c->grid_grad.as<float>(), c->n_grid / 2, 0.0f);// n_grid fp16 values
     // a gradient-only step leaves its gradients for reading; a full step's Adam pass clears them
     c->grid_grad_clear = !grad_only;
-    fill(s, c->loss.as<float>(), 1, 0.0f);
     if(n)
-        k_rc_train<<<nb, TRAIN_BLOCK, 0, s>>>(device_view(c), records, stride_f4, targets, n, n_dev,
-                                              c->grid_grad.as<half2v>(), c->grad_scale, c->partials.as<float>(),
-                                              c->loss.as<float>());
+    {
+        const uint32_t grid = XCDS * div_up(n, ENC_RECORDS);
+        c->train_enc.reserve((size_t)LEVELS * n * sizeof(bf16x2));
+        c->train_grad.reserve((size_t)LEVELS * n * sizeof(float2));
+        bf16x2 *enc = c->train_enc.as<bf16x2>();
+        float2 *enc_grad = c->train_grad.as<float2>();
+        k_rc_encode<<<grid, ENC_BLOCK, 0, s>>>(device_view(c), records, stride_f4, n, n_dev, enc, n, c->loss.as<float>());
+        k_rc_train<<<nb, TRAIN_BLOCK, 0, s>>>(device_view(c), records, stride_f4, targets, n, n_dev, enc, enc_grad, n,
+                                              c->partials.as<float>(), c->loss.as<float>());
+        k_rc_scatter<<<grid, ENC_BLOCK, 0, s>>>(device_view(c), records, stride_f4, n, n_dev, enc_grad, n,
+                                                c->grid_grad.as<half2v>(), c->grad_scale);
+    }
     else
+    {
+        fill(s, c->loss.as<float>(), 1, 0.0f);
         fill(s, c->partials.as<float>(), (uint64_t)nb * N_MLP, 0.0f);
+    }
     adam_consts a{};
     if(!grad_only)
     {
@@ -432,14 +503,15 @@ void train(vkrt_rc *c, const float4 *records, uint32_t stride_f4, const float4 *
                         (float)(1.0 / (1.0 - std::pow((double)p.beta1, (double)c->step))),
                         (float)(1.0 / (1.0 - std::pow((double)p.beta2, (double)c->step)))};
     }
-    k_rc_adam_mlp<<<div_up(N_MLP, 256), 256, 0, s>>>(c->mlp_master.as<float>(), c->mlp_m.as<float>(),
+    k_rc_adam_mlp<<<N_MLP / MLP_K, MLP_K * MLP_SUMS, 0, s>>>(c->mlp_master.as<float>(), c->mlp_m.as<float>(),
                                                        c->mlp_v.as<float>(), c->mlp_grad.as<float>(),
                                                        c->partials.as<float>(), n ? nb : 1, a, grad_only ? 0 : 1,
-                                                       c->w_fwd.as<__bf16>(), c->w_bwd.as<__bf16>());
+                                                       c->w_fwd.as<__bf16>(), c->w_bwd.as<__bf16>(),
+                                                       c->loss.as<float>(), c->host_loss);
     if(!grad_only)
-        k_rc_adam_grid<<<(uint32_t)((c->n_grid + 255) / 256), 256, 0, s>>>(
-            c->grid_master.as<float>(), c->grid_m.as<float>(), c->grid_v.as<float>(), c->grid_grad.as<_Float16>(),
-            1.0f / c->grad_scale, c->grid_half.as<__half>(), c->n_grid, a);
+        k_rc_adam_grid<<<(uint32_t)((c->n_grid / 2 + 255) / 256), 256, 0, s>>>(
+            c->grid_master.as<float2>(), c->grid_m.as<float2>(), c->grid_v.as<float2>(), c->grid_grad.as<uint32_t>(),
+            1.0f / c->grad_scale, c->grid_half.as<__half2>(), c->n_grid / 2, a);
     VKRT_HIP(hipGetLastError());
 }
 
@@ -448,8 +520,13 @@ void query(vkrt_rc *c, const float4 *records, uint32_t stride_f4, uint32_t n, fl
 {
     if(n == 0) return;
     const uint32_t per_block = QUERY_BLOCK / 64 * 16 * QUERY_TILES;
-    k_rc_query<<<div_up(n, per_block), QUERY_BLOCK, 0, c->ctx->stream>>>(device_view(c), records, stride_f4, n,
-                                                                         count_on_device, out, pixel_acc);
+    hipStream_t s = c->ctx->stream;
+    c->query_enc.reserve((size_t)LEVELS * n * sizeof(bf16x2));
+    bf16x2 *enc = c->query_enc.as<bf16x2>();
+    k_rc_encode<<<XCDS * div_up(n, ENC_RECORDS), ENC_BLOCK, 0, s>>>(device_view(c), records, stride_f4, n, count_on_device,
+                                                                  enc, n, nullptr);
+    k_rc_query<<<div_up(n, per_block), QUERY_BLOCK, 0, s>>>(device_view(c), records, stride_f4, n, count_on_device, enc, n,
+                                                            out, pixel_acc);
     VKRT_HIP(hipGetLastError());
 }
 
@@ -571,6 +648,7 @@ int vkrt_rc_create(vkrt_ctx *ctx, const vkrt_rc_params *params, uint32_t seed, v
         c->w_fwd.reserve(N_LAYERS * LAYER_ELEMS * 2);
         c->w_bwd.reserve(N_LAYERS * LAYER_ELEMS * 2);
         c->loss.reserve(256);
+        VKRT_HIP(hipHostMalloc(reinterpret_cast<void **>(&c->host_loss), 256));
         hipStream_t s = ctx->stream;
         // padding slots of the transposed W6 swizzle stay zero
         VKRT_HIP(hipMemsetAsync(c->w_bwd.ptr, 0, N_LAYERS * LAYER_ELEMS * 2, s));
@@ -643,10 +721,8 @@ int vkrt_rc_train(vkrt_rc *c, const float *records, const float *targets, uint32
         rc::train(c, rec, RECORD_F4, tg, n, (flags & VKRT_RC_GRAD_ONLY) != 0, nullptr, c->ctx->stream);
         if(loss)
         {
-            float sum = 0.f;
-            VKRT_HIP(hipMemcpyAsync(&sum, c->loss.ptr, 4, hipMemcpyDeviceToHost, ctx->stream));
             VKRT_HIP(hipStreamSynchronize(ctx->stream));
-            *loss = n ? sum / (float)n : 0.f;
+            *loss = n ? *c->host_loss / (float)n : 0.f;
         }
         finish_call(ctx, flags);
     });

@@ -22,6 +22,7 @@
 #include <cstdint>
 
 #include "context.hpp"
+#include "kernels.hpp"
 
 namespace vkrt::rc
 {
@@ -93,9 +94,12 @@ __device__ __forceinline__ void unit_position(const grid_desc &g, const float4 &
     p[2] = fminf(fmaxf((r0.z - g.bmin[2]) * g.inv_extent[2], 0.0f), 1.0f);
 }
 
-//! the 8 corner table indices and trilinear weights of one level; corner k = (k & 1, k >> 1 & 1, k >> 2)
-__device__ __forceinline__ void level_corners(const grid_desc &g, uint32_t level, const float p[3], uint32_t idx[8],
-                                              float w[8])
+//! Four of a cell's eight corners at one level, those with x offset `dx`: table indices and trilinear weights; corner j =
+//! (dx, j & 1, j >> 1). Two neighbouring lanes take a record's two halves: a corner and its x neighbour mostly share a
+//! cache line (dense levels: adjacent entries; hashed ones: the same but for the lowest bits), which one instruction then
+//! asks for once. Asked for one after the other, each was fetched on its own, 128 B a corner.
+__device__ __forceinline__ void level_corners(const grid_desc &g, uint32_t level, const float p[3], uint32_t dx,
+                                              uint32_t idx[4], float w[4])
 {
     const uint32_t n = g.res[level];
     const float nf = static_cast<float>(n);
@@ -110,43 +114,72 @@ __device__ __forceinline__ void level_corners(const grid_desc &g, uint32_t level
     }
     const bool dense = (g.dense_mask >> level) & 1u;
     const uint32_t mask = (1u << g.log2_t) - 1u;
+    const uint32_t cx = c0[0] + dx;
+    const float wx = dx ? f[0] : 1.0f - f[0];
 #pragma unroll
-    for(int k = 0; k < 8; ++k)
+    for(int j = 0; j < 4; ++j)
     {
-        const uint32_t dx = k & 1, dy = (k >> 1) & 1, dz = k >> 2;
-        const uint32_t cx = c0[0] + dx, cy = c0[1] + dy, cz = c0[2] + dz;
-        const float wx = dx ? f[0] : 1.0f - f[0];
+        const uint32_t dy = j & 1, dz = j >> 1;
+        const uint32_t cy = c0[1] + dy, cz = c0[2] + dz;
         const float wy = dy ? f[1] : 1.0f - f[1];
         const float wz = dz ? f[2] : 1.0f - f[2];
-        w[k] = (wx * wy) * wz;
-        idx[k] = dense ? cx + (n + 1u) * (cy + (n + 1u) * cz)
+        w[j] = (wx * wy) * wz;
+        idx[j] = dense ? cx + (n + 1u) * (cy + (n + 1u) * cz)
                        : ((cx * 1u) ^ (cy * 2654435761u) ^ (cz * 805459861u)) & mask;
     }
 }
 
-//! the 16 logical inputs 16 g .. 16 g + 15 that lane group g feeds to the first layer
-__device__ __forceinline__ void encode_group(const cache_dev &c, const float4 rec[4], uint32_t group, float v[16])
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
+//! one level's two features at unit position p, for the even lane of a pair whose lanes hold the cell's two halves (dx =
+//! the lane's lowest bit); every lane of the wave takes part
+__device__ __forceinline__ bf16x2 encode_level(const cache_dev &c, uint32_t level, const float p[3], uint32_t dx, bool valid)
 {
-    float p[3];
-    unit_position(c.g, rec[0], p);
-    const size_t table = size_t(1) << c.g.log2_t;
+    const __half2 *table = c.grid + ((size_t)level << c.g.log2_t);
+    uint32_t idx[4];
+    float w[4], t0[4], t1[4];
+    if(valid)
+    {
+        level_corners(c.g, level, p, dx, idx, w);
+#pragma unroll
+        for(int j = 0; j < 4; ++j)
+        {
+            const float2 e = __half22float2(table[idx[j]]);
+            t0[j] = w[j] * e.x;
+            t1[j] = w[j] * e.y;
+        }
+    }
+    else
+        for(int j = 0; j < 4; ++j) t0[j] = t1[j] = 0.0f;
+    // the eight corners' terms in order, x fastest
+    float f0 = 0.0f, f1 = 0.0f;
+#pragma unroll
+    for(int j = 0; j < 4; ++j)
+    {
+        f0 = f0 + t0[j];
+        f0 = f0 + __shfl_xor(t0[j], 1);
+        f1 = f1 + t1[j];
+        f1 = f1 + __shfl_xor(t1[j], 1);
+    }
+    return bf16x2{static_cast<__bf16>(f0), static_cast<__bf16>(f1)};
+}
+
+//! The two table levels that the workgroups of XCD x read or write (workgroup b runs on XCD b mod 8): a fine one with a
+//! coarse one. The L2s then hold two levels each (at most 4 MiB at 2^19 entries) instead of passing all 32 MiB through
+//! every one of them.
+__device__ __forceinline__ uint32_t xcd_level(uint32_t x, uint32_t k) { return k ? LEVELS - 1u - x : x; }
+
+//! the 16 logical inputs 16 g .. 16 g + 15 that lane group g feeds to the first layer: the features of its four levels
+//! (enc: [level][stride] as k_rc_encode left them, at this record), spherical harmonics and material
+__device__ __forceinline__ void input_group(const bf16x2 *__restrict__ enc, size_t stride, const float4 rec[4],
+                                            uint32_t group, bf16x8 b[2])
+{
 #pragma unroll
     for(uint32_t m = 0; m < 4; ++m)
     {
-        const uint32_t level = 4 * group + m;
-        uint32_t idx[8];
-        float w[8];
-        level_corners(c.g, level, p, idx, w);
-        float f0 = 0.0f, f1 = 0.0f;
-#pragma unroll
-        for(int k = 0; k < 8; ++k)
-        {
-            const float2 e = __half22float2(c.grid[level * table + idx[k]]);
-            f0 = f0 + w[k] * e.x;
-            f1 = f1 + w[k] * e.y;
-        }
-        v[2 * m] = f0;
-        v[2 * m + 1] = f1;
+        const bf16x2 e = enc[(4 * group + m) * stride];
+        b[0][2 * m] = e[0];
+        b[0][2 * m + 1] = e[1];
     }
     float sh[16];
     sh16(rec[1].x, rec[1].y, rec[1].z, sh);
@@ -155,17 +188,9 @@ __device__ __forceinline__ void encode_group(const cache_dev &c, const float4 re
 #pragma unroll
     for(uint32_t k = 0; k < 4; ++k)
     {
-        v[8 + k] = sh[4 * group + k];
-        v[12 + k] = extras[4 * group + k];
+        b[1][k] = static_cast<__bf16>(sh[4 * group + k]);
+        b[1][4 + k] = static_cast<__bf16>(extras[4 * group + k]);
     }
-}
-
-__device__ __forceinline__ bf16x8 pack8(const float *v)
-{
-    bf16x8 r;
-#pragma unroll
-    for(int j = 0; j < 8; ++j) r[j] = static_cast<__bf16>(v[j]);
-    return r;
 }
 
 //! D registers (4 row tiles x 4) -> the next layer's two B operands (K permutation phi)
@@ -283,6 +308,18 @@ struct vkrt_rc
     // grid_grad holds zeros: the last training step's Adam pass cleared every entry it read as non-zero
     bool grid_grad_clear = false;
     vkrt::device_buffer mlp_master, mlp_grad, mlp_m, mlp_v, w_fwd, w_bwd, partials, loss;
+    // per record: the encoder's features of a query or of a training step, and the latter's feature gradients. A
+    // training step may run beside a query, so each has its own
+    vkrt::device_buffer query_enc, train_enc, train_grad;
+    float *host_loss = nullptr;// the last training step's loss sum, in pinned memory
+
+    vkrt_rc() = default;
+    vkrt_rc(const vkrt_rc &) = delete;
+    vkrt_rc &operator=(const vkrt_rc &) = delete;
+    ~vkrt_rc()
+    {
+        if(host_loss) (void)hipHostFree(host_loss);
+    }
 };
 
 namespace vkrt::rc
