@@ -25,8 +25,8 @@ ANY_BYTES_PER_RAY = 33       # 32 B ray in + 1 B flag out
 
 
 # wave64 VALU instructions per second: 1,024 SIMDs of 32 FP32 lanes (157.3 TFLOP/s = 256 CUs x 4 SIMDs x 32
-# lanes x 2 flop x 2.4 GHz), 2 cycles per instruction; the brute-force kernel sustains 8.1e11/s, above what
-# 16-lane SIMDs (4 cycles, 6.1e11/s) could issue
+# lanes x 2 flop x 2.4 GHz), 2 cycles per instruction; 8.1e11/s were measured with a triangle test per pair of a
+# ray and a triangle, above what 16-lane SIMDs (4 cycles, 6.1e11/s) could issue
 MI355X_VALU_ISSUE = 1024 * 2.4e9 / 2
 
 
@@ -96,8 +96,9 @@ def cpu_baseline(tris, rays, budget_s):
 def brute_force_leg(ctx, reps=10):
     """the brute-force closest hit of 65,536 rays (origins U[-3,3]^3, directions uniform on S^2, seed 0)
     against the 20,480-triangle jittered icosphere (subdivision 5, radius 1, vertices N(0, 0.01)): one
-    ray-triangle test per pair, 1,342,177,280 per run, 52 FP32 operations each on the full path of
-    src/intersection.cpp:114-129 (no FMA). Timed on the GPU (HBM-resident arrays, hipEvents around `reps`
+    ray-triangle test per pair, 1,342,177,280 per run. The matrix cores sort out the pairs that can hit, 192
+    bf16 operations a pair (six 32x32x16 products per 1,024 pairs); those take the full test of
+    src/intersection.cpp:114-129. Timed on the GPU (HBM-resident arrays, hipEvents around `reps`
     runs) and, as the CPU baseline of this workload, the oracle's full run on every host thread (1 warm-up,
     median of 5) and a 4,096-ray sample on one thread. The GPU records are checked bit for bit against the
     oracle's full run."""
@@ -140,15 +141,15 @@ def brute_force_leg(ctx, reps=10):
     mismatch = int(np.sum((got["prim"] != want["prim"]) | (got["t"].view(np.uint32) != want["t"].view(np.uint32)) |
                           (got["u"].view(np.uint32) != want["u"].view(np.uint32)) |
                           (got["v"].view(np.uint32) != want["v"].view(np.uint32))))
-    flops = 52.0 * n_tests
+    flops = 192.0 * n_tests
     tflops = flops / (ms * 1e-3) / 1e12
     return {"workload": "brute-force closest hit, 65,536 rays x 20,480-triangle jittered icosphere (subdiv 5, "
                         "r 1, N(0, 0.01)), seed 0", "tests_per_run": n_tests,
             "gpu_ms": round(ms, 4), "gpu_tests_per_s": round(n_tests / (ms * 1e-3), 1),
             "gpu_rays_per_s": round(len(rays) / (ms * 1e-3), 1),
-            "roofline": {"bound": "fp32 valu", "kernel": "k_brute_closest (whole call: prep + fill + test + finalize)",
-                         "achieved": round(tflops, 3), "peak": 157.3, "unit": "TFLOP/s",
-                         "frac": round(tflops / 157.3, 5), "flop_per_test": 52, "flop_per_run": flops},
+            "roofline": {"bound": "bf16 mfma", "kernel": "k_brute (whole call: fill + filter and test + finalize)",
+                         "achieved": round(tflops, 3), "peak": 2516.6, "unit": "TFLOP/s",
+                         "frac": round(tflops / 2516.6, 5), "flop_per_test": 192, "flop_per_run": flops},
             "verified_vs_oracle_full_run": {"rays": len(rays), "mismatches": mismatch,
                                             "hits": int(np.sum(want["prim"] != 0xFFFFFFFF))},
             "cpu_full_run": {"threads": nthreads, "cpu_model": model, "median_s": round(cpu_s, 3),

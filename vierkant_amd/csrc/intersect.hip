@@ -2,10 +2,9 @@
 // closest/any-hit loop, for gfx950.
 //
 // Pairwise kernels evaluate the reference arithmetic (vierkant/rt_math.hpp) one element per lane.
-// The brute-force kernels tile (rays x triangle chunks): each wave64 holds 64 rays, walks one
-// triangle chunk whose addresses are wave-uniform (scalar loads feed the VALU directly), and merges
-// its best hit into a per-ray 64-bit key (ordered t << 32 | prim) with one atomic min, so ties on t
-// resolve to the lowest triangle index no matter which chunk finishes first.
+// The brute-force kernel tiles (rays x triangle chunks): the matrix cores sort out the pairs that can hit, those
+// take the reference's test, and a lane merges its best hit into a per-ray 64-bit key (ordered t << 32 | prim)
+// with one atomic min, so ties on t resolve to the lowest triangle index no matter which chunk finishes first.
 #include <cfloat>
 #include <mutex>
 
@@ -143,73 +142,215 @@ __global__ void k_fill_u8(uint8_t *__restrict__ p, uint32_t n, uint8_t value)
 }
 
 //! (v0, v1, v2) -> (v0, e1 = v1 - v0, e2 = v2 - v0): the first line of the reference test
-__global__ void k_tri_prep(const float *__restrict__ tris, uint32_t n, float *__restrict__ pre)
-{
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if(i >= n) return;
-    const float *t = tris + 9 * (size_t)i;
-    float *p = pre + 9 * (size_t)i;
-    vec3 v0 = ld3(t), e1 = ld3(t + 3) - v0, e2 = ld3(t + 6) - v0;
-    p[0] = v0.x, p[1] = v0.y, p[2] = v0.z;
-    p[3] = e1.x, p[4] = e1.y, p[5] = e1.z;
-    p[6] = e2.x, p[7] = e2.y, p[8] = e2.z;
-}
 
 // ---------------------------------------------------------------------------------------------
 // brute force
 // ---------------------------------------------------------------------------------------------
-// 65,536 rays x 20,480 triangles: 1.18 ms per launch against 1.23 one triangle at a time; eight at a time
-// (98 VGPRs) is no faster
-constexpr int BRUTE_UNROLL = 4;
+// A hit needs a = tvec.(d x e2), b = d.(tvec x e1) and c = det - a - b all of det's sign, and each of the three
+// is a product of a vector of the triangle and one of the ray, (edge, vertex x edge) . (o x d, d) in six
+// components about any origin: a contraction, so the matrix cores find the few pairs that can hit and only
+// those take the reference's test, whose decision and bits stand. With -ffp-contract=off that test is some 45
+// VALU instructions a pair; the filter leaves 3.5 of them (min3, max3, max, half a max3) beside six
+// 32x32x16 bf16 MFMAs per 32 x 32 pairs.
+//
+// The factors go in as two bf16 parts each, hi + mid, off by 2^-16 of the factor; a lane's half holds the
+// triangle's hi or mid parts and the two MFMAs of a product take the ray's hi and its mid parts. With
+// P = |d| E (|o| + V) (E the longest edge and V the farthest vertex of 32 triangles, all about the chunk's first
+// vertex) the parts are off by at most 2^-15 P, the 24 terms' sum by less than 2^-19 P, the reference's own
+// a, b and det by less than 2^-19 P: a pair whose three values are not all above -2^-14 P - 2^-70, nor all below
+// its negative, is no hit of the reference's. 2^-70 covers what is lost below the normal range while every
+// factor stays below 2^40; a ray or a tile beyond that, or with a NaN or an infinity, takes every pair.
+//
+// 65,536 rays x 20,480 triangles: 1,220 us with the reference's test for every pair, 237 so, the matrix cores busy
+// for 48 % of them and 69 VALU instructions a wave per 32 x 32 pairs, 48 of them the filter's. Two products of
+// 32 x 32 in flight per wave, at two or three waves a SIMD, are no faster: 248 - 255.
+constexpr float BRUTE_LIMIT = 0x1p40f;
+constexpr int BRUTE_STAGE = 256;// triangles in LDS at a time, one a thread
+constexpr int BRUTE_TILES = BRUTE_STAGE / 32;
 
-__global__ void __launch_bounds__(256) k_brute_closest(const float4 *__restrict__ rays, uint32_t n_ray,
-                                                       const float *__restrict__ pre, uint32_t n_tri,
-                                                       uint32_t chunk, uint64_t *__restrict__ keys)
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+//! six values as two bf16 parts each, two zeros behind
+__device__ __forceinline__ void split_bf16(const vec3 &p, const vec3 &q, bf16x8 &hi, bf16x8 &mid)
 {
-    const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t t0 = blockIdx.y * chunk;
-    const uint32_t t1 = min(n_tri, t0 + chunk);
-    vec3 o{0.f, 0.f, 0.f}, d{0.f, 0.f, 1.f};
-    float tmin = 0.f, tmax = -1.f;// an empty interval for lanes past the end
-    if(r < n_ray) load_ray(rays, r, o, tmin, d, tmax);
-    float best = tmax;
-    uint32_t best_i = VKRT_INVALID_PRIM;
-    // the triangle index is wave-uniform, so records come through scalar loads, four at a time: one wider
-    // request and one loop step per four tests (the loop's scalar work competes with the tests for issue)
-    uint32_t i = t0;
-    for(; i + BRUTE_UNROLL <= t1; i += BRUTE_UNROLL)
+    const float x[8] = {p.x, p.y, p.z, q.x, q.y, q.z, 0.f, 0.f};
+#pragma unroll
+    for(int k = 0; k < 8; ++k)
     {
-        const float *p = pre + 9 * (size_t)i;
-        float rec[9 * BRUTE_UNROLL];
+        hi[k] = static_cast<__bf16>(x[k]);
+        mid[k] = static_cast<__bf16>(x[k] - static_cast<float>(hi[k]));
+    }
+}
+
+//! no smaller than |v|, also where the squares underflow
+__device__ __forceinline__ float norm_above(const vec3 &v) { return sqrtf(dot(v, v)) + 0x1p-60f; }
+
+__device__ __forceinline__ uint32_t half_wave_max(uint32_t x)
+{
 #pragma unroll
-        for(int k = 0; k < 9 * BRUTE_UNROLL; ++k) rec[k] = p[k];
+    for(int off = 16; off > 0; off >>= 1) x = max(x, static_cast<uint32_t>(__shfl_xor(static_cast<int>(x), off)));
+    return x;
+}
+
+//! the smallest of three values, and of their negatives: neither reaches zero unless all lie on one side of it
+__device__ __forceinline__ float above(float a, float b, float c) { return fminf(fminf(a, b), c); }
+__device__ __forceinline__ float below(float a, float b, float c) { return fminf(fminf(-a, -b), -c); }
+
+//! a wave takes 32 * GROUPS rays over its workgroup's triangles; lanes l and l + 32 hold one ray, and 16
+//! triangles each of every 32
+template<bool ANY, int GROUPS>
+__global__ void __launch_bounds__(256, GROUPS > 2 ? 3 : 4) k_brute(const float4 *__restrict__ rays, uint32_t n_ray,
+                                                  const float *__restrict__ tris, uint32_t n_tri, uint32_t chunk,
+                                                  uint64_t *__restrict__ keys, uint8_t *__restrict__ occluded)
+{
+    __shared__ bf16x8 parts[BRUTE_TILES][3][64];
+    __shared__ float4 records[BRUTE_STAGE][3];// v0, e1, e2 for the reference's test
+    __shared__ float2 extent[BRUTE_TILES];    // E, V
+
+    const uint32_t lane = threadIdx.x & 63u, half = lane >> 5;
+    const uint32_t t0 = blockIdx.y * chunk, count = min(n_tri - t0, chunk);
+    const vec3 centre = ld3(tris + 9 * (size_t)t0);
+
+    bf16x8 ray_hi[GROUPS], ray_mid[GROUPS];
+    float ray_d[GROUPS], ray_o[GROUPS], best[GROUPS];
+    uint32_t best_i[GROUPS];
+    const uint32_t first_ray = (blockIdx.x * 4u + (threadIdx.x >> 6)) * (32u * GROUPS) + (lane & 31u);
 #pragma unroll
-        for(int k = 0; k < BRUTE_UNROLL; ++k)
+    for(int g = 0; g < GROUPS; ++g)
+    {
+        const uint32_t r = first_ray + 32u * g;
+        vec3 o{0.f, 0.f, 0.f}, d{0.f, 0.f, 1.f};
+        float tmin = 0.f, tmax = -1.f;
+        if(r < n_ray) load_ray(rays, r, o, tmin, d, tmax);
+        o = o - centre;
+        split_bf16(cross(o, d), d, ray_hi[g], ray_mid[g]);
+        ray_o[g] = norm_above(o);
+        ray_d[g] = norm_above(d);
+        if(!(ray_o[g] < BRUTE_LIMIT && ray_d[g] < BRUTE_LIMIT && ray_o[g] * ray_d[g] < BRUTE_LIMIT))
+            ray_d[g] = __int_as_float(0x7fc00000);
+        if(!(tmin < tmax)) ray_d[g] = -__int_as_float(0x7f800000);// no t lies inside: no pair is taken
+        best[g] = tmax;
+        best_i[g] = VKRT_INVALID_PRIM;
+    }
+
+    for(uint32_t done = 0; done < count; done += BRUTE_STAGE)
+    {
+        const uint32_t base = t0 + done, n = min(count - done, static_cast<uint32_t>(BRUTE_STAGE));
+        if(done) __syncthreads();
         {
-            const float *q = rec + 9 * k;
-            float t, u, v;
-            if(mt_fast_window(o, d, vec3{q[0], q[1], q[2]}, vec3{q[3], q[4], q[5]}, vec3{q[6], q[7], q[8]}, tmin,
-                              best, t, u, v))
+            vec3 v0 = centre, e1{0.f, 0.f, 0.f}, e2{0.f, 0.f, 0.f};
+            if(threadIdx.x < n)
             {
-                best = t;
-                best_i = i + k;
+                const float *t = tris + 9 * (size_t)(base + threadIdx.x);
+                v0 = ld3(t);
+                e1 = ld3(t + 3) - v0;
+                e2 = ld3(t + 6) - v0;
+            }
+            records[threadIdx.x][0] = make_float4(v0.x, v0.y, v0.z, e1.x);
+            records[threadIdx.x][1] = make_float4(e1.y, e1.z, e2.x, e2.y);
+            records[threadIdx.x][2] = make_float4(e2.z, 0.f, 0.f, 0.f);
+            v0 = v0 - centre;
+            const vec3 e3 = e1 - e2;
+            const uint32_t tile = threadIdx.x >> 5, row = threadIdx.x & 31u;
+            bf16x8 hi, mid;
+            split_bf16(e2, cross(v0, e2), hi, mid);
+            parts[tile][0][row] = hi;
+            parts[tile][0][32 + row] = mid;
+            split_bf16(vec3{0.f, 0.f, 0.f} - e1, cross(e1, v0), hi, mid);
+            parts[tile][1][row] = hi;
+            parts[tile][1][32 + row] = mid;
+            split_bf16(e3, cross(v0 + e1, e3), hi, mid);
+            parts[tile][2][row] = hi;
+            parts[tile][2][32 + row] = mid;
+            const float l1 = norm_above(e1);
+            float e = fmaxf(fmaxf(l1, norm_above(e2)), norm_above(e3));
+            float v = norm_above(v0) + l1;
+            // compared as integers a NaN is above every number
+            if(!(e < BRUTE_LIMIT && v < BRUTE_LIMIT && e * v < BRUTE_LIMIT)) e = __int_as_float(0x7fc00000);
+            e = __uint_as_float(half_wave_max(__float_as_uint(e)));
+            v = __uint_as_float(half_wave_max(__float_as_uint(v) & 0x7fffffffu));
+            if(row == 0) extent[tile] = make_float2(e, v);
+        }
+        __syncthreads();
+
+        const uint32_t n_tile = (n + 31u) / 32u;
+        for(uint32_t tile = 0; tile < n_tile; ++tile)
+        {
+            bf16x8 part[3];
+#pragma unroll
+            for(int k = 0; k < 3; ++k) part[k] = parts[tile][k][lane];
+            const float2 ev = extent[tile];
+#pragma unroll
+            for(int g = 0; g < GROUPS; ++g)
+            {
+                f32x16 m[3];
+#pragma unroll
+                for(int k = 0; k < 3; ++k)
+                {
+                    const f32x16 zero = {};
+                    m[k] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(part[k], ray_hi[g], zero, 0, 0, 0);
+                    m[k] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(part[k], ray_mid[g], m[k], 0, 0, 0);
+                }
+                const float margin = ray_d[g] * ev.x * (ray_o[g] + ev.y) * 0x1p-14f + 0x1p-70f;
+                float nearest = -__int_as_float(0x7f800000);
+#pragma unroll
+                for(int i = 0; i < 16; ++i)
+                    nearest = fmaxf(fmaxf(nearest, above(m[0][i], m[1][i], m[2][i])),
+                                    below(m[0][i], m[1][i], m[2][i]));
+                if(nearest < -margin) continue;
+
+                // a NaN margin gets here for rays that take no pair too, and for those past the end
+                if(ray_d[g] == -__int_as_float(0x7f800000)) continue;
+                uint32_t mask = 0;
+#pragma unroll
+                for(int i = 0; i < 16; ++i)
+                    mask |= fmaxf(above(m[0][i], m[1][i], m[2][i]), below(m[0][i], m[1][i], m[2][i])) < -margin
+                                ? 0u
+                                : 1u << i;
+                vec3 o, d;
+                float tmin, tmax;
+                load_ray(rays, first_ray + 32u * g, o, tmin, d, tmax);
+                while(mask)
+                {
+                    const uint32_t i = __ffs(static_cast<int>(mask)) - 1;
+                    mask &= mask - 1u;
+                    const uint32_t row = 32u * tile + 8u * (i >> 2) + 4u * half + (i & 3u);
+                    if(row >= n) break;
+                    const float4 q0 = records[row][0], q1 = records[row][1], q2 = records[row][2];
+                    float t, u, v;
+                    if(mt_fast_window(o, d, vec3{q0.x, q0.y, q0.z}, vec3{q0.w, q1.x, q1.y}, vec3{q1.z, q1.w, q2.x},
+                                      tmin, best[g], t, u, v))
+                    {
+                        best_i[g] = base + row;
+                        if(ANY)
+                        {
+                            ray_d[g] = -__int_as_float(0x7f800000);
+                            break;
+                        }
+                        best[g] = t;
+                    }
+                }
+            }
+            if(ANY)
+            {
+                bool open = false;
+#pragma unroll
+                for(int g = 0; g < GROUPS; ++g) open |= !(ray_d[g] == -__int_as_float(0x7f800000));
+                if(!__any(open)) break;
             }
         }
     }
-    for(; i < t1; ++i)
+#pragma unroll
+    for(int g = 0; g < GROUPS; ++g)
     {
-        const float *p = pre + 9 * (size_t)i;
-        float t, u, v;
-        if(mt_fast_window(o, d, ld3(p), ld3(p + 3), ld3(p + 6), tmin, best, t, u, v))
-        {
-            best = t;
-            best_i = i;
-        }
+        if(best_i[g] == VKRT_INVALID_PRIM) continue;
+        if(ANY) occluded[first_ray + 32u * g] = 1;
+        else atomicMin((unsigned long long *)&keys[first_ray + 32u * g], hit_key(best[g], best_i[g]));
     }
-    if(best_i != VKRT_INVALID_PRIM) atomicMin((unsigned long long *)&keys[r], hit_key(best, best_i));
 }
 
-__global__ void k_brute_finalize(const float4 *__restrict__ rays, uint32_t n_ray, const float *__restrict__ pre,
+__global__ void k_brute_finalize(const float4 *__restrict__ rays, uint32_t n_ray, const float *__restrict__ tris,
                                  const uint64_t *__restrict__ keys, vkrt_hit *__restrict__ hits)
 {
     uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
@@ -222,52 +363,13 @@ __global__ void k_brute_finalize(const float4 *__restrict__ rays, uint32_t n_ray
         vec3 o, d;
         float tmin, tmax;
         load_ray(rays, r, o, tmin, d, tmax);
-        const float *p = pre + 9 * (size_t)prim;
+        const float *p = tris + 9 * (size_t)prim;
+        const vec3 v0 = ld3(p);
         float t = 0.f, u = 0.f, v = 0.f;
-        mt_reference(o, d, ld3(p), ld3(p + 3), ld3(p + 6), t, u, v);
+        mt_reference(o, d, v0, ld3(p + 3) - v0, ld3(p + 6) - v0, t, u, v);
         h = vkrt_hit{t, u, v, prim};
     }
     hits[r] = h;
-}
-
-__global__ void __launch_bounds__(256) k_brute_any(const float4 *__restrict__ rays, uint32_t n_ray,
-                                                   const float *__restrict__ pre, uint32_t n_tri, uint32_t chunk,
-                                                   uint8_t *__restrict__ occluded)
-{
-    const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t t0 = blockIdx.y * chunk;
-    const uint32_t t1 = min(n_tri, t0 + chunk);
-    vec3 o{0.f, 0.f, 0.f}, d{0.f, 0.f, 1.f};
-    float tmin = 0.f, tmax = -1.f;
-    if(r < n_ray) load_ray(rays, r, o, tmin, d, tmax);
-    int occ = (r < n_ray) ? 0 : 1;
-    // four records per loop step, as in k_brute_closest; the wave leaves once every lane is occluded
-    uint32_t i = t0;
-    for(; i + BRUTE_UNROLL <= t1; i += BRUTE_UNROLL)
-    {
-        if(__all(occ)) break;
-        const float *p = pre + 9 * (size_t)i;
-        float rec[9 * BRUTE_UNROLL];
-#pragma unroll
-        for(int k = 0; k < 9 * BRUTE_UNROLL; ++k) rec[k] = p[k];
-#pragma unroll
-        for(int k = 0; k < BRUTE_UNROLL; ++k)
-        {
-            const float *q = rec + 9 * k;
-            float t, u, v;
-            if(!occ && mt_fast_window(o, d, vec3{q[0], q[1], q[2]}, vec3{q[3], q[4], q[5]}, vec3{q[6], q[7], q[8]},
-                                      tmin, tmax, t, u, v))
-                occ = 1;
-        }
-    }
-    for(; i < t1; ++i)
-    {
-        if(__all(occ)) break;
-        const float *p = pre + 9 * (size_t)i;
-        float t, u, v;
-        if(!occ && mt_fast_window(o, d, ld3(p), ld3(p + 3), ld3(p + 6), tmin, tmax, t, u, v)) occ = 1;
-    }
-    if(r < n_ray && occ) occluded[r] = 1;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -435,12 +537,6 @@ __global__ void __launch_bounds__(SPHERE_BLOCK) k_sphere_grow(const float *__res
 // ---------------------------------------------------------------------------------------------
 // host launchers
 // ---------------------------------------------------------------------------------------------
-void launch_tri_prep(hipStream_t s, const float *tris, uint32_t n, float *pre)
-{
-    if(!n) return;
-    k_tri_prep<<<div_up(n, 256), 256, 0, s>>>(tris, n, pre);
-}
-
 void launch_fill_u64(hipStream_t s, uint64_t *p, uint32_t n, uint64_t value)
 {
     if(!n) return;
@@ -453,50 +549,48 @@ void launch_fill_u8(hipStream_t s, uint8_t *p, uint32_t n, uint8_t value)
     k_fill_u8<<<div_up(n, 256), 256, 0, s>>>(p, n, value);
 }
 
-static uint32_t brute_chunk(uint32_t n_ray, uint32_t n_tri)
+//! launches k_brute over (workgroups of rays) x (chunks of triangles)
+template<bool ANY>
+static void brute(vkrt_ctx *ctx, const float *tris, uint32_t n_tri, const float4 *rays, uint32_t n_ray,
+                  uint64_t *keys, uint8_t *occ)
 {
-    // enough (ray block x triangle chunk) tiles for >= 16k waves, chunks of >= 256 triangles
-    uint64_t ray_waves = div_up(n_ray, 64);
-    uint64_t want = (16384 + ray_waves - 1) / ray_waves;
-    uint64_t max_chunks = div_up(n_tri, 256);
-    uint64_t chunks = want < 1 ? 1 : (want > max_chunks ? max_chunks : want);
-    if(chunks > 65535) chunks = 65535;
-    return div_up(n_tri, chunks);
+    const uint32_t stages = div_up(n_tri, BRUTE_STAGE);
+    // 128 rays a wave spread a triangle's loads and its preparation over more products once each SIMD gets 16 such
+    // waves; with fewer, waves of 32 rays fill the card better. 65,536 rays x 80 / 1,280 triangles (512 / 2,560
+    // waves of 128): 21 / 34 us with 128 rays, 14 / 32 with 32; 16,384 x 20,480 (10,240): 82 and 78; 32,768 x
+    // 20,480 (20,480): 130 and 148
+    const bool few = static_cast<uint64_t>(div_up(n_ray, 128)) * stages < 16384;
+    const uint32_t blocks = div_up(n_ray, few ? 128 : 512);
+    // chunks of whole stages, as many as fill the card some five times over (2,048, 4,096 and 16,384 workgroups:
+    // 245, 242 and 255 us) and no more than a grid can have
+    const uint32_t chunks = min(stages, min(div_up(4096, blocks), 65535u));
+    const uint32_t chunk = min(static_cast<uint64_t>(div_up(stages, chunks)) * BRUTE_STAGE, static_cast<uint64_t>(n_tri));
+    const dim3 grid(blocks, div_up(n_tri, chunk));
+    if(few) k_brute<ANY, 1><<<grid, 256, 0, ctx->stream>>>(rays, n_ray, tris, n_tri, chunk, keys, occ);
+    else k_brute<ANY, 4><<<grid, 256, 0, ctx->stream>>>(rays, n_ray, tris, n_tri, chunk, keys, occ);
 }
 
-void brute_closest(vkrt_ctx *ctx, const float *pre, uint32_t n_tri, const float4 *rays, uint32_t n_ray,
+void brute_closest(vkrt_ctx *ctx, const float *tris, uint32_t n_tri, const float4 *rays, uint32_t n_ray,
                    uint64_t *keys, vkrt_hit *hits)
 {
-    hipStream_t s = ctx->stream;
-    launch_fill_u64(s, keys, n_ray, ~0ull);
-    if(n_tri)
-    {
-        uint32_t chunk = brute_chunk(n_ray, n_tri);
-        dim3 grid(div_up(n_ray, 256), div_up(n_tri, chunk));
-        k_brute_closest<<<grid, 256, 0, s>>>(rays, n_ray, pre, n_tri, chunk, keys);
-    }
-    k_brute_finalize<<<div_up(n_ray, 256), 256, 0, s>>>(rays, n_ray, pre, keys, hits);
+    launch_fill_u64(ctx->stream, keys, n_ray, ~0ull);
+    if(n_tri) brute<false>(ctx, tris, n_tri, rays, n_ray, keys, nullptr);
+    k_brute_finalize<<<div_up(n_ray, 256), 256, 0, ctx->stream>>>(rays, n_ray, tris, keys, hits);
 }
 
-void brute_any(vkrt_ctx *ctx, const float *pre, uint32_t n_tri, const float4 *rays, uint32_t n_ray, uint8_t *occ)
+void brute_any(vkrt_ctx *ctx, const float *tris, uint32_t n_tri, const float4 *rays, uint32_t n_ray, uint8_t *occ)
 {
-    hipStream_t s = ctx->stream;
-    launch_fill_u8(s, occ, n_ray, 0);
-    if(!n_tri) return;
-    uint32_t chunk = brute_chunk(n_ray, n_tri);
-    dim3 grid(div_up(n_ray, 256), div_up(n_tri, chunk));
-    k_brute_any<<<grid, 256, 0, s>>>(rays, n_ray, pre, n_tri, chunk, occ);
+    launch_fill_u8(ctx->stream, occ, n_ray, 0);
+    if(n_tri) brute<true>(ctx, tris, n_tri, rays, n_ray, nullptr, occ);
 }
 
 // ---------------------------------------------------------------------------------------------
-// allocation-free brute force: its scratch (the (v0, e1, e2) triangles, then the 64-bit hit keys) is
+// allocation-free brute force: its scratch (the 64-bit hit keys) is
 // a file-scope device array, so a call allocates nothing. Each GPU holds its own copy of the array;
 // the host reaches it only through the address hipGetSymbolAddress returns on that device (the
 // array's name on the host is a stand-in, not a device address).
 // ---------------------------------------------------------------------------------------------
-constexpr size_t NOALLOC_TRI_BYTES = (size_t)VKRT_NOALLOC_MAX_TRI * 9 * sizeof(float);
-constexpr size_t NOALLOC_BYTES = NOALLOC_TRI_BYTES + (size_t)VKRT_NOALLOC_MAX_RAY * sizeof(uint64_t);
-static_assert(NOALLOC_TRI_BYTES % 256 == 0, "the key area must stay 256-B aligned");
+constexpr size_t NOALLOC_BYTES = (size_t)VKRT_NOALLOC_MAX_RAY * sizeof(uint64_t);
 
 static __device__ __align__(256) unsigned char scratch[NOALLOC_BYTES];
 
@@ -668,11 +762,8 @@ int vkrt_intersect_brute_closest(vkrt_ctx *ctx, const float *tris, uint32_t n_tr
         const float *dt = input(ctx, 0, tris, (size_t)n_tri * 9, flags);
         const vkrt_ray *dr = input(ctx, 1, rays, n_ray, flags);
         vkrt_hit *dh = output(ctx, 2, out, n_ray, flags);
-        ctx->scratch[0].reserve((size_t)n_tri * 9 * sizeof(float));
         ctx->scratch[1].reserve((size_t)n_ray * sizeof(uint64_t));
-        float *pre = ctx->scratch[0].as<float>();
-        launch_tri_prep(ctx->stream, dt, n_tri, pre);
-        brute_closest(ctx, pre, n_tri, reinterpret_cast<const float4 *>(dr), n_ray, ctx->scratch[1].as<uint64_t>(),
+        brute_closest(ctx, dt, n_tri, reinterpret_cast<const float4 *>(dr), n_ray, ctx->scratch[1].as<uint64_t>(),
                       dh);
         VKRT_HIP(hipGetLastError());
         finish_output(ctx, 2, out, n_ray, flags);
@@ -693,13 +784,10 @@ int vkrt_intersect_brute_closest_noalloc(vkrt_ctx *ctx, const float *tris, uint3
                      "vkrt_intersect_brute_closest_noalloc: n_ray exceeds VKRT_NOALLOC_MAX_RAY (786432)");
         VKRT_REQUIRE(ctx->noalloc_scratch, "no allocation-free scratch on this device");
         if(n_ray == 0) return;
-        unsigned char *base = static_cast<unsigned char *>(ctx->noalloc_scratch);
-        float *pre = reinterpret_cast<float *>(base);
-        uint64_t *keys = reinterpret_cast<uint64_t *>(base + NOALLOC_TRI_BYTES);
-        // every word brute_closest reads is written first in the same call: the triangles by the prep
-        // kernel, the keys by a fill kernel, so nothing left by an earlier call is read
-        launch_tri_prep(ctx->stream, tris, n_tri, pre);
-        brute_closest(ctx, pre, n_tri, reinterpret_cast<const float4 *>(rays), n_ray, keys, out);
+        uint64_t *keys = static_cast<uint64_t *>(ctx->noalloc_scratch);
+        // every key brute_closest reads is written first in the same call, by a fill kernel, so nothing left by
+        // an earlier call is read
+        brute_closest(ctx, tris, n_tri, reinterpret_cast<const float4 *>(rays), n_ray, keys, out);
         VKRT_HIP(hipGetLastError());
         finish_call(ctx, flags);
     });
@@ -714,10 +802,7 @@ int vkrt_intersect_brute_any(vkrt_ctx *ctx, const float *tris, uint32_t n_tri, c
         const float *dt = input(ctx, 0, tris, (size_t)n_tri * 9, flags);
         const vkrt_ray *dr = input(ctx, 1, rays, n_ray, flags);
         uint8_t *docc = output(ctx, 2, occluded, n_ray, flags);
-        ctx->scratch[0].reserve((size_t)n_tri * 9 * sizeof(float));
-        float *pre = ctx->scratch[0].as<float>();
-        launch_tri_prep(ctx->stream, dt, n_tri, pre);
-        brute_any(ctx, pre, n_tri, reinterpret_cast<const float4 *>(dr), n_ray, docc);
+        brute_any(ctx, dt, n_tri, reinterpret_cast<const float4 *>(dr), n_ray, docc);
         VKRT_HIP(hipGetLastError());
         finish_output(ctx, 2, occluded, n_ray, flags);
         finish_call(ctx, flags);
