@@ -342,7 +342,8 @@ __device__ __forceinline__ vec3 xyz(const float4 &f) { return vec3{f.x, f.y, f.z
 __device__ __forceinline__ float frac(float x) { return x - floorf(x); }
 
 //! the start of pixel p's path of a sample: the pixel's RNG state and sample offset (first sample), the lens sample,
-//! the camera ray and a fresh path state with the given flags
+//! the camera ray and the given flags. What every path starts with alike (throughput, radiance, refraction stack,
+//! cone, media) is not written: shade_path knows it at depth 0, which saves 56 B a path here and as many there
 __device__ __forceinline__ void begin_path(const pt_frame &f, const pt_buffers &b, uint32_t sample, uint32_t p,
                                            uint32_t flags)
 {
@@ -383,11 +384,6 @@ __device__ __forceinline__ void begin_path(const pt_frame &f, const pt_buffers &
     vec3 dir = normalize3(f.right * dv.x + f.up * dv.y - f.forward * dv.z);
     b.ray_o[p] = make_float4(origin.x, origin.y, origin.z, EPS);
     b.ray_d[p] = make_float4(dir.x, dir.y, dir.z, DEFAULT_TMAX);
-    b.beta[p] = make_float4(1.f, 1.f, 1.f, 0.f);
-    b.rad[p] = make_float4(0.f, 0.f, 0.f, 0.f);
-    b.iors[p] = make_float4(1.f, 1.f, 1.f, 1.f);
-    if(f.any_volume) b.media[p] = make_uint2(0xffffffffu, 0xffffffffu);
-    b.cone[p] = make_float2(f.cone_spread, 0.f);
 }
 
 //! pixels first .. first + n - 1: the whole image, or one of the pixel groups of a batch without a cache
@@ -430,18 +426,6 @@ __global__ void __launch_bounds__(PT_BLOCK) k_pt_begin(pt_frame f, pt_buffers b,
 __global__ void __launch_bounds__(PT_BLOCK) k_pt_zero(uint32_t *c, uint32_t n)
 {
     for(uint32_t i = threadIdx.x; i < n; i += PT_BLOCK) c[i] = 0u;
-}
-
-//! before a depth: the next queue, the shadow-ray count and the trace kernel's claim counters start at zero
-//! (one thread per claim counter)
-__global__ void k_pt_reset_depth(uint32_t *c, int next)
-{
-    if(threadIdx.x == 0)
-    {
-        c[C_QUEUE + next * COUNTER_LINE] = 0u;
-        c[C_SHADOW] = 0u;
-    }
-    c[PT_CLAIMS + threadIdx.x * COUNTER_STRIDE] = 0u;
 }
 
 //! the closest hit of path p's current ray at this depth; back faces are culled while the path is in air.
@@ -497,6 +481,13 @@ k_pt_trace(const vkrt_bvh_node *__restrict__ nodes, const float4 *__restrict__ t
            uint32_t depth, pt_tlas tl)
 {
     __shared__ int32_t smem[PT_LDS * PT_TRACE_BLOCK];
+    // nothing reads these between the last depth's shading and this depth's: the next queue's size, the shadow rays'
+    // number (a launch of its own for them cost 5 us a depth and a sample)
+    if(blockIdx.x == 0u && threadIdx.x == 0u)
+    {
+        b.counter[C_QUEUE + (in ^ 1) * COUNTER_LINE] = 0u;
+        b.counter[C_SHADOW] = 0u;
+    }
     const uint32_t count = b.counter[C_QUEUE + in * COUNTER_LINE];
     const uint32_t tiles = (count + PT_TRACE_BLOCK - 1) / PT_TRACE_BLOCK;
     const uint32_t home = blockIdx.x % XCDS;
@@ -609,19 +600,20 @@ __device__ __forceinline__ void shade_path(const pt_frame &f, const pt_buffers &
     uint32_t flags = st.y;
     float4 ro = b.ray_o[p], rd = b.ray_d[p];
     vec3 dir = xyz(rd);
-    const float4 beta4 = b.beta[p];
+    const bool fresh = depth == 0u;
+    const float4 beta4 = fresh ? make_float4(1.f, 1.f, 1.f, 0.f) : b.beta[p];
     vec3 beta = xyz(beta4);
     float prev_pdf = beta4.w;// payload.prev_bsdf_pdf
     // the traced segment, for the ghost-light pass after shading
     const vec3 seg_o = xyz(ro), seg_d = dir, seg_beta = beta;
     const float seg_tmin = ro.w, seg_tmax = rd.w, seg_prev_pdf = prev_pdf;
     const bool seg_caustic = (flags & F_CAUSTIC) != 0u;
-    vec3 radiance = xyz(b.rad[p]);
-    float2 cone = b.cone[p];// ray cone: spread angle, width (half precision values)
-    float4 iors = b.iors[p];
+    vec3 radiance = fresh ? vec3{0.f, 0.f, 0.f} : xyz(b.rad[p]);
+    float2 cone = fresh ? make_float2(f.cone_spread, 0.f) : b.cone[p];// ray cone: spread angle, width (half precision values)
+    float4 iors = fresh ? make_float4(1.f, 1.f, 1.f, 1.f) : b.iors[p];
     float ior_stack[MEDIA_STACK] = {iors.x, iors.y, iors.z, iors.w};
     uint32_t media_index = flags & F_MEDIA_MASK;
-    uint2 media = f.any_volume ? b.media[p] : make_uint2(0xffffffffu, 0xffffffffu);
+    uint2 media = f.any_volume && !fresh ? b.media[p] : make_uint2(0xffffffffu, 0xffffffffu);
     uint4 h = b.hit[p];
     bool stop = false;
     to_cache = false;
@@ -963,7 +955,8 @@ __device__ __forceinline__ void shade_path(const pt_frame &f, const pt_buffers &
         b.beta[p] = make_float4(beta.x, beta.y, beta.z, prev_pdf);
         b.rad[p] = make_float4(radiance.x, radiance.y, radiance.z, 0.f);
         b.cone[p] = cone;
-        b.iors[p] = make_float4(ior_stack[0], ior_stack[1], ior_stack[2], ior_stack[3]);
+        if(fresh || media_op == 1u)
+            b.iors[p] = make_float4(ior_stack[0], ior_stack[1], ior_stack[2], ior_stack[3]);
         if(f.any_volume) b.media[p] = media;
     }
     else
@@ -1051,6 +1044,8 @@ __global__ void __launch_bounds__(PT_BLOCK) k_pt_shade(pt_frame f, pt_buffers b,
 {
     const uint32_t count = b.counter[C_QUEUE + in * COUNTER_LINE];
     const uint32_t first = blockIdx.x * PT_BLOCK;
+    // this depth's trace is through, so its claim counters go back to zero for the next one
+    if(blockIdx.x == 0u && threadIdx.x < XCDS) b.counter[PT_CLAIMS + threadIdx.x * COUNTER_STRIDE] = 0u;
     if(first < count) shade_queue_entry<LIGHTS, INST>(f, b, s, depth, in, first + threadIdx.x, count);
 }
 
@@ -2089,7 +2084,6 @@ static void trace_batch(vkrt_pt *pt, const vkrt_camera &cam, uint32_t seed)
     auto depth_step = [&](const group &g, uint32_t depth, int in) {
         const pt_buffers &bb = g.b;
         hipStream_t st = g.stream;
-        k_pt_reset_depth<<<1, XCDS, 0, st>>>(bb.counter, in ^ 1);
         variant([&](auto a, auto in_) {
             using F = std::conditional_t<decltype(a)::value, alpha_filter, keep_all>;
             constexpr bool I = decltype(in_)::value;
