@@ -205,9 +205,7 @@ struct pt_tlas
     const vkrt_bvh4_node *tlas;
     int32_t root;
     uint32_t empty;
-    const uint32_t *order;
     const inst_dev *insts;
-    const blas_dev *blases;
 };
 
 //! transform_t applied to a point and to a direction (utils/transform.slang: rotate_quat, apply_transform)
@@ -451,8 +449,7 @@ __device__ __forceinline__ void trace_path(const vkrt_bvh_node *__restrict__ nod
             const bool in_air = (st.y & F_MEDIA_MASK) == 0u;
             if constexpr(F::active) flt.xi = rnd_peek(xxhash32(st.x, depth));
             t = rb.w;
-            scene_walk<false, BLOCK, PT_LDS, F>(tl.tlas, tl.root, tl.order, tl.insts, tl.blases, ra, rb, smem, t, u, v,
-                                                prim, inst, in_air, flt);
+            scene_walk<false, BLOCK, PT_LDS, F>(tl.tlas, tl.root, tl.insts, ra, rb, smem, t, u, v, prim, inst, in_air, flt);
         }
         b.hit_inst[p] = inst;
     }
@@ -1325,18 +1322,15 @@ __device__ float4 transmittance_walk_scene(const pt_tlas &tl, const gpu_material
             }
             else if(base < 0)
             {
-                uint32_t first, count;
-                leaf_decode(ref, first, count);
-                inst = tl.order[first];
+                inst = leaf_instance(ref);
                 const inst_dev I = tl.insts[inst];
-                const blas_dev B = tl.blases[I.blas];
-                if(!B.empty)
+                if(I.nodes)
                 {
                     r = object_ray(I, ra, rb);
-                    nodes = B.nodes;
-                    tris = B.tris;
+                    nodes = I.nodes;
+                    tris = I.tris;
                     base = sp;
-                    ref = B.root;
+                    ref = I.root;
                     continue;
                 }
             }
@@ -2626,7 +2620,7 @@ int vkrt_pt_set_instanced_scene(vkrt_pt *pt, const vkrt_pt_scene *sc, const uint
                                          &pt->scene);
         if(rc != VKRT_OK) throw error(rc, "instanced scene: " + pt->ctx->last_error);
         const scene_view v = scene_device_view(pt->scene);
-        pt->tlas = pt_tlas{v.tlas, v.root, v.empty, v.order, v.insts, v.blases};
+        pt->tlas = pt_tlas{v.tlas, v.root, v.empty, v.insts};
         pt->inst_xf.reserve(std::max<size_t>(1, xf.size()) * 16);
         if(!xf.empty())
             VKRT_HIP(hipMemcpyAsync(pt->inst_xf.ptr, xf.data(), xf.size() * 16, hipMemcpyHostToDevice, s));

@@ -29,9 +29,7 @@ constexpr int SCENE_LDS = 16;
 
 template<bool ANY, int BLOCK, int LDS_DEPTH>
 __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5))) k_scene_trace(const vkrt_bvh4_node *__restrict__ tlas, int32_t troot,
-                                                       uint32_t empty_scene, const uint32_t *__restrict__ order,
-                                                       const inst_dev *__restrict__ insts,
-                                                       const blas_dev *__restrict__ blases,
+                                                       uint32_t empty_scene, const inst_dev *__restrict__ insts,
                                                        const float4 *__restrict__ rays, uint32_t n,
                                                        void *__restrict__ out, uint32_t chunk)
 {
@@ -42,8 +40,8 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5)))
     float best_t = rb.w, best_u = 0.f, best_v = 0.f;
     uint32_t best_prim = VKRT_INVALID_PRIM, best_inst = VKRT_INVALID_PRIM;
     if(!empty_scene)
-        scene_walk<ANY, BLOCK, LDS_DEPTH>(tlas, troot, order, insts, blases, ra, rb, smem + threadIdx.x, best_t,
-                                          best_u, best_v, best_prim, best_inst);
+        scene_walk<ANY, BLOCK, LDS_DEPTH, keep_all, !ANY>(tlas, troot, insts, ra, rb, smem + threadIdx.x, best_t, best_u, best_v,
+                                          best_prim, best_inst);
     const bool hit = best_prim != VKRT_INVALID_PRIM;
     if(ANY) static_cast<uint8_t *>(out)[i] = hit ? 1 : 0;
     else
@@ -68,7 +66,8 @@ struct vkrt_scene
     vkrt_ctx *ctx = nullptr;
     std::vector<const vkrt_bvh *> blas;
     std::vector<vkrt_instance> instances;
-    vkrt::device_buffer nodes, order, insts, blases;
+    std::vector<vkrt::inst_dev> mesh;// per mesh what its instances share (nodes, tris, root)
+    vkrt::device_buffer nodes, insts;
     int32_t root = 0;
     bool empty = true;
     uint32_t n_nodes = 0, tlas_stack = 0, max_blas_stack = 0;
@@ -225,7 +224,7 @@ struct tlas_builder
     //! ref of the subtree over order[lo, hi): a leaf of one instance or a new 4-wide node
     int32_t build(uint32_t lo, uint32_t hi, uint32_t stack_in)
     {
-        if(hi - lo == 1) return static_cast<int32_t>(~(lo << 3));
+        if(hi - lo == 1) return static_cast<int32_t>(~order[lo]);
         uint32_t ranges[4][2];
         int cnt = 0;
         const uint32_t mid = split(lo, hi);
@@ -340,24 +339,20 @@ static void build_tlas(vkrt_scene *sc)
     hipStream_t s = sc->ctx->stream;
     sc->n_nodes = static_cast<uint32_t>(nodes.size());
     sc->nodes.reserve(std::max<size_t>(1, nodes.size()) * sizeof(vkrt_bvh4_node));
-    sc->order.reserve(std::max<size_t>(1, order.size()) * 4);
     std::vector<inst_dev> in(std::max<uint32_t>(1, n));
     for(uint32_t k = 0; k < n; ++k)
     {
         const float *w = sc->instances[k].world_to_object;
+        in[k] = sc->mesh[sc->instances[k].blas];
         in[k].w0 = make_float4(w[0], w[1], w[2], w[3]);
         in[k].w1 = make_float4(w[4], w[5], w[6], w[7]);
         in[k].w2 = make_float4(w[8], w[9], w[10], w[11]);
-        in[k].blas = sc->instances[k].blas;
         in[k].custom = sc->instances[k].custom_index;
-        in[k].pad0 = in[k].pad1 = 0;
     }
     sc->insts.reserve(in.size() * sizeof(inst_dev));
     if(!nodes.empty())
         VKRT_HIP(hipMemcpyAsync(sc->nodes.ptr, nodes.data(), nodes.size() * sizeof(vkrt_bvh4_node),
                                 hipMemcpyHostToDevice, s));
-    if(!order.empty())
-        VKRT_HIP(hipMemcpyAsync(sc->order.ptr, order.data(), order.size() * 4, hipMemcpyHostToDevice, s));
     VKRT_HIP(hipMemcpyAsync(sc->insts.ptr, in.data(), in.size() * sizeof(inst_dev), hipMemcpyHostToDevice, s));
     VKRT_HIP(hipStreamSynchronize(s));
 }
@@ -376,8 +371,7 @@ static void check_instances(const vkrt_scene *sc, const vkrt_instance *inst, uin
 
 scene_view scene_device_view(const vkrt_scene *sc)
 {
-    return scene_view{sc->nodes.as<vkrt_bvh4_node>(), sc->root, sc->empty ? 1u : 0u, sc->order.as<uint32_t>(),
-                      sc->insts.as<inst_dev>(), sc->blases.as<blas_dev>()};
+    return scene_view{sc->nodes.as<vkrt_bvh4_node>(), sc->root, sc->empty ? 1u : 0u, sc->insts.as<inst_dev>()};
 }
 
 template<bool ANY>
@@ -387,8 +381,8 @@ static void launch_scene(vkrt_scene *sc, const float4 *rays, uint32_t n, void *o
     const uint32_t chunk = sc->ctx->trace_cfg.xcd_chunk;
     k_scene_trace<ANY, SCENE_BLOCK, SCENE_LDS><<<xcd_grid(div_up(n, SCENE_BLOCK), chunk), SCENE_BLOCK, 0,
                                                  sc->ctx->stream>>>(
-            sc->nodes.as<vkrt_bvh4_node>(), sc->root, sc->empty ? 1u : 0u, sc->order.as<uint32_t>(),
-            sc->insts.as<inst_dev>(), sc->blases.as<blas_dev>(), rays, n, out, chunk);
+            sc->nodes.as<vkrt_bvh4_node>(), sc->root, sc->empty ? 1u : 0u, sc->insts.as<inst_dev>(), rays, n, out,
+            chunk);
     VKRT_HIP(hipGetLastError());
 }
 
@@ -407,7 +401,6 @@ int vkrt_scene_create(vkrt_ctx *ctx, vkrt_bvh *const *meshes, uint32_t n_meshes,
         VKRT_REQUIRE(n_meshes == 0 || meshes, "null mesh list");
         auto sc = std::make_unique<vkrt_scene>();
         sc->ctx = ctx;
-        std::vector<blas_dev> bd(std::max<uint32_t>(1, n_meshes));
         for(uint32_t m = 0; m < n_meshes; ++m)
         {
             const vkrt_bvh *b = meshes[m];
@@ -415,12 +408,16 @@ int vkrt_scene_create(vkrt_ctx *ctx, vkrt_bvh *const *meshes, uint32_t n_meshes,
             VKRT_REQUIRE(b->device == ctx->device, "mesh BVH belongs to another device");
             VKRT_REQUIRE(b->empty || b->wide, "mesh BVHs of a scene need the 4-wide layout (width 0 or 4)");
             sc->blas.push_back(b);
-            bd[m] = blas_dev{b->nodes4.as<vkrt_bvh4_node>(), b->tris.as<float4>(), b->root4, b->empty ? 1u : 0u};
+            inst_dev mesh{};
+            if(!b->empty)
+            {
+                mesh.nodes = b->nodes4.as<vkrt_bvh4_node>();
+                mesh.tris = b->tris.as<float4>();
+                mesh.root = b->root4;
+            }
+            sc->mesh.push_back(mesh);
             sc->max_blas_stack = std::max(sc->max_blas_stack, b->stack4);
         }
-        sc->blases.reserve(bd.size() * sizeof(blas_dev));
-        VKRT_HIP(hipMemcpyAsync(sc->blases.ptr, bd.data(), bd.size() * sizeof(blas_dev), hipMemcpyHostToDevice,
-                                ctx->stream));
         check_instances(sc.get(), instances, n_instances);
         sc->instances.assign(instances, instances + n_instances);
         build_tlas(sc.get());

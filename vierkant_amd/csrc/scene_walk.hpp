@@ -14,19 +14,20 @@ namespace vkrt
 
 constexpr int SCENE_STACK = 96;  // top-level + BLAS entries per ray; checked at build time
 
+//! an instance and its mesh: one read starts a mesh walk. (The mesh in a table of its own, and a leaf naming its
+//! instance through a second one, are two more round trips to memory in a row, for every instance the top level keeps:
+//! 1M rays into 1,000 instances and a heightfield 719 -> 710 us.)
 struct inst_dev
 {
     float4 w0, w1, w2;// world-to-object rows
-    uint32_t blas, custom, pad0, pad1;
-};
-
-struct blas_dev
-{
-    const vkrt_bvh4_node *nodes;
+    const vkrt_bvh4_node *nodes;// null: an empty mesh
     const float4 *tris;
     int32_t root;
-    uint32_t empty;
+    uint32_t custom, pad0, pad1;
 };
+
+//! the instance a top-level leaf holds
+__host__ __device__ __forceinline__ uint32_t leaf_instance(int32_t ref) { return static_cast<uint32_t>(~ref); }
 
 //! object-space setup of world ray (ra, rb) for instance I: each row ((w0 x + w1 y) + w2 z) + w3, the direction
 //! keeping its length (so t is shared by both spaces)
@@ -44,8 +45,9 @@ __device__ __forceinline__ ray_setup object_ray(const inst_dev &I, const float4 
 constexpr int SCENE_CAND = 4;     // instances kept per top-level pass of scene_walk
 
 //! one mesh leaf's triangles against the object ray, (t, instance, triangle) order; true when one became the
-//! best record
-template<bool ANY, class F>
+//! best record. PAIR: the first two records are asked for together (one round trip for a leaf of the default size;
+//! twelve more VGPRs, which the scene's closest-hit kernel has: 631 -> 615 us, and the path tracer's has not)
+template<bool ANY, bool PAIR, class F>
 __device__ __forceinline__ bool mesh_leaf(const float4 *__restrict__ tris, int32_t ref, const ray_setup &r,
                                           uint32_t inst, float &best_t, float &best_u, float &best_v,
                                           uint32_t &best_prim, uint32_t &best_inst, bool cull_back, const F &filter)
@@ -53,11 +55,24 @@ __device__ __forceinline__ bool mesh_leaf(const float4 *__restrict__ tris, int32
     uint32_t first, count;
     leaf_decode(ref, first, count);
     bool found = false;
+    size_t tb = (size_t)TRI_BYTES * first;
+    float4 p0 = load_global_f4(tris, tb), p1 = load_global_f4(tris, tb + 16), p2 = load_global_f4(tris, tb + 32);
+    float4 n0, n1, n2;
+    if constexpr(PAIR)
+    {
+        const size_t tb2 = tb + (count > 1u ? TRI_BYTES : 0u);
+        n0 = load_global_f4(tris, tb2), n1 = load_global_f4(tris, tb2 + 16), n2 = load_global_f4(tris, tb2 + 32);
+        // (the empty asm keeps the loads together, before the first test)
+        asm volatile("" : "+v"(p0.x), "+v"(p1.x), "+v"(p2.x), "+v"(n0.x), "+v"(n1.x), "+v"(n2.x));
+    }
     for(uint32_t k = 0; k < count; ++k)
     {
-        const size_t tb = (size_t)TRI_BYTES * (first + k);
-        const float4 p0 = load_global_f4(tris, tb), p1 = load_global_f4(tris, tb + 16),
-                     p2 = load_global_f4(tris, tb + 32);
+        if(PAIR && k == 1u) p0 = n0, p1 = n1, p2 = n2;
+        if(k > (PAIR ? 1u : 0u))
+        {
+            tb = (size_t)TRI_BYTES * (first + k);
+            p0 = load_global_f4(tris, tb), p1 = load_global_f4(tris, tb + 16), p2 = load_global_f4(tris, tb + 32);
+        }
         float t, u, v;
         const bool cull = cull_back && !(__float_as_uint(p2.w) & TRI_TWO_SIDED);
         if(vierkant::rt::mt_fast(r.o, r.d, vec3{p0.x, p0.y, p0.z}, vec3{p0.w, p1.x, p1.y}, vec3{p1.z, p1.w, p2.x}, t,
@@ -85,7 +100,7 @@ __device__ __forceinline__ bool mesh_leaf(const float4 *__restrict__ tris, int32
 //! one instance's mesh walked with its object ray, which stays fixed for the whole walk (the loop then
 //! carries no ray state from one level to another), the best record carried in and out; the step
 //! structure of the flat 4-wide walk. Returns true when ANY found a hit
-template<bool ANY, int BLOCK, int LDS_DEPTH, class F>
+template<bool ANY, bool PAIR, int BLOCK, int LDS_DEPTH, class F>
 __device__ __forceinline__ bool mesh_walk(const vkrt_bvh4_node *__restrict__ nodes, const float4 *__restrict__ tris,
                                           int32_t root, const ray_setup &r, lane_stack<BLOCK, LDS_DEPTH> &st,
                                           uint32_t inst, float &best_t, float &best_u, float &best_v,
@@ -121,7 +136,7 @@ __device__ __forceinline__ bool mesh_walk(const vkrt_bvh4_node *__restrict__ nod
                 continue;
             }
         }
-        else if(mesh_leaf<ANY, F>(tris, ref, r, inst, best_t, best_u, best_v, best_prim, best_inst, cull_back,
+        else if(mesh_leaf<ANY, PAIR, F>(tris, ref, r, inst, best_t, best_u, best_v, best_prim, best_inst, cull_back,
                                   filter) &&
                 ANY)
             return true;
@@ -142,10 +157,9 @@ __device__ __forceinline__ bool mesh_walk(const vkrt_bvh4_node *__restrict__ nod
 //! cull_back drops candidates seen from behind (object-space determinant below zero) unless their record is
 //! flagged TRI_TWO_SIDED; a candidate that would become the closest and whose record is flagged
 //! TRI_ALPHA_MASK is kept only if filter(record's last float4, u, v) says so (keep_all: no any-hit stage)
-template<bool ANY, int BLOCK, int LDS_DEPTH, class F = keep_all>
+template<bool ANY, int BLOCK, int LDS_DEPTH, class F = keep_all, bool PAIR = false>
 __device__ __forceinline__ void scene_walk(const vkrt_bvh4_node *__restrict__ tlas, int32_t troot,
-                                           const uint32_t *__restrict__ order, const inst_dev *__restrict__ insts,
-                                           const blas_dev *__restrict__ blases, const float4 &ra, const float4 &rb,
+                                           const inst_dev *__restrict__ insts, const float4 &ra, const float4 &rb,
                                            int32_t *lds, float &best_t, float &best_u, float &best_v,
                                            uint32_t &best_prim, uint32_t &best_inst, bool cull_back = false,
                                            const F &filter = F{})
@@ -198,9 +212,7 @@ __device__ __forceinline__ void scene_walk(const vkrt_bvh4_node *__restrict__ tl
         if(troot < 0)
         {
             // a single instance: no box to enter, walked whatever the ray
-            uint32_t first, count;
-            leaf_decode(troot, first, count);
-            keep(-__int_as_float(0x7f800000), order[first]);
+            keep(-__int_as_float(0x7f800000), leaf_instance(troot));
         }
         else
         {
@@ -232,11 +244,7 @@ __device__ __forceinline__ void scene_walk(const vkrt_bvh4_node *__restrict__ tl
                 auto take = [&](float q, int32_t c) {
                     if(!(q < KEY_MISSED)) return;
                     if(c < 0)
-                    {
-                        uint32_t first, count;
-                        leaf_decode(c, first, count);
-                        keep(q, order[first]);
-                    }
+                        keep(q, leaf_instance(c));
                     else
                     {
                         if(have) st.put(sp++, next);
@@ -272,10 +280,9 @@ __device__ __forceinline__ void scene_walk(const vkrt_bvh4_node *__restrict__ tl
             lb_k = ck[j];
             lb_i = inst;
             const inst_dev I = insts[inst];
-            const blas_dev B = blases[I.blas];
-            if(B.empty) continue;
+            if(!I.nodes) continue;
             const ray_setup ro = object_ray(I, ra, rb);
-            if(mesh_walk<ANY, BLOCK, LDS_DEPTH, F>(B.nodes, B.tris, B.root, ro, st, inst, best_t, best_u, best_v,
+            if(mesh_walk<ANY, PAIR, BLOCK, LDS_DEPTH, F>(I.nodes, I.tris, I.root, ro, st, inst, best_t, best_u, best_v,
                                                    best_prim, best_inst, cull_back, filter))
                 return;
         }
@@ -284,15 +291,13 @@ __device__ __forceinline__ void scene_walk(const vkrt_bvh4_node *__restrict__ tl
     }
 }
 
-//! device pointers of a two-level scene's top level, instances and meshes (kept by the scene object)
+//! device pointers of a two-level scene's top level and instances (kept by the scene object)
 struct scene_view
 {
     const vkrt_bvh4_node *tlas;
     int32_t root;
     uint32_t empty;
-    const uint32_t *order;
     const inst_dev *insts;
-    const blas_dev *blases;
 };
 
 scene_view scene_device_view(const vkrt_scene *sc);
