@@ -56,6 +56,23 @@ def test_brute_over_magnitudes(ctx, centre, scale):
     check(ctx, *soup(np.random.default_rng(9), 700, 400, centre, scale), f"{centre} {scale}")
 
 
+@pytest.mark.parametrize("distance", [1e2, 1e3, 1e5, 1e8, 1e14])
+def test_brute_from_far_away(ctx, distance):
+    """rays whose origins lie far from the triangles, with directions from tiny to long"""
+    rng = np.random.default_rng(15)
+    tris, rays = soup(rng, 600, 500)
+    d = rng.normal(size=(500, 3))
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    o = -distance * d + rng.uniform(-0.7, 0.7, (500, 3))
+    d *= 10.0 ** rng.integers(-25, 6, (500, 1))
+    for k, axis in enumerate("xyz"):
+        rays["o" + axis], rays["d" + axis] = o[:, k].astype(np.float32), d[:, k].astype(np.float32)
+    rays["tmin"], rays["tmax"] = 0.0, np.inf
+    want = check(ctx, tris, rays, f"from {distance}")
+    if distance < 1e5:
+        assert (want["prim"] != 0xFFFFFFFF).sum() > 30
+
+
 def test_brute_with_large_small_and_non_finite(ctx):
     """triangles of 1e-3 beside ones of 1e5, sparse NaNs, infinities and huge vertices, directions of any length, and
     rays with NaN or infinite parts or intervals: the first triangle of a chunk among them"""

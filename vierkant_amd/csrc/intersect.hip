@@ -155,13 +155,18 @@ __global__ void k_fill_u8(uint8_t *__restrict__ p, uint32_t n, uint8_t value)
 //
 // The factors go in as two bf16 parts each, hi + mid, off by 2^-16 of the factor; a lane's half holds the
 // triangle's hi or mid parts and the two MFMAs of a product take the ray's hi and its mid parts. With
-// P = |d| E (|o| + V) (E the longest edge and V the farthest vertex of 32 triangles, all about the chunk's first
-// vertex) the parts are off by at most 2^-15 P, the 24 terms' sum by less than 2^-19 P, the reference's own
-// a, b and det by less than 2^-19 P: a pair whose three values are not all above -2^-14 P - 2^-70, nor all below
-// its negative, is no hit of the reference's. 2^-70 covers what is lost below the normal range while every
-// factor stays below 2^40; a ray or a tile beyond that, or with a NaN or an infinity, takes every pair.
+// P = |d| E (|f| + V) (E the longest edge and V the farthest vertex of 32 triangles, f the point of the ray's line
+// nearest to the origin, all about the chunk's first vertex; o x d = f x d, so rays from far away lose no more than near
+// ones) the parts are off by at most 2^-15 P, the 24 terms' sum by less than 2^-19 P, and f itself and the reference's
+// own a, b and det by less than 2^-18 |d| E (|o| + V): a pair whose three values are not all above
+// -|d| E (2^-14 (|f| + V) + 2^-18 |o|) - 2^-70, nor all below its negative, is no hit of the reference's. 2^-70 covers
+// what is lost below the normal range while every factor stays below 2^40; a ray or a tile beyond that, or with a NaN or
+// an infinity, takes every pair: 1.3 times the time of a test for every pair where that is all tiles (one NaN in 32
+// triangles), 0.6 with one in 320. Constants that keep such a triangle alone out of the filter made every other case 5 %
+// slower.
 //
-// 65,536 rays x 20,480 triangles: 1,220 us with the reference's test for every pair, 237 so, the matrix cores busy
+// 65,536 rays x 20,480 triangles: 1,210 us with the reference's test for every pair, 239 so (origins a thousand radii
+// away 369, without f 1,630), the matrix cores busy
 // for 48 % of them and 69 VALU instructions a wave per 32 x 32 pairs, 48 of them the filter's. Two products of
 // 32 x 32 in flight per wave, at two or three waves a SIMD, are no faster: 248 - 255.
 constexpr float BRUTE_LIMIT = 0x1p40f;
@@ -224,8 +229,10 @@ __global__ void __launch_bounds__(256, GROUPS > 2 ? 3 : 4) k_brute(const float4 
         float tmin = 0.f, tmax = -1.f;
         if(r < n_ray) load_ray(rays, r, o, tmin, d, tmax);
         o = o - centre;
-        split_bf16(cross(o, d), d, ray_hi[g], ray_mid[g]);
-        ray_o[g] = norm_above(o);
+        const float dd = dot(d, d);
+        const vec3 foot = dd > 0x1p-100f ? o - d * (dot(o, d) / dd) : o;
+        split_bf16(cross(foot, d), d, ray_hi[g], ray_mid[g]);
+        ray_o[g] = norm_above(foot) + 0x1p-4f * norm_above(o);
         ray_d[g] = norm_above(d);
         if(!(ray_o[g] < BRUTE_LIMIT && ray_d[g] < BRUTE_LIMIT && ray_o[g] * ray_d[g] < BRUTE_LIMIT))
             ray_d[g] = __int_as_float(0x7fc00000);
@@ -302,34 +309,42 @@ __global__ void __launch_bounds__(256, GROUPS > 2 ? 3 : 4) k_brute(const float4 
 
                 // a NaN margin gets here for rays that take no pair too, and for those past the end
                 if(ray_d[g] == -__int_as_float(0x7f800000)) continue;
+                vec3 o, d;
+                float tmin, tmax;
+                load_ray(rays, first_ray + 32u * g, o, tmin, d, tmax);
+                auto test = [&](uint32_t row) {
+                    const float4 q0 = records[row][0], q1 = records[row][1], q2 = records[row][2];
+                    float t, u, v;
+                    if(!mt_fast_window(o, d, vec3{q0.x, q0.y, q0.z}, vec3{q0.w, q1.x, q1.y}, vec3{q1.z, q1.w, q2.x},
+                                       tmin, best[g], t, u, v))
+                        return;
+                    // (ANY: the ray takes no pair any more)
+                    if(ANY) ray_d[g] = -__int_as_float(0x7f800000);
+                    else best[g] = t;
+                    best_i[g] = base + row;
+                };
+                const uint32_t row0 = 32u * tile + 4u * half;
+                if(__any(!(margin < __int_as_float(0x7f800000))))
+                {
+                    // no bound for some ray: every pair, a step's records asked for ahead of its tests
+#pragma unroll 4
+                    for(uint32_t i = 0; i < 16; ++i)
+                        if(row0 + 8u * (i >> 2) + (i & 3u) < n) test(row0 + 8u * (i >> 2) + (i & 3u));
+                    continue;
+                }
                 uint32_t mask = 0;
 #pragma unroll
                 for(int i = 0; i < 16; ++i)
                     mask |= fmaxf(above(m[0][i], m[1][i], m[2][i]), below(m[0][i], m[1][i], m[2][i])) < -margin
                                 ? 0u
                                 : 1u << i;
-                vec3 o, d;
-                float tmin, tmax;
-                load_ray(rays, first_ray + 32u * g, o, tmin, d, tmax);
                 while(mask)
                 {
-                    const uint32_t i = __ffs(static_cast<int>(mask)) - 1;
+                    const uint32_t i = __ffs(static_cast<int>(mask)) - 1, row = row0 + 8u * (i >> 2) + (i & 3u);
                     mask &= mask - 1u;
-                    const uint32_t row = 32u * tile + 8u * (i >> 2) + 4u * half + (i & 3u);
                     if(row >= n) break;
-                    const float4 q0 = records[row][0], q1 = records[row][1], q2 = records[row][2];
-                    float t, u, v;
-                    if(mt_fast_window(o, d, vec3{q0.x, q0.y, q0.z}, vec3{q0.w, q1.x, q1.y}, vec3{q1.z, q1.w, q2.x},
-                                      tmin, best[g], t, u, v))
-                    {
-                        best_i[g] = base + row;
-                        if(ANY)
-                        {
-                            ray_d[g] = -__int_as_float(0x7f800000);
-                            break;
-                        }
-                        best[g] = t;
-                    }
+                    test(row);
+                    if(ANY && ray_d[g] == -__int_as_float(0x7f800000)) break;
                 }
             }
             if(ANY)
