@@ -166,9 +166,9 @@ __global__ void k_fill_u8(uint8_t *__restrict__ p, uint32_t n, uint8_t value)
 // slower.
 //
 // 65,536 rays x 20,480 triangles: 1,210 us with the reference's test for every pair, 239 so (origins a thousand radii
-// away 369, without f 1,630), the matrix cores busy
-// for 48 % of them and 69 VALU instructions a wave per 32 x 32 pairs, 48 of them the filter's. Two products of
-// 32 x 32 in flight per wave, at two or three waves a SIMD, are no faster: 248 - 255.
+// away 369, without f 1,630), the matrix cores busy for 48 % of them and 69 VALU instructions a wave per 32 x 32 pairs,
+// 48 of them the filter's. Two products of 32 x 32 in flight per wave, at two or three waves a SIMD, are no faster:
+// 248 - 255.
 constexpr float BRUTE_LIMIT = 0x1p40f;
 constexpr int BRUTE_STAGE = 256;// triangles in LDS at a time, one a thread
 constexpr int BRUTE_TILES = BRUTE_STAGE / 32;
