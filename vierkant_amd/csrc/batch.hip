@@ -42,8 +42,9 @@ constexpr uint32_t N_COUNTERS = CLAIM_COUNTERS;
 __global__ void k_batch_reset(uint32_t *counter) { counter[threadIdx.x] = 0u; }
 
 //! (8 waves per SIMD where the LDS stack allows it: the traversal fits 64 VGPRs with a spill or two of the
-//! loop state, against 72 unconstrained, which holds 7)
-template<int BLOCK, int LDS>
+//! loop state, against 72 unconstrained, which holds 7). JOINT: every 4-wide item's nodes and records are within reach
+//! of one base
+template<int BLOCK, int LDS, bool JOINT>
 __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8))) k_batch_trace(const batch_item_dev *__restrict__ items, uint32_t n_items,
                                                        const uint32_t *__restrict__ tile_prefix, uint32_t tile,
                                                        uint32_t *__restrict__ counters, uint32_t chunk)
@@ -81,8 +82,8 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8)))
             if(!it.empty)
             {
                 ray_setup rs = setup_ray(it.rays, r);
-                hit = it.wide ? traverse4<false, BLOCK, LDS>(it.nodes4, it.tris, it.root4, rs, smem + threadIdx.x, bt,
-                                                             bu, bv, prim)
+                hit = it.wide ? traverse4<false, BLOCK, LDS, keep_all, JOINT>(it.nodes4, it.tris, it.root4, rs,
+                                                                              smem + threadIdx.x, bt, bu, bv, prim)
                               : traverse<false, BLOCK, LDS>(it.nodes, it.tris, it.root, rs, smem + threadIdx.x, bt, bu,
                                                             bv, prim);
             }
@@ -93,26 +94,27 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8)))
 }
 
 template<int BLOCK, int LDS>
-static void launch_batch(hipStream_t s, uint32_t grid, const batch_item_dev *items, uint32_t n_items,
+static void launch_batch(hipStream_t s, uint32_t grid, bool joint, const batch_item_dev *items, uint32_t n_items,
                          const uint32_t *prefix, uint32_t tile, uint32_t *counter, uint32_t chunk)
 {
-    k_batch_trace<BLOCK, LDS><<<grid, BLOCK, 0, s>>>(items, n_items, prefix, tile, counter, chunk);
+    if(joint) k_batch_trace<BLOCK, LDS, true><<<grid, BLOCK, 0, s>>>(items, n_items, prefix, tile, counter, chunk);
+    else k_batch_trace<BLOCK, LDS, false><<<grid, BLOCK, 0, s>>>(items, n_items, prefix, tile, counter, chunk);
 }
 
 template<int BLOCK>
-static void launch_batch_lds(hipStream_t s, uint32_t lds, uint32_t grid, const batch_item_dev *items,
+static void launch_batch_lds(hipStream_t s, uint32_t lds, uint32_t grid, bool joint, const batch_item_dev *items,
                              uint32_t n_items, const uint32_t *prefix, uint32_t tile, uint32_t *counter,
                              uint32_t chunk)
 {
     switch(lds)
     {
-        case 0: launch_batch<BLOCK, 0>(s, grid, items, n_items, prefix, tile, counter, chunk); break;
-        case 8: launch_batch<BLOCK, 8>(s, grid, items, n_items, prefix, tile, counter, chunk); break;
-        case 16: launch_batch<BLOCK, 16>(s, grid, items, n_items, prefix, tile, counter, chunk); break;
-        case 24: launch_batch<BLOCK, 24>(s, grid, items, n_items, prefix, tile, counter, chunk); break;
-        case 32: launch_batch<BLOCK, 32>(s, grid, items, n_items, prefix, tile, counter, chunk); break;
-        case 48: launch_batch<BLOCK, 48>(s, grid, items, n_items, prefix, tile, counter, chunk); break;
-        default: launch_batch<BLOCK, 64>(s, grid, items, n_items, prefix, tile, counter, chunk); break;
+        case 0: launch_batch<BLOCK, 0>(s, grid, joint, items, n_items, prefix, tile, counter, chunk); break;
+        case 8: launch_batch<BLOCK, 8>(s, grid, joint, items, n_items, prefix, tile, counter, chunk); break;
+        case 16: launch_batch<BLOCK, 16>(s, grid, joint, items, n_items, prefix, tile, counter, chunk); break;
+        case 24: launch_batch<BLOCK, 24>(s, grid, joint, items, n_items, prefix, tile, counter, chunk); break;
+        case 32: launch_batch<BLOCK, 32>(s, grid, joint, items, n_items, prefix, tile, counter, chunk); break;
+        case 48: launch_batch<BLOCK, 48>(s, grid, joint, items, n_items, prefix, tile, counter, chunk); break;
+        default: launch_batch<BLOCK, 64>(s, grid, joint, items, n_items, prefix, tile, counter, chunk); break;
     }
 }
 
@@ -172,6 +174,7 @@ struct vkrt_batch
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     uint64_t total_rays = 0;
+    bool joint = true;// no item's walk is WALK_APART
 };
 
 namespace vkrt
@@ -210,9 +213,9 @@ static void prepare(vkrt_batch *b)
     const uint32_t ld = b->cfg.lds_stack_depth, tl = b->cfg.tile, ch = b->cfg.xcd_chunk;
     switch(b->cfg.block_size)
     {
-        case 64: launch_batch_lds<64>(s, ld, grid, items, n, pre, tl, counter, ch); break;
-        case 128: launch_batch_lds<128>(s, ld, grid, items, n, pre, tl, counter, ch); break;
-        default: launch_batch_lds<256>(s, ld, grid, items, n, pre, tl, counter, ch); break;
+        case 64: launch_batch_lds<64>(s, ld, grid, b->joint, items, n, pre, tl, counter, ch); break;
+        case 128: launch_batch_lds<128>(s, ld, grid, b->joint, items, n, pre, tl, counter, ch); break;
+        default: launch_batch_lds<256>(s, ld, grid, b->joint, items, n, pre, tl, counter, ch); break;
     }
     hipError_t launch_err = hipGetLastError();
     hipError_t end_err = hipStreamEndCapture(s, &b->graph);
@@ -269,7 +272,8 @@ int vkrt_batch_create(vkrt_ctx *ctx, const vkrt_batch_item *items, uint32_t n_it
             d.empty = it.bvh->empty ? 1u : 0u;
             d.n_rays = it.n_rays;
             d.root4 = it.bvh->root4;
-            d.wide = it.bvh->wide && it.bvh->joint ? 1u : 0u;
+            d.wide = it.bvh->wide ? 1u : 0u;
+            if(it.bvh->walk() == WALK_APART) b->joint = false;
             b->items.push_back(d);
             b->n_rays.push_back(it.n_rays);
             b->total_rays += it.n_rays;

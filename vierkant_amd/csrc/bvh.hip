@@ -1527,8 +1527,8 @@ static void build_tree(vkrt_ctx *ctx, vkrt_bvh *bvh, const mesh_view &mesh, cons
     // the 4-wide walk addresses nodes with 32-bit byte offsets (node4_intervals)
     bvh->wide = bvh->allow_wide && bvh->stack4 <= (uint32_t)STACK_SIZE &&
                 (uint64_t)bvh->n_nodes4 * sizeof(vkrt_bvh4_node) <= 0xffffffffull;
-    if(bvh->wide && bvh->joint) return;
-    // the binary tree stays where traversal or a refit uses it
+    if(bvh->wide) return;
+    // the binary tree stays where traversal uses it
     const size_t ni = n - 1u;
     place(bvh->binary, {{&bvh->nodes, ni * sizeof(vkrt_bvh_node)}, {&bvh->child, ni * sizeof(int2)},
                         {&bvh->range, ni * sizeof(uint2)}});

@@ -25,6 +25,18 @@ struct vkrt_bvh4_node
     int4 pad;
 };
 
+namespace vkrt
+{
+//! the walk that a BVH's layout takes: the binary tree, or the 4-wide collapse with nodes and records within reach of
+//! one base (joint) or each from its own
+enum walk_layout : uint32_t
+{
+    WALK_BINARY = 0,
+    WALK_JOINT = 1,
+    WALK_APART = 2
+};
+}// namespace vkrt
+
 struct vkrt_bvh
 {
     //! a part of the BVH's one allocation
@@ -46,13 +58,13 @@ struct vkrt_bvh
     bool empty = true;
     // One allocation holds the 4-wide collapse, used by traversal when its worst-case stack fits (wide == true), the
     // leaf records behind it, so that a walk reaches both with 32-bit offsets from one base (joint == true unless
-    // they pass 4 GiB), and what a refit needs: the mesh's indices, the leaves' order and the run of leaves below
+    // they pass 4 GiB, from some 41M triangles at two a leaf), and what a refit needs: the mesh's indices, the leaves' order and the run of leaves below
     // each 4-wide node. (Freeing a large allocation takes 250 to 500 us: eight of them took 1.7 of the 4.1 ms that
     // building and destroying a 1.8M-triangle BVH took.)
     vkrt::device_buffer memory;
     part nodes4, tris, indices, order, wide_range;
     uint32_t node_cap = 0;// 4-wide nodes there is room for
-    // the binary tree with its children and runs, kept only where traversal walks it: no 4-wide collapse, or not joint
+    // the binary tree with its children and runs, kept only where traversal walks it: no 4-wide collapse
     vkrt::device_buffer binary;
     part nodes, child, range;
     bool joint = true;
@@ -60,8 +72,9 @@ struct vkrt_bvh
     uint32_t n_nodes4 = 0, stack4 = 0;
     bool wide = false, allow_wide = true;
     vkrt_bvh_info info{};
-};
 
+    vkrt::walk_layout walk() const { return !wide ? vkrt::WALK_BINARY : joint ? vkrt::WALK_JOINT : vkrt::WALK_APART; }
+};
 
 namespace vkrt
 {

@@ -434,7 +434,7 @@ __global__ void __launch_bounds__(PT_BLOCK) k_pt_zero(uint32_t *c, uint32_t n)
 template<int BLOCK = PT_BLOCK, class F = alpha_filter, bool INST = false>
 __device__ __forceinline__ void trace_path(const vkrt_bvh_node *__restrict__ nodes, const float4 *__restrict__ tris,
                                            int32_t root, bool empty, const vkrt_bvh4_node *__restrict__ nodes4,
-                                           int32_t root4, bool wide, const pt_buffers &b, uint32_t p, int32_t *smem,
+                                           int32_t root4, uint32_t walk, const pt_buffers &b, uint32_t p, int32_t *smem,
                                            F flt, uint32_t depth, const pt_tlas &tl = pt_tlas{})
 {
     float t = 0.f, u = 0.f, v = 0.f;
@@ -460,8 +460,10 @@ __device__ __forceinline__ void trace_path(const vkrt_bvh_node *__restrict__ nod
         const bool in_air = (st.y & F_MEDIA_MASK) == 0u;
         if constexpr(F::active) flt.xi = rnd_peek(xxhash32(st.x, depth));
         // the shade kernel recovers HitKind (back face: negative determinant) from the vertices
-        if(wide)
+        if(walk == WALK_JOINT)
             traverse4<false, BLOCK, PT_LDS>(nodes4, tris, root4, r, smem, t, u, v, prim, in_air, flt);
+        else if(walk == WALK_APART)
+            traverse4<false, BLOCK, PT_LDS, F, false>(nodes4, tris, root4, r, smem, t, u, v, prim, in_air, flt);
         else
             traverse<false, BLOCK, PT_LDS>(nodes, tris, root, r, smem, t, u, v, prim, in_air, flt);
     }
@@ -474,7 +476,7 @@ template<class F, bool INST>
 __global__ void __launch_bounds__(PT_TRACE_BLOCK) __attribute__((amdgpu_waves_per_eu(
         INST ? PT_TRACE_INST_WAVES_PER_SIMD : (F::active ? PT_TRACE_WAVES_PER_SIMD : PT_TRACE_PLAIN_WAVES_PER_SIMD))))
 k_pt_trace(const vkrt_bvh_node *__restrict__ nodes, const float4 *__restrict__ tris, int32_t root, bool empty,
-           const vkrt_bvh4_node *__restrict__ nodes4, int32_t root4, bool wide, pt_buffers b, int in, F flt,
+           const vkrt_bvh4_node *__restrict__ nodes4, int32_t root4, uint32_t walk, pt_buffers b, int in, F flt,
            uint32_t depth, pt_tlas tl)
 {
     __shared__ int32_t smem[PT_LDS * PT_TRACE_BLOCK];
@@ -505,7 +507,7 @@ k_pt_trace(const vkrt_bvh_node *__restrict__ nodes, const float4 *__restrict__ t
         if(t >= tiles) break;
         const uint32_t q = t * PT_TRACE_BLOCK + threadIdx.x;
         if(q < count)
-            trace_path<PT_TRACE_BLOCK, F, INST>(nodes, tris, root, empty, nodes4, root4, wide, b, b.queue[in][q],
+            trace_path<PT_TRACE_BLOCK, F, INST>(nodes, tris, root, empty, nodes4, root4, walk, b, b.queue[in][q],
                                                 smem + threadIdx.x, flt, depth, tl);
     }
 }
@@ -1122,7 +1124,7 @@ constexpr int TR_STACK = 64;
 //! else the product of transmission * color over the transmissive hits in ascending (t, triangle) order
 template<class F = alpha_filter>
 __device__ float4 transmittance_walk(const vkrt_bvh_node *__restrict__ nodes2, int32_t root2,
-                                     const vkrt_bvh4_node *__restrict__ nodes4, int32_t root4, bool wide, bool empty,
+                                     const vkrt_bvh4_node *__restrict__ nodes4, int32_t root4, uint32_t walk, bool empty,
                                      const float4 *__restrict__ tris, const gpu_material *__restrict__ mats,
                                      const ray_setup &r, bool cull, int32_t *lds, const F &flt)
 {
@@ -1152,14 +1154,14 @@ __device__ float4 transmittance_walk(const vkrt_bvh_node *__restrict__ nodes2, i
         float bound = r.tmax;
         const float lo = first_pass ? r.tmin : fmaxf(r.tmin, lb_t);
         int sp = 0;
-        int32_t ref = wide ? root4 : root2;
+        int32_t ref = walk != WALK_BINARY ? root4 : root2;
         while(true)
         {
             if(ref >= 0)
             {
                 int32_t c[4];
                 int nc;
-                if(wide) nc = visit4(nodes4, ref, r, bound, c, lo);
+                if(walk != WALK_BINARY) nc = visit4(nodes4, ref, r, bound, c, lo);
                 else
                 {
                     const vkrt_bvh_node nd = nodes2[ref];
@@ -1435,7 +1437,7 @@ __device__ float4 transmittance_walk_scene(const pt_tlas &tl, const gpu_material
 template<bool INST>
 __global__ void __launch_bounds__(PT_BLOCK) k_pt_transmittance(const vkrt_bvh_node *__restrict__ nodes2,
                                                                int32_t root2, const vkrt_bvh4_node *__restrict__ nodes4,
-                                                               int32_t root4, bool wide, bool empty,
+                                                               int32_t root4, uint32_t walk, bool empty,
                                                                const float4 *__restrict__ tris,
                                                                const gpu_material *__restrict__ mats,
                                                                const float4 *__restrict__ rays, uint32_t n, bool cull,
@@ -1448,14 +1450,14 @@ __global__ void __launch_bounds__(PT_BLOCK) k_pt_transmittance(const vkrt_bvh_no
         out[i] = transmittance_walk_scene(tl, mats, rays[2 * (size_t)i], rays[2 * (size_t)i + 1], cull,
                                           smem + threadIdx.x, flt);
     else
-        out[i] = transmittance_walk(nodes2, root2, nodes4, root4, wide, empty, tris, mats, setup_ray(rays, i), cull,
+        out[i] = transmittance_walk(nodes2, root2, nodes4, root4, walk, empty, tris, mats, setup_ray(rays, i), cull,
                                     smem + threadIdx.x, flt);
 }
 
 //! trace one shadow record and add its next-event estimate to the pixel (and to its training vertex)
 template<class F = alpha_filter, bool INST = false>
 __device__ __forceinline__ void shadow_path(const vkrt_bvh_node *__restrict__ nodes2, int32_t root2,
-                                            const vkrt_bvh4_node *__restrict__ nodes4, int32_t root4, bool wide,
+                                            const vkrt_bvh4_node *__restrict__ nodes4, int32_t root4, uint32_t walk,
                                             bool empty, const float4 *__restrict__ tris,
                                             const gpu_material *__restrict__ mats, const pt_frame &f,
                                             const pt_buffers &b, const float4 (&rec)[SHADOW_F4], int32_t *smem,
@@ -1469,7 +1471,7 @@ __device__ __forceinline__ void shadow_path(const vkrt_bvh_node *__restrict__ no
     }
     float4 T;
     if constexpr(INST) T = transmittance_walk_scene(tl, mats, o, d, false, smem, flt);
-    else T = transmittance_walk(nodes2, root2, nodes4, root4, wide, empty, tris, mats, make_ray_setup(o, d), false, smem,
+    else T = transmittance_walk(nodes2, root2, nodes4, root4, walk, empty, tris, mats, make_ray_setup(o, d), false, smem,
                                 flt);
     if(!(T.x > 0.0f || T.y > 0.0f || T.z > 0.0f)) return;
     const float4 lr = rec[2], fc = rec[3], bp = rec[4], id = rec[5];
@@ -1498,7 +1500,7 @@ template<class F, bool INST>
 __global__ void __launch_bounds__(PT_BLOCK)
 __attribute__((amdgpu_waves_per_eu(INST || F::active ? 1 : PT_SHADOW_PLAIN_WAVES_PER_SIMD))) k_pt_shadow(const vkrt_bvh_node *__restrict__ nodes2, int32_t root2,
                                                         const vkrt_bvh4_node *__restrict__ nodes4, int32_t root4,
-                                                        bool wide, bool empty, const float4 *__restrict__ tris,
+                                                        uint32_t walk, bool empty, const float4 *__restrict__ tris,
                                                         const gpu_material *__restrict__ mats, pt_frame f,
                                                         pt_buffers b, F flt, pt_tlas tl)
 {
@@ -1509,7 +1511,7 @@ __attribute__((amdgpu_waves_per_eu(INST || F::active ? 1 : PT_SHADOW_PLAIN_WAVES
         const float4 *rec = b.shadow + (size_t)i * SHADOW_F4;
         float4 r[SHADOW_F4];
         for(uint32_t k = 0; k < SHADOW_F4; ++k) r[k] = rec[k];
-        shadow_path<F, INST>(nodes2, root2, nodes4, root4, wide, empty, tris, mats, f, b, r, smem + threadIdx.x, flt,
+        shadow_path<F, INST>(nodes2, root2, nodes4, root4, walk, empty, tris, mats, f, b, r, smem + threadIdx.x, flt,
                              tl);
     }
 }
@@ -1522,7 +1524,7 @@ template<bool LIGHTS, bool INST>
 __global__ void __launch_bounds__(PT_BLOCK) k_pt_train_paths(const vkrt_bvh_node *__restrict__ nodes2,
                                                              const float4 *__restrict__ tris, int32_t root2,
                                                              bool empty, const vkrt_bvh4_node *__restrict__ nodes4,
-                                                             int32_t root4, bool wide, pt_frame f, pt_buffers b,
+                                                             int32_t root4, uint32_t walk, pt_frame f, pt_buffers b,
                                                              pt_scene_dev s, pt_tlas tl)
 {
     __shared__ int32_t smem[PT_LDS * PT_BLOCK];
@@ -1534,7 +1536,7 @@ __global__ void __launch_bounds__(PT_BLOCK) k_pt_train_paths(const vkrt_bvh_node
     uint32_t segments = 0;
     for(uint32_t depth = 0; depth < f.max_depth; ++depth)
     {
-        trace_path<PT_BLOCK, alpha_filter, INST>(nodes2, tris, root2, empty, nodes4, root4, wide, b, p,
+        trace_path<PT_BLOCK, alpha_filter, INST>(nodes2, tris, root2, empty, nodes4, root4, walk, b, p,
                                                  smem + threadIdx.x, flt, depth, tl);
         bool alive = false, to_cache = false, need_shadow = false;
         float4 shadow_rec[SHADOW_F4];
@@ -1542,7 +1544,7 @@ __global__ void __launch_bounds__(PT_BLOCK) k_pt_train_paths(const vkrt_bvh_node
         shade_path<LIGHTS, INST>(f, b, s, depth, p, alive, to_cache, need_shadow, shadow_rec, qfeat);
         ++segments;
         if(LIGHTS && need_shadow)
-            shadow_path<alpha_filter, INST>(nodes2, root2, nodes4, root4, wide, empty, tris, s.mats, f, b, shadow_rec,
+            shadow_path<alpha_filter, INST>(nodes2, root2, nodes4, root4, walk, empty, tris, s.mats, f, b, shadow_rec,
                                             smem + threadIdx.x, shadow_flt, tl);
         if(!alive) break;
     }
@@ -1554,21 +1556,21 @@ __global__ void __launch_bounds__(PT_BLOCK) k_pt_train_paths(const vkrt_bvh_node
 template<bool LIGHTS, class F, bool INST>
 __device__ __forceinline__ uint32_t finish_path(const vkrt_bvh_node *__restrict__ nodes2, const float4 *__restrict__ tris,
                                                 int32_t root2, bool empty, const vkrt_bvh4_node *__restrict__ nodes4,
-                                                int32_t root4, bool wide, const pt_frame &f, const pt_buffers &b,
+                                                int32_t root4, uint32_t walk, const pt_frame &f, const pt_buffers &b,
                                                 const pt_scene_dev &s, const F &flt, const F &shadow_flt, uint32_t d0,
                                                 uint32_t p, int32_t *smem, const pt_tlas &tl)
 {
     uint32_t segments = 0;
     for(uint32_t depth = d0; depth < f.max_depth; ++depth)
     {
-        trace_path<PT_BLOCK, F, INST>(nodes2, tris, root2, empty, nodes4, root4, wide, b, p, smem, flt, depth, tl);
+        trace_path<PT_BLOCK, F, INST>(nodes2, tris, root2, empty, nodes4, root4, walk, b, p, smem, flt, depth, tl);
         bool alive = false, to_cache = false, need_shadow = false;
         float4 shadow_rec[SHADOW_F4];
         float4 qfeat[QUERY_F4];
         shade_path<LIGHTS, INST>(f, b, s, depth, p, alive, to_cache, need_shadow, shadow_rec, qfeat);
         ++segments;
         if(LIGHTS && need_shadow)
-            shadow_path<F, INST>(nodes2, root2, nodes4, root4, wide, empty, tris, s.mats, f, b, shadow_rec, smem,
+            shadow_path<F, INST>(nodes2, root2, nodes4, root4, walk, empty, tris, s.mats, f, b, shadow_rec, smem,
                                  shadow_flt, tl);
         if(!alive) break;
     }
@@ -1586,7 +1588,7 @@ template<bool LIGHTS, class F, bool INST, bool SAMPLES>
 __global__ void __launch_bounds__(PT_BLOCK) k_pt_finish(const vkrt_bvh_node *__restrict__ nodes2,
                                                         const float4 *__restrict__ tris, int32_t root2, bool empty,
                                                         const vkrt_bvh4_node *__restrict__ nodes4, int32_t root4,
-                                                        bool wide, pt_frame f, pt_buffers b, pt_scene_dev s, F flt,
+                                                        uint32_t walk, pt_frame f, pt_buffers b, pt_scene_dev s, F flt,
                                                         F shadow_flt, uint32_t d0, int in, uint32_t n, pt_tlas tl)
 {
     __shared__ int32_t smem[PT_LDS * PT_BLOCK];
@@ -1603,11 +1605,11 @@ __global__ void __launch_bounds__(PT_BLOCK) k_pt_finish(const vkrt_bvh_node *__r
             for(uint32_t sample = 0; sample < f.num_samples; ++sample)
             {
                 begin_path(f, b, sample, p, 0u);
-                segments += finish_path<LIGHTS, F, INST>(nodes2, tris, root2, empty, nodes4, root4, wide, f, b, s, flt,
+                segments += finish_path<LIGHTS, F, INST>(nodes2, tris, root2, empty, nodes4, root4, walk, f, b, s, flt,
                                                          shadow_flt, 0u, p, smem + threadIdx.x, tl);
             }
         else
-            segments = finish_path<LIGHTS, F, INST>(nodes2, tris, root2, empty, nodes4, root4, wide, f, b, s, flt,
+            segments = finish_path<LIGHTS, F, INST>(nodes2, tris, root2, empty, nodes4, root4, walk, f, b, s, flt,
                                                     shadow_flt, d0, p, smem + threadIdx.x, tl);
     }
     if(segments) atomicAdd(&s_segments, (unsigned long long)segments);
@@ -2017,7 +2019,8 @@ static void trace_batch(vkrt_pt *pt, const vkrt_camera &cam, uint32_t seed)
     const vkrt_bvh4_node *nodes4 = bvh ? bvh->nodes4.as<vkrt_bvh4_node>() : nullptr;
     const float4 *tris = bvh ? bvh->tris.as<float4>() : nullptr;
     const int32_t root_ref = bvh ? bvh->root_ref : 0, root4 = bvh ? bvh->root4 : 0;
-    const bool flat_empty = bvh ? bvh->empty : true, wide = bvh && bvh->wide && bvh->joint;
+    const bool flat_empty = bvh ? bvh->empty : true;
+    const uint32_t walk = bvh ? bvh->walk() : WALK_BINARY;
     // one depth of a queue of paths: trace, shade, and the shadow rays of next-event estimation
     // scenes with no alpha-tested material take the trace and shadow kernels without the any-hit filter
     const bool alpha = pt->any_alpha;
@@ -2082,13 +2085,13 @@ static void trace_batch(vkrt_pt *pt, const vkrt_camera &cam, uint32_t seed)
             using F = std::conditional_t<decltype(a)::value, alpha_filter, keep_all>;
             constexpr bool I = decltype(in_)::value;
             k_pt_trace<F, I><<<g.trace_grid, PT_TRACE_BLOCK, 0, st>>>(nodes2, tris, root_ref, flat_empty, nodes4,
-                                                                      root4, wide, bb, in, filter_of<F>(flt),
+                                                                      root4, walk, bb, in, filter_of<F>(flt),
                                                                       depth, tl);
             if(f.n_lights)
             {
                 k_pt_shade<true, I><<<g.blocks, PT_BLOCK, 0, st>>>(f, bb, sc, depth, in);
                 k_pt_shadow<F, I><<<g.shadow_grid, PT_BLOCK, 0, st>>>(nodes2, root_ref, nodes4, root4,
-                                                                      wide, flat_empty, tris, sc.mats, f, bb,
+                                                                      walk, flat_empty, tris, sc.mats, f, bb,
                                                                       filter_of<F>(shadow_flt), tl);
             }
             else
@@ -2103,7 +2106,7 @@ static void trace_batch(vkrt_pt *pt, const vkrt_camera &cam, uint32_t seed)
             constexpr bool I = decltype(in_)::value;
             auto launch = [&](auto lights, auto samples) {
                 k_pt_finish<decltype(lights)::value, F, I, decltype(samples)::value>
-                        <<<g.blocks, PT_BLOCK, 0, g.stream>>>(nodes2, tris, root_ref, flat_empty, nodes4, root4, wide, f,
+                        <<<g.blocks, PT_BLOCK, 0, g.stream>>>(nodes2, tris, root_ref, flat_empty, nodes4, root4, walk, f,
                                                               g.b, sc, filter_of<F>(flt), filter_of<F>(shadow_flt),
                                                               depth ? depth : g.first, in, g.n, tl);
             };
@@ -2161,7 +2164,7 @@ static void trace_batch(vkrt_pt *pt, const vkrt_camera &cam, uint32_t seed)
             auto train = [&](auto lights, auto in_) {
                 k_pt_train_paths<decltype(lights)::value, decltype(in_)::value>
                         <<<tgrid, PT_BLOCK, 0, side>>>(nodes2, tris, root_ref, flat_empty, nodes4,
-                                                                   root4, wide, f, bt, sc, tl);
+                                                                   root4, walk, f, bt, sc, tl);
             };
             if(f.n_lights && inst) train(std::true_type{}, std::true_type{});
             else if(f.n_lights) train(std::true_type{}, std::false_type{});
@@ -2657,7 +2660,7 @@ int vkrt_pt_trace_transmittance(vkrt_pt *pt, const vkrt_ray *rays, uint32_t n, f
         {
             const vkrt_bvh *b = pt->bvh;
             k_pt_transmittance<false><<<div_up(n, PT_BLOCK), PT_BLOCK, 0, ctx->stream>>>(
-                    b->nodes.as<vkrt_bvh_node>(), b->root_ref, b->nodes4.as<vkrt_bvh4_node>(), b->root4, b->wide && b->joint,
+                    b->nodes.as<vkrt_bvh_node>(), b->root_ref, b->nodes4.as<vkrt_bvh4_node>(), b->root4, b->walk(),
                     b->empty, b->tris.as<float4>(), pt->mats.as<gpu_material>(), r4, n, cull, dout, flt, pt->tlas);
         }
         VKRT_HIP(hipGetLastError());

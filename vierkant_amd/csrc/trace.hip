@@ -16,7 +16,16 @@
 namespace vkrt
 {
 
-template<bool ANY, int BLOCK, int LDS_DEPTH, bool POSTPONE>
+//! the loops of the walk: the 4-wide walk step by step with nodes and records joint or apart, or with leaves postponed
+//! (a binary tree has one loop, whichever is asked for)
+enum trace_loop
+{
+    LOOP_JOINT,
+    LOOP_APART,
+    LOOP_POSTPONED
+};
+
+template<bool ANY, int BLOCK, int LDS_DEPTH, trace_loop LOOP>
 __global__ void __launch_bounds__(BLOCK) k_trace(const vkrt_bvh_node *__restrict__ nodes,
                                                  const float4 *__restrict__ tris, int32_t root, bool empty,
                                                  const vkrt_bvh4_node *__restrict__ nodes4, int32_t root4, bool wide,
@@ -33,10 +42,11 @@ __global__ void __launch_bounds__(BLOCK) k_trace(const vkrt_bvh_node *__restrict
     {
         ray_setup r = setup_ray(rays, i);
         if(!wide) hit = traverse<ANY, BLOCK, LDS_DEPTH>(nodes, tris, root, r, smem + threadIdx.x, t, u, v, prim);
-        else if(POSTPONE)
+        else if(LOOP == LOOP_POSTPONED)
             hit = traverse4_postponed<ANY, BLOCK, LDS_DEPTH>(nodes4, tris, root4, r, smem + threadIdx.x, t, u, v, prim);
         else
-            hit = traverse4<ANY, BLOCK, LDS_DEPTH>(nodes4, tris, root4, r, smem + threadIdx.x, t, u, v, prim);
+            hit = traverse4<ANY, BLOCK, LDS_DEPTH, keep_all, LOOP == LOOP_JOINT>(nodes4, tris, root4, r,
+                                                                                 smem + threadIdx.x, t, u, v, prim);
     }
     if(ANY) static_cast<uint8_t *>(out)[i] = hit ? 1 : 0;
     else
@@ -44,32 +54,36 @@ __global__ void __launch_bounds__(BLOCK) k_trace(const vkrt_bvh_node *__restrict
                                               : vkrt_hit{__int_as_float(0x7f800000), 0.f, 0.f, VKRT_INVALID_PRIM};
 }
 
-template<bool ANY, int BLOCK, int LDS, bool POSTPONE>
-static void launch_one(hipStream_t s, const vkrt_bvh *bvh, const float4 *rays, uint32_t n, void *out, uint32_t chunk)
+template<bool ANY, int BLOCK, int LDS>
+static void launch_one(hipStream_t s, trace_loop loop, const vkrt_bvh *bvh, const float4 *rays, uint32_t n, void *out,
+                       uint32_t chunk)
 {
-    k_trace<ANY, BLOCK, LDS, POSTPONE><<<xcd_grid(div_up(n, BLOCK), chunk), BLOCK, 0, s>>>(
-            bvh->nodes.as<vkrt_bvh_node>(), bvh->tris.as<float4>(), bvh->root_ref, bvh->empty,
-            bvh->nodes4.as<vkrt_bvh4_node>(), bvh->root4, bvh->wide, rays, n, out, chunk);
+    auto launch = [&](auto kernel) {
+        kernel<<<xcd_grid(div_up(n, BLOCK), chunk), BLOCK, 0, s>>>(
+                bvh->nodes.as<vkrt_bvh_node>(), bvh->tris.as<float4>(), bvh->root_ref, bvh->empty,
+                bvh->nodes4.as<vkrt_bvh4_node>(), bvh->root4, bvh->wide, rays, n, out, chunk);
+    };
+    if(loop == LOOP_JOINT) launch(k_trace<ANY, BLOCK, LDS, LOOP_JOINT>);
+    else if(loop == LOOP_APART) launch(k_trace<ANY, BLOCK, LDS, LOOP_APART>);
+    else launch(k_trace<ANY, BLOCK, LDS, LOOP_POSTPONED>);
 }
 
 template<bool ANY, int BLOCK>
 static void launch_block(vkrt_ctx *ctx, const vkrt_trace_config &cfg, const vkrt_bvh *bvh, const float4 *rays,
                          uint32_t n, void *out)
 {
-    // (the step loop reaches nodes and records from one base with 32-bit offsets; the other loop has one for each)
-    const bool p = cfg.traversal == VKRT_TRAVERSAL_POSTPONED || !bvh->joint;
+    // nodes and records apart, 50M triangles: 4-wide step by step 1.41 ms for 2M camera rays, postponed 1.56
+    const trace_loop loop = cfg.traversal == VKRT_TRAVERSAL_POSTPONED ? LOOP_POSTPONED
+                            : bvh->walk() == WALK_APART               ? LOOP_APART
+                                                                      : LOOP_JOINT;
     const uint32_t x = cfg.xcd_chunk;
     hipStream_t s = ctx->stream;
     switch(cfg.lds_stack_depth)
     {
-        case 0: p ? launch_one<ANY, BLOCK, 0, true>(s, bvh, rays, n, out, x)
-                  : launch_one<ANY, BLOCK, 0, false>(s, bvh, rays, n, out, x); break;
-        case 8: p ? launch_one<ANY, BLOCK, 8, true>(s, bvh, rays, n, out, x)
-                  : launch_one<ANY, BLOCK, 8, false>(s, bvh, rays, n, out, x); break;
-        case 16: p ? launch_one<ANY, BLOCK, 16, true>(s, bvh, rays, n, out, x)
-                   : launch_one<ANY, BLOCK, 16, false>(s, bvh, rays, n, out, x); break;
-        case 32: p ? launch_one<ANY, BLOCK, 32, true>(s, bvh, rays, n, out, x)
-                   : launch_one<ANY, BLOCK, 32, false>(s, bvh, rays, n, out, x); break;
+        case 0: launch_one<ANY, BLOCK, 0>(s, loop, bvh, rays, n, out, x); break;
+        case 8: launch_one<ANY, BLOCK, 8>(s, loop, bvh, rays, n, out, x); break;
+        case 16: launch_one<ANY, BLOCK, 16>(s, loop, bvh, rays, n, out, x); break;
+        case 32: launch_one<ANY, BLOCK, 32>(s, loop, bvh, rays, n, out, x); break;
         default: throw error(VKRT_E_INVALID_ARG, "lds_stack_depth must be 0, 8, 16 or 32");
     }
 }

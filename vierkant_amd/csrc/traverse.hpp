@@ -168,16 +168,23 @@ __device__ __forceinline__ void child_intervals(const fetch7 &f, const ray_setup
     }
 }
 
-__device__ __forceinline__ void node4_intervals(const vkrt_bvh4_node *__restrict__ nodes, int32_t ref,
-                                                const ray_setup &r, float tn[4], float tf[4], int4 &child)
+//! the seven words of node `ref` alone
+__device__ __forceinline__ fetch7 fetch_node(const void *__restrict__ nodes, int32_t ref, const ray_setup &r)
 {
     const uint32_t nb = static_cast<uint32_t>(ref) * static_cast<uint32_t>(sizeof(vkrt_bvh4_node));
     const uint32_t ax = nb + r.nx, ay = nb + r.ny, az = nb + r.nz;
     const float4 nx = load_global_f4(nodes, ax), fx = load_global_f4(nodes, ax ^ 16u);
     const float4 ny = load_global_f4(nodes, ay), fy = load_global_f4(nodes, ay ^ 16u);
     const float4 nz = load_global_f4(nodes, az), fz = load_global_f4(nodes, az ^ 16u);
-    child = load_global_i4(nodes, nb + 96u);
-    child_intervals(fetch7{nx, fx, ny, fy, nz, fz, child}, r, tn, tf);
+    return fetch7{nx, fx, ny, fy, nz, fz, load_global_i4(nodes, nb + 96u)};
+}
+
+__device__ __forceinline__ void node4_intervals(const vkrt_bvh4_node *__restrict__ nodes, int32_t ref,
+                                                const ray_setup &r, float tn[4], float tf[4], int4 &child)
+{
+    const fetch7 f = fetch_node(nodes, ref, r);
+    child = f.c;
+    child_intervals(f, r, tn, tf);
 }
 
 //! the candidate filter of a traversal: a candidate that would become the closest hit and whose record is
@@ -367,18 +374,25 @@ __device__ __forceinline__ void trav_init(trav_state &s, const ray_setup &r, int
 
 //! one step of the 4-wide walk: a node (children whose padded interval meets [tmin, best_t] are entered
 //! nearest first, the others pushed farthest first) or a leaf, then a pop. Returns true when the ray is
-//! finished (stack empty, or the first hit when ANY). `base` holds the nodes and, from tri_offset on, the leaf
-//! records. `lds` is this lane's column of a [LDS_DEPTH][BLOCK] array; `spill` holds entries past LDS_DEPTH. A
+//! finished (stack empty, or the first hit when ANY). JOINT: the records lie within 4 GiB behind the nodes, and one
+//! fetch serves both; otherwise a node and a leaf are read by loads of their own. `lds` is this lane's column of a [LDS_DEPTH][BLOCK] array; `spill` holds entries past LDS_DEPTH. A
 //! child is entered under the same condition as in traverse(), and the closest-hit rule does not depend on the
 //! visiting order, so the result is the same.
-template<bool ANY, int BLOCK, int LDS_DEPTH, class F = keep_all>
-__device__ __forceinline__ bool step4(const void *base, uint32_t tri_offset, trav_state &s, int32_t *lds, int32_t *spill,
-                                      bool cull_back, const F &filter = F{})
+template<bool ANY, int BLOCK, int LDS_DEPTH, class F = keep_all, bool JOINT = true>
+__device__ __forceinline__ bool step4(const vkrt_bvh4_node *nodes, const float4 *tris, trav_state &s, int32_t *lds,
+                                      int32_t *spill, bool cull_back, const F &filter = F{})
 {
     const ray_setup &r = s.r;
     const bool node = s.ref >= 0;
-    const uint32_t at = walk_offset(s.ref, tri_offset);
-    const fetch7 f = fetch_step(base, at, node, r);
+    uint32_t at = 0;
+    fetch7 f;
+    if constexpr(JOINT)
+    {
+        at = walk_offset(s.ref, static_cast<uint32_t>(reinterpret_cast<uintptr_t>(tris) -
+                                                      reinterpret_cast<uintptr_t>(nodes)));
+        f = fetch_step(nodes, at, node, r);
+    }
+    else if(node) f = fetch_node(nodes, s.ref, r);
     if(node)
     {
         float tn[4], tf[4];
@@ -412,6 +426,14 @@ __device__ __forceinline__ bool step4(const void *base, uint32_t tri_offset, tra
             return false;
         }
     }
+    else if constexpr(!JOINT)
+    {
+        uint32_t first, count;
+        leaf_decode(s.ref, first, count);
+        if(test_leaf<ANY, F>(tris, (size_t)TRI_BYTES * first, 0, count, r, s.best_t, s.best_u, s.best_v, s.best_prim,
+                             cull_back, filter))
+            return true;
+    }
     else
     {
         const uint32_t count = (static_cast<uint32_t>(~s.ref) & 7u) + 1u;
@@ -423,7 +445,7 @@ __device__ __forceinline__ bool step4(const void *base, uint32_t tri_offset, tra
                                          __int_as_float(f.c.w));
             if(test_record<ANY, F>(f.z0, f.z1, c, r, s.best_t, s.best_u, s.best_v, s.best_prim, cull_back, filter))
                 return true;
-            if(test_leaf<ANY, F>(base, at, 2, count, r, s.best_t, s.best_u, s.best_v, s.best_prim, cull_back, filter))
+            if(test_leaf<ANY, F>(nodes, at, 2, count, r, s.best_t, s.best_u, s.best_v, s.best_prim, cull_back, filter))
                 return true;
         }
     }
@@ -484,19 +506,17 @@ struct lane_stack
 
 constexpr int spill_entries(int lds_depth) { return STACK_SIZE - lds_depth > 0 ? STACK_SIZE - lds_depth : 1; }
 
-//! the whole 4-wide walk for one ray (see step4) through a BVH whose nodes and records are joint
-template<bool ANY, int BLOCK, int LDS_DEPTH, class F = keep_all>
-__device__ __forceinline__ bool traverse4(const vkrt_bvh4_node *nodes, const float4 *tris, int32_t root, const ray_setup &r, int32_t *lds, float &best_t,
-                                          float &best_u, float &best_v, uint32_t &best_prim, bool cull_back = false,
+//! the whole 4-wide walk for one ray (see step4); JOINT as vkrt_bvh::walk says
+template<bool ANY, int BLOCK, int LDS_DEPTH, class F = keep_all, bool JOINT = true>
+__device__ __forceinline__ bool traverse4(const vkrt_bvh4_node *nodes, const float4 *tris, int32_t root,
+                                          const ray_setup &r, int32_t *lds, float &best_t, float &best_u,
+                                          float &best_v, uint32_t &best_prim, bool cull_back = false,
                                           const F &filter = F{})
 {
     int32_t spill[spill_entries(LDS_DEPTH)];
     trav_state s;
     trav_init(s, r, root);
-    // (nodes and records are one allocation, vkrt_bvh::walk)
-    const uint32_t tri_offset =
-            static_cast<uint32_t>(reinterpret_cast<uintptr_t>(tris) - reinterpret_cast<uintptr_t>(nodes));
-    while(!step4<ANY, BLOCK, LDS_DEPTH, F>(nodes, tri_offset, s, lds, spill, cull_back, filter)) {}
+    while(!step4<ANY, BLOCK, LDS_DEPTH, F, JOINT>(nodes, tris, s, lds, spill, cull_back, filter)) {}
     best_t = s.best_t;
     best_u = s.best_u;
     best_v = s.best_v;
