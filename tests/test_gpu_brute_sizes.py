@@ -1,8 +1,11 @@
 """Brute force at the sizes where its tiles (32 triangles, 32 rays a lane pair), stages of 256 triangles, workgroups
 of 128 and 512 rays and triangle chunks end, and on inputs whose magnitudes its filter cannot bound: every record and
 flag is the oracle's, bit for bit."""
+import time
+
 import numpy as np
 import pytest
+import torch
 
 import oracle_binding as orc
 from parity import assert_hits_equal
@@ -90,3 +93,43 @@ def test_brute_with_large_small_and_non_finite(ctx):
         rays[f][rng.integers(0, 600, 8)] = bad
     want = check(ctx, tris, rays, "mixed")
     assert (want["prim"] != 0xFFFFFFFF).sum() > 100
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf, -np.inf, 1e30])
+@pytest.mark.parametrize("where", ["first", "middle", "last", "ends", "tile", "all"])
+def test_brute_stray_triangles(ctx, bad, where):
+    """non-finite and far-off vertices where a chunk takes its origin from, in a whole tile, and everywhere; and rays with
+    such parts, tmin below zero among them (an infinite direction then gives t = +-0)"""
+    rng = np.random.default_rng(31)
+    tris, rays = soup(rng, 512 + 40, 300)
+    at = {"first": [0, 256, 512], "middle": [128, 276, 384], "last": [255, 511, 551], "ends": [0, 276, 551],
+          "tile": slice(64, 96), "all": slice(None)}[where]
+    tris[at, rng.integers(0, 9)] = bad
+    rays["tmin"][::3] = -1.0
+    for k, f in enumerate(("ox", "oy", "oz", "dx", "dy", "dz")):
+        rays[f][10 + k::40] = bad
+    check(ctx, tris, rays, f"{bad} {where}")
+
+
+def test_brute_non_finite_parts_cost_no_more(ctx):
+    """65,536 rays and the 20,480-triangle icosphere with every 256th triangle and every 32nd ray NaN take about as long
+    as without (a chunk, or a wave, that gives its filter up for them takes four times as long and more)"""
+    pos, idx, rays = W.icosphere_rays(65536)
+    tris = W.flat_triangles(pos, idx).astype(np.float32)
+    times = []
+    for bad in (False, True):
+        if bad:
+            tris, rays = tris.copy(), rays.copy()
+            tris[::256, 0] = np.nan
+            rays["ox"][::32] = np.nan
+        t = torch.from_numpy(tris).cuda()
+        r = torch.from_numpy(rays.view(np.float32).reshape(-1, 8).copy()).cuda()
+        out = torch.zeros((65536, 4), dtype=torch.int32, device="cuda")
+        torch.cuda.synchronize()
+        best = float("inf")
+        for _ in range(12):
+            t0 = time.perf_counter()
+            ctx.brute_closest(t, r, out=out)
+            best = min(best, time.perf_counter() - t0)
+        times.append(best)
+    assert times[1] < 2.5 * times[0], times

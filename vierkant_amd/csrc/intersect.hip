@@ -141,8 +141,6 @@ __global__ void k_fill_u8(uint8_t *__restrict__ p, uint32_t n, uint8_t value)
     if(i < n) p[i] = value;
 }
 
-//! (v0, v1, v2) -> (v0, e1 = v1 - v0, e2 = v2 - v0): the first line of the reference test
-
 // ---------------------------------------------------------------------------------------------
 // brute force
 // ---------------------------------------------------------------------------------------------
@@ -156,17 +154,18 @@ __global__ void k_fill_u8(uint8_t *__restrict__ p, uint32_t n, uint8_t value)
 // The factors go in as two bf16 parts each, hi + mid, off by 2^-16 of the factor; a lane's half holds the
 // triangle's hi or mid parts and the two MFMAs of a product take the ray's hi and its mid parts. With
 // P = |d| E (|f| + V) (E the longest edge and V the farthest vertex of 32 triangles, f the point of the ray's line
-// nearest to the origin, all about the chunk's first vertex; o x d = f x d, so rays from far away lose no more than near
+// nearest to the origin, all about a vertex of the chunk; o x d = f x d, so rays from far away lose no more than near
 // ones) the parts are off by at most 2^-15 P, the 24 terms' sum by less than 2^-19 P, and f itself and the reference's
 // own a, b and det by less than 2^-18 |d| E (|o| + V): a pair whose three values are not all above
 // -|d| E (2^-14 (|f| + V) + 2^-18 |o|) - 2^-70, nor all below its negative, is no hit of the reference's. 2^-70 covers
-// what is lost below the normal range while every factor stays below 2^40; a ray or a tile beyond that, or with a NaN or
-// an infinity, takes every pair: 1.3 times the time of a test for every pair where that is all tiles (one NaN in 32
-// triangles), 0.6 with one in 320. Constants that keep such a triangle alone out of the filter made every other case 5 %
-// slower.
+// what is lost below the normal range while every factor stays below 2^40; a ray or a tile beyond that takes every pair.
+// A triangle with a NaN or an infinity is never hit (det is not finite, so t comes out NaN or 0 x infinity): it takes the
+// place of another one of its tile in the filter and fails the reference's test where that one is asked for.
 //
-// 65,536 rays x 20,480 triangles: 1,210 us with the reference's test for every pair, 239 so (origins a thousand radii
-// away 369, without f 1,630), the matrix cores busy for 48 % of them and 69 VALU instructions a wave per 32 x 32 pairs,
+// 65,536 rays x 20,480 triangles: 1,210 us with the reference's test for every pair, 242 so (origins a thousand radii
+// away 375, without f 1,630; the scene at 1e13, where nothing has a bound, 1,196, and 1,590 where a record is read for
+// each ray of a lane; a NaN in every 256th triangle or every 32nd ray 270, and 1,540 where it takes its chunk's or its
+// wave's bound with it), the matrix cores busy for 48 % of them and 69 VALU instructions a wave per 32 x 32 pairs,
 // 48 of them the filter's. Two products of 32 x 32 in flight per wave, at two or three waves a SIMD, are no faster:
 // 248 - 255.
 constexpr float BRUTE_LIMIT = 0x1p40f;
@@ -191,6 +190,11 @@ __device__ __forceinline__ void split_bf16(const vec3 &p, const vec3 &q, bf16x8 
 //! no smaller than |v|, also where the squares underflow
 __device__ __forceinline__ float norm_above(const vec3 &v) { return sqrtf(dot(v, v)) + 0x1p-60f; }
 
+__device__ __forceinline__ bool finite3(const vec3 &v)
+{
+    return __builtin_isfinite(v.x) && __builtin_isfinite(v.y) && __builtin_isfinite(v.z);
+}
+
 __device__ __forceinline__ uint32_t half_wave_max(uint32_t x)
 {
 #pragma unroll
@@ -201,6 +205,9 @@ __device__ __forceinline__ uint32_t half_wave_max(uint32_t x)
 //! the smallest of three values, and of their negatives: neither reaches zero unless all lie on one side of it
 __device__ __forceinline__ float above(float a, float b, float c) { return fminf(fminf(a, b), c); }
 __device__ __forceinline__ float below(float a, float b, float c) { return fminf(fminf(-a, -b), -c); }
+
+//! the middle one of three values; of those that are numbers where one or two are NaN
+__device__ __forceinline__ float middle(float a, float b, float c) { return fmaxf(fminf(a, b), fminf(fmaxf(a, b), c)); }
 
 //! a wave takes 32 * GROUPS rays over its workgroup's triangles; lanes l and l + 32 hold one ray, and 16
 //! triangles each of every 32
@@ -215,11 +222,20 @@ __global__ void __launch_bounds__(256, GROUPS > 2 ? 3 : 4) k_brute(const float4 
 
     const uint32_t lane = threadIdx.x & 63u, half = lane >> 5;
     const uint32_t t0 = blockIdx.y * chunk, count = min(n_tri - t0, chunk);
-    const vec3 centre = ld3(tris + 9 * (size_t)t0);
+    // the origin for the chunk, a vertex that one stray or non-finite triangle does not carry off
+    const vec3 c0 = ld3(tris + 9 * (size_t)t0), c1 = ld3(tris + 9 * (size_t)(t0 + count / 2u)),
+               c2 = ld3(tris + 9 * (size_t)(t0 + count - 1u));
+    auto origin = [](float a, float b, float c) {
+        const float m = middle(a, b, c);
+        // (a scalar: the same in every lane, which the compiler does not see)
+        return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(fabsf(m) < BRUTE_LIMIT ? m : 0.f)));
+    };
+    const vec3 centre{origin(c0.x, c1.x, c2.x), origin(c0.y, c1.y, c2.y), origin(c0.z, c1.z, c2.z)};
 
     bf16x8 ray_hi[GROUPS], ray_mid[GROUPS];
     float ray_d[GROUPS], ray_o[GROUPS], best[GROUPS];
     uint32_t best_i[GROUPS];
+    bool unbounded = true;// each group has a ray that takes every pair
     const uint32_t first_ray = (blockIdx.x * 4u + (threadIdx.x >> 6)) * (32u * GROUPS) + (lane & 31u);
 #pragma unroll
     for(int g = 0; g < GROUPS; ++g)
@@ -234,13 +250,30 @@ __global__ void __launch_bounds__(256, GROUPS > 2 ? 3 : 4) k_brute(const float4 
         split_bf16(cross(foot, d), d, ray_hi[g], ray_mid[g]);
         ray_o[g] = norm_above(foot) + 0x1p-4f * norm_above(o);
         ray_d[g] = norm_above(d);
+        bool none = !(tmin < tmax);// no t lies inside
         if(!(ray_o[g] < BRUTE_LIMIT && ray_d[g] < BRUTE_LIMIT && ray_o[g] * ray_d[g] < BRUTE_LIMIT))
+        {
             ray_d[g] = __int_as_float(0x7fc00000);
-        if(!(tmin < tmax)) ray_d[g] = -__int_as_float(0x7f800000);// no t lies inside: no pair is taken
+            // a NaN or an infinite origin makes every t a NaN or infinite, an infinite direction makes it NaN or +-0
+            none |= !finite3(o) || d.x != d.x || d.y != d.y || d.z != d.z || (tmin >= 0.f && !finite3(d));
+        }
+        if(none) ray_d[g] = -__int_as_float(0x7f800000);// no pair is taken
         best[g] = tmax;
         best_i[g] = VKRT_INVALID_PRIM;
+        unbounded = unbounded && __any(ray_d[g] != ray_d[g]);
     }
 
+    auto test = [&](int g, const vec3 &o, const vec3 &d, float tmin, const float4 &q0, const float4 &q1,
+                    const float4 &q2, uint32_t prim) {
+        float t, u, v;
+        if(!mt_fast_window(o, d, vec3{q0.x, q0.y, q0.z}, vec3{q0.w, q1.x, q1.y}, vec3{q1.z, q1.w, q2.x}, tmin, best[g],
+                           t, u, v))
+            return;
+        // (ANY: the ray takes no pair any more)
+        if(ANY) ray_d[g] = -__int_as_float(0x7f800000);
+        else best[g] = t;
+        best_i[g] = prim;
+    };
     for(uint32_t done = 0; done < count; done += BRUTE_STAGE)
     {
         const uint32_t base = t0 + done, n = min(count - done, static_cast<uint32_t>(BRUTE_STAGE));
@@ -258,6 +291,32 @@ __global__ void __launch_bounds__(256, GROUPS > 2 ? 3 : 4) k_brute(const float4 
             records[threadIdx.x][1] = make_float4(e1.y, e1.z, e2.x, e2.y);
             records[threadIdx.x][2] = make_float4(e2.z, 0.f, 0.f, 0.f);
             v0 = v0 - centre;
+            float e, v;// E and V of this triangle, E NaN where it has no bound
+            auto measure = [&] {
+                const float l1 = norm_above(e1);
+                e = fmaxf(fmaxf(l1, norm_above(e2)), norm_above(e1 - e2));
+                v = norm_above(v0) + l1;
+                const bool bounded = e < BRUTE_LIMIT && v < BRUTE_LIMIT && e * v < BRUTE_LIMIT;
+                if(!bounded) e = __int_as_float(0x7fc00000);
+                return bounded;
+            };
+            if(__any(!measure()))
+            {
+                // (stand-ins for triangles that are never hit; a tile of nothing else lies below every bound)
+                const bool whole = threadIdx.x < n && finite3(v0) && finite3(e1) && finite3(e2);
+                const uint64_t wave_whole = __ballot(whole);
+                const uint32_t tile_whole = static_cast<uint32_t>(half ? wave_whole >> 32 : wave_whole);
+                const int from = static_cast<int>(32u * half) + max(__ffs(static_cast<int>(tile_whole)) - 1, 0);
+                float *part[9] = {&v0.x, &v0.y, &v0.z, &e1.x, &e1.y, &e1.z, &e2.x, &e2.y, &e2.z};
+#pragma unroll
+                for(int k = 0; k < 9; ++k)
+                {
+                    const float x = __shfl(*part[k], from);
+                    if(!whole) *part[k] = tile_whole ? x : 0.f;
+                }
+                measure();
+                if(!tile_whole) e = -__int_as_float(0x7f800000);
+            }
             const vec3 e3 = e1 - e2;
             const uint32_t tile = threadIdx.x >> 5, row = threadIdx.x & 31u;
             bf16x8 hi, mid;
@@ -270,11 +329,7 @@ __global__ void __launch_bounds__(256, GROUPS > 2 ? 3 : 4) k_brute(const float4 
             split_bf16(e3, cross(v0 + e1, e3), hi, mid);
             parts[tile][2][row] = hi;
             parts[tile][2][32 + row] = mid;
-            const float l1 = norm_above(e1);
-            float e = fmaxf(fmaxf(l1, norm_above(e2)), norm_above(e3));
-            float v = norm_above(v0) + l1;
-            // compared as integers a NaN is above every number
-            if(!(e < BRUTE_LIMIT && v < BRUTE_LIMIT && e * v < BRUTE_LIMIT)) e = __int_as_float(0x7fc00000);
+            // compared as integers a NaN is above every number, and -infinity above that
             e = __uint_as_float(half_wave_max(__float_as_uint(e)));
             v = __uint_as_float(half_wave_max(__float_as_uint(v) & 0x7fffffffu));
             if(row == 0) extent[tile] = make_float2(e, v);
@@ -282,12 +337,39 @@ __global__ void __launch_bounds__(256, GROUPS > 2 ? 3 : 4) k_brute(const float4 
         __syncthreads();
 
         const uint32_t n_tile = (n + 31u) / 32u;
+        float bound = extent[0].x;
+#pragma unroll
+        for(int tile = 1; tile < BRUTE_TILES; ++tile) bound = fminf(bound, extent[tile].x);
+        if(unbounded || bound != bound)
+        {
+            // no bound in the whole stage: every pair, a record read once for the lane's rays
+            vec3 o[GROUPS], d[GROUPS];
+            float tmin[GROUPS];
+#pragma unroll
+            for(int g = 0; g < GROUPS; ++g)
+            {
+                float tmax;
+                o[g] = d[g] = vec3{0.f, 0.f, 0.f};
+                tmin[g] = __int_as_float(0x7f800000);
+                if(!(ray_d[g] == -__int_as_float(0x7f800000)))
+                    load_ray(rays, first_ray + 32u * g, o[g], tmin[g], d[g], tmax);
+            }
+#pragma unroll 1
+            for(uint32_t row = half; row < n; row += 2u)
+            {
+                const float4 q0 = records[row][0], q1 = records[row][1], q2 = records[row][2];
+#pragma unroll
+                for(int g = 0; g < GROUPS; ++g) test(g, o[g], d[g], tmin[g], q0, q1, q2, base + row);
+            }
+            continue;
+        }
         for(uint32_t tile = 0; tile < n_tile; ++tile)
         {
             bf16x8 part[3];
 #pragma unroll
             for(int k = 0; k < 3; ++k) part[k] = parts[tile][k][lane];
             const float2 ev = extent[tile];
+            const uint32_t row0 = 32u * tile + 4u * half;
 #pragma unroll
             for(int g = 0; g < GROUPS; ++g)
             {
@@ -312,24 +394,15 @@ __global__ void __launch_bounds__(256, GROUPS > 2 ? 3 : 4) k_brute(const float4 
                 vec3 o, d;
                 float tmin, tmax;
                 load_ray(rays, first_ray + 32u * g, o, tmin, d, tmax);
-                auto test = [&](uint32_t row) {
-                    const float4 q0 = records[row][0], q1 = records[row][1], q2 = records[row][2];
-                    float t, u, v;
-                    if(!mt_fast_window(o, d, vec3{q0.x, q0.y, q0.z}, vec3{q0.w, q1.x, q1.y}, vec3{q1.z, q1.w, q2.x},
-                                       tmin, best[g], t, u, v))
-                        return;
-                    // (ANY: the ray takes no pair any more)
-                    if(ANY) ray_d[g] = -__int_as_float(0x7f800000);
-                    else best[g] = t;
-                    best_i[g] = base + row;
+                auto test_row = [&](uint32_t row) {
+                    test(g, o, d, tmin, records[row][0], records[row][1], records[row][2], base + row);
                 };
-                const uint32_t row0 = 32u * tile + 4u * half;
                 if(__any(!(margin < __int_as_float(0x7f800000))))
                 {
                     // no bound for some ray: every pair, a step's records asked for ahead of its tests
 #pragma unroll 4
                     for(uint32_t i = 0; i < 16; ++i)
-                        if(row0 + 8u * (i >> 2) + (i & 3u) < n) test(row0 + 8u * (i >> 2) + (i & 3u));
+                        if(row0 + 8u * (i >> 2) + (i & 3u) < n) test_row(row0 + 8u * (i >> 2) + (i & 3u));
                     continue;
                 }
                 uint32_t mask = 0;
@@ -343,7 +416,7 @@ __global__ void __launch_bounds__(256, GROUPS > 2 ? 3 : 4) k_brute(const float4 
                     const uint32_t i = __ffs(static_cast<int>(mask)) - 1, row = row0 + 8u * (i >> 2) + (i & 3u);
                     mask &= mask - 1u;
                     if(row >= n) break;
-                    test(row);
+                    test_row(row);
                     if(ANY && ray_d[g] == -__int_as_float(0x7f800000)) break;
                 }
             }
