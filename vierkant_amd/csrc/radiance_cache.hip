@@ -35,6 +35,18 @@ __device__ __forceinline__ void load_record(const float4 *records, uint32_t stri
     rec[3] = r[3];
 }
 
+//! How many records a pass over the encoder's buffers takes: a query and a training step of more of them are several
+//! passes, so the buffers are made with the cache and no call allocates.
+constexpr uint32_t QUERY_CHUNK = 1u << 20, TRAIN_CHUNK = 1u << 16;
+
+//! the records of a pass that begins at record `base` and has room for `cap`: with n_dev the device's count decides
+__device__ __forceinline__ uint32_t pass_count(uint32_t base, uint32_t cap, const uint32_t *__restrict__ n_dev)
+{
+    if(!n_dev) return cap;
+    const uint32_t n = *n_dev;
+    return n > base ? min(n - base, cap) : 0u;
+}
+
 //! a record's position word, read past the caches' least recently used order
 __device__ __forceinline__ float4 load_position(const float4 *rec)
 {
@@ -48,13 +60,13 @@ __device__ __forceinline__ float4 load_position(const float4 *rec)
 //! in every wave took 184. *loss, if given, is set to zero.
 constexpr uint32_t ENC_BLOCK = 256, ENC_RECORDS = ENC_BLOCK / 2;
 __global__ void __launch_bounds__(ENC_BLOCK) k_rc_encode(cache_dev c, const float4 *__restrict__ records,
-                                                         uint32_t stride_f4, uint32_t n_host,
+                                                         uint32_t stride_f4, uint32_t base, uint32_t n_cap,
                                                          const uint32_t *__restrict__ n_dev,
                                                          bf16x2 *__restrict__ enc, size_t enc_stride,
                                                          float *__restrict__ loss)
 {
     if(loss && blockIdx.x == 0 && threadIdx.x == 0) *loss = 0.0f;
-    const uint32_t n = n_dev ? min(*n_dev, n_host) : n_host;
+    const uint32_t n = pass_count(base, n_cap, n_dev);
     const uint32_t i = (blockIdx.x / XCDS) * ENC_RECORDS + threadIdx.x / 2, dx = threadIdx.x & 1u;
     float p[3] = {0.f, 0.f, 0.f};
     if(i < n) unit_position(c.g, load_position(records + (size_t)i * stride_f4), p);
@@ -71,12 +83,12 @@ __global__ void __launch_bounds__(ENC_BLOCK) k_rc_encode(cache_dev c, const floa
 }
 
 __global__ void __launch_bounds__(QUERY_BLOCK) k_rc_query(cache_dev c, const float4 *__restrict__ records,
-                                                          uint32_t stride_f4, uint32_t n_host,
+                                                          uint32_t stride_f4, uint32_t first, uint32_t n_cap,
                                                           const uint32_t *__restrict__ n_dev,
                                                           const bf16x2 *__restrict__ enc, size_t enc_stride,
                                                           float4 *__restrict__ out, float4 *__restrict__ pixel_acc)
 {
-    const uint32_t n = n_dev ? *n_dev : n_host;
+    const uint32_t n = pass_count(first, n_cap, n_dev);
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const uint32_t base = (blockIdx.x * (QUERY_BLOCK / 64) + wave) * (16 * QUERY_TILES);
     if(base >= n) return;// whole wave idle; the MLP below needs all 64 lanes
@@ -122,13 +134,14 @@ __global__ void __launch_bounds__(QUERY_BLOCK) k_rc_query(cache_dev c, const flo
 
 __global__ void __launch_bounds__(TRAIN_BLOCK) k_rc_train(cache_dev c, const float4 *__restrict__ records,
                                                           uint32_t stride_f4, const float4 *__restrict__ targets,
-                                                          uint32_t n_cap, const uint32_t *__restrict__ n_dev,
+                                                          uint32_t base, uint32_t n_cap, uint32_t n_all,
+                                                          const uint32_t *__restrict__ n_dev,
                                                           const bf16x2 *__restrict__ enc, float2 *__restrict__ enc_grad,
                                                           size_t enc_stride, float *__restrict__ partials,
                                                           float *__restrict__ loss_sum)
 {
-    // sample count: n_cap, or the device counter clamped to n_cap
-    const uint32_t n = n_dev ? min(*n_dev, n_cap) : n_cap;
+    const uint32_t n = pass_count(base, n_cap, n_dev);
+    const float nf = static_cast<float>(pass_count(0u, n_all, n_dev));// the samples of all passes
     __shared__ __bf16 act[N_LAYERS][WIDTH][LDS_ROW];// a_0 = x0, a_i = h_i (i = 1..5), [feature][sample]
     __shared__ __bf16 dzs[WIDTH][LDS_ROW];          // the current layer's output gradient, [feature][sample]
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, group = lane >> 4, col = lane & 15u;
@@ -136,10 +149,18 @@ __global__ void __launch_bounds__(TRAIN_BLOCK) k_rc_train(cache_dev c, const flo
 
     f32x4 dw[N_HIDDEN][4];// W1..W5: row tile = wave, column tiles 0..3
     f32x4 dw6 = {0.f, 0.f, 0.f, 0.f};
+    float *part = partials + (size_t)blockIdx.x * N_MLP;// logical [out][in] layout
+    // (a later pass goes on with the sums that the one before left)
 #pragma unroll
-    for(int l = 0; l < (int)N_HIDDEN; ++l)
+    for(uint32_t li = 0; li < N_HIDDEN; ++li)
 #pragma unroll
-        for(int q = 0; q < 4; ++q) dw[l][q] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for(int q = 0; q < 4; ++q)
+#pragma unroll
+            for(int i = 0; i < 4; ++i)
+                dw[li][q][i] = base ? part[layer_offset(li) + (16 * wave + 4 * group + i) * WIDTH + 16 * q + col] : 0.f;
+    if(base)
+#pragma unroll
+        for(int i = 0; i < 4; ++i) dw6[i] = part[layer_offset(N_HIDDEN) + (4 * group + i) * WIDTH + 16 * wave + col];
     float loss_lane = 0.0f;
     const uint32_t iterations = (n + TRAIN_SAMPLES - 1) / TRAIN_SAMPLES;
 
@@ -200,7 +221,6 @@ __global__ void __launch_bounds__(TRAIN_BLOCK) k_rc_train(cache_dev c, const flo
             const float denom = ybar * ybar + LOSS_EPS;
             const float d0 = y[0] - tg.x, d1 = y[1] - tg.y, d2 = y[2] - tg.z;
             loss_lane += ((d0 * d0) / denom + (d1 * d1) / denom) + (d2 * d2) / denom;
-            const float nf = static_cast<float>(n);
             dy[0] = (2.0f * d0 / denom) / nf;
             dy[1] = (2.0f * d1 / denom) / nf;
             dy[2] = (2.0f * d2 / denom) / nf;
@@ -275,8 +295,7 @@ __global__ void __launch_bounds__(TRAIN_BLOCK) k_rc_train(cache_dev c, const flo
                     enc_grad[(4 * r + 2 * group + h) * enc_stride + m] = make_float2(dh[r][2 * h], dh[r][2 * h + 1]);
     }
 
-    // ---- per-block weight gradients, logical [out][in] layout ------------------------------------------
-    float *part = partials + (size_t)blockIdx.x * N_MLP;
+    // ---- per-block weight gradients --------------------------------------------------------------------
 #pragma unroll
     for(uint32_t li = 0; li < N_HIDDEN; ++li)
 #pragma unroll
@@ -302,12 +321,12 @@ __global__ void __launch_bounds__(TRAIN_BLOCK) k_rc_train(cache_dev c, const flo
 //! entry's updates then meet in one L2, and a corner's with its neighbour's in one request (16,384 records: 61 us, 114
 //! with a corner a lane)
 __global__ void __launch_bounds__(ENC_BLOCK) k_rc_scatter(cache_dev c, const float4 *__restrict__ records,
-                                                          uint32_t stride_f4, uint32_t n_cap,
+                                                          uint32_t stride_f4, uint32_t base, uint32_t n_cap,
                                                           const uint32_t *__restrict__ n_dev,
                                                           const float2 *__restrict__ enc_grad, size_t enc_stride,
                                                           half2v *__restrict__ grid_grad, float grad_scale)
 {
-    const uint32_t n = n_dev ? min(*n_dev, n_cap) : n_cap;
+    const uint32_t n = pass_count(base, n_cap, n_dev);
     const uint32_t i = (blockIdx.x / XCDS) * ENC_RECORDS + threadIdx.x / 2, dx = threadIdx.x & 1u;
     if(i >= n) return;
     float p[3];
@@ -446,11 +465,11 @@ static void fill(hipStream_t s, float *p, uint64_t n, float value)
     if(n) k_rc_fill<<<(uint32_t)((n + 255) / 256), 256, 0, s>>>(p, n, value);
 }
 
-static uint32_t train_blocks(vkrt_rc *c, uint32_t n)
+static uint32_t train_blocks(const vkrt_ctx *ctx, uint32_t n)
 {
     // one 4-wave block per CU (the kernel runs one wave per SIMD)
     const uint32_t iterations = div_up(n, TRAIN_SAMPLES);
-    return std::max<uint32_t>(1u, std::min<uint32_t>(iterations, (uint32_t)c->ctx->cu_count));
+    return std::max<uint32_t>(1u, std::min<uint32_t>(iterations, (uint32_t)ctx->cu_count));
 }
 
 //! power-of-two loss scale of the fp16 grid gradient: per-sample gradients scale as 1 / n, so the scaled
@@ -470,24 +489,27 @@ __global__ void k_rc_grid_grad_f32(const _Float16 *__restrict__ g, float inv_sca
 void train(vkrt_rc *c, const float4 *records, uint32_t stride_f4, const float4 *targets, uint32_t n, bool grad_only,
            const uint32_t *n_dev, hipStream_t s)
 {
-    const uint32_t nb = train_blocks(c, n);
-    c->partials.reserve((size_t)nb * N_MLP * 4);
+    const uint32_t nb = train_blocks(c->ctx, std::min(n, TRAIN_CHUNK));
     c->grad_scale = grid_grad_scale(n);
     if(!c->grid_grad_clear) fill(s, c->grid_grad.as<float>(), c->n_grid / 2, 0.0f);// n_grid fp16 values
     // a gradient-only step leaves its gradients for reading; a full step's Adam pass clears them
     c->grid_grad_clear = !grad_only;
     if(n)
     {
-        const uint32_t grid = XCDS * div_up(n, ENC_RECORDS);
-        c->train_enc.reserve((size_t)LEVELS * n * sizeof(bf16x2));
-        c->train_grad.reserve((size_t)LEVELS * n * sizeof(float2));
         bf16x2 *enc = c->train_enc.as<bf16x2>();
         float2 *enc_grad = c->train_grad.as<float2>();
-        k_rc_encode<<<grid, ENC_BLOCK, 0, s>>>(device_view(c), records, stride_f4, n, n_dev, enc, n, c->loss.as<float>());
-        k_rc_train<<<nb, TRAIN_BLOCK, 0, s>>>(device_view(c), records, stride_f4, targets, n, n_dev, enc, enc_grad, n,
-                                              c->partials.as<float>(), c->loss.as<float>());
-        k_rc_scatter<<<grid, ENC_BLOCK, 0, s>>>(device_view(c), records, stride_f4, n, n_dev, enc_grad, n,
-                                                c->grid_grad.as<half2v>(), c->grad_scale);
+        for(uint32_t base = 0, m; base < n; base += m)
+        {
+            m = std::min(n - base, TRAIN_CHUNK);
+            const uint32_t grid = XCDS * div_up(m, ENC_RECORDS);
+            const float4 *rec = records + (size_t)base * stride_f4;
+            k_rc_encode<<<grid, ENC_BLOCK, 0, s>>>(device_view(c), rec, stride_f4, base, m, n_dev, enc, m,
+                                                   base ? nullptr : c->loss.as<float>());
+            k_rc_train<<<nb, TRAIN_BLOCK, 0, s>>>(device_view(c), rec, stride_f4, targets + base, base, m, n, n_dev,
+                                                  enc, enc_grad, m, c->partials.as<float>(), c->loss.as<float>());
+            k_rc_scatter<<<grid, ENC_BLOCK, 0, s>>>(device_view(c), rec, stride_f4, base, m, n_dev, enc_grad, m,
+                                                    c->grid_grad.as<half2v>(), c->grad_scale);
+        }
     }
     else
     {
@@ -521,12 +543,16 @@ void query(vkrt_rc *c, const float4 *records, uint32_t stride_f4, uint32_t n, fl
     if(n == 0) return;
     const uint32_t per_block = QUERY_BLOCK / 64 * 16 * QUERY_TILES;
     hipStream_t s = c->ctx->stream;
-    c->query_enc.reserve((size_t)LEVELS * n * sizeof(bf16x2));
     bf16x2 *enc = c->query_enc.as<bf16x2>();
-    k_rc_encode<<<XCDS * div_up(n, ENC_RECORDS), ENC_BLOCK, 0, s>>>(device_view(c), records, stride_f4, n, count_on_device,
-                                                                  enc, n, nullptr);
-    k_rc_query<<<div_up(n, per_block), QUERY_BLOCK, 0, s>>>(device_view(c), records, stride_f4, n, count_on_device, enc, n,
-                                                            out, pixel_acc);
+    for(uint32_t base = 0, m; base < n; base += m)
+    {
+        m = std::min(n - base, QUERY_CHUNK);
+        const float4 *rec = records + (size_t)base * stride_f4;
+        k_rc_encode<<<XCDS * div_up(m, ENC_RECORDS), ENC_BLOCK, 0, s>>>(device_view(c), rec, stride_f4, base, m,
+                                                                      count_on_device, enc, m, nullptr);
+        k_rc_query<<<div_up(m, per_block), QUERY_BLOCK, 0, s>>>(device_view(c), rec, stride_f4, base, m, count_on_device,
+                                                                enc, m, out ? out + base : nullptr, pixel_acc);
+    }
     VKRT_HIP(hipGetLastError());
 }
 
@@ -648,6 +674,10 @@ int vkrt_rc_create(vkrt_ctx *ctx, const vkrt_rc_params *params, uint32_t seed, v
         c->w_fwd.reserve(N_LAYERS * LAYER_ELEMS * 2);
         c->w_bwd.reserve(N_LAYERS * LAYER_ELEMS * 2);
         c->loss.reserve(256);
+        c->query_enc.reserve((size_t)LEVELS * QUERY_CHUNK * sizeof(bf16x2));
+        c->train_enc.reserve((size_t)LEVELS * TRAIN_CHUNK * sizeof(bf16x2));
+        c->train_grad.reserve((size_t)LEVELS * TRAIN_CHUNK * sizeof(float2));
+        c->partials.reserve((size_t)train_blocks(ctx, TRAIN_CHUNK) * N_MLP * 4);
         VKRT_HIP(hipHostMalloc(reinterpret_cast<void **>(&c->host_loss), 256));
         hipStream_t s = ctx->stream;
         // padding slots of the transposed W6 swizzle stay zero

@@ -308,8 +308,8 @@ struct vkrt_rc
     // grid_grad holds zeros: the last training step's Adam pass cleared every entry it read as non-zero
     bool grid_grad_clear = false;
     vkrt::device_buffer mlp_master, mlp_grad, mlp_m, mlp_v, w_fwd, w_bwd, partials, loss;
-    // per record: the encoder's features of a query or of a training step, and the latter's feature gradients. A
-    // training step may run beside a query, so each has its own
+    // the encoder's features of up to QUERY_CHUNK records of a query and up to TRAIN_CHUNK of a training step, and the
+    // latter's feature gradients. A training step may run beside a query, so each has its own
     vkrt::device_buffer query_enc, train_enc, train_grad;
     float *host_loss = nullptr;// the last training step's loss sum, in pinned memory
 
