@@ -17,23 +17,38 @@ def room():
     return W.room_scene(n_spheres=40)
 
 
+def render(ctx, scene, size, spp, lit, tail, batches=2, depth=6):
+    """the pixels' bytes and the last batch's segments; tail None: the shape the tracer chooses"""
+    s = vk.default_settings()
+    s.resolution[0], s.resolution[1] = size
+    s.num_samples, s.max_trace_depth = spp, depth
+    pt = vk.PathTracer(ctx, s, seed=9)
+    if isinstance(scene, tuple):
+        pt.set_instanced_scene(*scene)
+    else:
+        pt.set_scene(scene)
+    if lit:
+        pt.set_lights(W.room_lights())
+    if tail is not None:
+        pt.set_launch_mode(vk.PT_LAUNCH_FULL_GRID, tail)
+    for _ in range(batches):
+        pt.render(W.room_camera())
+    got = pt.pixels().tobytes(), pt.stats().segments
+    pt.close()
+    return got
+
+
 @pytest.mark.parametrize("lit", [False, True])
 @pytest.mark.parametrize("size", SIZES)
 def test_chosen_shape_gives_the_same_image(ctx, room, size, lit):
-    got = []
-    for tail in (None, vk.PT_NO_TAIL):
-        s = vk.default_settings()
-        s.resolution[0], s.resolution[1] = size
-        s.num_samples, s.max_trace_depth = 2, 6
-        pt = vk.PathTracer(ctx, s, seed=9)
-        pt.set_scene(room)
-        if lit:
-            pt.set_lights(W.room_lights())
-        if tail is not None:
-            pt.set_launch_mode(vk.PT_LAUNCH_FULL_GRID, tail)
-        for _ in range(2):
-            pt.render(W.room_camera())
-        got.append((pt.pixels().tobytes(), pt.stats().segments))
-        pt.close()
-    assert got[0][1] >= 2 * size[0] * size[1]
-    assert got[0] == got[1]
+    got, want = (render(ctx, room, size, 2, lit, tail) for tail in (None, vk.PT_NO_TAIL))
+    assert want[1] >= 2 * size[0] * size[1]
+    assert got == want
+
+
+@pytest.mark.parametrize("lit", [False, True])
+@pytest.mark.parametrize("spp", [63, 64, 65, 129])
+def test_runs_of_samples_give_the_same_image(ctx, room, spp, lit):
+    """a small image's launches take 64 samples each"""
+    got, want = (render(ctx, room, (47, 31), spp, lit, tail) for tail in (None, vk.PT_NO_TAIL))
+    assert got == want

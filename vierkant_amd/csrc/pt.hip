@@ -1581,9 +1581,11 @@ __device__ __forceinline__ uint32_t finish_path(const vkrt_bvh_node *__restrict_
 //! remaining depth with no kernel boundary between depths. Past the first few depths the live queue fills a fraction
 //! of the GPU and each per-depth launch lasts as long as its slowest wave's traversal (a chain of dependent node
 //! loads); here a wave's lanes run their depths back to back and the waves overlap. SAMPLES true: the same from the
-//! camera on, for every sample of pixels d0 .. d0 + n - 1, a lane each: a small image fills so little of the GPU
-//! that every launch is such a tail (see shape_of). Each path performs the operations of the per-depth kernels in
+//! camera on, for up to PT_SAMPLE_RUN samples from sample `in` on of pixels d0 .. d0 + n - 1, a lane each: a small image
+//! fills so little of the GPU that every launch is such a tail (see shape_of). Each path performs the operations of the per-depth kernels in
 //! the same order (trace, shade, shadow ray, next depth), so the image is bit for bit the same.
+//! (a launch of every sample of a batch would hold the GPU for seconds at thousands of samples a pixel)
+constexpr uint32_t PT_SAMPLE_RUN = 64;
 template<bool LIGHTS, class F, bool INST, bool SAMPLES>
 __global__ void __launch_bounds__(PT_BLOCK) k_pt_finish(const vkrt_bvh_node *__restrict__ nodes2,
                                                         const float4 *__restrict__ tris, int32_t root2, bool empty,
@@ -1602,12 +1604,15 @@ __global__ void __launch_bounds__(PT_BLOCK) k_pt_finish(const vkrt_bvh_node *__r
     {
         const uint32_t p = SAMPLES ? d0 + q : b.queue[in][q];
         if constexpr(SAMPLES)
-            for(uint32_t sample = 0; sample < f.num_samples; ++sample)
+        {
+            const uint32_t first = static_cast<uint32_t>(in), end = first + min(f.num_samples - first, PT_SAMPLE_RUN);
+            for(uint32_t sample = first; sample < end; ++sample)
             {
                 begin_path(f, b, sample, p, 0u);
                 segments += finish_path<LIGHTS, F, INST>(nodes2, tris, root2, empty, nodes4, root4, walk, f, b, s, flt,
                                                          shadow_flt, 0u, p, smem + threadIdx.x, tl);
             }
+        }
         else
             segments = finish_path<LIGHTS, F, INST>(nodes2, tris, root2, empty, nodes4, root4, walk, f, b, s, flt,
                                                     shadow_flt, d0, p, smem + threadIdx.x, tl);
@@ -1945,7 +1950,7 @@ static F filter_of(const alpha_filter &a)
 }
 
 //! How a batch without a cache is launched: pixel groups (one on the side stream), and the depth from which paths
-//! finish in one lane (0: from the camera on, every sample, in one launch).
+//! finish in one lane (0: from the camera on, PT_SAMPLE_RUN samples a launch).
 //!
 //! A per-depth launch lasts at least as long as its longest ray (150 us, lit 190), so the fewer pixels share it the
 //! earlier the one-lane kernel is the better one, although it holds only 2 waves per SIMD, 131,072 lanes of 256 CUs.
@@ -2098,9 +2103,9 @@ static void trace_batch(vkrt_pt *pt, const vkrt_camera &cam, uint32_t seed)
                 k_pt_shade<false, I><<<g.blocks, PT_BLOCK, 0, st>>>(f, bb, sc, depth, in);
         });
     };
-    // the survivors at the tail depth finish in one lane each; from depth 0 on, all samples in one launch
-    auto finish = [&](const group &g, uint32_t depth) {
-        const int in = static_cast<int>(depth & 1u);
+    // the survivors at the tail depth finish in one lane each; from depth 0 on, a run of samples from `sample` on
+    auto finish = [&](const group &g, uint32_t depth, uint32_t sample = 0) {
+        const int in = static_cast<int>(depth ? depth & 1u : sample);
         variant([&](auto a, auto in_) {
             using F = std::conditional_t<decltype(a)::value, alpha_filter, keep_all>;
             constexpr bool I = decltype(in_)::value;
@@ -2124,7 +2129,8 @@ static void trace_batch(vkrt_pt *pt, const vkrt_camera &cam, uint32_t seed)
         VKRT_HIP(hipStreamWaitEvent(side, pt->ev_fork, 0));
     }
     const bool whole = !f.cache_on && shape.tail == 0u;
-    for(uint32_t g = 0; whole && g < n_groups; ++g) finish(groups[g], 0u);
+    for(uint32_t sample = 0; whole && sample < f.num_samples; sample += PT_SAMPLE_RUN)
+        for(uint32_t g = 0; g < n_groups; ++g) finish(groups[g], 0u, sample);
     for(uint32_t sample = 0; !whole && sample < f.num_samples; ++sample)
     {
         uint32_t main_depths = f.max_depth;
