@@ -3,6 +3,10 @@ tracer chooses by itself gives the image, the segment count and the running mean
 import pytest
 
 import vierkant_amd as vk
+from test_gpu_media import _absorbing_room
+from test_gpu_pt import _alpha_room
+from test_gpu_textures import fully_textured_room
+from test_pt_oracle_instanced import _glassy
 from vierkant_amd import workloads as W
 
 pytestmark = pytest.mark.gpu
@@ -52,3 +56,27 @@ def test_runs_of_samples_give_the_same_image(ctx, room, spp, lit):
     """a small image's launches take 64 samples each"""
     got, want = (render(ctx, room, (47, 31), spp, lit, tail) for tail in (None, vk.PT_NO_TAIL))
     assert got == want
+
+
+@pytest.fixture(scope="module")
+def scenes():
+    """the kernels' other variants: instances, alpha-tested materials, interior media, textures"""
+    sc, mf, inst = W.room_instanced()
+    flat = W.room_scene(n_spheres=40)
+    absorbing = _absorbing_room(flat)
+    return {"instanced": (_glassy(sc, mf), mf, inst), "instanced alpha": (_alpha_room(sc), mf, inst),
+            "absorbing": absorbing, "absorbing instanced": (absorbing, *W.object_meshes(absorbing)),
+            "textured": fully_textured_room(), "alpha": _alpha_room(flat)}
+
+
+@pytest.mark.parametrize("lit", [False, True])
+@pytest.mark.parametrize("size", [(47, 31), (331, 397), (811, 811)])
+@pytest.mark.parametrize("name", ["instanced", "instanced alpha", "absorbing", "absorbing instanced", "textured",
+                                  "alpha"])
+def test_shapes_of_other_scenes_give_the_same_image(ctx, scenes, name, size, lit):
+    """one lane from the camera on, a tail, and two pixel groups with a tail, against one launch per depth; and the
+    smaller two images with a tail from depth 2"""
+    want = render(ctx, scenes[name], size, 2, lit, vk.PT_NO_TAIL)
+    assert want[1] > 2 * size[0] * size[1]
+    for tail in (None, 2) if size[0] < 800 else (None,):
+        assert render(ctx, scenes[name], size, 2, lit, tail) == want, tail
