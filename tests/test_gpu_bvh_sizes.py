@@ -13,9 +13,8 @@ pytestmark = pytest.mark.gpu
 SIZES = [1, 2, 3, 8, 9, 63, 64, 65, 129, 255, 256, 257, 511, 513, 1023, 1024, 1025, 2047, 2049, 4097, 65537, 262145]
 
 
-@pytest.mark.parametrize("builder", [vk.BUILDER_LBVH, vk.BUILDER_PLOC])
-@pytest.mark.parametrize("n_tri", SIZES)
-def test_build_and_refit_at_tile_edges(ctx, builder, n_tri):
+def check_build_and_refit(ctx, n_tri, shapes, **build):
+    """a soup of n_tri triangles, built at each (leaf size, width), before and after its vertices move"""
     rng = np.random.default_rng(n_tri)
     corner = rng.uniform(-1, 1, (n_tri, 1, 3))
     size = 2.0 * n_tri ** (-1 / 3)
@@ -24,8 +23,8 @@ def test_build_and_refit_at_tile_edges(ctx, builder, n_tri):
     pos = np.ascontiguousarray(pos[np.argsort(idx)])
     o = rng.uniform(-2, 2, (1000, 3)).astype(np.float32)
     rays = W.make_rays(o, W.glm_normalize(rng.normal(size=(1000, 3)).astype(np.float32)))
-    for leaf, width in ((0, 0), (8, 0), (1, 2)):
-        bvh = ctx.bvh_build(pos, idx, builder=builder, max_leaf_size=leaf, width=width)
+    for leaf, width in shapes:
+        bvh = ctx.bvh_build(pos, idx, max_leaf_size=leaf, width=width, **build)
         info = bvh.info()
         assert info.n_tri == n_tri and info.depth <= 64
         moved = pos + np.float32(0.25) * np.sin(3.0 * pos[:, ::-1]).astype(np.float32)
@@ -35,8 +34,22 @@ def test_build_and_refit_at_tile_edges(ctx, builder, n_tri):
             check = bvh.validate(p)
             assert check["ok"], check
             assert_hits_equal(ctx.trace_closest(bvh, rays), ctx.brute_closest(W.flat_triangles(p, idx), rays),
-                              f"{n_tri} triangles, leaf {leaf}, width {width}")
+                              f"{n_tri} triangles, leaf {leaf}, width {width}, {build}")
         bvh.close()
+
+
+@pytest.mark.parametrize("builder", [vk.BUILDER_LBVH, vk.BUILDER_PLOC])
+@pytest.mark.parametrize("n_tri", SIZES)
+def test_build_and_refit_at_tile_edges(ctx, builder, n_tri):
+    check_build_and_refit(ctx, n_tri, ((0, 0), (8, 0), (1, 2)), builder=builder)
+
+
+@pytest.mark.parametrize("n_tri", [900, 1025, 2049, 65537])
+@pytest.mark.parametrize("radius", [1, 3, 31, 32])
+def test_ploc_radii(ctx, radius, n_tri):
+    """the neighbour search's tile, span and LDS places depend on the radius: one workgroup's clusters, a few tiles and
+    many"""
+    check_build_and_refit(ctx, n_tri, ((0, 0), (1, 2)), builder=vk.BUILDER_PLOC, ploc_radius=radius)
 
 
 @pytest.mark.parametrize("builder", [vk.BUILDER_LBVH, vk.BUILDER_PLOC])

@@ -39,7 +39,8 @@ def test_queries_do_not_depend_on_the_batch(cache):
 @pytest.mark.parametrize("n", SIZES)
 def test_gradients_at_tile_edges(cache, n):
     """against the numpy restatement: only its entries are touched, and values agree to 12 roundings to bfloat16 (6
-    layers forward, 6 back, 2^-8 each: 4.7 %) of the largest one"""
+    layers forward, 6 back, 2^-8 each: 4.7 %) of the largest one; entries that only the last record, the one at the
+    tile's edge, touches agree to as much of that record's largest"""
     rec = base.world_records(n, 22)
     tg = np.random.default_rng(23).uniform(0, 2, (n, 3)).astype(np.float32)
     cache.train(rec, tg, grad_only=True)
