@@ -225,7 +225,7 @@ typedef struct vkrt_bvh_info
     uint32_t depth;
     float sah_cost;
     float build_ms;
-    uint64_t device_bytes;
+    uint64_t device_bytes;  /* device memory that the BVH holds */
     float bounds[6];
     uint32_t n_wide_nodes;  /* nodes of the 4-wide collapse (0 when traversal uses the binary tree) */
     uint32_t wide_stack;    /* worst-case traversal stack depth of the 4-wide collapse */

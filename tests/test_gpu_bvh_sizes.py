@@ -27,6 +27,11 @@ def check_build_and_refit(ctx, n_tri, shapes, **build):
         bvh = ctx.bvh_build(pos, idx, max_leaf_size=leaf, width=width, **build)
         info = bvh.info()
         assert info.n_tri == n_tri and info.depth <= 64
+        # a record, three indices and a place in the order per triangle; a 4-wide node and its run, or a binary one,
+        # its children and its run (and room for more 4-wide nodes than there came to be)
+        least = n_tri * (64 + 12 + 4) + info.n_wide_nodes * (128 + 8) + (0 if info.n_wide_nodes else info.n_nodes * 80)
+        if n_tri > leaf:
+            assert least <= info.device_bytes <= 2 * least + 4096
         moved = pos + np.float32(0.25) * np.sin(3.0 * pos[:, ::-1]).astype(np.float32)
         for p in (pos, moved):
             if p is moved:

@@ -1542,8 +1542,7 @@ static void refresh_info(vkrt_bvh *bvh)
 {
     bvh->info.n_tri = bvh->n_tri;
     bvh->info.n_nodes = bvh->n_nodes;
-    bvh->info.device_bytes = bvh->nodes.bytes + (uint64_t)bvh->n_tri * TRI_BYTES +
-                             (uint64_t)bvh->n_nodes4 * sizeof(vkrt_bvh4_node);
+    bvh->info.device_bytes = bvh->memory.bytes + bvh->binary.bytes;
     bvh->info.n_wide_nodes = bvh->wide ? bvh->n_nodes4 : 0;
     bvh->info.wide_stack = bvh->stack4;
 }
