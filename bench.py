@@ -96,12 +96,12 @@ def cpu_baseline(tris, rays, budget_s):
 def brute_force_leg(ctx, reps=10):
     """the brute-force closest hit of 65,536 rays (origins U[-3,3]^3, directions uniform on S^2, seed 0)
     against the 20,480-triangle jittered icosphere (subdivision 5, radius 1, vertices N(0, 0.01)): one
-    ray-triangle test per pair, 1,342,177,280 per run. The matrix cores sort out the pairs that can hit, 192
-    bf16 operations a pair (six 32x32x16 products per 1,024 pairs); those take the full test of
-    src/intersection.cpp:114-129. Timed on the GPU (HBM-resident arrays, hipEvents around `reps`
-    runs) and, as the CPU baseline of this workload, the oracle's full run on every host thread (1 warm-up,
-    median of 5) and a 4,096-ray sample on one thread. The GPU records are checked bit for bit against the
-    oracle's full run."""
+    ray-triangle test per pair, 1,342,177,280 per run. The matrix cores sort out the pairs that can hit, 144
+    bf16 operations a pair (six 32x32x16 products per 1,024 pairs, twelve of each sixteen terms values and the
+    others padding, which is not counted); those take the full test of src/intersection.cpp:114-129. Timed on
+    the GPU (HBM-resident arrays, hipEvents around `reps` runs) and, as the CPU baseline of this workload, the
+    oracle's full run on every host thread (1 warm-up, median of 5) and a 4,096-ray sample on one thread. The
+    GPU records are checked bit for bit against the oracle's full run."""
     import numpy as np
     import vierkant_amd as vk
     from vierkant_amd import workloads as W
@@ -141,7 +141,7 @@ def brute_force_leg(ctx, reps=10):
     mismatch = int(np.sum((got["prim"] != want["prim"]) | (got["t"].view(np.uint32) != want["t"].view(np.uint32)) |
                           (got["u"].view(np.uint32) != want["u"].view(np.uint32)) |
                           (got["v"].view(np.uint32) != want["v"].view(np.uint32))))
-    flops = 192.0 * n_tests
+    flops = 144.0 * n_tests
     tflops = flops / (ms * 1e-3) / 1e12
     return {"workload": "brute-force closest hit, 65,536 rays x 20,480-triangle jittered icosphere (subdiv 5, "
                         "r 1, N(0, 0.01)), seed 0", "tests_per_run": n_tests,
@@ -149,7 +149,7 @@ def brute_force_leg(ctx, reps=10):
             "gpu_rays_per_s": round(len(rays) / (ms * 1e-3), 1),
             "roofline": {"bound": "bf16 mfma", "kernel": "k_brute (whole call: fill + filter and test + finalize)",
                          "achieved": round(tflops, 3), "peak": 2516.6, "unit": "TFLOP/s",
-                         "frac": round(tflops / 2516.6, 5), "flop_per_test": 192, "flop_per_run": flops},
+                         "frac": round(tflops / 2516.6, 5), "flop_per_test": 144, "flop_per_run": flops},
             "verified_vs_oracle_full_run": {"rays": len(rays), "mismatches": mismatch,
                                             "hits": int(np.sum(want["prim"] != 0xFFFFFFFF))},
             "cpu_full_run": {"threads": nthreads, "cpu_model": model, "median_s": round(cpu_s, 3),

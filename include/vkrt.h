@@ -669,7 +669,8 @@ int vkrt_pt_set_lights(vkrt_pt *pt, const vkrt_light *lights, uint32_t n);
  * the workgroups the GPU holds at once that claim the live queue's tiles with atomics. tail_depth (>= 1,
  * VKRT_PT_TAIL_DEPTH_DEFAULT for large images): outside the radiance-cache mode the paths alive at that depth finish in
  * one lane each, every remaining depth in one kernel; VKRT_PT_NO_TAIL keeps one launch per depth to the end. A
- * tracer on which this was never called chooses the depth by the number of pixels.
+ * tracer on which this was never called chooses the depth by the number of pixels; a call fixes it for good, at
+ * VKRT_PT_TAIL_DEPTH_DEFAULT as at any other.
  * Every combination gives the same image bit for bit. */
 enum
 {

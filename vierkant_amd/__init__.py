@@ -817,7 +817,8 @@ class PathTracer:
 
     def set_launch_mode(self, mode, tail_depth=PT_TAIL_DEPTH_DEFAULT):
         """PT_LAUNCH_FULL_GRID (default) or PT_LAUNCH_PERSISTENT per-depth launches; paths alive at tail_depth
-        finish in one lane each (PT_NO_TAIL: per-depth launches to the end). Every choice gives the same image"""
+        finish in one lane each (PT_NO_TAIL: per-depth launches to the end). Every choice gives the same image. A
+        tracer on which this is not called chooses the depth by the number of pixels"""
         self.ctx.check(lib().vkrt_pt_set_launch_mode(self._h, mode, tail_depth))
 
     def set_lights(self, lights):

@@ -45,9 +45,9 @@ __global__ void k_batch_reset(uint32_t *counter) { counter[threadIdx.x] = 0u; }
 //! loop state, against 72 unconstrained, which holds 7). JOINT: every 4-wide item's nodes and records are within reach
 //! of one base
 template<int BLOCK, int LDS, bool JOINT>
-__global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8))) k_batch_trace(const batch_item_dev *__restrict__ items, uint32_t n_items,
-                                                       const uint32_t *__restrict__ tile_prefix, uint32_t tile,
-                                                       uint32_t *__restrict__ counters, uint32_t chunk)
+__global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(8)))
+k_batch_trace(const batch_item_dev *__restrict__ items, uint32_t n_items, const uint32_t *__restrict__ tile_prefix,
+              uint32_t tile, uint32_t *__restrict__ counters, uint32_t chunk)
 {
     __shared__ int32_t smem[LDS > 0 ? LDS * BLOCK : 1];
     __shared__ uint32_t s_tile;

@@ -58,9 +58,9 @@ struct vkrt_bvh
     bool empty = true;
     // One allocation holds the 4-wide collapse, used by traversal when its worst-case stack fits (wide == true), the
     // leaf records behind it, so that a walk reaches both with 32-bit offsets from one base (joint == true unless
-    // they pass 4 GiB, from some 41M triangles at two a leaf), and what a refit needs: the mesh's indices, the leaves' order and the run of leaves below
-    // each 4-wide node. (Freeing a large allocation takes 250 to 500 us: eight of them took 1.7 of the 4.1 ms that
-    // building and destroying a 1.8M-triangle BVH took.)
+    // they pass 4 GiB, from some 41M triangles at two a leaf), and what a refit needs: the mesh's indices, the
+    // leaves' order and the run of leaves below each 4-wide node. (Freeing a large allocation takes 250 to 500 us:
+    // eight of them took 1.7 of the 4.1 ms that building and destroying a 1.8M-triangle BVH took.)
     vkrt::device_buffer memory;
     part nodes4, tris, indices, order, wide_range;
     uint32_t node_cap = 0;// 4-wide nodes there is room for

@@ -1498,11 +1498,10 @@ __device__ __forceinline__ void shadow_path(const vkrt_bvh_node *__restrict__ no
 //! throughput joins the pixel's sample sum; a training vertex also records the unscaled estimate
 template<class F, bool INST>
 __global__ void __launch_bounds__(PT_BLOCK)
-__attribute__((amdgpu_waves_per_eu(INST || F::active ? 1 : PT_SHADOW_PLAIN_WAVES_PER_SIMD))) k_pt_shadow(const vkrt_bvh_node *__restrict__ nodes2, int32_t root2,
-                                                        const vkrt_bvh4_node *__restrict__ nodes4, int32_t root4,
-                                                        uint32_t walk, bool empty, const float4 *__restrict__ tris,
-                                                        const gpu_material *__restrict__ mats, pt_frame f,
-                                                        pt_buffers b, F flt, pt_tlas tl)
+__attribute__((amdgpu_waves_per_eu(INST || F::active ? 1 : PT_SHADOW_PLAIN_WAVES_PER_SIMD)))
+k_pt_shadow(const vkrt_bvh_node *__restrict__ nodes2, int32_t root2, const vkrt_bvh4_node *__restrict__ nodes4,
+            int32_t root4, uint32_t walk, bool empty, const float4 *__restrict__ tris,
+            const gpu_material *__restrict__ mats, pt_frame f, pt_buffers b, F flt, pt_tlas tl)
 {
     __shared__ int32_t smem[PT_LDS * PT_BLOCK];
     const uint32_t count = b.counter[C_SHADOW];
@@ -1963,7 +1962,10 @@ static F filter_of(const alpha_filter &a)
 //!  2,073,600          - 2.94 2.08 1.65 1.49   - 8.42 6.01 4.70 4.16
 //! Two groups, one tracing its last long paths while the other fills the chip, gain from about a million pixels on
 //! (921,600 pixels .95 -> .92 and 2.79 -> 2.73 ms, 2,073,600 1.49 -> 1.35 and 4.16 -> 3.77) and cost below (230,400
-//! .58 -> .61). Three gain 2 % more there.
+//! .58 -> .61). Three gain 2 % more there. The lines between the measured sizes are interpolated, at one, two and a
+//! half, five and ten times the lanes. They were not drawn for other scenes, where this shape is nowhere slower than
+//! a tail at depth 4 in one group: over flat, alpha-tested, glass, instanced and instanced alpha-tested rooms, lit and
+//! unlit, at 57,600 to 921,600 pixels and max_trace_depth 3, 8 and 24 (14,400 to 2,073,600 at 8).
 struct batch_shape
 {
     uint32_t groups, tail;
@@ -1972,7 +1974,11 @@ struct batch_shape
 static batch_shape shape_of(const vkrt_pt *pt, uint32_t n_pix)
 {
     const uint32_t lanes = static_cast<uint32_t>(pt->ctx->cu_count) * 4u * 2u * 64u;
-    const uint32_t tail = n_pix <= lanes ? 0u : n_pix <= 5 * lanes / 2 ? 1u : n_pix <= 5 * lanes ? 2u : n_pix <= 10 * lanes ? 3u : 4u;
+    const uint32_t tail = n_pix <= lanes           ? 0u
+                          : n_pix <= 5 * lanes / 2 ? 1u
+                          : n_pix <= 5 * lanes     ? 2u
+                          : n_pix <= 10 * lanes    ? 3u
+                                                   : 4u;
     return batch_shape{n_pix <= 5 * lanes ? 1u : PT_MAX_GROUPS, pt->tail_depth == PT_TAIL_AUTO ? tail : pt->tail_depth};
 }
 

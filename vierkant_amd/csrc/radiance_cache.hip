@@ -373,7 +373,8 @@ __device__ __forceinline__ void publish_weight(uint32_t k, float w, __bf16 *w_fw
 }
 
 //! MLP_K weights a workgroup; the partials of blocks j mod 8 are summed by thread row j, the eight sums combined in a
-//! fixed order: deterministic. The step's loss goes to pinned host memory on the way. (All eight sums by one thread per weight left 172 CUs idle: 15.5 us, 5.4 now.)
+//! fixed order: deterministic. The step's loss goes to pinned host memory on the way. (All eight sums by one thread
+//! per weight left 172 CUs idle: 15.5 us, 5.4 now.)
 constexpr uint32_t MLP_K = 32, MLP_SUMS = 8;
 __global__ void __launch_bounds__(MLP_K *MLP_SUMS) k_rc_adam_mlp(float *__restrict__ master, float *__restrict__ mom,
                                                                  float *__restrict__ vel, float *__restrict__ grad_out,

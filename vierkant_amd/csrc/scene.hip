@@ -28,10 +28,10 @@ constexpr int SCENE_BLOCK = 64;   // with the context's XCD chunk: 3.02 Grays/s 
 constexpr int SCENE_LDS = 16;
 
 template<bool ANY, int BLOCK, int LDS_DEPTH>
-__global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5))) k_scene_trace(const vkrt_bvh4_node *__restrict__ tlas, int32_t troot,
-                                                       uint32_t empty_scene, const inst_dev *__restrict__ insts,
-                                                       const float4 *__restrict__ rays, uint32_t n,
-                                                       void *__restrict__ out, uint32_t chunk)
+__global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5)))
+k_scene_trace(const vkrt_bvh4_node *__restrict__ tlas, int32_t troot, uint32_t empty_scene,
+              const inst_dev *__restrict__ insts, const float4 *__restrict__ rays, uint32_t n, void *__restrict__ out,
+              uint32_t chunk)
 {
     __shared__ int32_t smem[LDS_DEPTH > 0 ? LDS_DEPTH * BLOCK : 1];
     const uint32_t i = xcd_block(blockIdx.x, chunk) * BLOCK + threadIdx.x;
@@ -40,8 +40,8 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(5)))
     float best_t = rb.w, best_u = 0.f, best_v = 0.f;
     uint32_t best_prim = VKRT_INVALID_PRIM, best_inst = VKRT_INVALID_PRIM;
     if(!empty_scene)
-        scene_walk<ANY, BLOCK, LDS_DEPTH, keep_all, !ANY>(tlas, troot, insts, ra, rb, smem + threadIdx.x, best_t, best_u, best_v,
-                                          best_prim, best_inst);
+        scene_walk<ANY, BLOCK, LDS_DEPTH, keep_all, !ANY>(tlas, troot, insts, ra, rb, smem + threadIdx.x, best_t,
+                                                          best_u, best_v, best_prim, best_inst);
     const bool hit = best_prim != VKRT_INVALID_PRIM;
     if(ANY) static_cast<uint8_t *>(out)[i] = hit ? 1 : 0;
     else

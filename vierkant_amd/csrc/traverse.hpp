@@ -87,12 +87,6 @@ __device__ __forceinline__ void slab_interval(const ray_setup &r, float lox, flo
 
 static_assert(sizeof(vkrt_bvh4_node) == 128, "4-wide node layout: lo/hi float4 pairs at 0/16, 32/48, 64/80");
 
-//! the padded intervals of a 4-wide node's four children and its child refs. Each axis's near-plane float4
-//! is loaded from the offset the ray chose at setup and the far-plane float4 from that offset ^ 16, so a
-//! child costs two fmas per axis and one max/min per end: for a valid box (lo <= hi) the near plane's
-//! value is the smaller of the two on every axis, the same value slab_interval's per-axis min picks. For a
-//! box with lo > hi (the empty box of non-finite triangles) the interval comes out empty. Node offsets are
-//! 32-bit: the build keeps the 4-wide layout only while the nodes fit 4 GiB.
 //! BVH nodes and triangle records always live in device global memory; saying so lets a pointer that a kernel
 //! read from memory (a batch item, a scene record) take global loads with a scalar base and a 32-bit lane
 //! offset instead of flat loads with a 64-bit address per lane (two VGPRs per load in flight)
@@ -151,6 +145,10 @@ __device__ __forceinline__ fetch7 fetch_step(const void *base, uint32_t at, bool
     return f;
 }
 
+//! the padded intervals of a 4-wide node's four children. A child costs two fmas per axis and one max/min per end:
+//! for a valid box (lo <= hi) the near plane's value is the smaller of the two on every axis, the same value
+//! slab_interval's per-axis min picks. For a box with lo > hi (the empty box of non-finite triangles) the interval
+//! comes out empty
 __device__ __forceinline__ void child_intervals(const fetch7 &f, const ray_setup &r, float tn[4], float tf[4])
 {
     const float n0[4] = {f.x0.x, f.x0.y, f.x0.z, f.x0.w}, f0[4] = {f.x1.x, f.x1.y, f.x1.z, f.x1.w};
@@ -168,7 +166,9 @@ __device__ __forceinline__ void child_intervals(const fetch7 &f, const ray_setup
     }
 }
 
-//! the seven words of node `ref` alone
+//! the seven words of node `ref` alone: each axis's near-plane float4 from the offset the ray chose at setup, the
+//! far-plane float4 from that offset ^ 16. Node offsets are 32-bit: the build keeps the 4-wide layout only while the
+//! nodes fit 4 GiB
 __device__ __forceinline__ fetch7 fetch_node(const void *__restrict__ nodes, int32_t ref, const ray_setup &r)
 {
     const uint32_t nb = static_cast<uint32_t>(ref) * static_cast<uint32_t>(sizeof(vkrt_bvh4_node));
@@ -324,11 +324,10 @@ __device__ __forceinline__ bool traverse(const vkrt_bvh_node *__restrict__ nodes
     return best_prim != VKRT_INVALID_PRIM;
 }
 
-//! sort key of a 4-wide node's child: +inf when the ray misses it, else its entry distance clamped below
-//! +inf (so a hit child never sorts with the missed ones)
 constexpr float KEY_MISSED = __builtin_huge_valf();
-//! a child that meets the interval has an entry below +inf (an entry n = +inf pads to fma(-inf, T_PAD, inf) =
-//! NaN, which fails every comparison of child_hit), so its own entry is its key
+//! sort key of a 4-wide node's child: +inf when the ray misses it, else its entry distance. A child that meets the
+//! interval has an entry below +inf (an entry n = +inf pads to fma(-inf, T_PAD, inf) = NaN, which fails every
+//! comparison of child_hit), so a hit child never sorts with the missed ones
 __device__ __forceinline__ float sort_key(bool hit, float k) { return hit ? k : KEY_MISSED; }
 
 //! does the ray's padded interval [tn, tf] of child c meet [tmin, best_t]? The terms are joined with '&',
@@ -375,9 +374,9 @@ __device__ __forceinline__ void trav_init(trav_state &s, const ray_setup &r, int
 //! one step of the 4-wide walk: a node (children whose padded interval meets [tmin, best_t] are entered
 //! nearest first, the others pushed farthest first) or a leaf, then a pop. Returns true when the ray is
 //! finished (stack empty, or the first hit when ANY). JOINT: the records lie within 4 GiB behind the nodes, and one
-//! fetch serves both; otherwise a node and a leaf are read by loads of their own. `lds` is this lane's column of a [LDS_DEPTH][BLOCK] array; `spill` holds entries past LDS_DEPTH. A
-//! child is entered under the same condition as in traverse(), and the closest-hit rule does not depend on the
-//! visiting order, so the result is the same.
+//! fetch serves both; otherwise a node and a leaf are read by loads of their own. `lds` is this lane's column of a
+//! [LDS_DEPTH][BLOCK] array; `spill` holds entries past LDS_DEPTH. A child is entered under the same condition as in
+//! traverse(), and the closest-hit rule does not depend on the visiting order, so the result is the same.
 template<bool ANY, int BLOCK, int LDS_DEPTH, class F = keep_all, bool JOINT = true>
 __device__ __forceinline__ bool step4(const vkrt_bvh4_node *nodes, const float4 *tris, trav_state &s, int32_t *lds,
                                       int32_t *spill, bool cull_back, const F &filter = F{})
@@ -404,8 +403,8 @@ __device__ __forceinline__ bool step4(const vkrt_bvh4_node *nodes, const float4 
         bool v2 = child_hit(cr.z, k2, tf[2], r.tmin, s.best_t);
         bool v3 = child_hit(cr.w, k3, tf[3], r.tmin, s.best_t);
         int32_t c0 = cr.x, c1 = cr.y, c2 = cr.z, c3 = cr.w;
-        // sort nearest first with the missed children last (sort keys: +inf for them, the entry distance
-        // clamped below +inf for the others): five branchless compare-exchanges of (key, ref)
+        // sort nearest first with the missed children last (sort keys: +inf for them, the entry distance for the
+        // others): five branchless compare-exchanges of (key, ref)
         float q0 = sort_key(v0, k0), q1 = sort_key(v1, k1), q2 = sort_key(v2, k2), q3 = sort_key(v3, k3);
         compare_exchange(q0, c0, q1, c1);
         compare_exchange(q2, c2, q3, c3);
