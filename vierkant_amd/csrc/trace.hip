@@ -30,7 +30,7 @@ __global__ void __launch_bounds__(BLOCK) k_trace(const vkrt_bvh_node *__restrict
                                                  const float4 *__restrict__ tris, int32_t root, bool empty,
                                                  const vkrt_bvh4_node *__restrict__ nodes4, int32_t root4, bool wide,
                                                  const float4 *__restrict__ rays, uint32_t n, void *__restrict__ out,
-                                                 uint32_t chunk)
+                                                 uint32_t chunk, bool gather)
 {
     __shared__ int32_t smem[LDS_DEPTH > 0 ? LDS_DEPTH * BLOCK : 1];
     const uint32_t i = xcd_block(blockIdx.x, chunk) * BLOCK + threadIdx.x;
@@ -41,7 +41,9 @@ __global__ void __launch_bounds__(BLOCK) k_trace(const vkrt_bvh_node *__restrict
     if(!empty)
     {
         ray_setup r = setup_ray(rays, i);
-        if(!wide) hit = traverse<ANY, BLOCK, LDS_DEPTH>(nodes, tris, root, r, smem + threadIdx.x, t, u, v, prim);
+        if(!wide)
+            hit = traverse<ANY, BLOCK, LDS_DEPTH>(nodes, tris, root, r, smem + threadIdx.x, t, u, v, prim, false,
+                                                  keep_all{}, gather);
         else if(LOOP == LOOP_POSTPONED)
             hit = traverse4_postponed<ANY, BLOCK, LDS_DEPTH>(nodes4, tris, root4, r, smem + threadIdx.x, t, u, v, prim);
         else
@@ -61,7 +63,8 @@ static void launch_one(hipStream_t s, trace_loop loop, const vkrt_bvh *bvh, cons
     auto launch = [&](auto kernel) {
         kernel<<<xcd_grid(div_up(n, BLOCK), chunk), BLOCK, 0, s>>>(
                 bvh->nodes.as<vkrt_bvh_node>(), bvh->tris.as<float4>(), bvh->root_ref, bvh->empty,
-                bvh->nodes4.as<vkrt_bvh4_node>(), bvh->root4, bvh->wide, rays, n, out, chunk);
+                bvh->nodes4.as<vkrt_bvh4_node>(), bvh->root4, bvh->wide, rays, n, out, chunk,
+                !ANY || bvh->max_leaf > 4u);
     };
     if(loop == LOOP_JOINT) launch(k_trace<ANY, BLOCK, LDS, LOOP_JOINT>);
     else if(loop == LOOP_APART) launch(k_trace<ANY, BLOCK, LDS, LOOP_APART>);
