@@ -67,6 +67,8 @@ __global__ void __launch_bounds__(ENC_BLOCK) k_rc_encode(cache_dev c, const floa
 {
     if(loss && blockIdx.x == 0 && threadIdx.x == 0) *loss = 0.0f;
     const uint32_t n = pass_count(base, n_cap, n_dev);
+    // (the path tracer's queries: the room for them is the image, their number the device's)
+    if((blockIdx.x / XCDS) * ENC_RECORDS >= n) return;
     const uint32_t i = (blockIdx.x / XCDS) * ENC_RECORDS + threadIdx.x / 2, dx = threadIdx.x & 1u;
     float p[3] = {0.f, 0.f, 0.f};
     if(i < n) unit_position(c.g, load_position(records + (size_t)i * stride_f4), p);
